@@ -1002,6 +1002,88 @@ struct PostNorm {
     const float *y, *ls;
     float *h_out;
 };
+// The staging of NORM 1 - 3: rows of x (see above) -> normalised f32 values, element i of row b handed to put(b, i, v)
+// (which may write it to xn + b k + i).  Every wave of the workgroup takes part; the last barrier is the caller's.  LDS
+// at xn: [BP][k] rows, [2][k] scale and bias, partial sums, statistics (NORM == 3: then [BP][k] residual rows).
+template <int BP, int NORM, class Put>
+__device__ __forceinline__ void stage_normed_rows(float *xn, const float *__restrict__ x, uint64_t k, uint32_t batch,
+                                                  const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
+                                                  uint64_t ldx, const PostNorm &post, Put put) {
+    const uint32_t ld = (uint32_t)k;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+    // One trip to memory: the rows, the scale and the bias all go to LDS first; the two
+    // statistics passes and the normalisation then work from there.
+    float *gs = xn + (size_t)BP * ld, *bs = gs + k;  // scale, bias
+    float *red = bs + k;                            // [16 waves][BP] partial sums
+    float *stat = red + 16 * BP;                    // [0][b] mean, [1][b] standard deviation
+    float *hs = stat + 32;                          // NORM == 3: [BP][k] residual rows
+    float ps[BP];
+#pragma unroll
+    for (int b = 0; b < BP; b++) ps[b] = 0.f;
+    for (uint64_t i = threadIdx.x; i < k; i += blockDim.x) {
+        gs[i] = nscale[i];
+        if (NORM == 1) bs[i] = nbias ? nbias[i] : 0.f;
+        if (NORM == 3) bs[i] = post.ls ? post.ls[i] : 1.0f;
+#pragma unroll
+        for (int b = 0; b < BP; b++)
+            if (b < (int)batch) {
+                const float v = NORM == 3 ? post.y[(uint64_t)b * k + i] : x[(uint64_t)b * ldx + i];
+                xn[(uint32_t)b * ld + i] = v;
+                if (NORM == 3) hs[(uint32_t)b * ld + i] = x[(uint64_t)b * ldx + i];
+                ps[b] += v;
+            }
+    }
+    // every wave's partial per row -> wave 0 finishes row b = lane
+    auto finish = [&](float (&p)[BP]) -> float {
+#pragma unroll
+        for (int b = 0; b < BP; b++) {
+            const float t = wave_sum(p[b]);
+            if (lane == 0) red[wave * BP + b] = t;
+        }
+        __syncthreads();
+        float tot = 0.f;
+        if (wave == 0 && lane < BP)
+            for (uint32_t w = 0; w < nwaves; w++) tot += red[w * BP + lane];
+        return tot;
+    };
+    if (NORM == 1) {
+        const float tot = finish(ps);
+        if (wave == 0 && lane < BP) stat[lane] = tot / (float)k;
+        __syncthreads();
+    } else if (threadIdx.x < BP) {
+        stat[threadIdx.x] = 0.f;  // a root-mean-square norm subtracts no mean
+    }
+#pragma unroll
+    for (int b = 0; b < BP; b++) ps[b] = 0.f;
+    if (NORM >= 2) __syncthreads();  // the rows and the zero means are in LDS
+    for (uint64_t i = threadIdx.x; i < k; i += blockDim.x)
+#pragma unroll
+        for (int b = 0; b < BP; b++)
+            if (b < (int)batch) {
+                const float d = xn[(uint32_t)b * ld + i] - stat[b];
+                ps[b] = fmaf(d, d, ps[b]);
+            }
+    {
+        const float tot = finish(ps);
+        if (wave == 0 && lane < BP) stat[16 + lane] = sqrtf(tot / (float)k + eps);
+        __syncthreads();
+    }
+    for (uint64_t i = threadIdx.x; i < k; i += blockDim.x) {
+        const float g = gs[i], bi = NORM == 1 ? bs[i] : 0.f;
+#pragma unroll
+        for (int b = 0; b < BP; b++)
+            if (b < (int)batch) {
+                if (NORM == 3) {
+                    const float v = fmaf(xn[(uint32_t)b * ld + i] / stat[16 + b] * g, bs[i], hs[(uint32_t)b * ld + i]);
+                    put((uint32_t)b, (uint32_t)i, v);
+                    if (blockIdx.x == 0) post.h_out[(uint64_t)b * k + i] = v;
+                } else {
+                    put((uint32_t)b, (uint32_t)i, g * (xn[(uint32_t)b * ld + i] - stat[b]) / stat[16 + b] + bi);
+                }
+            }
+    }
+}
+
 template <bool BF16, int BP, int NORM>
 __global__ __launch_bounds__(1024) void gemv_dense_kernel(const void *__restrict__ wdata,
                                                           const float *__restrict__ x, uint64_t k,
@@ -1037,77 +1119,8 @@ __global__ __launch_bounds__(1024) void gemv_dense_kernel(const void *__restrict
     }
     const float *xs = x;  // where the main loop reads activation row b: xs + b * k
     if (NORM) {
-        // One trip to memory: the rows, the scale and the bias all go to LDS first; the two
-        // statistics passes and the normalisation then work from there.
-        float *gs = xn + (size_t)BP * k, *bs = gs + k;  // scale, bias
-        float *red = bs + k;                            // [16 waves][BP] partial sums
-        float *stat = red + 16 * BP;                    // [0][b] mean, [1][b] standard deviation
-        float *hs = stat + 32;                          // NORM == 3: [BP][k] residual rows
-        float ps[BP];
-#pragma unroll
-        for (int b = 0; b < BP; b++) ps[b] = 0.f;
-        for (uint64_t i = threadIdx.x; i < k; i += blockDim.x) {
-            gs[i] = nscale[i];
-            if (NORM == 1) bs[i] = nbias ? nbias[i] : 0.f;
-            if (NORM == 3) bs[i] = post.ls ? post.ls[i] : 1.0f;
-#pragma unroll
-            for (int b = 0; b < BP; b++)
-                if (b < (int)batch) {
-                    const float v = NORM == 3 ? post.y[(uint64_t)b * k + i] : x[(uint64_t)b * ldx + i];
-                    xn[(uint64_t)b * k + i] = v;
-                    if (NORM == 3) hs[(uint64_t)b * k + i] = x[(uint64_t)b * ldx + i];
-                    ps[b] += v;
-                }
-        }
-        // every wave's partial per row -> wave 0 finishes row b = lane
-        auto finish = [&](float (&p)[BP]) -> float {
-#pragma unroll
-            for (int b = 0; b < BP; b++) {
-                const float t = wave_sum(p[b]);
-                if (lane == 0) red[wave * BP + b] = t;
-            }
-            __syncthreads();
-            float tot = 0.f;
-            if (wave == 0 && lane < BP)
-                for (uint32_t w = 0; w < nwaves; w++) tot += red[w * BP + lane];
-            return tot;
-        };
-        if (NORM == 1) {
-            const float tot = finish(ps);
-            if (wave == 0 && lane < BP) stat[lane] = tot / (float)k;
-            __syncthreads();
-        } else if (threadIdx.x < BP) {
-            stat[threadIdx.x] = 0.f;  // a root-mean-square norm subtracts no mean
-        }
-#pragma unroll
-        for (int b = 0; b < BP; b++) ps[b] = 0.f;
-        if (NORM >= 2) __syncthreads();  // the rows and the zero means are in LDS
-        for (uint64_t i = threadIdx.x; i < k; i += blockDim.x)
-#pragma unroll
-            for (int b = 0; b < BP; b++)
-                if (b < (int)batch) {
-                    const float d = xn[(uint64_t)b * k + i] - stat[b];
-                    ps[b] = fmaf(d, d, ps[b]);
-                }
-        {
-            const float tot = finish(ps);
-            if (wave == 0 && lane < BP) stat[16 + lane] = sqrtf(tot / (float)k + eps);
-            __syncthreads();
-        }
-        for (uint64_t i = threadIdx.x; i < k; i += blockDim.x) {
-            const float g = gs[i], bi = NORM == 1 ? bs[i] : 0.f;
-#pragma unroll
-            for (int b = 0; b < BP; b++)
-                if (b < (int)batch) {
-                    if (NORM == 3) {
-                        const float v = fmaf(xn[(uint64_t)b * k + i] / stat[16 + b] * g, bs[i], hs[(uint64_t)b * k + i]);
-                        xn[(uint64_t)b * k + i] = v;
-                        if (blockIdx.x == 0) post.h_out[(uint64_t)b * k + i] = v;
-                    } else {
-                        xn[(uint64_t)b * k + i] = g * (xn[(uint64_t)b * k + i] - stat[b]) / stat[16 + b] + bi;
-                    }
-                }
-        }
+        stage_normed_rows<BP, NORM>(xn, x, k, batch, nscale, nbias, eps, ldx, post,
+                                    [&](uint32_t b, uint32_t i, float v) { xn[(uint64_t)b * k + i] = v; });
         __syncthreads();
         xs = xn;
     }
@@ -1182,6 +1195,249 @@ __global__ __launch_bounds__(1024) void gemv_dense_kernel(const void *__restrict
             if (b < (int)batch) epi_store<true>(e, b, j, acc[b]);
 }
 
+// ---------------------------------------------------------------- bf16 rows on the matrix cores (2 - 16 rows)
+// y[b, j] for a tile of 16 weight rows j and all b at once: v_mfma_f32_16x16x32_bf16 with the weights as they are
+// stored and every activation as the sum of three bf16 (8 mantissa bits each: x exactly), three instructions per 32
+// of k into one f32 accumulator.  The products are those of the f32 form; what changes is the order of the sums.
+//
+// gemv_dense_kernel (a wave per weight row, activations by f32 FMA) reads `batch` f32 activations per weight: at batch
+// 4 that is eight times the weights' bytes, out of L2 where a row does not fit the first-level cache.  Here a tile's
+// 16 rows share them, and they are split once per wave.  Us per launch, there / here, distinct weights in turn:
+//              batch 2        4            8            16
+//   2048 x 2048   5.8 / 4.8    7.4 / 4.9   10.5 / 5.3    16.7 / 6.6
+//   5632 x 2048  11.6 / 8.2   15.4 / 8.6   21.9 / 10.7   35.2 / 14.1
+//   4096 x 22016   47 / 34     73 / 36      118 / 40      215 / 55
+//   768 x 50257    28 / 14     41 / 14       68 / 16      127 / 18
+// (one row: 4.2, 8.7, 33, 18.5 there, which keeps it: a wave per row needs no sum over waves.)  The large ones are
+// at 5 TB/s of weights.  An infinite weight makes its output NaN (times the pieces of an activation that are zero).
+//
+// The workgroup's waves take a share of k each, in pairs of 32-wide chunks: a wave request is 8 rows x 128 bytes, as
+// the weights lie, and passes through a corner of LDS that is the wave's own to where the matrix cores want it (a
+// lane: 8 consecutive k of one row).  Loaded the way they are multiplied (16 rows x 64 bytes, neighbouring lanes in
+// different rows) the same weights take a third longer: 4096 x 22016 at batch 4 in 51 against 40 us.  The activations
+// travel likewise.  PD pairs are in flight per wave across the ends of tiles; the waves' partial tiles meet in LDS.
+
+// Two values -> their three bf16, a pair of upper halves per piece.  What is left of an infinity is zero (its own
+// difference would be a NaN).
+struct Split2 { uint32_t p[3]; };
+__device__ __forceinline__ Split2 split2(float a, float b) {
+    uint32_t v[2] = {__float_as_uint(a), __float_as_uint(b)};
+    Split2 s;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        s.p[i] = __builtin_amdgcn_perm(v[1], v[0], 0x07060302u);
+        if (i == 2) break;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float f = __uint_as_float(v[j]), h = __uint_as_float(v[j] & 0xffff0000u);
+            v[j] = __float_as_uint(i == 0 && f == h ? 0.f : f - h);
+        }
+    }
+    return s;
+}
+struct Split3 { uint4 p[3]; };  // eight values of a row
+
+__device__ __forceinline__ float4_t mfma_split3(const uint4 &w, const Split3 &x, float4_t acc) {
+    union { uint4 u; bf16x8_t v; } uw, ux;
+    uw.u = w;
+#pragma unroll
+    for (int i = 2; i >= 0; i--) {
+        ux.u = x.p[i];
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(uw.v, ux.v, acc, 0, 0, 0);
+    }
+    return acc;
+}
+
+// The tiles blockIdx.x, + grid, .. of the workgroup.  XQ > 0: f32 activation rows x [batch][k] in global memory, read
+// four to a request (XQ requests cover the batch) and split on their way into the wave's corner.  XQ == 0: `stage`,
+// which runs behind the first requests, puts them into LDS: piece i of row b at xs.at(i, b).
+// k % 64 == 0 and at least one pair of chunks per wave.
+// KEEP: a wave's share of k is at most PD pairs, and its split activations stay in registers from tile to tile.
+// lds: mfma_wave_lds(XQ) uint4 per wave.
+struct SplitRows {
+    uint16_t *p;
+    uint32_t k, rows;  // (rows 8 elements longer than k: at a multiple of 256 bytes apart they would share their banks)
+    __device__ uint16_t *at(int i, uint32_t b) const { return p + (i * rows + b) * (k + 8); }
+    __device__ void put(uint32_t b, uint32_t i, float v) const {
+        const Split2 s = split2(v, 0.f);
+#pragma unroll
+        for (int j = 0; j < 3; j++) at(j, b)[i] = (uint16_t)s.p[j];
+    }
+    __device__ void put2(uint32_t b, uint32_t i, float2 v) const {
+        const Split2 s = split2(v.x, v.y);
+#pragma unroll
+        for (int j = 0; j < 3; j++) *(uint32_t *)(at(j, b) + i) = s.p[j];
+    }
+};
+static constexpr size_t split_rows_bytes(size_t rows, size_t k) { return 3 * rows * (k + 8) * 2; }
+static constexpr uint32_t mfma_wave_lds(int xq) { return 128 + 96 * xq; }
+template <int PD, bool KEEP, int XQ, class Stage>
+__device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const float *__restrict__ x, uint32_t k, uint32_t n,
+                                          uint32_t batch, uint32_t nw, uint32_t grid, const EpiArgs &e, uint4 *lds,
+                                          const SplitRows &xs, Stage stage) {
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t c = lane & 15, g = lane >> 4, cb = min(c, batch - 1);
+    const uint32_t pairs = k >> 6, pb = pairs * wave / nw, np = pairs * (wave + 1) / nw - pb, groups = (np + PD - 1) / PD;
+    const uint32_t tiles = (n + 15) / 16;
+    uint4 *wl = lds + wave * mfma_wave_lds(XQ), *xl = wl + 128;
+    // (a pair behind the wave's share is the share's last one again: no branches around the requests)
+    auto pair_at = [&](uint32_t i) { return min(i, np - 1) * 64; };
+    struct WRows { const uint16_t *p[2]; };
+    auto tile_rows = [&](uint32_t tile) {
+        WRows r;
+#pragma unroll
+        for (int q = 0; q < 2; q++) r.p[q] = w + (uint64_t)min(tile * 16 + 8 * q + (lane >> 3), n - 1) * k + pb * 64 + (lane & 7) * 8;
+        return r;
+    };
+    const float *xr[XQ ? XQ : 1];
+    uint4 wr[PD][2];
+    u32x4_t xv[XQ ? PD : 1][XQ ? XQ : 1];  // (arrays of the struct type would be copied through scratch memory)
+    auto x_request = [&](int s, uint32_t i) {
+#pragma unroll
+        for (int q = 0; q < XQ; q++) xv[s][q] = *(const u32x4_t *)(xr[q] + pair_at(i));
+    };
+    auto w_request = [&](int s, const WRows &r, uint32_t i) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) wr[s][q] = load_stream((const uint4 *)(r.p[q] + pair_at(i)));
+    };
+    // 16-byte pieces of a row change places with the row, so that neither side's lanes share banks
+    auto x_put = [&](int s) {
+#pragma unroll
+        for (int q = 0; q < XQ; q++) {
+            const uint32_t r = 4 * q + (lane >> 4), at = (r * 8 + (((lane & 15) >> 1) ^ ((r >> 1) & 7))) * 2 + (lane & 1);
+            const u32x4_t v = xv[s][q];
+            const Split2 lo = split2(__uint_as_float(v.x), __uint_as_float(v.y)), hi = split2(__uint_as_float(v.z), __uint_as_float(v.w));
+#pragma unroll
+            for (int i = 0; i < 3; i++) *((uint2 *)(xl + i * 32 * XQ) + at) = make_uint2(lo.p[i], hi.p[i]);
+        }
+    };
+    auto w_put = [&](int s) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const uint32_t r = 8 * q + (lane >> 3);
+            wl[r * 8 + ((lane & 7) ^ (r >> 1))] = wr[s][q];
+        }
+    };
+    auto x_get = [&](uint32_t i, int h) {  // chunk h of pair i
+        Split3 f;
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            f.p[j] = XQ ? xl[j * 32 * XQ + cb * 8 + ((4 * h + g) ^ (cb >> 1))]
+                        : *(const uint4 *)(xs.at(j, cb) + pb * 64 + pair_at(i) + h * 32 + g * 8);
+        return f;
+    };
+    if (XQ) {
+#pragma unroll
+        for (int q = 0; q < XQ; q++) xr[q] = x + (uint64_t)min(4 * q + (lane >> 4), batch - 1) * k + pb * 64 + (lane & 15) * 4;
+    }
+    uint32_t tile = blockIdx.x, gi = 0;
+    WRows wp = tile_rows(tile);
+    // Loads return in order.  Activations that stay in registers go first: they are split while the weights travel.
+    // Else the order is the loop's: in any other one a wait of the loop would be for the fewest requests that either
+    // order leaves behind the awaited one.
+    if (XQ && KEEP) {
+#pragma unroll
+        for (int s = 0; s < PD; s++) x_request(s, s);
+    }
+#pragma unroll
+    for (int s = 0; s < PD; s++) {
+        if (XQ && !KEEP) x_request(s, s);
+        w_request(s, wp, s);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!XQ) stage();
+    Split3 kept[KEEP ? PD : 1][2];
+    if (KEEP) {
+#pragma unroll
+        for (int s = 0; s < PD; s++) {
+            x_put(s);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int h = 0; h < 2; h++) kept[KEEP ? s : 0][h] = x_get(s, h);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    auto group = [&](uint32_t i0, const WRows &next, uint32_t n0, auto request) {
+#pragma unroll
+        for (int s = 0; s < PD; s++) {
+            // (LDS serves a wave's stores and loads in order: nothing here waits for another wave)
+            if (!KEEP) x_put(s);
+            w_put(s);
+            __builtin_amdgcn_wave_barrier();
+            if (request()) {
+                if (!KEEP) x_request(s, n0 + s);
+                w_request(s, next, n0 + s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (i0 + s < np) {
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const uint4 wf = wl[c * 8 + ((4 * h + g) ^ (c >> 1))];
+                    if constexpr (KEEP) acc = mfma_split3(wf, kept[s][h], acc);
+                    else acc = mfma_split3(wf, x_get(i0 + s, h), acc);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    for (;;) {
+        const bool ends = gi + 1 == groups;
+        const uint32_t ntile = ends ? tile + grid : tile, ngi = ends ? 0 : gi + 1;
+        const bool more = ntile < tiles;
+        if (more) {
+            if (ends) wp = tile_rows(ntile);
+            group(gi * PD, wp, ngi * PD, [] { return true; });
+        } else {
+            group(gi * PD, wp, 0, [] { return false; });
+        }
+        if (ends) {
+            // lane (c, g) holds outputs 16 tile + 4 g .. + 3 of row c; a wave's corner of LDS is free
+            if (c < batch) *(float4_t *)(wl + lane) = acc;
+            acc = float4_t{0.f, 0.f, 0.f, 0.f};
+            lds_barrier();
+            const uint32_t row = tile * 16 + c;
+            for (uint32_t b = wave; b < batch; b += nw) {
+                // lane (c, g) adds output c of every fourth wave
+                float sum = 0.f;
+                for (uint32_t v = g; v < nw; v += 4)
+                    sum += ((const float *)(lds + v * mfma_wave_lds(XQ) + (c >> 2) * 16 + b))[c & 3];
+                sum = xor32_sum(xor16_sum(sum));
+                if (epi_gated(e.act)) {
+                    const float up = lane_xor1(sum);
+                    if (g == 0 && (c & 1) == 0 && row + 1 < n) epi_store_gated(e, b, row / 2, sum, up);
+                } else if (g == 0 && row < n) {
+                    epi_store<true>(e, b, row, sum);
+                }
+            }
+            if (more) lds_barrier();
+        }
+        if (!more) break;
+        tile = ntile;
+        gi = ngi;
+    }
+}
+
+// NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
+template <int BP, int NORM, int PD, bool KEEP>
+__global__ __launch_bounds__(1024) void gemv_mfma_kernel(const uint16_t *__restrict__ w, const float *__restrict__ x, uint32_t k,
+                                                         uint32_t n, uint32_t batch, uint32_t waves, uint32_t grid, EpiArgs e,
+                                                         const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
+                                                         uint64_t ldx, PostNorm post) {
+    extern __shared__ uint4 mlds[];
+    constexpr int XQ = NORM ? 0 : BP / 4;
+    // a folded norm: the split rows first; what its staging needs lies where the corners will be
+    const SplitRows xs{(uint16_t *)mlds, k, (uint32_t)BP};
+    uint4 *corners = NORM ? (uint4 *)(xs.p + 3 * BP * (k + 8)) : mlds;
+    mfma_rows<PD, KEEP, XQ>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
+        if constexpr (NORM != 0) {
+            stage_normed_rows<BP, NORM>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post,
+                                        [&](uint32_t b, uint32_t i, float v) { xs.put(b, i, v); });
+            __syncthreads();
+        }
+    });
+}
+
 static const size_t kDenseNormLdsLimit = 64 * 1024;
 // rows + scale + bias + per-wave partial sums + statistics
 static size_t gemv_dense_norm_lds(uint64_t k, uint32_t bp) { return ((size_t)(bp + 2) * k + 16 * bp + 32) * 4; }
@@ -1193,6 +1449,10 @@ bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch) {
     return gemv_dense_norm_lds(w.k, pad_batch(batch)) <= kDenseNormLdsLimit;
 }
 
+// Batches of 2 and more on bf16 weights whose rows are whole pairs of chunks, one for every wave at least.
+static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves) {
+    return w.dtype == COEUS_W_BF16 && batch >= 2 && w.k % 64 == 0 && w.k / 64 >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
+}
 static size_t gemv_dense_post_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)bp * k * 4; }
 bool gemv_can_fuse_post_norm(const Weight &w, uint64_t batch) {
     if (w.dtype >= COEUS_W_Q8_0 || batch < 1 || batch > 16) return false;
@@ -1248,13 +1508,15 @@ int launch_hyper_fold(const float *mix, const float *out, const float *in, float
     return COEUS_OK;
 }
 
-template <bool BF16, int BP, int NIT>
+template <bool BF16, int BP, int NIT, bool MF = false>
 __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict__ wdata, const float *__restrict__ x,
                                                           const float *__restrict__ y, const float *__restrict__ norm,
                                                           const HyperFold *__restrict__ fold, uint32_t k, uint32_t batch_streams,
                                                           float *x_out, float eps, EpiArgs e) {
     constexpr int NS = kFusedStreams, SL = 4;
-    extern __shared__ float xn[];  // [BP][k]
+    // [BP][k]; MF: the waves' corners (mfma_rows), the rows' pieces
+    extern __shared__ __attribute__((aligned(16))) float hyper_lds[];
+    float *xn = MF ? hyper_lds + 16 * 4 * mfma_wave_lds(0) : hyper_lds;
     __shared__ float2 red[16][BP];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), S = batch_streams >> 16,
                    batch = batch_streams & 0xffffu;
@@ -1277,6 +1539,8 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
     };
     // Where element i of the normalised rows lies: the two quads of every eight in halves of their own, so that the
     // lanes of a read of quads are neighbours.
+    // (MF: split, as mfma_rows takes them)
+    const SplitRows xs{(uint16_t *)xn, k, (uint32_t)BP};
     auto place = [&](uint32_t i) { return vec ? (i & 4 ? k / 2 : 0) + (i >> 3) * 4 + (i & 3) : i; };
     // The streams are requested before the weights: loads return in order, and the norm needs only the streams.
     // (No branches here: a lane behind the end re-reads the last elements, a stream that is not there the last one.)
@@ -1293,6 +1557,97 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
             yv[it][b] = *(const float2 *)(y + (uint64_t)row * k + i);
         }
     }
+    auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
+    auto normalise = [&]() {
+        float2 v[NIT][BP];
+        float cnt = 0.f;  // elements of this wave
+#pragma unroll
+        for (int it = 0; it < NIT; it++) {
+            const uint32_t i = 2 * (tid + 1024 * it), w0 = 2 * (64 * wave + 1024 * it);
+            cnt += w0 < k ? (float)min(128u, k - w0) : 0.f;
+#pragma unroll
+            for (int b = 0; b < BP; b++) {
+                float2 o = make_float2(fold->cy * yv[it][b].x, fold->cy * yv[it][b].y);
+#pragma unroll
+                for (int s = 0; s < NS; s++) { o.x = fmaf(fold->cs[s], xv[it][b][s].x, o.x); o.y = fmaf(fold->cs[s], xv[it][b][s].y, o.y); }
+                v[it][b] = i < k ? o : make_float2(0.f, 0.f);
+            }
+        }
+        if (blockIdx.x == 0 && x_out) {
+#pragma unroll
+            for (int it = 0; it < NIT; it++) {
+                const uint32_t i = 2 * (tid + 1024 * it);
+#pragma unroll
+                for (int b = 0; b < BP; b++) {
+                    if (b >= (int)batch || i >= k) continue;
+#pragma unroll
+                    for (int u = 0; u < NS; u++) {
+                        if (u >= (int)S) continue;
+                        float2 nv = make_float2(fold->om[u] * yv[it][b].x, fold->om[u] * yv[it][b].y);
+#pragma unroll
+                        for (int s = 0; s < NS; s++) {
+                            nv.x = fmaf(fold->mix[s][u], xv[it][b][s].x, nv.x);
+                            nv.y = fmaf(fold->mix[s][u], xv[it][b][s].y, nv.y);
+                        }
+                        *(float2 *)(x_out + ((uint64_t)b * S + u) * k + i) = nv;
+                    }
+                }
+            }
+        }
+        const float inv_cnt = cnt > 0.f ? 1.0f / cnt : 0.f;
+#pragma unroll
+        for (int b = 0; b < BP; b++) {
+            if (b >= (int)batch) continue;
+            float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+            for (int it = 0; it < NIT; it++) s1 += v[it][b].x + v[it][b].y;
+            const float own = row_sum(s1), mw = own * inv_cnt;
+#pragma unroll
+            for (int it = 0; it < NIT; it++)
+                if (2 * (tid + 1024 * it) < k) {
+                    const float dx = v[it][b].x - mw, dy = v[it][b].y - mw;
+                    s2 = fmaf(dx, dx, s2); s2 = fmaf(dy, dy, s2);
+                }
+            s2 = row_sum(s2);
+            if (lane == 0) red[wave][b] = make_float2(own, s2);
+        }
+        __syncthreads();
+        {
+            // lane w of 16 takes wave w's record
+            const uint32_t w = lane & 15;
+            float cw = 0.f;
+#pragma unroll
+            for (int it = 0; it < NIT; it++) {
+                const uint32_t w0 = 2 * (64 * w + 1024 * it);
+                cw += w0 < k ? (float)min(128u, k - w0) : 0.f;
+            }
+#pragma unroll
+            for (int b = 0; b < BP; b++) {
+                if (b >= (int)batch) continue;
+                const float2 rec = red[w][b];
+                const float mean = group_sum<16>(rec.x) / (float)k, dm = cw > 0.f ? rec.x / cw - mean : 0.f;
+                const float rs = 1.0f / sqrtf(group_sum<16>(fmaf(cw * dm, dm, rec.y)) / (float)k + eps);
+#pragma unroll
+                for (int it = 0; it < NIT; it++) {
+                    const uint32_t i = 2 * (tid + 1024 * it);
+                    const float2 o = make_float2((v[it][b].x - mean) * rs * g[it].x, (v[it][b].y - mean) * rs * g[it].y);
+                    if (i < k) {
+                        if (MF) xs.put2(b, i, o);
+                        else *(float2 *)(xn + (size_t)b * k + place(i)) = o;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    };
+    if constexpr (MF) {
+        __builtin_amdgcn_sched_barrier(0);
+        mfma_rows<2, true, 0>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
+            __builtin_amdgcn_sched_barrier(0);
+            normalise();
+        });
+        return;
+    }
     __builtin_amdgcn_sched_barrier(0);
     uint4 wa[SL], wb[SL];
 #pragma unroll
@@ -1301,83 +1656,7 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
         if (vec) wload(wa[q], wb[q]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    float2 v[NIT][BP];
-    float cnt = 0.f;  // elements of this wave
-#pragma unroll
-    for (int it = 0; it < NIT; it++) {
-        const uint32_t i = 2 * (tid + 1024 * it), w0 = 2 * (64 * wave + 1024 * it);
-        cnt += w0 < k ? (float)min(128u, k - w0) : 0.f;
-#pragma unroll
-        for (int b = 0; b < BP; b++) {
-            float2 o = make_float2(fold->cy * yv[it][b].x, fold->cy * yv[it][b].y);
-#pragma unroll
-            for (int s = 0; s < NS; s++) { o.x = fmaf(fold->cs[s], xv[it][b][s].x, o.x); o.y = fmaf(fold->cs[s], xv[it][b][s].y, o.y); }
-            v[it][b] = i < k ? o : make_float2(0.f, 0.f);
-        }
-    }
-    if (blockIdx.x == 0 && x_out) {
-#pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            const uint32_t i = 2 * (tid + 1024 * it);
-#pragma unroll
-            for (int b = 0; b < BP; b++) {
-                if (b >= (int)batch || i >= k) continue;
-#pragma unroll
-                for (int u = 0; u < NS; u++) {
-                    if (u >= (int)S) continue;
-                    float2 nv = make_float2(fold->om[u] * yv[it][b].x, fold->om[u] * yv[it][b].y);
-#pragma unroll
-                    for (int s = 0; s < NS; s++) {
-                        nv.x = fmaf(fold->mix[s][u], xv[it][b][s].x, nv.x);
-                        nv.y = fmaf(fold->mix[s][u], xv[it][b][s].y, nv.y);
-                    }
-                    *(float2 *)(x_out + ((uint64_t)b * S + u) * k + i) = nv;
-                }
-            }
-        }
-    }
-    auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
-    const float inv_cnt = cnt > 0.f ? 1.0f / cnt : 0.f;
-#pragma unroll
-    for (int b = 0; b < BP; b++) {
-        if (b >= (int)batch) continue;
-        float s1 = 0.f, s2 = 0.f;
-#pragma unroll
-        for (int it = 0; it < NIT; it++) s1 += v[it][b].x + v[it][b].y;
-        const float own = row_sum(s1), mw = own * inv_cnt;
-#pragma unroll
-        for (int it = 0; it < NIT; it++)
-            if (2 * (tid + 1024 * it) < k) {
-                const float dx = v[it][b].x - mw, dy = v[it][b].y - mw;
-                s2 = fmaf(dx, dx, s2); s2 = fmaf(dy, dy, s2);
-            }
-        s2 = row_sum(s2);
-        if (lane == 0) red[wave][b] = make_float2(own, s2);
-    }
-    __syncthreads();
-    {
-        // lane w of 16 takes wave w's record
-        const uint32_t w = lane & 15;
-        float cw = 0.f;
-#pragma unroll
-        for (int it = 0; it < NIT; it++) {
-            const uint32_t w0 = 2 * (64 * w + 1024 * it);
-            cw += w0 < k ? (float)min(128u, k - w0) : 0.f;
-        }
-#pragma unroll
-        for (int b = 0; b < BP; b++) {
-            if (b >= (int)batch) continue;
-            const float2 rec = red[w][b];
-            const float mean = group_sum<16>(rec.x) / (float)k, dm = cw > 0.f ? rec.x / cw - mean : 0.f;
-            const float rs = 1.0f / sqrtf(group_sum<16>(fmaf(cw * dm, dm, rec.y)) / (float)k + eps);
-#pragma unroll
-            for (int it = 0; it < NIT; it++) {
-                const uint32_t i = 2 * (tid + 1024 * it);
-                if (i < k) *(float2 *)(xn + (size_t)b * k + place(i)) = make_float2((v[it][b].x - mean) * rs * g[it].x, (v[it][b].y - mean) * rs * g[it].y);
-            }
-        }
-    }
-    __syncthreads();
+    normalise();
     float acc[BP], gate[BP];
 #pragma unroll
     for (int b = 0; b < BP; b++) acc[b] = gate[b] = 0.f;
@@ -1456,14 +1735,25 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
         nf.bias || (nf.y && (!nf.h_out || nf.h_out == nf.h)))
         return fail(COEUS_INVALID_INPUT, "folded hyper-connections: bad arguments or too many streams");
     const uint32_t bp = pad_batch(batch), b = (uint32_t)batch, k = (uint32_t)w.k, nit = hyper_pairs(w.k);
-    const size_t lds = (size_t)bp * k * 4;
+    const bool mf = BF16 && nit == 1 && gemv_uses_mfma(w, batch, 16);
+    const size_t lds = mf ? 16 * 16 * mfma_wave_lds(0) + split_rows_bytes(bp, k) : (size_t)bp * k * 4;
     const uint32_t bs = b | nf.streams << 16;
     const HyperFold *fold = (const HyperFold *)nf.fold;
     const float *y = nf.y ? nf.y : nf.h;  // (without an output of a sublayer before its weight is zero)
     float *x_out = nf.y ? nf.h_out : nullptr;
     if (w.n > 0x7fffffffull) return fail(COEUS_INVALID_INPUT, "folded hyper-connections: too many rows");
     const uint64_t units = epi_gated(e.act) ? w.n / 2 : w.n;
-    const dim3 grid((unsigned)std::min<uint64_t>(256, units)), block(1024);  // (a workgroup per compute unit)
+    const dim3 grid((unsigned)std::min<uint64_t>(256, mf ? ceil_div(w.n, 16) : units)), block(1024);  // (a workgroup per compute unit)
+    if constexpr (BF16) {
+        if (mf) {
+            if (bp == 4)
+                hipLaunchKernelGGL((gemv_hyper_kernel<true, 4, 1, true>), grid, block, lds, st, w.data, nf.h, y, nf.scale, fold, k, bs, x_out, nf.eps, e);
+            else
+                hipLaunchKernelGGL((gemv_hyper_kernel<true, 2, 1, true>), grid, block, lds, st, w.data, nf.h, y, nf.scale, fold, k, bs, x_out, nf.eps, e);
+            COEUS_HIP(hipGetLastError());
+            return COEUS_OK;
+        }
+    }
 #define COEUS_GH(BPV, NV) \
     hipLaunchKernelGGL((gemv_hyper_kernel<BF16, BPV, NV>), grid, block, lds, st, w.data, nf.h, y, nf.scale, fold, k, bs, x_out, nf.eps, e)
     if (bp == 4) COEUS_GH(4, 1);
@@ -1500,6 +1790,40 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     const float *xin = nf ? nf->h : x;
     const float *ns = nf ? nf->scale : nullptr, *nb = nf ? nf->bias : nullptr;
     const float eps = nf ? nf->eps : 0.f;
+    if constexpr (BF16) {
+        // plain: as many waves as have two pairs of chunks each, workgroups enough to fill the compute units' 16 waves;
+        // a folded norm: one workgroup of 16 waves per compute unit, which stages the rows once
+        const uint32_t pairs = (uint32_t)std::min<uint64_t>(w.k / 64, 1u << 20), mw = nf ? 16u : std::max(1u, std::min(16u, (pairs + 1) / 2));
+        const size_t corners = (size_t)mw * 16 * mfma_wave_lds(nf ? 0 : std::max(bp, 4u) / 4),
+                     mlds = nf ? split_rows_bytes(bp, w.k) + std::max(corners, lds) : corners;
+        if (gemv_uses_mfma(w, batch, nf ? 16 : mw) && mlds <= 160 * 1024) {
+            const uint32_t tiles = (uint32_t)ceil_div(w.n, 16), np = (pairs + mw - 1) / mw;
+            const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
+#define COEUS_MFMA4(BPV, NV, PV, KV)                                                                                          \
+    do {                                                                                                                      \
+        static const bool once = [] { (void)hipFuncSetAttribute((const void *)gemv_mfma_kernel<BPV, NV, PV, KV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); return true; }(); \
+        (void)once;                                                                                                           \
+        hipLaunchKernelGGL((gemv_mfma_kernel<BPV, NV, PV, KV>), mgrid, mblock, mlds, st, (const uint16_t *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
+    } while (0)
+#define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (np % 3 == 0 || np == 5) COEUS_MFMA4(BPV, NV, 3, false); else COEUS_MFMA4(BPV, NV, 4, false); } while (0)
+#define COEUS_MFMA(BPV) do { if (norm == 1) COEUS_MFMA3(BPV, 1); else if (norm == 2) COEUS_MFMA3(BPV, 2); else COEUS_MFMA3(BPV, 3); } while (0)
+            if (norm == 0 && bp <= 4) COEUS_MFMA3(4, 0);
+            else if (norm == 0 && bp == 8 && np <= 2) COEUS_MFMA4(8, 0, 2, true);
+            else if (norm == 0 && bp == 8 && np % 3 == 0) COEUS_MFMA4(8, 0, 3, false);  // (four pairs do not fit the registers)
+            else if (norm == 0 && bp == 8) COEUS_MFMA4(8, 0, 2, false);
+            else if (norm == 0 && np <= 2) COEUS_MFMA4(16, 0, 2, true);
+            else if (norm == 0) COEUS_MFMA4(16, 0, 2, false);
+            else if (bp == 2) COEUS_MFMA(2);
+            else if (bp == 4) COEUS_MFMA(4);
+            else if (bp == 8) COEUS_MFMA(8);
+            else COEUS_MFMA(16);
+#undef COEUS_MFMA
+#undef COEUS_MFMA3
+#undef COEUS_MFMA4
+            COEUS_HIP(hipGetLastError());
+            return COEUS_OK;
+        }
+    }
 #define COEUS_GEMVD2(BPV, NV) \
     hipLaunchKernelGGL((gemv_dense_kernel<BF16, BPV, NV>), grid, block, lds, st, w.data, xin, w.k, b, e, ns, nb, eps, ldx, post)
 #define COEUS_GEMVD(BPV) \

@@ -734,7 +734,11 @@ int layered_decode(Session &s, hipStream_t st, int only, uint64_t *launches, uin
     auto stream_gemv = [&](const Weight &w, const Around &to, const Epilogue &e) -> int {
         const float *const this_fold = fold;
         if (fold) fold += kHyperFoldFloats;
-        const bool fuse = s.fuse && (cfg.streams || w.n <= 16384) &&
+        // (Hyper-connections of 3 and 4 rows in front of bf16 weights are a launch of their own: folded, every
+        // compute unit reads four streams and y of every row, 42 MB out of L2 at 4 rows of 2048: 16.7 us against
+        // 4.3 + 8.4 for 11264 rows of the weight.)
+        const bool folds = !cfg.streams || w.dtype != COEUS_W_BF16 || B <= 2;
+        const bool fuse = s.fuse && folds && (cfg.streams || w.n <= 16384) &&
                           (cfg.streams ? gemv_can_fuse_hyper(w, B, cfg.streams) : pending && gemv_can_fuse_post_norm(w, B));
         if (fuse) {
             NormFuse nf;

@@ -396,7 +396,7 @@ int launch_norm_residual(const float *y, uint64_t rows, uint64_t hidden, const f
 // 4): the streams pass through registers 16 bytes at a time, the weighted sum stays there for the norm.
 // SMAX >= streams.  out may be h.y itself (a thread reads y where it writes out).
 template <int SMAX, int VM>
-__global__ __launch_bounds__(256) void hyper_kernel(float *__restrict__ x, uint32_t hidden, HyperStep h, float *out,
+__global__ __launch_bounds__(VM == 1 ? 1024 : 256) void hyper_kernel(float *__restrict__ x, uint32_t hidden, HyperStep h, float *out,
                                                     uint16_t *__restrict__ out_lp, uint64_t lp_ld, bool lp_bf16) {
     __shared__ float sh[16];
     const uint64_t row = blockIdx.x;
@@ -409,12 +409,12 @@ __global__ __launch_bounds__(256) void hyper_kernel(float *__restrict__ x, uint3
         const uint32_t i = threadIdx.x + blockDim.x * u;
         v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (i >= n4) continue;
-        float4 a[SMAX];
+        float4 a[SMAX], y;
+        if (h.y) y = *(const float4 *)(h.y + row * hidden + 4 * i);
 #pragma unroll
         for (int s = 0; s < SMAX; s++)
             if (s < (int)S) a[s] = *(const float4 *)(xr + (uint64_t)s * hidden + 4 * i);
         if (h.y) {
-            const float4 y = *(const float4 *)(h.y + row * hidden + 4 * i);
 #pragma unroll
             for (int t = 0; t < SMAX; t++) {
                 if (t >= (int)S) continue;
@@ -524,10 +524,13 @@ int launch_hyper(float *x, uint64_t rows, uint64_t hidden, const HyperStep &h, f
     const bool bf = u_lp && u_lp->bf16;
     const dim3 grid((unsigned)rows);
     if ((hidden & 3) == 0 && hidden <= 8192 && (ld & 3) == 0) {
-        const uint64_t n4 = hidden / 4, threads = std::min<uint64_t>(256, round_up(n4, 64)), vm = ceil_div(n4, threads);
+        // The few rows of a decode step: a thread per 16 bytes of the row (what bounds them is the one trip to memory
+        // and the two sums behind it: 4 rows of 2048, 6.4 us with 256 threads).
+        const uint64_t n4 = hidden / 4, most = rows <= 64 && n4 <= 1024 ? 1024 : 256;
+        const uint64_t threads = std::min<uint64_t>(most, round_up(n4, 64)), vm = ceil_div(n4, threads);
 #define COEUS_HY2(SV, VV) \
     hipLaunchKernelGGL((hyper_kernel<SV, VV>), grid, dim3((unsigned)threads), 0, st, x, (uint32_t)hidden, h, u, lp, ld, bf)
-#define COEUS_HY(SV) do { if (vm <= 2) COEUS_HY2(SV, 2); else if (vm <= 4) COEUS_HY2(SV, 4); else COEUS_HY2(SV, 8); } while (0)
+#define COEUS_HY(SV) do { if (vm == 1) COEUS_HY2(SV, 1); else if (vm <= 2) COEUS_HY2(SV, 2); else if (vm <= 4) COEUS_HY2(SV, 4); else COEUS_HY2(SV, 8); } while (0)
         if (h.streams <= 2) COEUS_HY(2);
         else if (h.streams == 3) COEUS_HY(3);
         else if (h.streams == 4) COEUS_HY(4);
