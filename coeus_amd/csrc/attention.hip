@@ -7,7 +7,7 @@
 //   kv_append_kernel      scatters the k|v thirds of a projected qkv buffer into the cache.
 //   attn_generic_kernel   one wave per (query row, head, sequence); lanes own keys for q.k and
 //                         own output dimensions for P.V.  Any head_dim, any cache type.
-//   attn_decode_kernel    one query per (sequence, head), head_dim 64 or 128, 16-bit cache: the
+//   attn_decode_kernel    one query per (sequence, head), head_dim 64 or 128: the
 //                         context is split over workgroups (flash-decoding); every lane streams
 //                         16-byte pieces of K and V with the same (key, dims) ownership in both
 //                         phases, so probabilities never leave registers; a second kernel merges
@@ -104,18 +104,31 @@ __global__ __launch_bounds__(256) void attn_generic_kernel(const float *__restri
 
 // ---------------------------------------------------------------- flash-decoding (n == 1)
 constexpr uint32_t kAttnMaxSplits = 32;  // splits per (sequence, head): bounds the merge's LDS
-// Lane l owns 16-byte piece (l % CPK) of key (l / CPK) of every wave-wide load, CPK = HD/8.
-template <int HD, bool BF16, int NW = 4>
+// Lane l owns 16-byte piece (l % CPK) of key (l / CPK) of every wave-wide load: CPK pieces of EPL elements a key.  KV: the
+// cache's type (COEUS_KV_*).
+template <int KV, int EPL>
+__device__ __forceinline__ void kv_piece(const uint4 &r, float (&v)[EPL]) {
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        if constexpr (KV == COEUS_KV_F32) v[u] = __uint_as_float(w[u]);
+        else if constexpr (KV == COEUS_KV_BF16) { v[2 * u] = __uint_as_float(w[u] << 16); v[2 * u + 1] = __uint_as_float(w[u] & 0xffff0000u); }
+        else { union { uint32_t u32; half2_t h2; } cv; cv.u32 = w[u]; v[2 * u] = (float)cv.h2.x; v[2 * u + 1] = (float)cv.h2.y; }
+    }
+}
+template <int HD, int KV, int NW = 4>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__restrict__ qkv,
-                                                          const uint16_t *__restrict__ kc,
-                                                          const uint16_t *__restrict__ vc,
+                                                          const void *__restrict__ kc,
+                                                          const void *__restrict__ vc,
                                                           uint32_t heads, uint32_t max_ctx,
                                                           uint32_t pos0, const uint32_t *pos_dev,
                                                           uint32_t keys_per_split, float *part,
                                                           uint32_t *counters, float *out,
                                                           __half *out_xq, uint32_t bp) {
-    constexpr int CPK = HD / 8, KPL = 64 / CPK;  // pieces per key, keys per wave load
-    constexpr int TILE = 16;                     // wave loads kept in flight per phase
+    constexpr int EPL = KV == COEUS_KV_F32 ? 4 : 8, CPK = HD / EPL, KPL = 64 / CPK;  // pieces per key, keys per wave load
+    // wave loads kept in flight per phase.  (f32: 32 keys of 64 a wave, so that four waves share the shortest contexts;
+    // 12 heads of 64 at contexts of 24 - 124, which attn_generic_kernel's one wave a head walked in 11.2 us: 5.0 us)
+    constexpr int TILE = KV == COEUS_KV_F32 ? 8 : 16;
     __shared__ float sm[NW], sl[NW], sacc[NW][HD];
     __shared__ float srec[kAttnMaxSplits * (HD + 2)];  // the partial records, for the merging split
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -123,20 +136,20 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
     const uint32_t inner = heads * HD;
     const uint32_t ctx = (pos_dev ? *pos_dev : pos0) + 1;
     const uint32_t piece = lane % CPK, ksub = lane / CPK;
-    float q[8];
+    float q[EPL];
 #pragma unroll
-    for (int t = 0; t < 8; t++) q[t] = qkv[(uint64_t)b * 3 * inner + h * HD + piece * 8 + t];
+    for (int t = 0; t < EPL; t++) q[t] = qkv[(uint64_t)b * 3 * inner + h * HD + piece * EPL + t];
     const uint64_t base = ((uint64_t)b * heads + h) * max_ctx * HD;
-    const uint4 *k4 = (const uint4 *)(kc + base), *v4 = (const uint4 *)(vc + base);
+    const uint4 *k4 = (const uint4 *)kc + base / EPL, *v4 = (const uint4 *)vc + base / EPL;
     const uint32_t k_begin = split * keys_per_split;
     const uint32_t k_end = min(ctx, k_begin + keys_per_split);
     // scores and running maxima are kept in base 2: s = (q . k) * scale * log2(e), p = 2^(s - m):
     // one hardware exponential per key instead of expf's range reduction (this wave's sixteen keys
     // are evaluated after its last line has arrived, on the launch's tail)
     const float scale = 1.4426950408889634f / sqrtf((float)HD);
-    float m = -INFINITY, l = 0.f, acc[8];
+    float m = -INFINITY, l = 0.f, acc[EPL];
 #pragma unroll
-    for (int t = 0; t < 8; t++) acc[t] = 0.f;
+    for (int t = 0; t < EPL; t++) acc[t] = 0.f;
 
     // each wave takes tiles of TILE*KPL keys, interleaved over the NW waves
     for (uint32_t t0 = k_begin + wave * TILE * KPL; t0 < k_end; t0 += NW * TILE * KPL) {
@@ -164,18 +177,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
         float s[TILE], tmax = -INFINITY;
 #pragma unroll
         for (int t = 0; t < TILE; t++) {
-            const uint32_t w[4] = {kr[t].x, kr[t].y, kr[t].z, kr[t].w};
-            float dot = 0.f;
+            float kv[EPL], dot = 0.f;
+            kv_piece<KV>(kr[t], kv);
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                float lo, hi;
-                if (BF16) { lo = __uint_as_float(w[u] << 16); hi = __uint_as_float(w[u] & 0xffff0000u); }
-                else { union { uint32_t u32; half2_t h2; } cv; cv.u32 = w[u]; lo = (float)cv.h2.x; hi = (float)cv.h2.y; }
-                dot = fmaf(q[2 * u], lo, dot);
-                dot = fmaf(q[2 * u + 1], hi, dot);
-            }
-            // sum the CPK pieces of a key (the lanes of one key are an aligned group of 8 or 16)
-            dot = group_sum<CPK>(dot);
+            for (int u = 0; u < EPL; u++) dot = fmaf(q[u], kv[u], dot);
+            // sum the CPK pieces of a key (the lanes of one key are an aligned group)
+            dot = group_sum<CPK == 32 ? 16 : CPK>(dot);
+            if (CPK == 32) dot = xor16_sum(dot);
             const uint32_t key = t0 + t * KPL + ksub;
             s[t] = key < k_end ? dot * scale : -INFINITY;
             tmax = fmaxf(tmax, s[t]);
@@ -184,20 +192,15 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
         const float corr = __builtin_amdgcn_exp2f(m - m_new);
         float psum = 0.f;
 #pragma unroll
-        for (int t = 0; t < 8; t++) acc[t] *= corr;
+        for (int t = 0; t < EPL; t++) acc[t] *= corr;
 #pragma unroll
         for (int t = 0; t < TILE; t++) {
             const float p = __builtin_amdgcn_exp2f(s[t] - m_new);  // 2^(-inf) = 0 for keys past the end
             psum += p;
-            const uint32_t w[4] = {vr[t].x, vr[t].y, vr[t].z, vr[t].w};
+            float vv[EPL];
+            kv_piece<KV>(vr[t], vv);
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                float lo, hi;
-                if (BF16) { lo = __uint_as_float(w[u] << 16); hi = __uint_as_float(w[u] & 0xffff0000u); }
-                else { union { uint32_t u32; half2_t h2; } cv; cv.u32 = w[u]; lo = (float)cv.h2.x; hi = (float)cv.h2.y; }
-                acc[2 * u] = fmaf(p, lo, acc[2 * u]);
-                acc[2 * u + 1] = fmaf(p, hi, acc[2 * u + 1]);
-            }
+            for (int u = 0; u < EPL; u++) acc[u] = fmaf(p, vv[u], acc[u]);
         }
         // every lane of a key holds the same p: count each key once
         l = l * corr + wave_sum(psum) * (1.0f / CPK);
@@ -205,14 +208,15 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
     }
     // fold the KPL key-subsets of the wave: lanes with equal piece hold partial sums
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
+    for (int t = 0; t < EPL; t++) {
         if (CPK == 8) acc[t] += dpp_f32<DPP_ROW_ROR8>(acc[t]);  // the other 8 lanes of the row
-        acc[t] = xor32_sum(xor16_sum(acc[t]));
+        if (CPK < 32) acc[t] = xor16_sum(acc[t]);
+        acc[t] = xor32_sum(acc[t]);
     }
     if (lane == 0) { sm[wave] = m; sl[wave] = l; }
     if (lane < CPK)
 #pragma unroll
-        for (int t = 0; t < 8; t++) sacc[wave][lane * 8 + t] = acc[t];
+        for (int t = 0; t < EPL; t++) sacc[wave][lane * EPL + t] = acc[t];
     __syncthreads();
     // merge the waves; thread d < HD finishes output dimension d
     if (threadIdx.x < HD) {
@@ -728,33 +732,33 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
     if (max_ctx * hd > 0xffffffffull)
         return fail(COEUS_INVALID_INPUT, "attention: max_ctx %llu x head_dim %llu exceeds 2^32 elements per head",
                     (unsigned long long)max_ctx, (unsigned long long)hd);
-    const bool fast = n == 1 && (hd == 64 || hd == 128) && kv_dtype != COEUS_KV_F32 &&
-                      part_scratch && nsplit >= 1;
+    const bool fast = n == 1 && (hd == 64 || hd == 128) && part_scratch && nsplit >= 1;
     if (fast) {
         if (counters && nsplit > kAttnMaxSplits)
             return fail(COEUS_INVALID_INPUT, "attention: at most %u splits with the in-kernel merge",
                         kAttnMaxSplits);
         const uint32_t kps = (uint32_t)round_up(ceil_div(max_ctx, nsplit), 64);
         const dim3 grid(nsplit, (unsigned)heads, (unsigned)batch);
-        const bool bf = kv_dtype == COEUS_KV_BF16;
         // One workgroup per CU at most and splits of 512 keys or more: 8 waves per workgroup, a tile
         // of 64 keys each at once, instead of 4 waves walking two tiles each (7B shape, batch 1,
         // context 4096: 1.768 -> 1.759 ms per step over five alternations; with shorter splits the
         // extra waves have nothing to take and the step is 0.5 % slower).
         const bool wide = batch * heads * nsplit <= 256 && kps >= 512;
-#define COEUS_AD(HDV, BFV) do {                                                                    \
+#define COEUS_AD(HDV, KVV) do {                                                                    \
     if (wide)                                                                                      \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, BFV, 8>), grid, dim3(512), 0, st, qkv,             \
-                       (const uint16_t *)kc, (const uint16_t *)vc, (uint32_t)heads,                \
+    hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV, 8>), grid, dim3(512), 0, st, qkv,             \
+                       kc, vc, (uint32_t)heads,                \
                        (uint32_t)max_ctx, (uint32_t)pos0, pos_dev, kps, part_scratch, counters,    \
                        out, out_xq, bp);                                                           \
     else                                                                                           \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, BFV>), grid, dim3(256), 0, st, qkv,                \
-                       (const uint16_t *)kc, (const uint16_t *)vc, (uint32_t)heads,                \
+    hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV>), grid, dim3(256), 0, st, qkv,                \
+                       kc, vc, (uint32_t)heads,                \
                        (uint32_t)max_ctx, (uint32_t)pos0, pos_dev, kps, part_scratch, counters,    \
                        out, out_xq, bp); } while (0)
-        if (hd == 64) { if (bf) COEUS_AD(64, true); else COEUS_AD(64, false); }
-        else { if (bf) COEUS_AD(128, true); else COEUS_AD(128, false); }
+#define COEUS_ADH(HDV) do { if (kv_dtype == COEUS_KV_F32) COEUS_AD(HDV, COEUS_KV_F32); \
+        else if (kv_dtype == COEUS_KV_BF16) COEUS_AD(HDV, COEUS_KV_BF16); else COEUS_AD(HDV, COEUS_KV_F16); } while (0)
+        if (hd == 64) COEUS_ADH(64); else COEUS_ADH(128);
+#undef COEUS_ADH
 #undef COEUS_AD
         COEUS_HIP(hipGetLastError());
         if (counters || nsplit == 1) return COEUS_OK;  // merged by the last split of each (sequence, head)
