@@ -218,7 +218,7 @@ static bool gemm_f32_is_small(const Weight &w, uint64_t m) {
 // order and runs the epilogue (8 + 5 us).  Below 48 slices the second launch costs what the split
 // saves (768-long k, 128 rows: 16.5 us unsplit, 17.7 + 4.7 us in two shares).
 static uint32_t gemm_f32_splits_wanted(const Weight &w, uint64_t m) {
-    if (w.dtype != COEUS_W_F32 || m == 0 || !gemm_f32_is_small(w, m)) return 1;
+    if (w.dtype != COEUS_W_F32 || m == 0 || !gemm_f32_is_small(w, m) || gemv_takes_f32_rows(w, m)) return 1;
     const uint64_t wgs = ceil_div(w.n, SN) * ceil_div(m, SM), slices = ceil_div(w.k, BK);
     if (slices < 48) return 1;
     uint64_t s = 768 / wgs;
@@ -229,6 +229,9 @@ static uint32_t gemm_f32_splits_wanted(const Weight &w, uint64_t m) {
 
 static int launch_gemm_f32(const Weight &w, const float *a, uint64_t m, const Epilogue &ep,
                            const GemmScratch &scr, hipStream_t st) {
+    // Up to 16 rows: the decode matmul, which gives a weight row's k to 16 waves instead of 4 and requests all of it at
+    // once (5 rows, 768 x 2304 / 768 x 768 / 768 x 3072 / 3072 x 768: 11.5 / 12.3 / 12.1 / 7.9 + 4.7 us here).
+    if (gemv_takes_f32_rows(w, m) && scr.repeat <= 1 && !scr.ev_begin) return launch_gemv(w, a, m, ep, st);
     const EpiArgs e = make_epi(ep, w.n);
     const dim3 grid((unsigned)ceil_div(w.n, BN), (unsigned)ceil_div(m, BM));
     const bool small = gemm_f32_is_small(w, m);

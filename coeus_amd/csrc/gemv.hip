@@ -1195,10 +1195,11 @@ __global__ __launch_bounds__(1024) void gemv_dense_kernel(const void *__restrict
             if (b < (int)batch) epi_store<true>(e, b, j, acc[b]);
 }
 
-// ---------------------------------------------------------------- bf16 rows on the matrix cores (2 - 16 rows)
-// y[b, j] for a tile of 16 weight rows j and all b at once: v_mfma_f32_16x16x32_bf16 with the weights as they are
-// stored and every activation as the sum of three bf16 (8 mantissa bits each: x exactly), three instructions per 32
-// of k into one f32 accumulator.  The products are those of the f32 form; what changes is the order of the sums.
+// ---------------------------------------------------------------- dense rows on the matrix cores (2 - 16 rows)
+// y[b, j] for a tile of 16 weight rows j and all b at once.  bf16 weights: v_mfma_f32_16x16x32_bf16 with the weights as
+// they are stored and every activation as the sum of three bf16 (8 mantissa bits each: x exactly), three instructions
+// per 32 of k into one f32 accumulator.  f32 weights: v_mfma_f32_16x16x4_f32.  The products are those of the f32 form;
+// what changes is the order of the sums.
 //
 // gemv_dense_kernel (a wave per weight row, activations by f32 FMA) reads `batch` f32 activations per weight: at batch
 // 4 that is eight times the weights' bytes, out of L2 where a row does not fit the first-level cache.  Here a tile's
@@ -1208,6 +1209,7 @@ __global__ __launch_bounds__(1024) void gemv_dense_kernel(const void *__restrict
 //   5632 x 2048  11.6 / 8.2   15.4 / 8.6   21.9 / 10.7   35.2 / 14.1
 //   4096 x 22016   47 / 34     73 / 36      118 / 40      215 / 55
 //   768 x 50257    28 / 14     41 / 14       68 / 16      127 / 18
+// f32: 768 x 3072 9.0 / 4.4 at batch 8, 768 x 50257 79 / 30, 4096 x 4096 31 / 15.
 // (one row: 4.2, 8.7, 33, 18.5 there, which keeps it: a wave per row needs no sum over waves.)  The large ones are
 // at 5 TB/s of weights.  An infinite weight makes its output NaN (times the pieces of an activation that are zero).
 //
@@ -1235,28 +1237,17 @@ __device__ __forceinline__ Split2 split2(float a, float b) {
     }
     return s;
 }
-struct Split3 { uint4 p[3]; };  // eight values of a row
-
-__device__ __forceinline__ float4_t mfma_split3(const uint4 &w, const Split3 &x, float4_t acc) {
-    union { uint4 u; bf16x8_t v; } uw, ux;
-    uw.u = w;
-#pragma unroll
-    for (int i = 2; i >= 0; i--) {
-        ux.u = x.p[i];
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(uw.v, ux.v, acc, 0, 0, 0);
-    }
-    return acc;
-}
-
 // The tiles blockIdx.x, + grid, .. of the workgroup.  XQ > 0: f32 activation rows x [batch][k] in global memory, read
 // four to a request (XQ requests cover the batch) and split on their way into the wave's corner.  XQ == 0: `stage`,
 // which runs behind the first requests, puts them into LDS: piece i of row b at xs.at(i, b).
 // k % 64 == 0 and at least one pair of chunks per wave.
 // KEEP: a wave's share of k is at most PD pairs, and its split activations stay in registers from tile to tile.
 // lds: mfma_wave_lds(XQ) uint4 per wave.
-struct SplitRows {
+// (Rows 16 bytes longer than k: at a multiple of 256 bytes apart they would share their banks.)
+struct SplitRows {  // bf16 weights: three pieces
     uint16_t *p;
-    uint32_t k, rows;  // (rows 8 elements longer than k: at a multiple of 256 bytes apart they would share their banks)
+    uint32_t k, rows;
+    static constexpr size_t bytes(size_t rows, size_t k) { return 3 * rows * (k + 8) * 2; }
     __device__ uint16_t *at(int i, uint32_t b) const { return p + (i * rows + b) * (k + 8); }
     __device__ void put(uint32_t b, uint32_t i, float v) const {
         const Split2 s = split2(v, 0.f);
@@ -1269,29 +1260,75 @@ struct SplitRows {
         for (int j = 0; j < 3; j++) *(uint32_t *)(at(j, b) + i) = s.p[j];
     }
 };
-static constexpr size_t split_rows_bytes(size_t rows, size_t k) { return 3 * rows * (k + 8) * 2; }
-static constexpr uint32_t mfma_wave_lds(int xq) { return 128 + 96 * xq; }
-template <int PD, bool KEEP, int XQ, class Stage>
-__device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const float *__restrict__ x, uint32_t k, uint32_t n,
-                                          uint32_t batch, uint32_t nw, uint32_t grid, const EpiArgs &e, uint4 *lds,
-                                          const SplitRows &xs, Stage stage) {
+struct PlainRows {  // f32 weights
+    float *p;
+    uint32_t k, rows;
+    static constexpr size_t bytes(size_t rows, size_t k) { return rows * (k + 4) * 4; }
+    __device__ float *at(int, uint32_t b) const { return p + b * (k + 4); }
+    __device__ void put(uint32_t b, uint32_t i, float v) const { at(0, b)[i] = v; }
+};
+// What the two weight types do differently.  bf16: 64 k per 128 bytes of a row, activations in three pieces; f32: 32 k,
+// four 16x16x4 products per 16-byte piece.
+template <bool BF16> struct MfmaType;
+template <> struct MfmaType<true> {
+    typedef uint16_t W;
+    typedef SplitRows Rows;
+    static constexpr uint32_t KU = 64;
+    static constexpr int PIECES = 3, XROWS = 4;  // rows of x that a wave request covers
+    struct Frag { uint4 p[3]; };
+    static __device__ __forceinline__ float4_t mul(const uint4 &w, const Frag &x, float4_t acc) {
+        union { uint4 u; bf16x8_t v; } uw, ux;
+        uw.u = w;
+#pragma unroll
+        for (int i = 2; i >= 0; i--) {
+            ux.u = x.p[i];
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(uw.v, ux.v, acc, 0, 0, 0);
+        }
+        return acc;
+    }
+};
+template <> struct MfmaType<false> {
+    typedef float W;
+    typedef PlainRows Rows;
+    static constexpr uint32_t KU = 32;
+    static constexpr int PIECES = 1, XROWS = 8;
+    struct Frag { uint4 p[1]; };
+    static __device__ __forceinline__ float4_t mul(const uint4 &w, const Frag &x, float4_t acc) {
+        union { uint4 u; float4_t v; } uw, ux;
+        uw.u = w;
+        ux.u = x.p[0];
+        return mfma4(uw.v, ux.v, acc);
+    }
+};
+// uint4 of a wave's corner: 16 weight rows x 128 bytes; per request of x its rows' KU values in pieces
+template <bool BF16>
+static constexpr uint32_t mfma_wave_lds(int xq) { return 128 + (BF16 ? 96 : 64) * xq; }
+template <bool BF16, int PD, bool KEEP, int XQ, class Stage>
+__device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
+                                          uint32_t n, uint32_t batch, uint32_t nw, uint32_t grid, const EpiArgs &e, uint4 *lds,
+                                          const typename MfmaType<BF16>::Rows &xs, Stage stage) {
+    typedef MfmaType<BF16> MT;
+    typedef typename MT::W W;
+    typedef typename MT::Frag Frag;
+    constexpr uint32_t KU = MT::KU, EPP = KU / 8;  // k per pair, elements per 16-byte piece
+    constexpr int XR = MT::XROWS, XN = XQ ? XQ : 1;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t c = lane & 15, g = lane >> 4, cb = min(c, batch - 1);
-    const uint32_t pairs = k >> 6, pb = pairs * wave / nw, np = pairs * (wave + 1) / nw - pb, groups = (np + PD - 1) / PD;
+    const uint32_t pairs = k / KU, pb = pairs * wave / nw, np = pairs * (wave + 1) / nw - pb, groups = (np + PD - 1) / PD;
     const uint32_t tiles = (n + 15) / 16;
-    uint4 *wl = lds + wave * mfma_wave_lds(XQ), *xl = wl + 128;
+    uint4 *wl = lds + wave * mfma_wave_lds<BF16>(XQ), *xl = wl + 128;
     // (a pair behind the wave's share is the share's last one again: no branches around the requests)
-    auto pair_at = [&](uint32_t i) { return min(i, np - 1) * 64; };
-    struct WRows { const uint16_t *p[2]; };
+    auto pair_at = [&](uint32_t i) { return min(i, np - 1) * KU; };
+    struct WRows { const W *p[2]; };
     auto tile_rows = [&](uint32_t tile) {
         WRows r;
 #pragma unroll
-        for (int q = 0; q < 2; q++) r.p[q] = w + (uint64_t)min(tile * 16 + 8 * q + (lane >> 3), n - 1) * k + pb * 64 + (lane & 7) * 8;
+        for (int q = 0; q < 2; q++) r.p[q] = w + (uint64_t)min(tile * 16 + 8 * q + (lane >> 3), n - 1) * k + pb * KU + (lane & 7) * EPP;
         return r;
     };
-    const float *xr[XQ ? XQ : 1];
+    const float *xr[XN];
     uint4 wr[PD][2];
-    u32x4_t xv[XQ ? PD : 1][XQ ? XQ : 1];  // (arrays of the struct type would be copied through scratch memory)
+    u32x4_t xv[XQ ? PD : 1][XN];  // (arrays of the struct type would be copied through scratch memory)
     auto x_request = [&](int s, uint32_t i) {
 #pragma unroll
         for (int q = 0; q < XQ; q++) xv[s][q] = *(const u32x4_t *)(xr[q] + pair_at(i));
@@ -1304,11 +1341,16 @@ __device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const 
     auto x_put = [&](int s) {
 #pragma unroll
         for (int q = 0; q < XQ; q++) {
-            const uint32_t r = 4 * q + (lane >> 4), at = (r * 8 + (((lane & 15) >> 1) ^ ((r >> 1) & 7))) * 2 + (lane & 1);
             const u32x4_t v = xv[s][q];
-            const Split2 lo = split2(__uint_as_float(v.x), __uint_as_float(v.y)), hi = split2(__uint_as_float(v.z), __uint_as_float(v.w));
+            if constexpr (BF16) {
+                const uint32_t r = 4 * q + (lane >> 4), at = (r * 8 + (((lane & 15) >> 1) ^ ((r >> 1) & 7))) * 2 + (lane & 1);
+                const Split2 lo = split2(__uint_as_float(v.x), __uint_as_float(v.y)), hi = split2(__uint_as_float(v.z), __uint_as_float(v.w));
 #pragma unroll
-            for (int i = 0; i < 3; i++) *((uint2 *)(xl + i * 32 * XQ) + at) = make_uint2(lo.p[i], hi.p[i]);
+                for (int i = 0; i < 3; i++) *((uint2 *)(xl + i * 32 * XQ) + at) = make_uint2(lo.p[i], hi.p[i]);
+            } else {
+                const uint32_t r = 8 * q + (lane >> 3);
+                *(u32x4_t *)(xl + r * 8 + ((lane & 7) ^ ((r >> 1) & 7))) = v;
+            }
         }
     };
     auto w_put = [&](int s) {
@@ -1318,17 +1360,18 @@ __device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const 
             wl[r * 8 + ((lane & 7) ^ (r >> 1))] = wr[s][q];
         }
     };
-    auto x_get = [&](uint32_t i, int h) {  // chunk h of pair i
-        Split3 f;
+    auto x_get = [&](uint32_t i, int h) {  // half h of pair i
+        Frag f;
 #pragma unroll
-        for (int j = 0; j < 3; j++)
-            f.p[j] = XQ ? xl[j * 32 * XQ + cb * 8 + ((4 * h + g) ^ (cb >> 1))]
-                        : *(const uint4 *)(xs.at(j, cb) + pb * 64 + pair_at(i) + h * 32 + g * 8);
+        for (int j = 0; j < MT::PIECES; j++)
+            f.p[j] = XQ ? xl[j * 8 * XR * XN + cb * 8 + ((4 * h + g) ^ (cb >> 1))]
+                        : *(const uint4 *)(xs.at(j, cb) + pb * KU + pair_at(i) + (4 * h + g) * EPP);
         return f;
     };
     if (XQ) {
+        constexpr uint32_t LPR = 64 / XR;  // lanes per row
 #pragma unroll
-        for (int q = 0; q < XQ; q++) xr[q] = x + (uint64_t)min(4 * q + (lane >> 4), batch - 1) * k + pb * 64 + (lane & 15) * 4;
+        for (int q = 0; q < XQ; q++) xr[q] = x + (uint64_t)min(XR * q + lane / LPR, batch - 1) * k + pb * KU + (lane % LPR) * 4;
     }
     uint32_t tile = blockIdx.x, gi = 0;
     WRows wp = tile_rows(tile);
@@ -1346,7 +1389,7 @@ __device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const 
         __builtin_amdgcn_sched_barrier(0);
     }
     if (!XQ) stage();
-    Split3 kept[KEEP ? PD : 1][2];
+    Frag kept[KEEP ? PD : 1][2];
     if (KEEP) {
 #pragma unroll
         for (int s = 0; s < PD; s++) {
@@ -1374,8 +1417,8 @@ __device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const 
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const uint4 wf = wl[c * 8 + ((4 * h + g) ^ (c >> 1))];
-                    if constexpr (KEEP) acc = mfma_split3(wf, kept[s][h], acc);
-                    else acc = mfma_split3(wf, x_get(i0 + s, h), acc);
+                    if constexpr (KEEP) acc = MT::mul(wf, kept[s][h], acc);
+                    else acc = MT::mul(wf, x_get(i0 + s, h), acc);
                 }
             }
             __builtin_amdgcn_wave_barrier();
@@ -1401,7 +1444,7 @@ __device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const 
                 // lane (c, g) adds output c of every fourth wave
                 float sum = 0.f;
                 for (uint32_t v = g; v < nw; v += 4)
-                    sum += ((const float *)(lds + v * mfma_wave_lds(XQ) + (c >> 2) * 16 + b))[c & 3];
+                    sum += ((const float *)(lds + v * mfma_wave_lds<BF16>(XQ) + (c >> 2) * 16 + b))[c & 3];
                 sum = xor32_sum(xor16_sum(sum));
                 if (epi_gated(e.act)) {
                     const float up = lane_xor1(sum);
@@ -1419,17 +1462,18 @@ __device__ __forceinline__ void mfma_rows(const uint16_t *__restrict__ w, const 
 }
 
 // NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
-template <int BP, int NORM, int PD, bool KEEP>
-__global__ __launch_bounds__(1024) void gemv_mfma_kernel(const uint16_t *__restrict__ w, const float *__restrict__ x, uint32_t k,
+template <bool BF16, int BP, int NORM, int PD, bool KEEP>
+__global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
                                                          uint32_t n, uint32_t batch, uint32_t waves, uint32_t grid, EpiArgs e,
                                                          const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
                                                          uint64_t ldx, PostNorm post) {
     extern __shared__ uint4 mlds[];
-    constexpr int XQ = NORM ? 0 : BP / 4;
+    typedef typename MfmaType<BF16>::Rows Rows;
+    constexpr int XQ = NORM ? 0 : (BP + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
     // a folded norm: the split rows first; what its staging needs lies where the corners will be
-    const SplitRows xs{(uint16_t *)mlds, k, (uint32_t)BP};
-    uint4 *corners = NORM ? (uint4 *)(xs.p + 3 * BP * (k + 8)) : mlds;
-    mfma_rows<PD, KEEP, XQ>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
+    const Rows xs{(decltype(Rows::p))mlds, k, (uint32_t)BP};
+    uint4 *corners = NORM ? (uint4 *)((char *)mlds + Rows::bytes(BP, k)) : mlds;
+    mfma_rows<BF16, PD, KEEP, XQ>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
         if constexpr (NORM != 0) {
             stage_normed_rows<BP, NORM>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post,
                                         [&](uint32_t b, uint32_t i, float v) { xs.put(b, i, v); });
@@ -1449,9 +1493,18 @@ bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch) {
     return gemv_dense_norm_lds(w.k, pad_batch(batch)) <= kDenseNormLdsLimit;
 }
 
-// Batches of 2 and more on bf16 weights whose rows are whole pairs of chunks, one for every wave at least.
+// Batches of 2 and more on weights whose rows are whole pairs of chunks (128 bytes), one for every wave at least.
 static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves) {
-    return w.dtype == COEUS_W_BF16 && batch >= 2 && w.k % 64 == 0 && w.k / 64 >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
+    const uint64_t ku = w.dtype == COEUS_W_BF16 ? 64 : 32;
+    // (f32, two or three rows on fewer than 64 tiles: a wave per row keeps more compute units busy, 6.7 against 7.9 us
+    // for 2 rows of 3072 x 768; four rows 8.7 against 8.1)
+    if (w.dtype == COEUS_W_F32 && batch < 4 && w.n <= 63 * 16) return false;
+    return w.dtype <= COEUS_W_BF16 && batch >= 2 && w.k % ku == 0 && w.k / ku >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
+}
+// Waves of a plain launch: as many as have two pairs of chunks each.
+static uint32_t gemv_mfma_waves(uint64_t pairs) { return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (pairs + 1) / 2)); }
+bool gemv_takes_f32_rows(const Weight &w, uint64_t rows) {
+    return w.dtype == COEUS_W_F32 && rows <= 16 && gemv_uses_mfma(w, rows, gemv_mfma_waves(w.k / 32));
 }
 static size_t gemv_dense_post_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)bp * k * 4; }
 bool gemv_can_fuse_post_norm(const Weight &w, uint64_t batch) {
@@ -1516,7 +1569,7 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
     constexpr int NS = kFusedStreams, SL = 4;
     // [BP][k]; MF: the waves' corners (mfma_rows), the rows' pieces
     extern __shared__ __attribute__((aligned(16))) float hyper_lds[];
-    float *xn = MF ? hyper_lds + 16 * 4 * mfma_wave_lds(0) : hyper_lds;
+    float *xn = MF ? hyper_lds + 16 * 4 * mfma_wave_lds<true>(0) : hyper_lds;
     __shared__ float2 red[16][BP];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), S = batch_streams >> 16,
                    batch = batch_streams & 0xffffu;
@@ -1642,7 +1695,7 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
     };
     if constexpr (MF) {
         __builtin_amdgcn_sched_barrier(0);
-        mfma_rows<2, true, 0>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
+        mfma_rows<true, 2, true, 0>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
             __builtin_amdgcn_sched_barrier(0);
             normalise();
         });
@@ -1736,7 +1789,7 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
         return fail(COEUS_INVALID_INPUT, "folded hyper-connections: bad arguments or too many streams");
     const uint32_t bp = pad_batch(batch), b = (uint32_t)batch, k = (uint32_t)w.k, nit = hyper_pairs(w.k);
     const bool mf = BF16 && nit == 1 && gemv_uses_mfma(w, batch, 16);
-    const size_t lds = mf ? 16 * 16 * mfma_wave_lds(0) + split_rows_bytes(bp, k) : (size_t)bp * k * 4;
+    const size_t lds = mf ? 16 * 16 * mfma_wave_lds<true>(0) + SplitRows::bytes(bp, k) : (size_t)bp * k * 4;
     const uint32_t bs = b | nf.streams << 16;
     const HyperFold *fold = (const HyperFold *)nf.fold;
     const float *y = nf.y ? nf.y : nf.h;  // (without an output of a sublayer before its weight is zero)
@@ -1790,27 +1843,29 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     const float *xin = nf ? nf->h : x;
     const float *ns = nf ? nf->scale : nullptr, *nb = nf ? nf->bias : nullptr;
     const float eps = nf ? nf->eps : 0.f;
-    if constexpr (BF16) {
-        // plain: as many waves as have two pairs of chunks each, workgroups enough to fill the compute units' 16 waves;
+    {
+        // plain: workgroups enough to fill the compute units' 16 waves;
         // a folded norm: one workgroup of 16 waves per compute unit, which stages the rows once
-        const uint32_t pairs = (uint32_t)std::min<uint64_t>(w.k / 64, 1u << 20), mw = nf ? 16u : std::max(1u, std::min(16u, (pairs + 1) / 2));
-        const size_t corners = (size_t)mw * 16 * mfma_wave_lds(nf ? 0 : std::max(bp, 4u) / 4),
-                     mlds = nf ? split_rows_bytes(bp, w.k) + std::max(corners, lds) : corners;
+        const uint32_t pairs = (uint32_t)std::min<uint64_t>(w.k / MfmaType<BF16>::KU, 1u << 20), mw = nf ? 16u : gemv_mfma_waves(pairs);
+        const uint32_t xbp = std::max(bp, 4u), xq = nf ? 0 : (xbp + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
+        const size_t corners = (size_t)mw * 16 * mfma_wave_lds<BF16>(xq),
+                     mlds = nf ? MfmaType<BF16>::Rows::bytes(bp, w.k) + std::max(corners, lds) : corners;
         if (gemv_uses_mfma(w, batch, nf ? 16 : mw) && mlds <= 160 * 1024) {
             const uint32_t tiles = (uint32_t)ceil_div(w.n, 16), np = (pairs + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
 #define COEUS_MFMA4(BPV, NV, PV, KV)                                                                                          \
     do {                                                                                                                      \
-        static const bool once = [] { (void)hipFuncSetAttribute((const void *)gemv_mfma_kernel<BPV, NV, PV, KV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); return true; }(); \
+        static const bool once = [] { (void)hipFuncSetAttribute((const void *)gemv_mfma_kernel<BF16, BPV, NV, PV, KV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); return true; }(); \
         (void)once;                                                                                                           \
-        hipLaunchKernelGGL((gemv_mfma_kernel<BPV, NV, PV, KV>), mgrid, mblock, mlds, st, (const uint16_t *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
+        hipLaunchKernelGGL((gemv_mfma_kernel<BF16, BPV, NV, PV, KV>), mgrid, mblock, mlds, st, (const typename MfmaType<BF16>::W *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
     } while (0)
 #define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (np % 3 == 0 || np == 5) COEUS_MFMA4(BPV, NV, 3, false); else COEUS_MFMA4(BPV, NV, 4, false); } while (0)
 #define COEUS_MFMA(BPV) do { if (norm == 1) COEUS_MFMA3(BPV, 1); else if (norm == 2) COEUS_MFMA3(BPV, 2); else COEUS_MFMA3(BPV, 3); } while (0)
+            constexpr int P8 = BF16 ? 2 : 4;  // (bf16, 8 rows: four pairs do not fit the registers)
             if (norm == 0 && bp <= 4) COEUS_MFMA3(4, 0);
             else if (norm == 0 && bp == 8 && np <= 2) COEUS_MFMA4(8, 0, 2, true);
-            else if (norm == 0 && bp == 8 && np % 3 == 0) COEUS_MFMA4(8, 0, 3, false);  // (four pairs do not fit the registers)
-            else if (norm == 0 && bp == 8) COEUS_MFMA4(8, 0, 2, false);
+            else if (norm == 0 && bp == 8 && np % 3 == 0) COEUS_MFMA4(8, 0, 3, false);
+            else if (norm == 0 && bp == 8) COEUS_MFMA4(8, 0, P8, false);
             else if (norm == 0 && np <= 2) COEUS_MFMA4(16, 0, 2, true);
             else if (norm == 0) COEUS_MFMA4(16, 0, 2, false);
             else if (bp == 2) COEUS_MFMA(2);

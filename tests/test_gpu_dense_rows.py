@@ -1,5 +1,5 @@
-"""The decode matmul of several rows on bf16 weights (matrix cores, activations as three bf16 each) against a
-float64 product of the same weights and activations."""
+"""The decode matmul of several rows on dense weights (matrix cores; with bf16 weights the activations as three bf16
+each) against a float64 product of the same weights and activations."""
 import numpy as np
 import pytest
 
@@ -19,15 +19,18 @@ def bound(x, w, k):
 @pytest.mark.parametrize("k,n", [(64, 1), (64, 16), (192, 33), (320, 50), (768, 130), (1024, 17), (2048, 70), (2112, 40), (3072, 31),
                                  (4096, 48), (5632, 20), (11008, 18), (128, 65552), (1024, 5003)])
 @pytest.mark.parametrize("batch", [2, 3, 4, 5, 8, 9, 16])
-def test_rows_match_float64(orc, k, n, batch):
+@pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_F32])
+def test_rows_match_float64(orc, dtype, k, n, batch):
     rng = np.random.default_rng(k + 31 * n + batch)
     w = (rng.standard_normal((k, n)) * 0.02).astype(np.float32)
     # magnitudes over forty binary orders: every piece of an activation counts
     x = (rng.standard_normal((batch, k)) * np.exp2(rng.integers(-20, 20, (batch, k)))).astype(np.float32)
-    wt = Weight(_lib.W_BF16, w)
-    wd = oracle_roundtrip(orc, _lib.W_BF16, w).astype(np.float64)
-    y = wt.gemv(dev(x))
-    assert (np.abs(y - x.astype(np.float64) @ wd) <= bound(x, wd, k)).all()
+    wt = Weight(dtype, w)
+    wd = oracle_roundtrip(orc, dtype, w).astype(np.float64)
+    want = x.astype(np.float64) @ wd
+    assert (np.abs(wt.gemv(dev(x)) - want) <= bound(x, wd, k)).all()
+    if dtype == _lib.W_F32:  # a short prompt takes the same kernel
+        assert (np.abs(wt.gemm(dev(x)) - want) <= bound(x, wd, k)).all()
 
 
 @pytest.mark.parametrize("batch", [2, 5, 16])
@@ -48,14 +51,15 @@ def test_gated_pairs_and_bias(orc, batch):
 
 
 @pytest.mark.parametrize("batch", [2, 16])
-def test_infinities_and_nan_stay_in_their_row(orc, batch):
+@pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_F32])
+def test_infinities_and_nan_stay_in_their_row(orc, dtype, batch):
     rng = np.random.default_rng(batch)
     k, n = 256, 40
     w = (rng.standard_normal((k, n)) * 0.02).astype(np.float32)
     x = rng.standard_normal((batch, k)).astype(np.float32)
     x[0, 7] = np.inf
     x[1, 70] = np.nan
-    wd = oracle_roundtrip(orc, _lib.W_BF16, w).astype(np.float64)
-    y = Weight(_lib.W_BF16, w).gemv(dev(x))
+    wd = oracle_roundtrip(orc, dtype, w).astype(np.float64)
+    y = Weight(dtype, w).gemv(dev(x))
     assert np.array_equal(y[0], np.sign(wd[7]) * np.inf) and np.isnan(y[1]).all()
     assert (np.abs(y[2:] - x[2:].astype(np.float64) @ wd) <= bound(x[2:], wd, k)).all()
