@@ -127,7 +127,7 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
                                                           __half *out_xq, uint32_t bp) {
     constexpr int EPL = KV == COEUS_KV_F32 ? 4 : 8, CPK = HD / EPL, KPL = 64 / CPK;  // pieces per key, keys per wave load
     // wave loads kept in flight per phase.  (f32: 32 keys of 64 a wave, so that four waves share the shortest contexts;
-    // 12 heads of 64 at contexts of 24 - 124, which attn_generic_kernel's one wave a head walked in 11.2 us: 5.0 us)
+    // 12 heads of 64 at contexts of 24 - 124, which attn_generic_kernel walks with one wave a head in 11.2 us and more: 3.2 us)
     constexpr int TILE = KV == COEUS_KV_F32 ? 8 : 16;
     __shared__ float sm[NW], sl[NW], sacc[NW][HD];
     __shared__ float srec[kAttnMaxSplits * (HD + 2)];  // the partial records, for the merging split

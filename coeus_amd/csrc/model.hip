@@ -3,6 +3,9 @@
 // MT:791-919) and KV-cache sessions.  Configuration, parameter layout and errors are in host.hip.
 #include "model.hpp"
 
+#include <sys/mman.h>
+#include <unistd.h>
+
 #include <cmath>
 
 namespace coeus {
@@ -19,6 +22,56 @@ void DeviceBuf::release() {
     if (p) (void)hipFree(p);
     p = nullptr;
     bytes = 0;
+}
+
+// ---------------------------------------------------------------- results to the caller
+// Maps the pages of a buffer that is about to be written, without changing what they hold (a kernel that does not
+// know the advice leaves them to be faulted in).
+static void map_pages(void *p, uint64_t bytes) {
+#ifndef MADV_POPULATE_WRITE
+#define MADV_POPULATE_WRITE 23
+#endif
+    static const uint64_t page = (uint64_t)sysconf(_SC_PAGESIZE);
+    const uint64_t first = (uint64_t)p / page * page, last = round_up((uint64_t)p + bytes, page);
+    (void)madvise((void *)first, last - first, MADV_POPULATE_WRITE);
+}
+
+int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st) {
+    if (!pin && bytes > 4096) {
+        bool ok = hipHostMalloc((void **)&pin, kSlot * kSlots, hipHostMallocDefault) == hipSuccess;
+        for (uint64_t i = 0; i < kSlots && ok; i++) ok = hipEventCreateWithFlags(&done[i], hipEventDisableTiming) == hipSuccess;
+        if (!ok) {
+            release();
+            (void)hipGetLastError();
+        }
+    }
+    if (!pin || bytes <= 4096) {
+        COEUS_HIP(hipMemcpyAsync(dst, src_dev, bytes, hipMemcpyDeviceToHost, st));
+        COEUS_HIP(hipStreamSynchronize(st));
+        return COEUS_OK;
+    }
+    const uint64_t slots = ceil_div(bytes, kSlot);
+    auto size = [&](uint64_t i) { return i + 1 < slots ? kSlot : bytes - i * kSlot; };
+    auto request = [&](uint64_t i) -> hipError_t {
+        const hipError_t e = hipMemcpyAsync(pin + i % kSlots * kSlot, (const char *)src_dev + i * kSlot, size(i), hipMemcpyDeviceToHost, st);
+        return e == hipSuccess ? hipEventRecord(done[i % kSlots], st) : e;
+    };
+    for (uint64_t i = 0; i < slots && i < kSlots; i++) COEUS_HIP(request(i));
+    map_pages(dst, bytes);
+    for (uint64_t i = 0; i < slots; i++) {
+        COEUS_HIP(hipEventSynchronize(done[i % kSlots]));
+        std::memcpy((char *)dst + i * kSlot, pin + i % kSlots * kSlot, size(i));
+        if (i + kSlots < slots) COEUS_HIP(request(i + kSlots));
+    }
+    return COEUS_OK;
+}
+void HostCopy::release() {
+    for (hipEvent_t &e : done) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
 }
 
 static uint64_t kv_elem_size(uint32_t kv_dtype) { return kv_dtype == COEUS_KV_F32 ? 4 : 2; }
@@ -92,6 +145,7 @@ Model::~Model() {
     ws.release();
     tmp_k.release();
     tmp_v.release();
+    host_copy.release();
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -360,7 +414,7 @@ static int check_ids(const Model &m, const uint64_t *ids, uint64_t count) {
     return COEUS_OK;
 }
 
-// The rows of m.ws.h -> logits on the host (enqueued).
+// The rows of m.ws.h -> logits on the host.
 static int finish_forward(Model &m, uint64_t seq_len, float *logits_out, bool all_rows, hipStream_t st) {
     const coeus_config &c = m.cfg;
     const uint64_t H = c.hidden_dim, V = c.vocab_size;
@@ -374,9 +428,7 @@ static int finish_forward(Model &m, uint64_t seq_len, float *logits_out, bool al
     } else {
         COEUS_TRY(logits_gemv(m, m.ws, x + (seq_len - 1) * H, 1, logits, st));
     }
-    COEUS_HIP(hipMemcpyAsync(logits_out, logits, (all_rows ? seq_len : 1) * V * 4,
-                             hipMemcpyDeviceToHost, st));
-    return COEUS_OK;
+    return m.host_copy.out(logits_out, logits, (all_rows ? seq_len : 1) * V * 4, st);
 }
 
 int model_forward(Model &m, const uint64_t *ids, uint64_t seq_len, float *logits_out, bool all_rows) {
@@ -528,7 +580,7 @@ int session_prefill(Session &s, const uint64_t *ids, uint64_t n, float *logits_o
         COEUS_TRY(launch_norm(c.norm, COEUS_SCOPE_TOKEN, last, s.batch, H, m.fin_s, m.fin_b,
                               c.layer_norm_eps, x, nullptr, 0, st));
         COEUS_TRY(logits_gemv(m, s.ws, x, s.batch, (float *)s.dlogits.p, st));
-        COEUS_HIP(hipMemcpyAsync(logits_out, s.dlogits.p, s.batch * V * 4, hipMemcpyDeviceToHost, st));
+        COEUS_TRY(m.host_copy.out(logits_out, s.dlogits.p, s.batch * V * 4, st));
     }
     COEUS_HIP(hipStreamSynchronize(st));
     return COEUS_OK;
@@ -558,7 +610,7 @@ int session_feed(Session &s, const uint64_t *ids, uint64_t n, const uint64_t *wa
         COEUS_TRY(launch_gather_rows((const float *)s.ws.h.p, (const uint64_t *)s.drows.p, total, H, x, st));
         COEUS_TRY(launch_norm(c.norm, COEUS_SCOPE_TOKEN, x, total, H, m.fin_s, m.fin_b, c.layer_norm_eps, x, nullptr, 0, st));
         COEUS_TRY(logits_gemv(m, s.ws, x, total, (float *)s.ws.logits.p, st));
-        COEUS_HIP(hipMemcpyAsync(logits_out, s.ws.logits.p, total * V * 4, hipMemcpyDeviceToHost, st));
+        COEUS_TRY(m.host_copy.out(logits_out, s.ws.logits.p, total * V * 4, st));
     }
     COEUS_HIP(hipStreamSynchronize(st));
     return COEUS_OK;
@@ -697,11 +749,11 @@ static int enqueue_decode_step(Session &s, hipStream_t st, int only = STEP_ALL,
     return COEUS_OK;
 }
 
-static int upload_pos(Session &s, hipStream_t st) {
+// The step's tokens (nullable) and position go to the device with a kernel's arguments: two copies out of the
+// caller's memory cost a staging trip and a copy kernel each.
+static int upload_step(Session &s, const uint64_t *ids, hipStream_t st) {
     s.host_pos[0] = (uint32_t)s.pos;
-    s.host_pos[1] = 0;
-    COEUS_HIP(hipMemcpyAsync(s.dpos.p, s.host_pos, 8, hipMemcpyHostToDevice, st));
-    return COEUS_OK;
+    return launch_step_state(ids, ids ? s.batch : 0, (uint32_t)s.pos, (uint64_t *)s.dids.p, (uint32_t *)s.dpos.p, st);
 }
 
 int session_decode(Session &s, const uint64_t *ids, float *logits_out) {
@@ -713,13 +765,10 @@ int session_decode(Session &s, const uint64_t *ids, float *logits_out) {
                     (unsigned long long)(s.pos + 1), (unsigned long long)s.max_ctx);
     COEUS_TRY(check_ids(m, ids, s.batch));
     hipStream_t st = m.stream;
-    COEUS_HIP(hipMemcpyAsync(s.dids.p, ids, s.batch * 8, hipMemcpyHostToDevice, st));
-    COEUS_TRY(upload_pos(s, st));
+    COEUS_TRY(upload_step(s, ids, st));
     COEUS_TRY(enqueue_decode_step(s, st));
     s.pos += 1;
-    if (logits_out)
-        COEUS_HIP(hipMemcpyAsync(logits_out, s.dlogits.p, s.batch * m.cfg.vocab_size * 4,
-                                 hipMemcpyDeviceToHost, st));
+    if (logits_out) COEUS_TRY(m.host_copy.out(logits_out, s.dlogits.p, s.batch * m.cfg.vocab_size * 4, st));
     COEUS_HIP(hipStreamSynchronize(st));
     return COEUS_OK;
 }
@@ -757,8 +806,7 @@ int session_decode_greedy(Session &s, const uint64_t *first_ids, uint64_t n_step
     hipStream_t st = m.stream;
     const bool sample = sampling && sampling->temperature > 0.f;
     if (!sample && !s.graph_exec && s.use_graph) COEUS_TRY(build_greedy_graph(s, st));
-    COEUS_HIP(hipMemcpyAsync(s.dids.p, first_ids, s.batch * 8, hipMemcpyHostToDevice, st));
-    COEUS_TRY(upload_pos(s, st));
+    COEUS_TRY(upload_step(s, first_ids, st));
     for (uint64_t i = 0; i < n_steps; i++) {
         if (!sample && s.use_graph) {
             COEUS_HIP(hipGraphLaunch(s.graph_exec, st));
@@ -831,7 +879,7 @@ static int session_time_decode_part(Session &s, int only, uint64_t reps, float *
         // positions 0 .. that row, so a full session attends to its whole context
         const uint64_t keep = s.pos;
         if (s.pos >= s.max_ctx || only == STEP_ATTENTION) s.pos = (s.pos < s.max_ctx ? s.pos : s.max_ctx) - 1;
-        int rc0 = upload_pos(s, st);
+        int rc0 = upload_step(s, nullptr, st);
         s.pos = keep;
         COEUS_TRY(rc0);
     }

@@ -22,6 +22,20 @@ struct DeviceBuf {
     void release();
 };
 
+// Results on their way to the caller's memory.  hipMemcpyAsync into pageable memory goes through the runtime's own
+// staging buffer and, where the caller's pages have never been touched (a result array made for this call), faults
+// them in one by one while the GPU waits: 1.6 MB of logits took 0.45 ms behind a step of 0.53 ms.  Here the copy goes to
+// pinned slots of the model's, the caller's pages are mapped while the GPU still computes, and a slot is copied out
+// while the next one fills.
+struct HostCopy {
+    static constexpr uint64_t kSlot = 1 << 20, kSlots = 4;
+    char *pin = nullptr;
+    hipEvent_t done[kSlots] = {};
+    // dst[0 .. bytes) = src_dev, behind everything enqueued on st; returns when dst is written
+    int out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st);
+    void release();
+};
+
 struct LayerWeights {
     Weight qkv, o, up, down;  // up holds interleaved (gate, up) rows for a gated FFN
     const float *ln1_s = nullptr, *ln1_b = nullptr, *ln2_s = nullptr, *ln2_b = nullptr;
@@ -107,6 +121,7 @@ struct Model {
     std::mutex mu;  // serialises every call that touches the stream or the workspaces
     Workspace ws;
     DeviceBuf tmp_k, tmp_v;
+    HostCopy host_copy;
     // HBM that resident f16 copies of quantised weights may still take (prefill matmul operands)
     static constexpr uint64_t kExpandBudget = 64ull << 30;
     uint64_t expand_budget = kExpandBudget;
@@ -128,7 +143,7 @@ struct Session {
     uint32_t bp = 1, nsplit = 1;
     bool use_graph = true;
     bool fuse = true;  // fold norms into the decode matmuls where possible
-    uint32_t host_pos[2] = {0, 0};
+    uint32_t host_pos[1] = {0};  // the position of the step enqueued last
     DeviceBuf kc, vc;
     LayeredState state;  // layered models (instead of kc / vc)
     Workspace ws;  // prefill

@@ -746,4 +746,20 @@ int launch_advance(uint32_t *pos, uint32_t *step, hipStream_t st) {
     return COEUS_OK;
 }
 
+struct StepState { uint64_t ids[16]; uint32_t n, pos; };
+__global__ void step_state_kernel(StepState a, uint64_t *dids, uint32_t *dpos) {
+    if (threadIdx.x < a.n) dids[threadIdx.x] = a.ids[threadIdx.x];
+    if (threadIdx.x < 2) dpos[threadIdx.x] = threadIdx.x == 0 ? a.pos : 0u;
+}
+int launch_step_state(const uint64_t *ids, uint64_t n, uint32_t pos, uint64_t *dids, uint32_t *dpos, hipStream_t st) {
+    if (n > 16) return fail(COEUS_INVALID_INPUT, "a decode step has at most 16 sequences");
+    StepState a{};
+    for (uint64_t i = 0; i < n; i++) a.ids[i] = ids[i];
+    a.n = (uint32_t)n;
+    a.pos = pos;
+    hipLaunchKernelGGL(step_state_kernel, dim3(1), dim3(64), 0, st, a, dids, dpos);
+    COEUS_HIP(hipGetLastError());
+    return COEUS_OK;
+}
+
 }  // namespace coeus
