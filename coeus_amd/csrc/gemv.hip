@@ -1195,6 +1195,128 @@ __global__ __launch_bounds__(1024) void gemv_dense_kernel(const void *__restrict
             if (b < (int)batch) epi_store<true>(e, b, j, acc[b]);
 }
 
+// One activation row with the norm in front (NORM 1 or 2), k % 8 == 0, k <= 512 STEPS: no LDS and no barrier.  A wave
+// keeps the whole row in registers in the places of its weight loads (lane: 8 consecutive elements of every 512),
+// finds the statistics by itself and multiplies R weight rows, all of whose loads are out before the row is
+// normalised.  The kernel above normalises once for 16 rows, in five passes through LDS with a barrier behind each:
+// 6.9 - 7.1 us for 768 x 2304 and 768 x 3072 in f32 and 6.0 in bf16; here 4.9 - 5.1 and 4.0 - 4.2.
+constexpr int kRowR = 4;  // (2: 2-3 % slower steps of the 250M models)
+template <bool BF16, bool RMS, int STEPS, int R>
+__global__ __launch_bounds__(256) void gemv_row_kernel(const void *__restrict__ wdata, const float *__restrict__ x, uint32_t k,
+                                                       const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
+                                                       EpiArgs e) {
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t n = (uint32_t)e.n, j0 = (blockIdx.x * 4 + wave) * R;
+    float4 xv[STEPS][2], gv[STEPS][2], bv[STEPS][2];
+    const float *bp = RMS || !nbias ? nscale : nbias;  // (unused then)
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        const uint32_t i = min(512 * s + 8 * lane, k - 8);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            xv[s][h] = *(const float4 *)(x + i + 4 * h);
+            gv[s][h] = *(const float4 *)(nscale + i + 4 * h);
+            if (!RMS) bv[s][h] = *(const float4 *)(bp + i + 4 * h);
+        }
+    }
+    uint4 wv[R][STEPS][BF16 ? 1 : 2];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint32_t row = min(j0 + r, n - 1);
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) {
+            const uint64_t at = (uint64_t)row * k + min(512 * s + 8 * lane, k - 8);
+            if (BF16) wv[r][s][0] = load_stream((const uint4 *)((const uint16_t *)wdata + at));
+            else {
+                wv[r][s][0] = load_stream((const uint4 *)((const float *)wdata + at));
+                wv[r][s][BF16 ? 0 : 1] = load_stream((const uint4 *)((const float *)wdata + at + 4));
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
+    float v[STEPS][8];
+    float mean = 0.f, rs;
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        const bool in = 512 * s + 8 * lane < k;
+        const float t[8] = {xv[s][0].x, xv[s][0].y, xv[s][0].z, xv[s][0].w, xv[s][1].x, xv[s][1].y, xv[s][1].z, xv[s][1].w};
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[s][u] = in ? t[u] : 0.f;
+    }
+    if (!RMS) {
+        float sum = 0.f;
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
+#pragma unroll
+            for (int u = 0; u < 8; u++) sum += v[s][u];
+        mean = row_sum(sum) / (float)k;
+    }
+    {
+        float sq = 0.f;
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) {
+            const bool in = 512 * s + 8 * lane < k;
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const float d = in ? v[s][u] - mean : 0.f;
+                sq = fmaf(d, d, sq);
+            }
+        }
+        rs = 1.0f / sqrtf(row_sum(sq) / (float)k + eps);
+    }
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) {
+        const bool in = 512 * s + 8 * lane < k;
+        const float g[8] = {gv[s][0].x, gv[s][0].y, gv[s][0].z, gv[s][0].w, gv[s][1].x, gv[s][1].y, gv[s][1].z, gv[s][1].w};
+        float b[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (!RMS && nbias) {
+            const float t[8] = {bv[s][0].x, bv[s][0].y, bv[s][0].z, bv[s][0].w, bv[s][1].x, bv[s][1].y, bv[s][1].z, bv[s][1].w};
+#pragma unroll
+            for (int u = 0; u < 8; u++) b[u] = t[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[s][u] = in ? g[u] * (v[s][u] - mean) * rs + b[u] : 0.f;
+    }
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        acc[r] = 0.f;
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) {
+            const uint4 a = wv[r][s][0], c = wv[r][s][BF16 ? 0 : 1];
+            float w[8];
+            if (BF16) {
+                const uint32_t q[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+                for (int u = 0; u < 4; u++) { w[2 * u] = __uint_as_float(q[u] << 16); w[2 * u + 1] = __uint_as_float(q[u] & 0xffff0000u); }
+            } else {
+                const uint32_t q[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+                for (int u = 0; u < 8; u++) w[u] = __uint_as_float(q[u]);
+            }
+            const bool in = 512 * s + 8 * lane < k;  // (a lane behind the end re-read the last weights: an infinite one times 0)
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc[r] = fmaf(in ? w[u] : 0.f, v[s][u], acc[r]);
+        }
+        acc[r] = row_sum(acc[r]);
+    }
+    // lane r finishes row r (gated: lane m the pair 2m, 2m + 1)
+    if (epi_gated(e.act)) {
+        float g = acc[0], u = acc[R > 1 ? 1 : 0];
+#pragma unroll
+        for (int m = 1; m < R / 2; m++)
+            if (lane == (uint32_t)m) { g = acc[2 * m]; u = acc[2 * m + 1]; }
+        if (lane < R / 2 && j0 + 2 * lane + 1 < n) epi_store_gated(e, 0, j0 / 2 + lane, g, u);
+    } else {
+        float t = acc[0];
+#pragma unroll
+        for (int r = 1; r < R; r++)
+            if (lane == (uint32_t)r) t = acc[r];
+        if (lane < R && j0 + lane < n) epi_store<true>(e, 0, j0 + lane, t);
+    }
+}
+
 // ---------------------------------------------------------------- dense rows on the matrix cores (2 - 16 rows)
 // y[b, j] for a tile of 16 weight rows j and all b at once.  bf16 weights: v_mfma_f32_16x16x32_bf16 with the weights as
 // they are stored and every activation as the sum of three bf16 (8 mantissa bits each: x exactly), three instructions
@@ -1493,13 +1615,16 @@ bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch) {
     return gemv_dense_norm_lds(w.k, pad_batch(batch)) <= kDenseNormLdsLimit;
 }
 
-// Batches of 2 and more on weights whose rows are whole pairs of chunks (128 bytes), one for every wave at least.
+// Weights whose rows are whole pairs of chunks (128 bytes), one for every wave at least.
 static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves) {
     const uint64_t ku = w.dtype == COEUS_W_BF16 ? 64 : 32;
     // (f32, two or three rows on fewer than 64 tiles: a wave per row keeps more compute units busy, 6.7 against 7.9 us
     // for 2 rows of 3072 x 768; four rows 8.7 against 8.1)
     if (w.dtype == COEUS_W_F32 && batch < 4 && w.n <= 63 * 16) return false;
-    return w.dtype <= COEUS_W_BF16 && batch >= 2 && w.k % ku == 0 && w.k / ku >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
+    // (one row of bf16 weights: long rows few of which there are, 11008 x 4096 20.8 us there, 18.9 here, 4096 x 4096 8.6 / 7.9;
+    // and short rows many of which there are, 768 x 50257 18.5 / 13.9; between them a wave per row: 2048 x 5632 7.1 / 8.4)
+    if (batch == 1 && (w.dtype != COEUS_W_BF16 || !((w.k >= 4096 && w.n <= 4096) || (w.k <= 1024 && w.n >= 16384)))) return false;
+    return w.dtype <= COEUS_W_BF16 && batch >= 1 && w.k % ku == 0 && w.k / ku >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
 }
 // Waves of a plain launch: as many as have two pairs of chunks each.
 static uint32_t gemv_mfma_waves(uint64_t pairs) { return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (pairs + 1) / 2)); }
@@ -1843,6 +1968,16 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     const float *xin = nf ? nf->h : x;
     const float *ns = nf ? nf->scale : nullptr, *nb = nf ? nf->bias : nullptr;
     const float eps = nf ? nf->eps : 0.f;
+    const bool aligned = (((uintptr_t)xin | (uintptr_t)ns | (uintptr_t)nb) & 15) == 0;  // 16-byte loads
+    // (up to 1024 elements: a wave's registers hold the row, its scale and bias and four weight rows)
+    if (bp == 1 && (norm == 1 || norm == 2) && aligned && w.k % 8 == 0 && w.k <= 1024 && w.n < (1ull << 31) - 64) {
+#define COEUS_ROW(SV, RMSV) hipLaunchKernelGGL((gemv_row_kernel<BF16, RMSV, SV, kRowR>), dim3((unsigned)ceil_div(w.n, 4 * kRowR)), dim3(256), 0, st, w.data, xin, (uint32_t)w.k, ns, nb, eps, e)
+        if (w.k <= 512) { if (norm == 1) COEUS_ROW(1, false); else COEUS_ROW(1, true); }
+        else { if (norm == 1) COEUS_ROW(2, false); else COEUS_ROW(2, true); }
+#undef COEUS_ROW
+        COEUS_HIP(hipGetLastError());
+        return COEUS_OK;
+    }
     {
         // plain: workgroups enough to fill the compute units' 16 waves;
         // a folded norm: one workgroup of 16 waves per compute unit, which stages the rows once
@@ -1850,7 +1985,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         const uint32_t xbp = std::max(bp, 4u), xq = nf ? 0 : (xbp + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
         const size_t corners = (size_t)mw * 16 * mfma_wave_lds<BF16>(xq),
                      mlds = nf ? MfmaType<BF16>::Rows::bytes(bp, w.k) + std::max(corners, lds) : corners;
-        if (gemv_uses_mfma(w, batch, nf ? 16 : mw) && mlds <= 160 * 1024) {
+        if (aligned && !(nf && batch == 1) && gemv_uses_mfma(w, batch, nf ? 16 : mw) && mlds <= 160 * 1024) {
             const uint32_t tiles = (uint32_t)ceil_div(w.n, 16), np = (pairs + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
 #define COEUS_MFMA4(BPV, NV, PV, KV)                                                                                          \

@@ -18,7 +18,7 @@ def bound(x, w, k):
 # do not fill a tile; more tiles than workgroups (16 * 4096 rows)
 @pytest.mark.parametrize("k,n", [(64, 1), (64, 16), (192, 33), (320, 50), (768, 130), (1024, 17), (2048, 70), (2112, 40), (3072, 31),
                                  (4096, 48), (5632, 20), (11008, 18), (128, 65552), (1024, 5003)])
-@pytest.mark.parametrize("batch", [2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("batch", [1, 2, 3, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_F32])
 def test_rows_match_float64(orc, dtype, k, n, batch):
     rng = np.random.default_rng(k + 31 * n + batch)
