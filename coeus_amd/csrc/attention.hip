@@ -116,7 +116,7 @@ __device__ __forceinline__ void kv_piece(const uint4 &r, float (&v)[EPL]) {
         else { union { uint32_t u32; half2_t h2; } cv; cv.u32 = w[u]; v[2 * u] = (float)cv.h2.x; v[2 * u + 1] = (float)cv.h2.y; }
     }
 }
-template <int HD, int KV, int NW = 4>
+template <int HD, int KV, int NW, int TILE>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__restrict__ qkv,
                                                           const void *__restrict__ kc,
                                                           const void *__restrict__ vc,
@@ -126,9 +126,6 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
                                                           uint32_t *counters, float *out,
                                                           __half *out_xq, uint32_t bp) {
     constexpr int EPL = KV == COEUS_KV_F32 ? 4 : 8, CPK = HD / EPL, KPL = 64 / CPK;  // pieces per key, keys per wave load
-    // wave loads kept in flight per phase.  (f32: 32 keys of 64 a wave, so that four waves share the shortest contexts;
-    // 12 heads of 64 at contexts of 24 - 124, which attn_generic_kernel walks with one wave a head in 11.2 us and more: 3.2 us)
-    constexpr int TILE = KV == COEUS_KV_F32 ? 8 : 16;
     __shared__ float sm[NW], sl[NW], sacc[NW][HD];
     __shared__ float srec[kAttnMaxSplits * (HD + 2)];  // the partial records, for the merging split
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -707,7 +704,7 @@ bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype) {
 }
 
 uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t max_ctx) {
-    // Aim for one workgroup per CU, at least 256 keys per split.  Measured at context 4096 with 32
+    // Aim for one workgroup per CU, at least 128 keys per split.  Measured at context 4096 with 32
     // heads of 128: batch 1, 8 splits 17.3 us against 17.8 with 16; batch 4, 2 splits 46.3 us
     // against 49.0 with 8; batch 16, 1 split 182.7 us against 187.9 with 2 (fewer partial records
     // to publish and merge; the kernel's two workgroups per CU stream at the same rate either way).
@@ -715,7 +712,11 @@ uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t max_ctx) {
     // ran 17.6 us at batch 8 x 12 heads of 64 against 14.0 us with four.
     uint64_t want = ceil_div(256, batch * heads);
     while (want & (want - 1)) want++;  // up to the next power of two
+    // 256 keys per split, but 128 up to eight splits (us per launch, 256 / 128 keys: 32 heads of 128 at 520 keys 8.3 / 7.0,
+    // at 1080 9.3 / 8.3; 12 heads of 64 at 560 5.9 / 5.3; at 2025, sixteen splits against eight, 7.3 / 6.3)
     uint64_t cap = ceil_div(max_ctx, 256);
+    const uint64_t fine = ceil_div(max_ctx, 128);
+    if (cap < 8) cap = fine < 8 ? fine : 8;
     uint64_t s = 1;
     while (s * 2 <= want && s * 2 <= cap && s * 2 <= kAttnMaxSplits) s *= 2;
     return (uint32_t)s;
@@ -744,22 +745,28 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
         // context 4096: 1.768 -> 1.759 ms per step over five alternations; with shorter splits the
         // extra waves have nothing to take and the step is 0.5 % slower).
         const bool wide = batch * heads * nsplit <= 256 && kps >= 512;
+        // TILE: wave loads kept in flight per phase, as many as the four waves need to take a split at once (a split of 128
+        // keys of 64 in 16 loads a wave is one wave's work; 12 heads of 64 at 560 keys: 6.1 -> 5.3 us).  f32: at most 8,
+        // half the keys per load (12 heads of 64 at 124 / 500 / 1000 keys, which attn_generic_kernel walks with one wave
+        // a head in 25 / 116 / 312 us: 3.2 / 5.5 / 5.9).
+        const uint32_t epl = kv_dtype == COEUS_KV_F32 ? 4 : 8, kpl = 64 / ((uint32_t)hd / epl);
+        const uint32_t once = 4 * kpl;
+        const int tile = kps <= 4 * once ? 4 : kps <= 8 * once || kv_dtype == COEUS_KV_F32 ? 8 : 16;
+#define COEUS_AD3(HDV, KVV, NWV, TV)                                                               \
+    hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV, NWV, TV>), grid, dim3(NWV * 64), 0, st, qkv,  \
+                       kc, vc, (uint32_t)heads, (uint32_t)max_ctx, (uint32_t)pos0, pos_dev, kps,   \
+                       part_scratch, counters, out, out_xq, bp)
 #define COEUS_AD(HDV, KVV) do {                                                                    \
-    if (wide)                                                                                      \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV, 8>), grid, dim3(512), 0, st, qkv,             \
-                       kc, vc, (uint32_t)heads,                \
-                       (uint32_t)max_ctx, (uint32_t)pos0, pos_dev, kps, part_scratch, counters,    \
-                       out, out_xq, bp);                                                           \
-    else                                                                                           \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV>), grid, dim3(256), 0, st, qkv,                \
-                       kc, vc, (uint32_t)heads,                \
-                       (uint32_t)max_ctx, (uint32_t)pos0, pos_dev, kps, part_scratch, counters,    \
-                       out, out_xq, bp); } while (0)
+    if (wide) COEUS_AD3(HDV, KVV, 8, (KVV == COEUS_KV_F32 ? 8 : 16));                              \
+    else if (tile == 4) COEUS_AD3(HDV, KVV, 4, 4);                                                 \
+    else if (tile == 8) COEUS_AD3(HDV, KVV, 4, 8);                                                 \
+    else COEUS_AD3(HDV, KVV, 4, (KVV == COEUS_KV_F32 ? 8 : 16)); } while (0)
 #define COEUS_ADH(HDV) do { if (kv_dtype == COEUS_KV_F32) COEUS_AD(HDV, COEUS_KV_F32); \
         else if (kv_dtype == COEUS_KV_BF16) COEUS_AD(HDV, COEUS_KV_BF16); else COEUS_AD(HDV, COEUS_KV_F16); } while (0)
         if (hd == 64) COEUS_ADH(64); else COEUS_ADH(128);
 #undef COEUS_ADH
 #undef COEUS_AD
+#undef COEUS_AD3
         COEUS_HIP(hipGetLastError());
         if (counters || nsplit == 1) return COEUS_OK;  // merged by the last split of each (sequence, head)
         const dim3 mg((unsigned)heads, (unsigned)batch);

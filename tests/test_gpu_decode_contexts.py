@@ -1,0 +1,34 @@
+"""Decode attention (split context): a session's step logits against the prompt pass over the same tokens, at contexts
+around the kernel's tiles and splits."""
+import numpy as np
+import pytest
+
+from coeus_amd import Transformer250MConfig, TransformerModelPlugin
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,hd", [(2, 64), (3, 128)])
+@pytest.mark.parametrize("max_ctx", [140, 520, 1300, 2300])
+@pytest.mark.parametrize("kv", ["f32", "f16", "bf16"])
+def test_steps_match_prompt_pass(heads, hd, max_ctx, kv):
+    cfg = Transformer250MConfig(hidden_dim=heads * hd, num_layers=2, num_heads=heads, intermediate_dim=256, vocab_size=160,
+                                max_seq_len=max_ctx, norm_scope="token", max_batch=3, kv_dtype=kv)
+    model = TransformerModelPlugin().create_builder().build(cfg, seed=5)
+    rng = np.random.default_rng(max_ctx + hd)
+    # 32 (16) keys of 64 (128) a wave, four or eight waves, splits of 64 or 256 and more keys
+    for ctx in (1, 2, 31, 32, 33, 64, 127, 128, 129, 255, 257, 512, 513, 1025, 2049, max_ctx):
+        if ctx > max_ctx:
+            continue
+        ids = rng.integers(0, cfg.vocab_size, (3, ctx), dtype=np.uint64)
+        s = model.session(batch=3, max_ctx=max_ctx)
+        if ctx > 1:
+            s.prefill(ids[:, :-1], want_logits=False)
+        got = s.decode(ids[:, -1])
+        s.close()
+        for b in range(3):
+            want = model.forward(ids[b])
+            # f32: two orders of sums over two layers, a few roundings of 2^-24 each (1e-6 measured).  16-bit caches: the
+            # prompt pass also rounds queries and weights of the softmax to the cache's type, 2^-11 and 2^-8 relative
+            tol = {"f32": 2e-5, "f16": 2e-3, "bf16": 1.6e-2}[kv]
+            assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), (ctx, b)
