@@ -54,12 +54,12 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
     auto size = [&](uint64_t i) { return i + 1 < slots ? kSlot : bytes - i * kSlot; };
     auto request = [&](uint64_t i) -> hipError_t {
         const hipError_t e = hipMemcpyAsync(pin + i % kSlots * kSlot, (const char *)src_dev + i * kSlot, size(i), hipMemcpyDeviceToHost, st);
-        return e == hipSuccess ? hipEventRecord(done[i % kSlots], st) : e;
+        return e == hipSuccess && i + 1 < slots ? hipEventRecord(done[i % kSlots], st) : e;
     };
     for (uint64_t i = 0; i < slots && i < kSlots; i++) COEUS_HIP(request(i));
     map_pages(dst, bytes);
     for (uint64_t i = 0; i < slots; i++) {
-        COEUS_HIP(hipEventSynchronize(done[i % kSlots]));
+        COEUS_HIP(i + 1 < slots ? hipEventSynchronize(done[i % kSlots]) : hipStreamSynchronize(st));
         std::memcpy((char *)dst + i * kSlot, pin + i % kSlots * kSlot, size(i));
         if (i + kSlots < slots) COEUS_HIP(request(i + kSlots));
     }
@@ -768,7 +768,7 @@ int session_decode(Session &s, const uint64_t *ids, float *logits_out) {
     COEUS_TRY(upload_step(s, ids, st));
     COEUS_TRY(enqueue_decode_step(s, st));
     s.pos += 1;
-    if (logits_out) COEUS_TRY(m.host_copy.out(logits_out, s.dlogits.p, s.batch * m.cfg.vocab_size * 4, st));
+    if (logits_out) return m.host_copy.out(logits_out, s.dlogits.p, s.batch * m.cfg.vocab_size * 4, st);
     COEUS_HIP(hipStreamSynchronize(st));
     return COEUS_OK;
 }
