@@ -1370,16 +1370,25 @@ static bool gemm_uses_h256(const Weight &w, uint64_t m) {
 // each tile walks all of k at about a microsecond per 32-wide slice.  Such launches are split along
 // k: `splits` workgroups per tile each take a share of the slices and store plain partial products,
 // and a second kernel sums them in split order (deterministic) and runs the epilogue.  At least 8
-// slices per split (the request pipeline is 3 deep), at most 16 splits (each adds a plane of
-// m x n floats to write and read back), no more workgroups than CUs (one workgroup fills a CU's LDS).
+// slices per split (the request pipeline is 3 deep), at most 16 splits, no more workgroups than CUs (one workgroup
+// fills a CU's LDS).  Each split adds a plane of m x n floats to write and read back: of the splits that fit, the one
+// with the shortest sum of 0.6 us per slice, 4.5 us for the second launch and the planes at 5.5 TB/s (us, the most
+// splits that fit / this rule: 201 rows of 4096 x 4096 34.6 / 31.5, of 768 x 3072 22.9 / 22.9; 512 rows of 768 x 3072
+// 29.5 / 24.9; 2000 rows of 768 x 2304 35.4 / 28.0).
 static uint32_t gemm_splits_wanted(const Weight &w, uint64_t m) {
     if (!gemm_uses_h256(w, m)) return 1;
     const uint64_t tiles = ceil_div(m, TM) * ceil_div(w.n, TN), slices = w.k / TK;
     if (tiles > 128) return 1;
-    uint64_t s = 256 / tiles;
-    if (s > slices / 8) s = slices / 8;
-    if (s > 16) s = 16;
-    return s < 2 ? 1 : (uint32_t)s;
+    uint64_t most = 256 / tiles;
+    if (most > slices / 8) most = slices / 8;
+    if (most > 16) most = 16;
+    uint32_t best = 1;
+    double best_us = 0.6 * (double)slices;
+    for (uint64_t s = 2; s <= most; s++) {
+        const double us = 0.6 * (double)ceil_div(slices, s) + 4.5 + (double)(s * m * w.n) * 8.0 / 5.5e6;
+        if (us < best_us) { best_us = us; best = (uint32_t)s; }
+    }
+    return best;
 }
 
 // A larger launch runs its tiles in rounds of 256 (one workgroup fills a CU), and the last round
