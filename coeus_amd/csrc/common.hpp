@@ -194,6 +194,8 @@ struct NormFuse {
     const float *g = nullptr;
     // Dense weights only: row stride of h (0: k), for rows that are part of a wider buffer.
     uint64_t ld = 0;
+    // f32 weights, LayerNorm only (gemv_can_fuse_whole_norm): one mean and variance over all the rows
+    bool whole = false;
     // Dense weights only, instead of a norm in front: the norm stands behind the previous sublayer, whose
     // bare output is y [batch, k].  The matmul multiplies h + y / rms(y) * scale (* ls) and stores these
     // rows to h_out (not h: every workgroup reads h).
@@ -211,6 +213,8 @@ bool gemv_can_fuse_norm(const Weight &w, uint64_t batch);
 // The same for f32 / bf16 weights (the normalised block [batch, k] f32 has to fit in LDS; the
 // statistics are computed inside the launch, NormFuse::stats is not used).
 bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch);
+// ... and for a LayerNorm over all rows together (NormFuse::whole) in front of f32 weights.
+bool gemv_can_fuse_whole_norm(const Weight &w, uint64_t batch);
 // ... and for the norm behind a sublayer (NormFuse::y): two rows per sequence have to fit.
 bool gemv_can_fuse_post_norm(const Weight &w, uint64_t batch);
 // ... and for hyper-connections (NormFuse::streams).

@@ -246,7 +246,14 @@ __device__ __forceinline__ float epi_store(const EpiArgs &e, uint64_t row, uint6
     if (KV && e.kv_k && j >= e.kv_inner) {
         // column j of q|k|v: key or value element (head, dim) of sequence `row` at position *kv_pos
         const uint32_t c = (uint32_t)(j % e.kv_inner), hh = c / e.kv_hd, d = c % e.kv_hd;
-        const uint64_t idx = ((row * e.kv_heads + hh) * e.kv_max_ctx + (pos_known ? pos : *e.kv_pos)) * e.kv_hd + d;
+        uint64_t seq = row, at;
+        if (e.kv_rows_per_seq) {  // a short prompt
+            seq = row / e.kv_rows_per_seq;
+            at = e.kv_pos0 + row % e.kv_rows_per_seq;
+        } else {
+            at = pos_known ? pos : *e.kv_pos;
+        }
+        const uint64_t idx = ((seq * e.kv_heads + hh) * e.kv_max_ctx + at) * e.kv_hd + d;
         kv_cache_store(j < 2 * (uint64_t)e.kv_inner ? e.kv_k : e.kv_v, e.kv_dtype, idx, v);
         return v;
     }

@@ -1002,7 +1002,7 @@ struct PostNorm {
     const float *y, *ls;
     float *h_out;
 };
-// The staging of NORM 1 - 3: rows of x (see above) -> normalised f32 values, element i of row b handed to put(b, i, v)
+// The staging of NORM 1 - 4: rows of x (see above; 4: LayerNorm over all rows together) -> normalised f32 values, element i of row b handed to put(b, i, v)
 // (which may write it to xn + b k + i).  Every wave of the workgroup takes part; the last barrier is the caller's.  LDS
 // at xn: [BP][k] rows, [2][k] scale and bias, partial sums, statistics (NORM == 3: then [BP][k] residual rows).
 template <int BP, int NORM, class Put>
@@ -1022,7 +1022,7 @@ __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__rest
     for (int b = 0; b < BP; b++) ps[b] = 0.f;
     for (uint64_t i = threadIdx.x; i < k; i += blockDim.x) {
         gs[i] = nscale[i];
-        if (NORM == 1) bs[i] = nbias ? nbias[i] : 0.f;
+        if (NORM == 1 || NORM == 4) bs[i] = nbias ? nbias[i] : 0.f;
         if (NORM == 3) bs[i] = post.ls ? post.ls[i] : 1.0f;
 #pragma unroll
         for (int b = 0; b < BP; b++)
@@ -1046,8 +1046,16 @@ __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__rest
             for (uint32_t w = 0; w < nwaves; w++) tot += red[w * BP + lane];
         return tot;
     };
-    if (NORM == 1) {
-        const float tot = finish(ps);
+    // NORM == 4: one mean and variance over all rows (wave 0, lanes 0 .. BP - 1 hold the rows' sums)
+    auto all_rows = [&](float t) {
+        float sum = 0.f;
+#pragma unroll
+        for (int b = 0; b < BP; b++) sum += b < (int)batch ? __shfl(t, b, 64) : 0.f;
+        return sum / (float)batch;
+    };
+    if (NORM == 1 || NORM == 4) {
+        float tot = finish(ps);
+        if (NORM == 4) tot = all_rows(tot);
         if (wave == 0 && lane < BP) stat[lane] = tot / (float)k;
         __syncthreads();
     } else if (threadIdx.x < BP) {
@@ -1055,7 +1063,7 @@ __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__rest
     }
 #pragma unroll
     for (int b = 0; b < BP; b++) ps[b] = 0.f;
-    if (NORM >= 2) __syncthreads();  // the rows and the zero means are in LDS
+    if (NORM == 2 || NORM == 3) __syncthreads();  // the rows and the zero means are in LDS
     for (uint64_t i = threadIdx.x; i < k; i += blockDim.x)
 #pragma unroll
         for (int b = 0; b < BP; b++)
@@ -1064,12 +1072,13 @@ __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__rest
                 ps[b] = fmaf(d, d, ps[b]);
             }
     {
-        const float tot = finish(ps);
+        float tot = finish(ps);
+        if (NORM == 4) tot = all_rows(tot);
         if (wave == 0 && lane < BP) stat[16 + lane] = sqrtf(tot / (float)k + eps);
         __syncthreads();
     }
     for (uint64_t i = threadIdx.x; i < k; i += blockDim.x) {
-        const float g = gs[i], bi = NORM == 1 ? bs[i] : 0.f;
+        const float g = gs[i], bi = NORM == 1 || NORM == 4 ? bs[i] : 0.f;
 #pragma unroll
         for (int b = 0; b < BP; b++)
             if (b < (int)batch) {
@@ -1376,6 +1385,11 @@ struct SplitRows {  // bf16 weights: three pieces
 #pragma unroll
         for (int j = 0; j < 3; j++) at(j, b)[i] = (uint16_t)s.p[j];
     }
+    __device__ void put4(uint32_t b, uint32_t i, const float4_t &v) const {
+        const Split2 lo = split2(v[0], v[1]), hi = split2(v[2], v[3]);
+#pragma unroll
+        for (int j = 0; j < 3; j++) *(uint2 *)(at(j, b) + i) = make_uint2(lo.p[j], hi.p[j]);
+    }
     __device__ void put2(uint32_t b, uint32_t i, float2 v) const {
         const Split2 s = split2(v.x, v.y);
 #pragma unroll
@@ -1388,6 +1402,7 @@ struct PlainRows {  // f32 weights
     static constexpr size_t bytes(size_t rows, size_t k) { return rows * (k + 4) * 4; }
     __device__ float *at(int, uint32_t b) const { return p + b * (k + 4); }
     __device__ void put(uint32_t b, uint32_t i, float v) const { at(0, b)[i] = v; }
+    __device__ void put4(uint32_t b, uint32_t i, const float4_t &v) const { *(float4_t *)(at(0, b) + i) = v; }
 };
 // What the two weight types do differently.  bf16: 64 k per 128 bytes of a row, activations in three pieces; f32: 32 k,
 // four 16x16x4 products per 16-byte piece.
@@ -1583,6 +1598,84 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
     }
 }
 
+// The staging of a folded norm for mfma_rows: wave b normalises row b in its registers (16 bytes of every 256 elements a
+// lane, k <= 256 VM) and puts it into LDS split.  stage_normed_rows spreads every row over all waves, a trip through
+// LDS and a barrier for each of two sums and a chain of 16 reads behind them: 13.9 us for a folded launch of 8 rows of
+// 768 x 2304 in f32, whose product alone takes 4.3.
+template <int NORM, int VM, class Rows>
+__device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__restrict__ x, uint32_t k, uint32_t batch,
+                                                   const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
+                                                   uint64_t ldx, const PostNorm &post, const Rows &xs) {
+    const uint32_t lane = threadIdx.x & 63, b = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n4 = k / 4;
+    const bool on = b < batch;
+    const float *row = NORM == 3 ? post.y + (uint64_t)b * k : x + (uint64_t)b * ldx;
+    auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
+    float4_t v[VM], g[VM];
+    if (on) {
+#pragma unroll
+        for (int u = 0; u < VM; u++) v[u] = *(const float4_t *)(row + 4 * min(lane + 64 * u, n4 - 1));
+#pragma unroll
+        for (int u = 0; u < VM; u++) g[u] = *(const float4_t *)(nscale + 4 * min(lane + 64 * u, n4 - 1));
+    }
+    float mean = 0.f;
+    if (NORM == 1 || NORM == 4) {
+        float sum = 0.f;
+        if (on) {
+#pragma unroll
+            for (int u = 0; u < VM; u++) sum += lane + 64 * u < n4 ? (v[u][0] + v[u][1]) + (v[u][2] + v[u][3]) : 0.f;
+            sum = row_sum(sum);
+        }
+        if (NORM == 4) {
+            if (lane == 0) sh[b] = sum;
+            __syncthreads();
+            sum = 0.f;
+            for (uint32_t w = 0; w < batch; w++) sum += sh[w];
+            sum /= (float)batch;
+        }
+        mean = sum / (float)k;
+    }
+    float sq = 0.f;
+    if (on) {
+#pragma unroll
+        for (int u = 0; u < VM; u++)
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const float d = lane + 64 * u < n4 ? v[u][t] - mean : 0.f;
+                sq = fmaf(d, d, sq);
+            }
+        sq = row_sum(sq);
+    }
+    if (NORM == 4) {
+        if (lane == 0) sh[16 + b] = sq;
+        __syncthreads();
+        sq = 0.f;
+        for (uint32_t w = 0; w < batch; w++) sq += sh[16 + w];
+        sq /= (float)batch;
+    }
+    if (!on) return;
+    const float rs = 1.0f / sqrtf(sq / (float)k + eps);
+#pragma unroll
+    for (int u = 0; u < VM; u++) {
+        const uint32_t i = 4 * (lane + 64 * u);
+        if (i >= k) continue;
+        float4_t o;
+        if (NORM == 3) {
+            const float4_t h = *(const float4_t *)(x + (uint64_t)b * ldx + i);
+            float4_t ls = {1.f, 1.f, 1.f, 1.f};
+            if (post.ls) ls = *(const float4_t *)(post.ls + i);
+#pragma unroll
+            for (int t = 0; t < 4; t++) o[t] = fmaf(v[u][t] * rs * g[u][t], ls[t], h[t]);
+            if (blockIdx.x == 0) *(float4_t *)(post.h_out + (uint64_t)b * k + i) = o;
+        } else {
+            float4_t bi = {0.f, 0.f, 0.f, 0.f};
+            if (NORM != 2 && nbias) bi = *(const float4_t *)(nbias + i);
+#pragma unroll
+            for (int t = 0; t < 4; t++) o[t] = g[u][t] * (v[u][t] - mean) * rs + bi[t];
+        }
+        xs.put4(b, i, o);
+    }
+}
+
 // NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
 template <bool BF16, int BP, int NORM, int PD, bool KEEP>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
@@ -1597,8 +1690,11 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType
     uint4 *corners = NORM ? (uint4 *)((char *)mlds + Rows::bytes(BP, k)) : mlds;
     mfma_rows<BF16, PD, KEEP, XQ>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
         if constexpr (NORM != 0) {
-            stage_normed_rows<BP, NORM>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post,
-                                        [&](uint32_t b, uint32_t i, float v) { xs.put(b, i, v); });
+            if (k <= 1024) stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
+            else if (k <= 2048) stage_rows_by_wave<NORM, 8>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
+            else
+                stage_normed_rows<BP, NORM>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post,
+                                            [&](uint32_t b, uint32_t i, float v) { xs.put(b, i, v); });
             __syncthreads();
         }
     });
@@ -1630,6 +1726,15 @@ static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves) {
 static uint32_t gemv_mfma_waves(uint64_t pairs) { return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (pairs + 1) / 2)); }
 bool gemv_takes_f32_rows(const Weight &w, uint64_t rows) {
     return w.dtype == COEUS_W_F32 && rows <= 16 && gemv_uses_mfma(w, rows, gemv_mfma_waves(w.k / 32));
+}
+static size_t gemv_mfma_norm_lds(const Weight &w, uint32_t bp, size_t staging) {
+    const bool bf = w.dtype == COEUS_W_BF16;
+    return (bf ? SplitRows::bytes(bp, w.k) : PlainRows::bytes(bp, w.k)) + std::max((size_t)16 * 16 * 128, staging);
+}
+bool gemv_can_fuse_whole_norm(const Weight &w, uint64_t batch) {
+    if (w.dtype != COEUS_W_F32 || batch < 2 || batch > 16 || !gemv_can_fuse_norm_dense(w, batch) || !gemv_uses_mfma(w, batch, 16)) return false;
+    const uint32_t bp = pad_batch(batch);
+    return gemv_mfma_norm_lds(w, bp, gemv_dense_norm_lds(w.k, bp)) <= 160 * 1024;
 }
 static size_t gemv_dense_post_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)bp * k * 4; }
 bool gemv_can_fuse_post_norm(const Weight &w, uint64_t batch) {
@@ -1962,13 +2067,16 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     const uint32_t waves = nf ? 16 : 4;
     const dim3 grid((unsigned)ceil_div(w.n, waves)), block(waves * 64);
     const size_t lds = !nf ? 0 : post_norm ? gemv_dense_post_lds(w.k, bp) : gemv_dense_norm_lds(w.k, bp);
-    const int norm = !nf ? 0 : post_norm ? 3 : nf->kind == COEUS_NORM_RMSNORM ? 2 : 1;
+    const int norm = !nf ? 0 : post_norm ? 3 : nf->whole ? 4 : nf->kind == COEUS_NORM_RMSNORM ? 2 : 1;
+    if (norm == 4 && (!gemv_can_fuse_whole_norm(w, batch) || nf->kind != COEUS_NORM_LAYERNORM))
+        return fail(COEUS_INVALID_INPUT, "a folded norm over all rows needs f32 weights, 2 to 16 rows and room in LDS");
     const uint64_t ldx = nf && nf->ld ? nf->ld : w.k;
     const PostNorm post = post_norm ? PostNorm{nf->y, nf->ls, nf->h_out} : PostNorm{nullptr, nullptr, nullptr};
     const float *xin = nf ? nf->h : x;
     const float *ns = nf ? nf->scale : nullptr, *nb = nf ? nf->bias : nullptr;
     const float eps = nf ? nf->eps : 0.f;
-    const bool aligned = (((uintptr_t)xin | (uintptr_t)ns | (uintptr_t)nb) & 15) == 0;  // 16-byte loads
+    // 16-byte loads
+    const bool aligned = (((uintptr_t)xin | (uintptr_t)ns | (uintptr_t)nb | (uintptr_t)post.y | (uintptr_t)post.ls | (uintptr_t)post.h_out | (nf ? ldx * 4 : 0)) & 15) == 0;
     // (up to 1024 elements: a wave's registers hold the row, its scale and bias and four weight rows)
     if (bp == 1 && (norm == 1 || norm == 2) && aligned && w.k % 8 == 0 && w.k <= 1024 && w.n < (1ull << 31) - 64) {
 #define COEUS_ROW(SV, RMSV) hipLaunchKernelGGL((gemv_row_kernel<BF16, RMSV, SV, kRowR>), dim3((unsigned)ceil_div(w.n, 4 * kRowR)), dim3(256), 0, st, w.data, xin, (uint32_t)w.k, ns, nb, eps, e)
@@ -1984,7 +2092,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         const uint32_t pairs = (uint32_t)std::min<uint64_t>(w.k / MfmaType<BF16>::KU, 1u << 20), mw = nf ? 16u : gemv_mfma_waves(pairs);
         const uint32_t xbp = std::max(bp, 4u), xq = nf ? 0 : (xbp + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
         const size_t corners = (size_t)mw * 16 * mfma_wave_lds<BF16>(xq),
-                     mlds = nf ? MfmaType<BF16>::Rows::bytes(bp, w.k) + std::max(corners, lds) : corners;
+                     mlds = nf ? gemv_mfma_norm_lds(w, bp, lds) : corners;
         if (aligned && !(nf && batch == 1) && gemv_uses_mfma(w, batch, nf ? 16 : mw) && mlds <= 160 * 1024) {
             const uint32_t tiles = (uint32_t)ceil_div(w.n, 16), np = (pairs + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
@@ -1995,7 +2103,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         hipLaunchKernelGGL((gemv_mfma_kernel<BF16, BPV, NV, PV, KV>), mgrid, mblock, mlds, st, (const typename MfmaType<BF16>::W *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
     } while (0)
 #define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (np % 3 == 0 || np == 5) COEUS_MFMA4(BPV, NV, 3, false); else COEUS_MFMA4(BPV, NV, 4, false); } while (0)
-#define COEUS_MFMA(BPV) do { if (norm == 1) COEUS_MFMA3(BPV, 1); else if (norm == 2) COEUS_MFMA3(BPV, 2); else COEUS_MFMA3(BPV, 3); } while (0)
+#define COEUS_MFMA(BPV) do { if (norm == 4) { if constexpr (!BF16) COEUS_MFMA3(BPV, 4); } else if (norm == 1) COEUS_MFMA3(BPV, 1); else if (norm == 2) COEUS_MFMA3(BPV, 2); else COEUS_MFMA3(BPV, 3); } while (0)
             constexpr int P8 = BF16 ? 2 : 4;  // (bf16, 8 rows: four pairs do not fit the registers)
             if (norm == 0 && bp <= 4) COEUS_MFMA3(4, 0);
             else if (norm == 0 && bp == 8 && np <= 2) COEUS_MFMA4(8, 0, 2, true);
@@ -2014,6 +2122,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
             return COEUS_OK;
         }
     }
+    if (norm == 4) return fail(COEUS_INVALID_INPUT, "a folded norm over all rows needs its vectors on 16-byte boundaries");
 #define COEUS_GEMVD2(BPV, NV) \
     hipLaunchKernelGGL((gemv_dense_kernel<BF16, BPV, NV>), grid, block, lds, st, w.data, xin, w.k, b, e, ns, nb, eps, ldx, post)
 #define COEUS_GEMVD(BPV) \

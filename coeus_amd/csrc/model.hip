@@ -342,24 +342,40 @@ int run_blocks_prefill(Model &m, Workspace &ws, const Cache &cache, uint64_t bat
     const LpOut x_lp{ws.a_lp.p, gemm_ld(H), lp_bf};
     const LpOut att_lp{ws.b_lp.p, gemm_ld(m.L.inner_dim), lp_bf};
     const LpOut ff_lp{ws.b_lp.p, gemm_ld(c.intermediate_dim), lp_bf};
+    // A prompt of a few rows on f32 weights: its matmuls are the decode kernel's, with the norms in front folded in and
+    // the cache rows written by the q|k|v epilogue (5 rows of the 250M model: 6.3 us per norm launch, 2.6 us per append).
+    const bool whole = c.norm_scope == COEUS_SCOPE_SEQUENCE;
+    auto folds = [&](const Weight &w) {
+        return whole ? c.norm == COEUS_NORM_LAYERNORM && gemv_can_fuse_whole_norm(w, rows) : gemv_can_fuse_norm_dense(w, rows);
+    };
+    const bool few = gemv_takes_f32_rows(m.layers[0].qkv, rows) && gemv_takes_f32_rows(m.layers[0].up, rows) && folds(m.layers[0].qkv) &&
+                     folds(m.layers[0].up);
+    auto normed = [&](const Weight &w, const float *ns, const float *nb, const Epilogue &e) -> int {
+        if (few) {
+            NormFuse nf;
+            nf.h = h; nf.scale = ns; nf.bias = nb; nf.eps = c.layer_norm_eps; nf.kind = c.norm; nf.whole = whole;
+            return launch_gemv(w, nullptr, rows, e, st, &nf);
+        }
+        COEUS_TRY(launch_norm(c.norm, c.norm_scope, h, rows, H, ns, nb, c.layer_norm_eps, lp ? nullptr : x, nullptr, 0, st,
+                              lp ? &x_lp : nullptr, (double *)ws.norm_part.p));
+        return launch_gemm(w, lp ? (const void *)ws.a_lp.p : (const void *)x, rows, e, ws.gs, st, lp);
+    };
     for (uint64_t l = 0; l < c.num_layers; l++) {
         const LayerWeights &lw = m.layers[l];
         char *kc = (char *)cache.k + (cache.per_layer ? l * cache.layer_bytes : 0);
         char *vc = (char *)cache.v + (cache.per_layer ? l * cache.layer_bytes : 0);
         // h -> LN1 -> q|k|v (MT:469, MT:185-214)
-        COEUS_TRY(launch_norm(c.norm, c.norm_scope, h, rows, H, lw.ln1_s, lw.ln1_b, c.layer_norm_eps,
-                              lp ? nullptr : x, nullptr, 0, st, lp ? &x_lp : nullptr, (double *)ws.norm_part.p));
         Epilogue e1;
         e1.bias = lw.b_qkv; e1.out_f32 = qkv;
         // the matrix-core matmul writes the key and value thirds straight into the cache
-        const bool fused_append = gemm_appends_kv(lw.qkv, rows, m.L.inner_dim, hd);
+        const bool fused_append = few || gemm_appends_kv(lw.qkv, rows, m.L.inner_dim, hd);
         if (fused_append) {
             e1.kv_k = kc; e1.kv_v = vc; e1.kv_dtype = c.kv_dtype;
             e1.kv_inner = (uint32_t)m.L.inner_dim; e1.kv_heads = (uint32_t)c.num_heads;
             e1.kv_hd = (uint32_t)hd; e1.kv_max_ctx = (uint32_t)cache.max_ctx;
             e1.kv_rows_per_seq = (uint32_t)n; e1.kv_pos0 = (uint32_t)pos0;
         }
-        COEUS_TRY(launch_gemm(lw.qkv, lp ? (const void *)ws.a_lp.p : (const void *)x, rows, e1, ws.gs, st, lp));
+        COEUS_TRY(normed(lw.qkv, lw.ln1_s, lw.ln1_b, e1));
         if (!fused_append)
             COEUS_TRY(launch_kv_append(qkv, kc, vc, c.kv_dtype, batch, n, c.num_heads, hd, cache.max_ctx,
                                        pos0, nullptr, st));
@@ -371,13 +387,11 @@ int run_blocks_prefill(Model &m, Workspace &ws, const Cache &cache, uint64_t bat
         e2.bias = lw.b_o; e2.residual = h; e2.out_f32 = h;
         COEUS_TRY(launch_gemm(lw.o, attn_lp ? (const void *)ws.b_lp.p : (const void *)att, rows, e2, ws.gs, st, attn_lp));
         // LN2 -> FFN -> residual (MT:488-496, MT:339-375)
-        COEUS_TRY(launch_norm(c.norm, c.norm_scope, h, rows, H, lw.ln2_s, lw.ln2_b, c.layer_norm_eps,
-                              lp ? nullptr : x, nullptr, 0, st, lp ? &x_lp : nullptr, (double *)ws.norm_part.p));
         Epilogue e3;
         e3.bias = lw.b_up;
         if (lp) e3.out_lp = ff_lp; else e3.out_f32 = ff;
         e3.act = c.activation == COEUS_ACT_SILU_GATED ? COEUS_EPI_SILU_GATE : COEUS_EPI_GELU;
-        COEUS_TRY(launch_gemm(lw.up, lp ? (const void *)ws.a_lp.p : (const void *)x, rows, e3, ws.gs, st, lp));
+        COEUS_TRY(normed(lw.up, lw.ln2_s, lw.ln2_b, e3));
         Epilogue e4;
         e4.bias = lw.b_down; e4.residual = h; e4.out_f32 = h;
         COEUS_TRY(launch_gemm(lw.down, lp ? (const void *)ws.b_lp.p : (const void *)ff, rows, e4, ws.gs, st, lp));

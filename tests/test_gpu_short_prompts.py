@@ -1,0 +1,47 @@
+"""Prompts of 2 - 16 rows on f32 weights (the decode matmul with the norms folded in, per row or over all rows, and the
+cache rows from its epilogue) against the float64 model."""
+import numpy as np
+import pytest
+
+import f64_model
+from coeus_amd import Transformer250MConfig, TransformerModelPlugin
+
+pytestmark = pytest.mark.gpu
+
+
+def build(orc, **kw):
+    cfg = Transformer250MConfig(num_layers=2, num_heads=16, intermediate_dim=608, vocab_size=150, max_seq_len=40, **kw)
+    oc = orc.config_from_kwargs({k: getattr(cfg, k) for k in ("num_layers", "num_heads", "intermediate_dim", "vocab_size", "max_seq_len", *kw)})
+    params = orc.init_seeded(oc, 11)
+    return TransformerModelPlugin().create_builder().build(cfg, parameters=params), oc, params
+
+
+# 512: one chunk pair per wave; 768, 1024: registers of a wave full or not; 1088, 2080: the next size of the staging, and
+# rows too long for it
+@pytest.mark.parametrize("hidden", [512, 768, 1024, 1088, 2080])
+@pytest.mark.parametrize("scope", ["sequence", "token"])
+def test_forward_matches_float64(orc, hidden, scope):
+    model, oc, params = build(orc, hidden_dim=hidden, norm_scope=scope)
+    rng = np.random.default_rng(hidden)
+    for rows in (2, 3, 4, 5, 8, 9, 16, 17):
+        ids = rng.integers(0, 150, rows, dtype=np.uint64)
+        want = f64_model.forward_all(oc, params, ids)
+        got = model.forward_all(ids)
+        # f32 sums of up to 2080 terms over two layers; the sinusoidal table's f32 angles (1e-6 at these positions)
+        assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max(), rows
+
+
+@pytest.mark.parametrize("batch,n", [(1, 7), (3, 5), (16, 1), (2, 8)])
+@pytest.mark.parametrize("kv", ["f32", "bf16"])
+def test_session_cache_rows(orc, batch, n, kv):
+    """The rows that the epilogue wrote are read by the steps behind the prompt; a second prompt starts behind the first."""
+    model, oc, params = build(orc, hidden_dim=512, norm_scope="token", max_batch=16, kv_dtype=kv)
+    ids = np.random.default_rng(batch).integers(0, 150, (batch, 2 * n + 1), dtype=np.uint64)
+    s = model.session(batch=batch, max_ctx=36)
+    s.prefill(ids[:, :n], want_logits=False)
+    s.prefill(ids[:, n:2 * n], want_logits=False)
+    got = s.decode(ids[:, 2 * n])
+    tol = 2e-5 if kv == "f32" else 2e-2  # (bf16 keys and values: 2^-9 each)
+    for b in range(batch):
+        want = f64_model.forward_all(oc, params, ids[b])[-1]
+        assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), b
