@@ -635,7 +635,7 @@ static int check_attention_decode_args(const float *qkv_dev, const void *k, cons
         return fail(COEUS_INVALID_INPUT, "Sequence length %llu out of range [1, %llu]", (unsigned long long)ctx,
                     (unsigned long long)max_ctx);
     if (merge > COEUS_MERGE_SEPARATE) return fail(COEUS_INVALID_INPUT, "unknown merge mode %u", merge);
-    if (*nsplit == 0) *nsplit = attn_decode_splits(batch, heads, max_ctx);
+    if (*nsplit == 0) *nsplit = attn_decode_splits(batch, heads, hd, kv_dtype, max_ctx);
     if (*nsplit > 32) return fail(COEUS_INVALID_INPUT, "decode attention: %u splits out of range [1, 32]", *nsplit);
     return COEUS_OK;
 }

@@ -703,15 +703,22 @@ bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype) {
     return n >= 16 && (hd == 64 || hd == 128) && kv_dtype != COEUS_KV_F32;
 }
 
-uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t max_ctx) {
-    // Aim for one workgroup per CU, at least 128 keys per split.  Measured at context 4096 with 32
-    // heads of 128: batch 1, 8 splits 17.3 us against 17.8 with 16; batch 4, 2 splits 46.3 us
-    // against 49.0 with 8; batch 16, 1 split 182.7 us against 187.9 with 2 (fewer partial records
-    // to publish and merge; the kernel's two workgroups per CU stream at the same rate either way).
-    // A power of two: three splits of 2048 keys (704 + 704 + 640, the wave tiles no longer line up)
-    // ran 17.6 us at batch 8 x 12 heads of 64 against 14.0 us with four.
-    uint64_t want = ceil_div(256, batch * heads);
-    while (want & (want - 1)) want++;  // up to the next power of two
+uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t hd, uint32_t kv_dtype, uint64_t max_ctx) {
+    // More than one split costs its records' two trips through memory, 1.5 - 2 us.  So one split where a head's keys fit
+    // the requests of one workgroup: 64 KiB of them (512 keys of 64 in 16 bits), and 128 KiB with at least 64 workgroups
+    // to fill the memory pipeline.  us per launch, two splits or four / one: 8 x 12 heads of 64 at 201 keys 5.6 / 3.6, at
+    // 500 6.1 / 4.8, at 700 7.3 / 6.7; 32 heads of 128 at 256 5.9 / 5.0; 4 x 32 of 128 at 500 9.2 / 8.7; but 32 of
+    // 128 at 500 6.4 / 7.1, 48 of 64 at 960 6.7 / 7.4.
+    const uint64_t pairs = batch * heads, key_bytes = max_ctx * hd * (kv_dtype == COEUS_KV_F32 ? 4 : 2);
+    if (key_bytes <= (64u << 10) || (pairs >= 64 && key_bytes <= (128u << 10))) return 1;
+    // Else as many as fill the CUs with one workgroup each, a power of two: three splits of 2048 keys (704 + 704 + 640, the
+    // wave tiles no longer line up) ran 17.6 us at batch 8 x 12 heads of 64 against 14.0 us with four.  More than 128
+    // heads stay whole (us, two splits / one of eight waves: 5 x 32 heads of 128 at 700 / 2000 / 4000 keys 14.9 / 33.0 / 63.5
+    // against 11.4 / 28.8 / 53.3; 16 x 12 of 64 at 1000 / 2000 11.3 / 19.1 against 9.3 / 17.1; 4 x 32 of 128 at 2000 24.0 / 27.4).
+    // At context 4096 with 32 heads of 128, batch 1, 8 splits 17.3 us against 17.8 with 16.
+    if (pairs > 128) return 1;
+    uint64_t want = ceil_div(256, pairs);
+    while (want & (want - 1)) want++;
     // 256 keys per split, but 128 up to eight splits (us per launch, 256 / 128 keys: 32 heads of 128 at 520 keys 8.3 / 7.0,
     // at 1080 9.3 / 8.3; 12 heads of 64 at 560 5.9 / 5.3; at 2025, sixteen splits against eight, 7.3 / 6.3)
     uint64_t cap = ceil_div(max_ctx, 256);
@@ -740,24 +747,26 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
                         kAttnMaxSplits);
         const uint32_t kps = (uint32_t)round_up(ceil_div(max_ctx, nsplit), 64);
         const dim3 grid(nsplit, (unsigned)heads, (unsigned)batch);
-        // One workgroup per CU at most and splits of 512 keys or more: 8 waves per workgroup, a tile
-        // of 64 keys each at once, instead of 4 waves walking two tiles each (7B shape, batch 1,
-        // context 4096: 1.768 -> 1.759 ms per step over five alternations; with shorter splits the
-        // extra waves have nothing to take and the step is 0.5 % slower).
-        const bool wide = batch * heads * nsplit <= 256 && kps >= 512;
-        // TILE: wave loads kept in flight per phase, as many as the four waves need to take a split at once (a split of 128
-        // keys of 64 in 16 loads a wave is one wave's work; 12 heads of 64 at 560 keys: 6.1 -> 5.3 us).  f32: at most 8,
-        // half the keys per load (12 heads of 64 at 124 / 500 / 1000 keys, which attn_generic_kernel walks with one wave
-        // a head in 25 / 116 / 312 us: 3.2 / 5.5 / 5.9).
+        // TILE: wave loads kept in flight per phase, as many as the waves need to take a split at once (a split of 128 keys of
+        // 64 in 16 loads a wave is one wave's work; 12 heads of 64 at 560 keys: 6.1 -> 5.3 us).  f32: at most 8, half the
+        // keys per load (12 heads of 64 at 124 / 500 / 1000 keys, which attn_generic_kernel walks with one wave a head in
+        // 25 / 116 / 312 us: 3.2 / 5.5 / 5.9).
         const uint32_t epl = kv_dtype == COEUS_KV_F32 ? 4 : 8, kpl = 64 / ((uint32_t)hd / epl);
-        const uint32_t once = 4 * kpl;
-        const int tile = kps <= 4 * once ? 4 : kps <= 8 * once || kv_dtype == COEUS_KV_F32 ? 8 : 16;
+        const uint32_t most = kv_dtype == COEUS_KV_F32 ? 8 : 16;
+        // One workgroup per CU at most and splits that four waves would walk in two trips (or 512 keys, where the trip is full): 8
+        // waves (us per launch, 4 waves / 8: 6 x 32 heads of 128 at 330 keys whole 8.6 / 7.6, at 2 splits of 350 9.9 / 9.4; 12
+        // heads of 64 in f32 at 200 4.6 / 4.1; 7B shape, batch 1, context 4096: 1.768 -> 1.759 ms per step).  With
+        // shorter splits the extra waves have nothing to take and the step is 0.5 % slower.
+        const bool wide = batch * heads * nsplit <= 256 && (kps > 4 * most * kpl || kps >= 512);
+        const uint32_t once = (wide ? 8 : 4) * kpl;
+        const uint32_t tile = !wide && kps <= 4 * once ? 4 : kps <= 8 * once ? 8 : most;
 #define COEUS_AD3(HDV, KVV, NWV, TV)                                                               \
     hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV, NWV, TV>), grid, dim3(NWV * 64), 0, st, qkv,  \
                        kc, vc, (uint32_t)heads, (uint32_t)max_ctx, (uint32_t)pos0, pos_dev, kps,   \
                        part_scratch, counters, out, out_xq, bp)
 #define COEUS_AD(HDV, KVV) do {                                                                    \
-    if (wide) COEUS_AD3(HDV, KVV, 8, (KVV == COEUS_KV_F32 ? 8 : 16));                              \
+    if (wide && tile == 8) COEUS_AD3(HDV, KVV, 8, 8);                                              \
+    else if (wide) COEUS_AD3(HDV, KVV, 8, (KVV == COEUS_KV_F32 ? 8 : 16));                         \
     else if (tile == 4) COEUS_AD3(HDV, KVV, 4, 4);                                                 \
     else if (tile == 8) COEUS_AD3(HDV, KVV, 4, 8);                                                 \
     else COEUS_AD3(HDV, KVV, 4, (KVV == COEUS_KV_F32 ? 8 : 16)); } while (0)

@@ -323,7 +323,7 @@ int launch_sample(const float *logits, uint64_t rows, uint64_t vocab, const coeu
 int launch_kv_append(const float *qkv, void *kc, void *vc, uint32_t kv_dtype, uint64_t batch,
                      uint64_t n, uint64_t heads, uint64_t hd, uint64_t max_ctx, uint64_t pos0,
                      const uint32_t *pos_dev, hipStream_t st);
-uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t max_ctx);
+uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t hd, uint32_t kv_dtype, uint64_t max_ctx);
 // True when n new rows per sequence take the matrix-core prefill kernel (which can write 16-bit
 // output rows) rather than the generic one.
 bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype);

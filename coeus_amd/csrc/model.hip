@@ -531,7 +531,7 @@ int session_create(Model &m, uint64_t batch, uint64_t max_ctx, Session **out) {
     COEUS_TRY(s->dids.ensure(batch * 8));
     COEUS_TRY(s->dpos.ensure(64));
     COEUS_TRY(s->dhist.ensure(batch * max_ctx * 8));
-    s->nsplit = attn_decode_splits(batch, c.num_heads, max_ctx);
+    s->nsplit = attn_decode_splits(batch, c.num_heads, hd, c.kv_dtype, max_ctx);
     COEUS_TRY(s->dpart.ensure(batch * c.num_heads * s->nsplit * (hd + 2) * 4));
     COEUS_TRY(s->dcount.ensure(batch * c.num_heads * 4));
     COEUS_HIP(hipMemset(s->dcount.p, 0, s->dcount.bytes));

@@ -16,7 +16,7 @@ def test_steps_match_prompt_pass(heads, hd, max_ctx, kv):
                                 max_seq_len=max_ctx, norm_scope="token", max_batch=3, kv_dtype=kv)
     model = TransformerModelPlugin().create_builder().build(cfg, seed=5)
     rng = np.random.default_rng(max_ctx + hd)
-    # 32 (16) keys of 64 (128) a wave, four or eight waves, splits of 64 or 256 and more keys
+    # 16-bit: 32 - 128 (16 - 64) keys of 64 (128) a wave, four or eight waves, one split or several of 64 keys and more
     for ctx in (1, 2, 31, 32, 33, 64, 127, 128, 129, 255, 257, 512, 513, 1025, 2049, max_ctx):
         if ctx > max_ctx:
             continue
@@ -32,3 +32,21 @@ def test_steps_match_prompt_pass(heads, hd, max_ctx, kv):
             # prompt pass also rounds queries and weights of the softmax to the cache's type, 2^-11 and 2^-8 relative
             tol = {"f32": 2e-5, "f16": 2e-3, "bf16": 1.6e-2}[kv]
             assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), (ctx, b)
+
+
+@pytest.mark.parametrize("heads,hd,max_ctx", [(4, 64, 1024), (4, 64, 1025), (4, 128, 512), (8, 64, 1030), (9, 64, 1500), (9, 128, 700)])
+@pytest.mark.parametrize("kv", ["f32", "f16"])
+def test_many_heads_match_prompt_pass(heads, hd, max_ctx, kv):
+    # 16 sequences: 64 heads and up to 128 KiB of keys a head whole, 64 - 128 heads split beyond that, more than 128 whole
+    cfg = Transformer250MConfig(hidden_dim=heads * hd, num_layers=1, num_heads=heads, intermediate_dim=256, vocab_size=160,
+                                max_seq_len=max_ctx, norm_scope="token", max_batch=16, kv_dtype=kv)
+    model = TransformerModelPlugin().create_builder().build(cfg, seed=6)
+    ids = np.random.default_rng(max_ctx).integers(0, cfg.vocab_size, (16, max_ctx), dtype=np.uint64)
+    s = model.session(batch=16, max_ctx=max_ctx)
+    s.prefill(ids[:, :-1], want_logits=False)
+    got = s.decode(ids[:, -1])
+    s.close()
+    tol = {"f32": 2e-5, "f16": 2e-3}[kv]  # as above
+    for b in (0, 7, 15):
+        want = model.forward(ids[b])
+        assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), b
