@@ -17,6 +17,10 @@
 //                      fragment with all four.  In both kernels the value used for every weight is
 //                      exactly its dequantised value q*d.
 //   gemv_dense_kernel  f32 / bf16 weights, one wave per output row, f32 FMA on the VALU.
+//   gemv_row_kernel    one activation row behind a norm of up to 1024 elements: the row in every
+//                      wave's registers, no LDS and no barrier.
+//   gemv_mfma_kernel   2 - 16 activation rows on f32 / bf16 weights: 16 output rows a workgroup on
+//                      the matrix cores (bf16: the f32 activations as three bf16 each).
 #include "device_utils.hpp"
 
 namespace coeus {
