@@ -2022,7 +2022,9 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
         nf.bias || (nf.y && (!nf.h_out || nf.h_out == nf.h)))
         return fail(COEUS_INVALID_INPUT, "folded hyper-connections: bad arguments or too many streams");
     const uint32_t bp = pad_batch(batch), b = (uint32_t)batch, k = (uint32_t)w.k, nit = hyper_pairs(w.k);
-    const bool mf = BF16 && nit == 1 && gemv_uses_mfma(w, batch, 16);
+    // (the matrix-core instances lay their LDS out for two or four rows: one row stays with a wave per weight row, also where
+    // gemv_uses_mfma takes one row of a plain launch)
+    const bool mf = BF16 && nit == 1 && bp >= 2 && gemv_uses_mfma(w, batch, 16);
     const size_t lds = mf ? 16 * 16 * mfma_wave_lds<true>(0) + SplitRows::bytes(bp, k) : (size_t)bp * k * 4;
     const uint32_t bs = b | nf.streams << 16;
     const HyperFold *fold = (const HyperFold *)nf.fold;
