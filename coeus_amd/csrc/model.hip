@@ -195,17 +195,21 @@ int model_create(const coeus_config &cfg, const float *params, uint64_t n_params
 
     // ---- small parameters (norm scales/biases, linear biases), assembled on the host
     const uint64_t up_rows = gated ? 2 * I : I;
-    const uint64_t per_layer = 2 * H + 3 * inner + H + 2 * H + up_rows + H;
-    std::vector<float> sm(cfg.num_layers * per_layer + 2 * H, 0.0f);
+    // Every vector starts on 16 bytes, whatever the sizes: the kernels that take a norm into a matmul load its scale
+    // and bias in 16-byte pieces (and a whole-slice norm has no other form there).
+    uint64_t per_layer = 0;
+    auto place = [&](uint64_t count) { const uint64_t at = per_layer; per_layer += round_up(count, 4); return at; };
+    const uint64_t ln1_s = place(H), ln1_b = place(H), b_qkv = place(3 * inner), b_o = place(H), ln2_s = place(H), ln2_b = place(H),
+                   b_up = place(up_rows), b_down = place(H);
+    std::vector<float> sm(cfg.num_layers * per_layer + 2 * round_up(H, 4), 0.0f);
     for (uint64_t l = 0; l < cfg.num_layers; l++) {
         const uint64_t base = L.first_layer_offset + l * L.layer_stride;
         float *d = sm.data() + l * per_layer;
-        for (uint64_t i = 0; i < H; i++) d[i] = value(base + L.ln1_scale + i, 1.0f);
-        for (uint64_t i = 0; i < H; i++) d[H + i] = value(base + L.ln1_bias + i, 0.0f);
-        float *bqkv = d + 2 * H, *bo = bqkv + 3 * inner, *ln2 = bo + H, *bup = ln2 + 2 * H,
-              *bdown = bup + up_rows;
-        for (uint64_t i = 0; i < H; i++) ln2[i] = value(base + L.ln2_scale + i, 1.0f);
-        for (uint64_t i = 0; i < H; i++) ln2[H + i] = value(base + L.ln2_bias + i, 0.0f);
+        for (uint64_t i = 0; i < H; i++) d[ln1_s + i] = value(base + L.ln1_scale + i, 1.0f);
+        for (uint64_t i = 0; i < H; i++) d[ln1_b + i] = value(base + L.ln1_bias + i, 0.0f);
+        float *bqkv = d + b_qkv, *bo = d + b_o, *bup = d + b_up, *bdown = d + b_down;
+        for (uint64_t i = 0; i < H; i++) d[ln2_s + i] = value(base + L.ln2_scale + i, 1.0f);
+        for (uint64_t i = 0; i < H; i++) d[ln2_b + i] = value(base + L.ln2_bias + i, 0.0f);
         if (bias) {
             for (uint64_t i = 0; i < inner; i++) {
                 bqkv[i] = value(base + L.bq + i, 0.0f);
@@ -227,7 +231,7 @@ int model_create(const coeus_config &cfg, const float *params, uint64_t n_params
     {
         float *d = sm.data() + cfg.num_layers * per_layer;
         for (uint64_t i = 0; i < H; i++) d[i] = value(L.final_ln_offset + i, 1.0f);
-        for (uint64_t i = 0; i < H; i++) d[H + i] = value(L.final_ln_offset + H + i, 0.0f);
+        for (uint64_t i = 0; i < H; i++) d[round_up(H, 4) + i] = value(L.final_ln_offset + H + i, 0.0f);
     }
     COEUS_HIP(hipMalloc((void **)&m->small, sm.size() * 4));
     COEUS_HIP(hipMemcpy(m->small, sm.data(), sm.size() * 4, hipMemcpyHostToDevice));
@@ -239,12 +243,12 @@ int model_create(const coeus_config &cfg, const float *params, uint64_t n_params
         const uint64_t base = L.first_layer_offset + l * L.layer_stride;
         LayerWeights &lw = m->layers[l];
         const float *d = m->small + l * per_layer;
-        lw.ln1_s = d; lw.ln1_b = d + H;
-        lw.b_qkv = bias ? d + 2 * H : nullptr;
-        lw.b_o = bias ? d + 2 * H + 3 * inner : nullptr;
-        lw.ln2_s = d + 2 * H + 3 * inner + H; lw.ln2_b = lw.ln2_s + H;
-        lw.b_up = bias ? lw.ln2_b + H : nullptr;
-        lw.b_down = bias ? lw.ln2_b + H + up_rows : nullptr;
+        lw.ln1_s = d + ln1_s; lw.ln1_b = d + ln1_b;
+        lw.b_qkv = bias ? d + b_qkv : nullptr;
+        lw.b_o = bias ? d + b_o : nullptr;
+        lw.ln2_s = d + ln2_s; lw.ln2_b = d + ln2_b;
+        lw.b_up = bias ? d + b_up : nullptr;
+        lw.b_down = bias ? d + b_down : nullptr;
         WeightSource src;
         src.params = dev_params;
         src.seed = seed;
@@ -267,7 +271,7 @@ int model_create(const coeus_config &cfg, const float *params, uint64_t n_params
         for (const Weight *w : {&lw.qkv, &lw.o, &lw.up, &lw.down}) COEUS_TRY(weight_expand(*w, &m->expand_budget, st));
     }
     m->fin_s = m->small + cfg.num_layers * per_layer;
-    m->fin_b = m->fin_s + H;
+    m->fin_b = m->fin_s + round_up(H, 4);
     {
         WeightSource src;
         src.params = dev_params; src.seed = seed;

@@ -10,8 +10,9 @@ pytestmark = pytest.mark.gpu
 
 
 def build(orc, **kw):
-    cfg = Transformer250MConfig(num_layers=2, num_heads=16, intermediate_dim=608, vocab_size=150, max_seq_len=40, **kw)
-    oc = orc.config_from_kwargs({k: getattr(cfg, k) for k in ("num_layers", "num_heads", "intermediate_dim", "vocab_size", "max_seq_len", *kw)})
+    kw = {"num_layers": 2, "num_heads": 16, "intermediate_dim": 608, **kw}
+    cfg = Transformer250MConfig(vocab_size=150, max_seq_len=40, **kw)
+    oc = orc.config_from_kwargs({k: getattr(cfg, k) for k in ("vocab_size", "max_seq_len", *kw)})
     params = orc.init_seeded(oc, 11)
     return TransformerModelPlugin().create_builder().build(cfg, parameters=params), oc, params
 
@@ -45,3 +46,17 @@ def test_session_cache_rows(orc, batch, n, kv):
     for b in range(batch):
         want = f64_model.forward_all(oc, params, ids[b])[-1]
         assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), b
+
+
+# biases of a layer whose lengths are no multiple of four: behind them no vector starts on 16 bytes unless it is padded
+@pytest.mark.parametrize("scope", ["sequence", "token"])
+@pytest.mark.parametrize("kw", [dict(intermediate_dim=770), dict(intermediate_dim=609), dict(intermediate_dim=609, activation="silu_gated"),
+                                dict(num_heads=3, head_dim=21), dict(num_heads=3, head_dim=21, intermediate_dim=611, use_bias=False)])
+def test_vectors_behind_odd_lengths(orc, kw, scope):
+    model, oc, params = build(orc, hidden_dim=512, num_layers=3, norm_scope=scope, **kw)
+    rng = np.random.default_rng(len(kw))
+    for rows in (1, 2, 5, 16, 17):
+        ids = rng.integers(0, 150, rows, dtype=np.uint64)
+        want = f64_model.forward_all(oc, params, ids)
+        got = model.forward_all(ids)
+        assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max(), rows  # (as above)
