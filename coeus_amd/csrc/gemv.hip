@@ -1006,24 +1006,39 @@ struct PostNorm {
     const float *y, *ls;
     float *h_out;
 };
+// 1 / standard deviation of a whole-slice norm, rounded once: the f32 value and a Newton step in f64 (a square root and a
+// division in f64 would spill the rows that wait in registers).
+__device__ __forceinline__ float whole_norm_rs(double var, float eps) {
+    const double v = var + (double)eps;
+    const float r = 1.0f / sqrtf((float)v);
+    const double d = r;
+    return r > 0.f && r < INFINITY ? (float)(d * fma(-0.5 * v * d, d, 1.5)) : r;
+}
+// 1 / n to 2^-46, in the registers that a wave has left (see above)
+__device__ __forceinline__ double inv_count(uint32_t n) {
+    const double r = 1.0f / (float)n;
+    return fma(fma(-(double)n, r, 1.0), r, r);
+}
 // The staging of NORM 1 - 4: rows of x (see above; 4: LayerNorm over all rows together) -> normalised f32 values, element i of row b handed to put(b, i, v)
 // (which may write it to xn + b k + i).  Every wave of the workgroup takes part; the last barrier is the caller's.  LDS
 // at xn: [BP][k] rows, [2][k] scale and bias, partial sums, statistics (NORM == 3: then [BP][k] residual rows).
+// The sums of NORM 4 are carried in f64, as where that norm is a launch of its own (norm_sequence_kernel).
 template <int BP, int NORM, class Put>
 __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__restrict__ x, uint64_t k, uint32_t batch,
                                                   const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
                                                   uint64_t ldx, const PostNorm &post, Put put) {
+    typedef typename std::conditional<NORM == 4, double, float>::type Sum;
     const uint32_t ld = (uint32_t)k;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
     // One trip to memory: the rows, the scale and the bias all go to LDS first; the two
     // statistics passes and the normalisation then work from there.
     float *gs = xn + (size_t)BP * ld, *bs = gs + k;  // scale, bias
-    float *red = bs + k;                            // [16 waves][BP] partial sums
-    float *stat = red + 16 * BP;                    // [0][b] mean, [1][b] standard deviation
+    Sum *red = (Sum *)(bs + k);                     // [16 waves][BP] partial sums (NORM 4: k is a multiple of 32)
+    float *stat = (float *)(red + 16 * BP);         // [0][b] mean, [1][b] standard deviation (NORM 4: its reciprocal)
     float *hs = stat + 32;                          // NORM == 3: [BP][k] residual rows
-    float ps[BP];
+    Sum ps[BP], mean = 0;                           // (mean: NORM 4, unrounded)
 #pragma unroll
-    for (int b = 0; b < BP; b++) ps[b] = 0.f;
+    for (int b = 0; b < BP; b++) ps[b] = 0;
     for (uint64_t i = threadIdx.x; i < k; i += blockDim.x) {
         gs[i] = nscale[i];
         if (NORM == 1 || NORM == 4) bs[i] = nbias ? nbias[i] : 0.f;
@@ -1037,47 +1052,51 @@ __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__rest
                 ps[b] += v;
             }
     }
-    // every wave's partial per row -> wave 0 finishes row b = lane
-    auto finish = [&](float (&p)[BP]) -> float {
+    // every wave's partial per row -> wave 0 finishes row b = lane; NORM 4: every wave finishes all rows together
+    auto finish = [&](Sum (&p)[BP]) -> Sum {
 #pragma unroll
         for (int b = 0; b < BP; b++) {
-            const float t = wave_sum(p[b]);
+            Sum t;
+            if constexpr (NORM == 4) t = wave_sum_f64(p[b]);
+            else t = wave_sum(p[b]);
             if (lane == 0) red[wave * BP + b] = t;
         }
         __syncthreads();
-        float tot = 0.f;
-        if (wave == 0 && lane < BP)
+        Sum tot = 0;
+        if (NORM == 4) {
+            for (uint32_t i = lane; i < nwaves * BP; i += 64) tot += red[i];  // (zero for the rows that are not there)
+            tot = wave_sum_f64(tot);
+            __syncthreads();  // (red is written again)
+        } else if (wave == 0 && lane < BP) {
             for (uint32_t w = 0; w < nwaves; w++) tot += red[w * BP + lane];
+        }
         return tot;
     };
-    // NORM == 4: one mean and variance over all rows (wave 0, lanes 0 .. BP - 1 hold the rows' sums)
-    auto all_rows = [&](float t) {
-        float sum = 0.f;
-#pragma unroll
-        for (int b = 0; b < BP; b++) sum += b < (int)batch ? __shfl(t, b, 64) : 0.f;
-        return sum / (float)batch;
-    };
-    if (NORM == 1 || NORM == 4) {
-        float tot = finish(ps);
-        if (NORM == 4) tot = all_rows(tot);
+    if (NORM == 4) {
+        mean = finish(ps) * inv_count((uint32_t)k * batch);
+    } else if (NORM == 1) {
+        const Sum tot = finish(ps);
         if (wave == 0 && lane < BP) stat[lane] = tot / (float)k;
         __syncthreads();
     } else if (threadIdx.x < BP) {
         stat[threadIdx.x] = 0.f;  // a root-mean-square norm subtracts no mean
     }
 #pragma unroll
-    for (int b = 0; b < BP; b++) ps[b] = 0.f;
+    for (int b = 0; b < BP; b++) ps[b] = 0;
     if (NORM == 2 || NORM == 3) __syncthreads();  // the rows and the zero means are in LDS
     for (uint64_t i = threadIdx.x; i < k; i += blockDim.x)
 #pragma unroll
         for (int b = 0; b < BP; b++)
             if (b < (int)batch) {
-                const float d = xn[(uint32_t)b * ld + i] - stat[b];
-                ps[b] = fmaf(d, d, ps[b]);
+                const Sum d = xn[(uint32_t)b * ld + i] - (NORM == 4 ? mean : (Sum)stat[b]);
+                ps[b] = fma(d, d, ps[b]);
             }
-    {
-        float tot = finish(ps);
-        if (NORM == 4) tot = all_rows(tot);
+    float whole_mean = 0.f, whole_rs = 0.f;
+    if constexpr (NORM == 4) {
+        whole_mean = (float)mean;
+        whole_rs = whole_norm_rs(finish(ps) * inv_count((uint32_t)k * batch), eps);
+    } else {
+        const Sum tot = finish(ps);
         if (wave == 0 && lane < BP) stat[16 + lane] = sqrtf(tot / (float)k + eps);
         __syncthreads();
     }
@@ -1090,6 +1109,8 @@ __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__rest
                     const float v = fmaf(xn[(uint32_t)b * ld + i] / stat[16 + b] * g, bs[i], hs[(uint32_t)b * ld + i]);
                     put((uint32_t)b, (uint32_t)i, v);
                     if (blockIdx.x == 0) post.h_out[(uint64_t)b * k + i] = v;
+                } else if (NORM == 4) {
+                    put((uint32_t)b, (uint32_t)i, g * (xn[(uint32_t)b * ld + i] - whole_mean) * whole_rs + bi);
                 } else {
                     put((uint32_t)b, (uint32_t)i, g * (xn[(uint32_t)b * ld + i] - stat[b]) / stat[16 + b] + bi);
                 }
@@ -1614,32 +1635,65 @@ __device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__res
     const bool on = b < batch;
     const float *row = NORM == 3 ? post.y + (uint64_t)b * k : x + (uint64_t)b * ldx;
     auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
-    float4_t v[VM], g[VM];
+    // (Sums in f64 next to a long row and its scale would spill.  Rows that long are at most eight, so that the last wave,
+    // which has none, brings the scale into LDS.)
+    constexpr bool SCALE_LDS = NORM == 4 && VM == 8;
+    float *gs = sh + 64;
+    float4_t v[VM], g[SCALE_LDS ? 1 : VM];
     if (on) {
 #pragma unroll
         for (int u = 0; u < VM; u++) v[u] = *(const float4_t *)(row + 4 * min(lane + 64 * u, n4 - 1));
+        if constexpr (!SCALE_LDS) {
 #pragma unroll
-        for (int u = 0; u < VM; u++) g[u] = *(const float4_t *)(nscale + 4 * min(lane + 64 * u, n4 - 1));
+            for (int u = 0; u < VM; u++) g[u] = *(const float4_t *)(nscale + 4 * min(lane + 64 * u, n4 - 1));
+        }
+    } else if (SCALE_LDS && b == 15) {
+#pragma unroll
+        for (int u = 0; u < VM; u++)
+            if (lane + 64 * u < n4) *(float4_t *)(gs + 4 * (lane + 64 * u)) = *(const float4_t *)(nscale + 4 * (lane + 64 * u));
     }
-    float mean = 0.f;
-    if (NORM == 1 || NORM == 4) {
-        float sum = 0.f;
+    float mean = 0.f, rs;
+    if constexpr (NORM == 4) {
+        // Whole slice: sums in f64 (as norm_sequence_kernel's, which serves the longer prompts).
+        double *shd = (double *)sh, sum = 0.0, sq = 0.0;
         if (on) {
 #pragma unroll
+            for (int u = 0; u < VM; u++) {
+                if (lane + 64 * u < n4) sum += ((double)v[u][0] + v[u][1]) + ((double)v[u][2] + v[u][3]);
+                __builtin_amdgcn_sched_barrier(0);  // (converted all at once, the row spills)
+            }
+            sum = wave_sum_f64(sum);
+            if (lane == 0) shd[b] = sum;
+        }
+        __syncthreads();
+        const double inv = inv_count(k * batch), m = wave_sum_f64(lane < batch ? shd[lane] : 0.0) * inv;
+        if (on) {
+#pragma unroll
+            for (int u = 0; u < VM; u++) {
+                if (lane + 64 * u < n4)
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        const double d = v[u][t] - m;
+                        sq = fma(d, d, sq);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            sq = wave_sum_f64(sq);
+            if (lane == 0) shd[16 + b] = sq;
+        }
+        __syncthreads();
+        if (!on) return;
+        mean = (float)m;
+        rs = whole_norm_rs(wave_sum_f64(lane < batch ? shd[16 + lane] : 0.0) * inv, eps);
+    } else {
+        if (!on) return;
+        if (NORM == 1) {
+            float sum = 0.f;
+#pragma unroll
             for (int u = 0; u < VM; u++) sum += lane + 64 * u < n4 ? (v[u][0] + v[u][1]) + (v[u][2] + v[u][3]) : 0.f;
-            sum = row_sum(sum);
+            mean = row_sum(sum) / (float)k;
         }
-        if (NORM == 4) {
-            if (lane == 0) sh[b] = sum;
-            __syncthreads();
-            sum = 0.f;
-            for (uint32_t w = 0; w < batch; w++) sum += sh[w];
-            sum /= (float)batch;
-        }
-        mean = sum / (float)k;
-    }
-    float sq = 0.f;
-    if (on) {
+        float sq = 0.f;
 #pragma unroll
         for (int u = 0; u < VM; u++)
 #pragma unroll
@@ -1647,34 +1701,27 @@ __device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__res
                 const float d = lane + 64 * u < n4 ? v[u][t] - mean : 0.f;
                 sq = fmaf(d, d, sq);
             }
-        sq = row_sum(sq);
+        rs = 1.0f / sqrtf(row_sum(sq) / (float)k + eps);
     }
-    if (NORM == 4) {
-        if (lane == 0) sh[16 + b] = sq;
-        __syncthreads();
-        sq = 0.f;
-        for (uint32_t w = 0; w < batch; w++) sq += sh[16 + w];
-        sq /= (float)batch;
-    }
-    if (!on) return;
-    const float rs = 1.0f / sqrtf(sq / (float)k + eps);
 #pragma unroll
     for (int u = 0; u < VM; u++) {
         const uint32_t i = 4 * (lane + 64 * u);
         if (i >= k) continue;
-        float4_t o;
+        float4_t o, gu;
+        if constexpr (SCALE_LDS) gu = *(const float4_t *)(gs + i);
+        else gu = g[u];
         if (NORM == 3) {
             const float4_t h = *(const float4_t *)(x + (uint64_t)b * ldx + i);
             float4_t ls = {1.f, 1.f, 1.f, 1.f};
             if (post.ls) ls = *(const float4_t *)(post.ls + i);
 #pragma unroll
-            for (int t = 0; t < 4; t++) o[t] = fmaf(v[u][t] * rs * g[u][t], ls[t], h[t]);
+            for (int t = 0; t < 4; t++) o[t] = fmaf(v[u][t] * rs * gu[t], ls[t], h[t]);
             if (blockIdx.x == 0) *(float4_t *)(post.h_out + (uint64_t)b * k + i) = o;
         } else {
             float4_t bi = {0.f, 0.f, 0.f, 0.f};
             if (NORM != 2 && nbias) bi = *(const float4_t *)(nbias + i);
 #pragma unroll
-            for (int t = 0; t < 4; t++) o[t] = g[u][t] * (v[u][t] - mean) * rs + bi[t];
+            for (int t = 0; t < 4; t++) o[t] = gu[t] * (v[u][t] - mean) * rs + bi[t];
         }
         xs.put4(b, i, o);
     }
@@ -1708,6 +1755,9 @@ static const size_t kDenseNormLdsLimit = 64 * 1024;
 // rows + scale + bias + per-wave partial sums + statistics
 static size_t gemv_dense_norm_lds(uint64_t k, uint32_t bp) { return ((size_t)(bp + 2) * k + 16 * bp + 32) * 4; }
 
+// (a norm over all rows: the partial sums in f64)
+static size_t gemv_whole_norm_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)16 * bp * 4; }
+
 // True when the dense decode matmul can take the normalisation into its staging: the normalised
 // activation block [batch padded, k] f32 has to fit in LDS.
 bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch) {
@@ -1738,7 +1788,7 @@ static size_t gemv_mfma_norm_lds(const Weight &w, uint32_t bp, size_t staging) {
 bool gemv_can_fuse_whole_norm(const Weight &w, uint64_t batch) {
     if (w.dtype != COEUS_W_F32 || batch < 2 || batch > 16 || !gemv_can_fuse_norm_dense(w, batch) || !gemv_uses_mfma(w, batch, 16)) return false;
     const uint32_t bp = pad_batch(batch);
-    return gemv_mfma_norm_lds(w, bp, gemv_dense_norm_lds(w.k, bp)) <= 160 * 1024;
+    return gemv_mfma_norm_lds(w, bp, gemv_whole_norm_lds(w.k, bp)) <= 160 * 1024;
 }
 static size_t gemv_dense_post_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)bp * k * 4; }
 bool gemv_can_fuse_post_norm(const Weight &w, uint64_t batch) {
@@ -2072,8 +2122,8 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     // plain: 4 rows per workgroup; folded norm: 16, so that the block is normalised once per 16 rows
     const uint32_t waves = nf ? 16 : 4;
     const dim3 grid((unsigned)ceil_div(w.n, waves)), block(waves * 64);
-    const size_t lds = !nf ? 0 : post_norm ? gemv_dense_post_lds(w.k, bp) : gemv_dense_norm_lds(w.k, bp);
     const int norm = !nf ? 0 : post_norm ? 3 : nf->whole ? 4 : nf->kind == COEUS_NORM_RMSNORM ? 2 : 1;
+    const size_t lds = norm == 0 ? 0 : norm == 3 ? gemv_dense_post_lds(w.k, bp) : norm == 4 ? gemv_whole_norm_lds(w.k, bp) : gemv_dense_norm_lds(w.k, bp);
     if (norm == 4 && (!gemv_can_fuse_whole_norm(w, batch) || nf->kind != COEUS_NORM_LAYERNORM))
         return fail(COEUS_INVALID_INPUT, "a folded norm over all rows needs f32 weights, 2 to 16 rows and room in LDS");
     const uint64_t ldx = nf && nf->ld ? nf->ld : w.k;

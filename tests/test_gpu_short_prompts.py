@@ -60,3 +60,42 @@ def test_vectors_behind_odd_lengths(orc, kw, scope):
         want = f64_model.forward_all(oc, params, ids)
         got = model.forward_all(ids)
         assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max(), rows  # (as above)
+
+
+@pytest.mark.parametrize("hidden,rows", [(512, 2), (768, 5), (1024, 16), (1088, 9), (2048, 4), (2080, 2), (2080, 4)])
+def test_whole_slice_far_from_zero(orc, hidden, rows):
+    """Statistics over all rows of values 2000 standard deviations from zero.  Attention adds nothing here, so the norm in
+    front of the feed-forward sees exactly the embedded rows; what comes behind is large against them and keeps its digits."""
+    cfg = dict(hidden_dim=hidden, num_layers=1, use_bias=False)
+    _, oc, params = build(orc, **cfg)
+    rng = np.random.default_rng(hidden + rows)
+    first, stride, rel = f64_model.offsets(oc)
+    params = params.copy()
+
+    def part(name, shape=None):
+        at, size = rel[name]
+        a = params[first + at:first + at + size]
+        return a.reshape(shape) if shape else a
+
+    table = params[:150 * hidden].reshape(150, hidden)
+    table[:] = 1000 + 0.5 * rng.standard_normal(table.shape)
+    part("wo")[:] = 0
+    part("w_down")[:] = 1e5 * rng.standard_normal(part("w_down").size)
+    model = TransformerModelPlugin().create_builder().build(
+        Transformer250MConfig(vocab_size=150, max_seq_len=40, num_heads=16, intermediate_dim=608, **cfg), parameters=params)
+    ids = rng.integers(0, 150, rows, dtype=np.uint64)
+    x = (table[ids.astype(int)] + orc.positional_encoding(40, hidden)[:rows]).astype(np.float64)
+    eps = np.float64(np.float32(oc.layer_norm_eps))
+
+    def norm(x, scale, bias):
+        # (the mean is rounded to f32 before it is subtracted, as where the norm is a launch of its own)
+        return scale * (x - np.float64(np.float32(x.mean()))) / np.sqrt(x.var() + eps) + bias
+
+    up = norm(x, part("ln2_s"), part("ln2_b")) @ part("w_up", (hidden, 608)).astype(np.float64)
+    x = x + f64_model.gelu(up) @ part("w_down", (608, hidden)).astype(np.float64)
+    at = first + stride
+    x = norm(x, params[at:at + hidden], params[at + hidden:at + 2 * hidden])
+    want = x @ params[at + 2 * hidden:at + 2 * hidden + 150 * hidden].reshape(hidden, 150).astype(np.float64)
+    # a mean that is off by one f32 step (6e-5 of values that spread by 0.5) moves every normalised value by 1.2e-4;
+    # f32 sums of the matmuls: a few 1e-7
+    assert np.abs(model.forward_all(ids) - want).max() <= 5e-6 * np.abs(want).max()
