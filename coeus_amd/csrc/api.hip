@@ -319,6 +319,7 @@ static int weight_create_common(uint32_t dtype, const float *host_w, uint64_t se
         src.base = 0;
     }
     rc = weight_pack(w->w, src, nullptr);
+    if (rc == COEUS_OK) rc = weights_check({&w->w}, nullptr);
     hipError_t e = hipDeviceSynchronize();
     if (dev) (void)hipFree(dev);
     if (rc == COEUS_OK && e != hipSuccess) rc = fail(COEUS_DEVICE_ERROR, "weight packing failed: %s", hipGetErrorString(e));

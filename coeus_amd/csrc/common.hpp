@@ -89,6 +89,7 @@ struct Weight {
     void *data = nullptr;        // weights (quants for Q*)
     __half *scales = nullptr;    // Q* only
     uint64_t bytes = 0;
+    bool infinite = false;       // bf16: some value is infinite (weights_check)
     __half *xq_scratch = nullptr; // [k_pad/8][16][8] f16 staging for the operator-level API
     // Q* only: dense f16 copy [n] rows of gemm_ld(k) elements for the prefill matmul, made on first
     // use and kept while the owner's budget lasts (7B: 13.7 GB next to 4.2 GB of quants; the card
@@ -115,6 +116,8 @@ int weight_pack(Weight &w, const WeightSource &src, hipStream_t st);
 // Q* only: makes the resident f16 copy for the prefill matmul (Weight::expanded) if `budget`
 // still covers it, and charges the budget; does nothing for other types or when it does not fit.
 int weight_expand(const Weight &w, uint64_t *budget, hipStream_t st);
+// Sets Weight::infinite of the bf16 weights among `list` (null and empty ones are passed over); waits for `st`.
+int weights_check(const std::vector<Weight *> &list, hipStream_t st);
 int weight_unpack_to_device(const Weight &w, float *dst_kn, hipStream_t st);
 
 // Host/device counter-based generator (see weights.hip).

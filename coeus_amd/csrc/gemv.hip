@@ -1367,7 +1367,7 @@ __global__ __launch_bounds__(256) void gemv_row_kernel(const void *__restrict__ 
 //   768 x 50257    28 / 14     41 / 14       68 / 16      127 / 18
 // f32: 768 x 3072 9.0 / 4.4 at batch 8, 768 x 50257 79 / 30, 4096 x 4096 31 / 15.
 // (one row: 4.2, 8.7, 33, 18.5 there, which keeps it: a wave per row needs no sum over waves.)  The large ones are
-// at 5 TB/s of weights.  An infinite weight makes its output NaN (times the pieces of an activation that are zero).
+// at 5 TB/s of weights.  A matrix with an infinite value stays there (times a piece that is zero it would be a NaN).
 //
 // The workgroup's waves take a share of k each, in pairs of 32-wide chunks: a wave request is 8 rows x 128 bytes, as
 // the weights lie, and passes through a corner of LDS that is the wave's own to where the matrix cores want it (a
@@ -1765,7 +1765,8 @@ bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch) {
     return gemv_dense_norm_lds(w.k, pad_batch(batch)) <= kDenseNormLdsLimit;
 }
 
-// Weights whose rows are whole pairs of chunks (128 bytes), one for every wave at least.
+// Weights whose rows are whole pairs of chunks (128 bytes), one for every wave at least, and none of whose values is infinite
+// (an activation's three bf16 may be zero).
 static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves) {
     const uint64_t ku = w.dtype == COEUS_W_BF16 ? 64 : 32;
     // (f32, two or three rows on fewer than 64 tiles: a wave per row keeps more compute units busy, 6.7 against 7.9 us
@@ -1774,7 +1775,7 @@ static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves) {
     // (one row of bf16 weights: long rows few of which there are, 11008 x 4096 20.8 us there, 18.9 here, 4096 x 4096 8.6 / 7.9;
     // and short rows many of which there are, 768 x 50257 18.5 / 13.9; between them a wave per row: 2048 x 5632 7.1 / 8.4)
     if (batch == 1 && (w.dtype != COEUS_W_BF16 || !((w.k >= 4096 && w.n <= 4096) || (w.k <= 1024 && w.n >= 16384)))) return false;
-    return w.dtype <= COEUS_W_BF16 && batch >= 1 && w.k % ku == 0 && w.k / ku >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
+    return w.dtype <= COEUS_W_BF16 && !w.infinite && batch >= 1 && w.k % ku == 0 && w.k / ku >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
 }
 // Waves of a plain launch: as many as have two pairs of chunks each.
 static uint32_t gemv_mfma_waves(uint64_t pairs) { return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (pairs + 1) / 2)); }

@@ -359,6 +359,9 @@ int build(const LayeredConfig &cfg, const SafeTensors *file, uint64_t seed, cons
         m->weight_bytes += table.bytes;
     }
     COEUS_HIP(hipDeviceSynchronize());
+    std::vector<Weight *> linear{&m->out};
+    for (LayeredLayer &ly : stack.layers) linear.insert(linear.end(), {&ly.in, &ly.o, &ly.up, &ly.down, &ly.uq, &ly.ukv});
+    COEUS_TRY(weights_check(linear, st));
     *out = m.release();
     return COEUS_OK;
 }

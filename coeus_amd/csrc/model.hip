@@ -280,6 +280,9 @@ int model_create(const coeus_config &cfg, const float *params, uint64_t n_params
         COEUS_TRY(weight_pack(m->out, src, st));
         m->weight_bytes += m->out.bytes;
     }
+    std::vector<Weight *> linear{&m->out};
+    for (LayerWeights &lw : m->layers) linear.insert(linear.end(), {&lw.qkv, &lw.o, &lw.up, &lw.down});
+    COEUS_TRY(weights_check(linear, st));
 
     // ---- token embedding: bf16 with bf16 weights, f32 otherwise
     m->embed_bf16 = wd == COEUS_W_BF16;

@@ -3,6 +3,8 @@
 // (GGML block_q8_0 / block_q4_0 value convention) and the counter-based synthetic generator.
 #include "common.hpp"
 
+#include <algorithm>
+
 // Everything in this file must reproduce the CPU arithmetic bit for bit (quantiser, generator):
 // no a*b+c may be fused into an FMA.  The build compiles this file with -ffp-contract=off.
 
@@ -375,6 +377,41 @@ int weight_pack(Weight &w, const WeightSource &ws, hipStream_t st) {
                                (uint32_t *)w.data, w.scales, w.k, w.n, nblk_pad, w.n_pad);
     }
     COEUS_HIP(hipGetLastError());
+    return COEUS_OK;
+}
+
+// The decode matmul of several rows multiplies bf16 weights with the parts of split activations, some of which are zero:
+// an infinite weight would make a NaN of what is an infinity.  Such a matrix is found once, when the weights are made.
+__global__ __launch_bounds__(256) void find_infinite_kernel(const uint16_t *__restrict__ w, uint64_t n, uint32_t *flag) {
+    const uint64_t n8 = n / 8, step = (uint64_t)gridDim.x * blockDim.x, t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    auto hit = [](uint32_t v) { return (v & 0x7fffu) == 0x7f80u || (v >> 16 & 0x7fffu) == 0x7f80u; };
+    bool found = false;
+    for (uint64_t i = t; i < n8; i += step) {
+        const uint4 v = ((const uint4 *)w)[i];
+        found |= hit(v.x) || hit(v.y) || hit(v.z) || hit(v.w);
+    }
+    if (t < n - 8 * n8) found |= hit(w[8 * n8 + t]);
+    if (found) *flag = 1u;  // (whoever writes, writes the same)
+}
+
+int weights_check(const std::vector<Weight *> &list, hipStream_t st) {
+    std::vector<Weight *> bf;
+    for (Weight *w : list)
+        if (w && w->data && w->dtype == COEUS_W_BF16) bf.push_back(w);
+    if (bf.empty()) return COEUS_OK;
+    std::vector<uint32_t> found(bf.size(), 0);
+    struct Flags { uint32_t *p = nullptr; ~Flags() { if (p) (void)hipFree(p); } } flags;
+    COEUS_HIP(hipMalloc((void **)&flags.p, found.size() * 4));
+    COEUS_HIP(hipMemcpyAsync(flags.p, found.data(), found.size() * 4, hipMemcpyHostToDevice, st));
+    for (size_t i = 0; i < bf.size(); i++) {
+        const uint64_t n = bf[i]->k * bf[i]->n;
+        hipLaunchKernelGGL(find_infinite_kernel, dim3((unsigned)std::min<uint64_t>(2048, ceil_div(n, 2048))), dim3(256), 0, st,
+                           (const uint16_t *)bf[i]->data, n, flags.p + i);
+    }
+    COEUS_HIP(hipGetLastError());
+    COEUS_HIP(hipMemcpyAsync(found.data(), flags.p, found.size() * 4, hipMemcpyDeviceToHost, st));
+    COEUS_HIP(hipStreamSynchronize(st));
+    for (size_t i = 0; i < bf.size(); i++) bf[i]->infinite = found[i] != 0;
     return COEUS_OK;
 }
 

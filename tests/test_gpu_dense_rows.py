@@ -3,7 +3,8 @@ each) against a float64 product of the same weights and activations."""
 import numpy as np
 import pytest
 
-from coeus_amd import _lib
+import layered_util as L
+from coeus_amd import PLUGINS, Transformer250MConfig, _lib, load_model
 from gpu_util import Weight, dev, oracle_roundtrip
 
 pytestmark = pytest.mark.gpu
@@ -63,3 +64,50 @@ def test_infinities_and_nan_stay_in_their_row(orc, dtype, batch):
     y = Weight(dtype, w).gemv(dev(x))
     assert np.array_equal(y[0], np.sign(wd[7]) * np.inf) and np.isnan(y[1]).all()
     assert (np.abs(y[2:] - x[2:].astype(np.float64) @ wd) <= bound(x[2:], wd, k)).all()
+
+
+@pytest.mark.parametrize("batch,k,n", [(1, 4096, 40), (1, 1024, 16400), (2, 256, 40), (5, 1024, 33), (16, 2048, 70)])
+@pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_F32])
+def test_infinite_weights(orc, dtype, batch, k, n):
+    rng = np.random.default_rng(k + batch)
+    w = (rng.standard_normal((k, n)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((batch, k)).astype(np.float32)
+    x[:, 1] = 1.0  # (one bf16: its other two pieces are zero)
+    w[1, 3], w[k - 1, 7], w[5, n - 1] = np.inf, -np.inf, np.inf
+    w[9, 11] = 3.4e38  # rounds to an infinite bf16
+    wd = oracle_roundtrip(orc, dtype, w).astype(np.float64)
+    want = x.astype(np.float64) @ np.where(np.isinf(wd), 0, wd)
+    bad = np.isinf(wd).any(0)
+    for r, c in np.argwhere(np.isinf(wd)):
+        want[:, c] = wd[r, c] * np.sign(x[:, r])
+    got = Weight(dtype, w).gemv(dev(x))
+    assert np.array_equal(got[:, bad], want[:, bad].astype(np.float32))
+    ok = np.setdiff1d(np.flatnonzero(~bad), [11])
+    assert (np.abs(got[:, ok] - want[:, ok]) <= bound(x, np.where(np.isinf(wd), 0, wd), k)[:, ok]).all()
+
+
+def test_infinite_weights_of_models(orc, tmp_path):
+    """Columns of the output projection with an infinite value each: infinite logits (capped ones: the cap), not NaN.  One
+    activation in 256 has a third bf16 that is zero; here 1120 and 3200 of them meet an infinity."""
+    rng = np.random.default_rng(3)
+    kw = dict(hidden_dim=1024, num_layers=1, num_heads=16, intermediate_dim=320, vocab_size=90, max_seq_len=16, norm_scope="token", weight_dtype="bf16",
+              kv_dtype="bf16", max_batch=16)
+    oc = orc.config_from_kwargs(kw)
+    params = orc.init_seeded(oc, 5)
+    out = params[orc.layout(oc).output_proj_offset:][:1024 * 90].reshape(1024, 90)
+    out[np.arange(20, 90) * 2, np.arange(20, 90)] = np.inf
+    s = PLUGINS["transformer_model"].create_builder().build(Transformer250MConfig(**kw), parameters=params).session(batch=16, max_ctx=16)
+    ids = rng.integers(0, 90, (16, 4), dtype=np.uint64)
+    s.prefill(ids)
+    y = s.decode(ids[:, 0])
+    assert np.isinf(y[:, 20:]).all() and np.isfinite(y[:, :20]).all()
+
+    cfg = L.CONFIGS["hyper_wide"]
+    w = L.weights(cfg, 6)
+    w["head"][np.arange(200), np.arange(200) % 128] = np.inf
+    model = load_model(L.write_folder(str(tmp_path / "m"), cfg, w), max_seq_len=16, max_batch=16)
+    s = model.session(batch=16, max_ctx=16)
+    ids = rng.integers(0, 200, (16, 4), dtype=np.uint64)
+    s.prefill(ids)
+    y = s.decode(ids[:, 0])
+    assert (np.abs(y) == 8.0).all()
