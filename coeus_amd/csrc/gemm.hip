@@ -231,7 +231,12 @@ static int launch_gemm_f32(const Weight &w, const float *a, uint64_t m, const Ep
                            const GemmScratch &scr, hipStream_t st) {
     // Up to 16 rows: the decode matmul, which gives a weight row's k to 16 waves instead of 4 and requests all of it at
     // once (5 rows, 768 x 2304 / 768 x 768 / 768 x 3072 / 3072 x 768: 11.5 / 12.3 / 12.1 / 7.9 + 4.7 us here).
-    if (gemv_takes_f32_rows(w, m) && scr.repeat <= 1 && !scr.ev_begin) return launch_gemv(w, a, m, ep, st);
+    if (gemv_takes_f32_rows(w, m)) {
+        if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
+        for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) COEUS_TRY(launch_gemv(w, a, m, ep, st));
+        if (scr.ev_end) COEUS_HIP(hipEventRecord(scr.ev_end, st));
+        return COEUS_OK;
+    }
     const EpiArgs e = make_epi(ep, w.n);
     const dim3 grid((unsigned)ceil_div(w.n, BN), (unsigned)ceil_div(m, BM));
     const bool small = gemm_f32_is_small(w, m);

@@ -1,10 +1,14 @@
 """The decode matmul of several rows on dense weights (matrix cores; with bf16 weights the activations as three bf16
 each) against a float64 product of the same weights and activations."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import layered_util as L
 from coeus_amd import PLUGINS, Transformer250MConfig, _lib, load_model
+from coeus_amd.device import DeviceArray
+from coeus_amd.plugin import _check
 from gpu_util import Weight, dev, oracle_roundtrip
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +36,16 @@ def test_rows_match_float64(orc, dtype, k, n, batch):
     assert (np.abs(wt.gemv(dev(x)) - want) <= bound(x, wd, k)).all()
     if dtype == _lib.W_F32:  # a short prompt takes the same kernel
         assert (np.abs(wt.gemm(dev(x)) - want) <= bound(x, wd, k)).all()
+
+
+@pytest.mark.parametrize("dtype,rows", [(_lib.W_F32, 2), (_lib.W_F32, 5), (_lib.W_F32, 16), (_lib.W_F32, 17), (_lib.W_BF16, 5)])
+def test_timed_matmul_is_the_one_that_runs(dtype, rows):
+    """What the repeated, timed launches leave is the bits of the plain call: the same kernel, in the same order of sums."""
+    rng = np.random.default_rng(rows)
+    w = Weight(dtype, (rng.standard_normal((3072, 768)) * 0.02).astype(np.float32))
+    x, y, ms = dev(rng.standard_normal((rows, 3072)).astype(np.float32)), DeviceArray((rows, 768)).zero_(), C.c_float()
+    _check(_lib.load().coeus_op_gemm_timed(w.h, x.ptr, rows, 0, y.ptr, 3, C.byref(ms), None))
+    assert ms.value > 0 and np.array_equal(y.to_host(), w.gemm(x))
 
 
 @pytest.mark.parametrize("batch", [2, 5, 16])
