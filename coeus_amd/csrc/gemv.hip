@@ -2073,10 +2073,10 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
         nf.bias || (nf.y && (!nf.h_out || nf.h_out == nf.h)))
         return fail(COEUS_INVALID_INPUT, "folded hyper-connections: bad arguments or too many streams");
     const uint32_t bp = pad_batch(batch), b = (uint32_t)batch, k = (uint32_t)w.k, nit = hyper_pairs(w.k);
-    // (the matrix-core instances lay their LDS out for two or four rows: one row stays with a wave per weight row, also where
-    // gemv_uses_mfma takes one row of a plain launch)
-    const bool mf = BF16 && nit == 1 && bp >= 2 && gemv_uses_mfma(w, batch, 16);
-    const size_t lds = mf ? 16 * 16 * mfma_wave_lds<true>(0) + SplitRows::bytes(bp, k) : (size_t)bp * k * 4;
+    // (the matrix-core instance lays its LDS out for two rows: one stays with a wave per weight row, also where gemv_uses_mfma
+    // takes one row of a plain launch; in front of three or four a model's step has a launch of its own)
+    const bool mf = BF16 && nit == 1 && bp == 2 && gemv_uses_mfma(w, batch, 16);
+    const size_t lds = mf ? 16 * 16 * mfma_wave_lds<true>(0) + SplitRows::bytes(bp, k) : (size_t)bp * k * 4;  // (57 KiB at most)
     const uint32_t bs = b | nf.streams << 16;
     const HyperFold *fold = (const HyperFold *)nf.fold;
     const float *y = nf.y ? nf.y : nf.h;  // (without an output of a sublayer before its weight is zero)
@@ -2086,10 +2086,7 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
     const dim3 grid((unsigned)std::min<uint64_t>(256, mf ? ceil_div(w.n, 16) : units)), block(1024);  // (a workgroup per compute unit)
     if constexpr (BF16) {
         if (mf) {
-            if (bp == 4)
-                hipLaunchKernelGGL((gemv_hyper_kernel<true, 4, 1, true>), grid, block, lds, st, w.data, nf.h, y, nf.scale, fold, k, bs, x_out, nf.eps, e);
-            else
-                hipLaunchKernelGGL((gemv_hyper_kernel<true, 2, 1, true>), grid, block, lds, st, w.data, nf.h, y, nf.scale, fold, k, bs, x_out, nf.eps, e);
+            hipLaunchKernelGGL((gemv_hyper_kernel<true, 2, 1, true>), grid, block, lds, st, w.data, nf.h, y, nf.scale, fold, k, bs, x_out, nf.eps, e);
             COEUS_HIP(hipGetLastError());
             return COEUS_OK;
         }

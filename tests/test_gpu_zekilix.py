@@ -69,7 +69,7 @@ def test_hyper_output_over_its_input():
 @pytest.mark.parametrize("with_y", [True, False])
 @pytest.mark.parametrize("batch,k,n,streams", [(1, 96, 40, 3), (3, 58, 131, 2), (4, 128, 64, 4), (2, 1024, 300, 1), (1, 4096, 52, 4), (3, 250, 17, 3),
                                                (1, 2050, 34, 2), (2, 4000, 20, 4), (1, 6000, 18, 3), (1, 520, 8230, 4), (2, 64, 9001, 2),
-                                               (1, 1024, 16400, 4)])
+                                               (1, 1024, 16400, 4), (2, 2048, 5003, 4), (3, 2048, 300, 4), (4, 1024, 520, 2)])
 def test_hyper_gemv(wd, with_y, batch, k, n, streams):
     rng = np.random.default_rng(k + n)
     w = rng.normal(size=(k, n)).astype(np.float32) / np.float32(np.sqrt(k))
