@@ -36,8 +36,17 @@ static void map_pages(void *p, uint64_t bytes) {
     (void)madvise((void *)first, last - first, MADV_POPULATE_WRITE);
 }
 
+// Memory that the runtime knows (pinned, managed or on a device): its own copy goes there in one piece.
+static bool known_to_runtime(const void *p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return false;
+}
+
 int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st) {
-    if (!pin && bytes > 4096) {
+    const bool slots_help = bytes > 4096 && !known_to_runtime(dst);
+    if (!pin && slots_help) {
         bool ok = hipHostMalloc((void **)&pin, kSlot * kSlots, hipHostMallocDefault) == hipSuccess;
         for (uint64_t i = 0; i < kSlots && ok; i++) ok = hipEventCreateWithFlags(&done[i], hipEventDisableTiming) == hipSuccess;
         if (!ok) {
@@ -45,7 +54,7 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
             (void)hipGetLastError();
         }
     }
-    if (!pin || bytes <= 4096) {
+    if (!pin || !slots_help) {
         COEUS_HIP(hipMemcpyAsync(dst, src_dev, bytes, hipMemcpyDeviceToHost, st));
         COEUS_HIP(hipStreamSynchronize(st));
         return COEUS_OK;

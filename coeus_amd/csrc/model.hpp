@@ -26,7 +26,7 @@ struct DeviceBuf {
 // staging buffer and, where the caller's pages have never been touched (a result array made for this call), faults
 // them in one by one while the GPU waits: 1.6 MB of logits took 0.45 ms behind a step of 0.53 ms.  Here the copy goes to
 // pinned slots of the model's, the caller's pages are mapped while the GPU still computes, and a slot is copied out
-// while the next one fills.
+// while the next one fills.  Into pinned (or device) memory the copy is the runtime's, without a stop.
 struct HostCopy {
     static constexpr uint64_t kSlot = 1 << 20, kSlots = 4;
     char *pin = nullptr;

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from coeus_amd import Transformer250MConfig, TransformerModelPlugin, _lib
+from coeus_amd.device import DeviceArray
 from coeus_amd.plugin import _check
 
 pytestmark = pytest.mark.gpu
@@ -32,3 +33,28 @@ def test_every_row_arrives(vocab, rows):
         s.prefill(ids[:-1].reshape(1, -1), want_logits=False)
         last = s.decode(ids[-1:])[0]
         assert np.abs(last - want[-1]).max() <= 2e-5 * np.abs(want[-1]).max()
+
+
+def test_into_pinned_and_device_memory():
+    """Results that the caller wants in pinned memory (26 slots' worth, and less than a slot), or on the device."""
+    vocab, rows = 50257, 128
+    cfg = Transformer250MConfig(hidden_dim=32, num_layers=1, num_heads=2, intermediate_dim=64, vocab_size=vocab, max_seq_len=rows,
+                                norm_scope="token")
+    model = TransformerModelPlugin().create_builder().build(cfg, seed=3)
+    lib, hip = _lib.load(), C.CDLL("libamdhip64.so", mode=C.RTLD_GLOBAL)
+    hip.hipHostMalloc.argtypes, hip.hipHostFree.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint], [C.c_void_p]
+    ids = np.random.default_rng(4).integers(0, vocab, rows, dtype=np.uint64)
+    for n, call, size in ((rows, lib.coeus_model_forward_all, rows * vocab), (rows, lib.coeus_model_forward, vocab)):
+        want = np.empty(size, np.float32)
+        _check(call(model._h, ids.ctypes.data, n, want.ctypes.data))
+        p = C.c_void_p()
+        assert hip.hipHostMalloc(C.byref(p), 4 * size + 4096, 0) == 0
+        buf = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_float)), (size + 1024,))
+        buf[:] = 7.0
+        _check(call(model._h, ids.ctypes.data, n, p.value + 4 * 17))
+        assert np.array_equal(buf[17:17 + size], want) and (buf[:17] == 7.0).all() and (buf[17 + size:] == 7.0).all()
+        del buf
+        assert hip.hipHostFree(p) == 0
+        d = DeviceArray((size,), np.float32)
+        _check(call(model._h, ids.ctypes.data, n, d.ptr))
+        assert np.array_equal(d.to_host(), want)
