@@ -186,13 +186,15 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
             tmax = fmaxf(tmax, s[t]);
         }
         const float m_new = fmaxf(m, wave_max(tmax));
-        const float corr = __builtin_amdgcn_exp2f(m - m_new);
+        // (keys whose scores are all -inf weigh nothing: -inf - -inf would make a NaN of a wave's share)
+        const float top = m_new == -INFINITY ? 0.f : m_new;
+        const float corr = __builtin_amdgcn_exp2f(m - top);
         float psum = 0.f;
 #pragma unroll
         for (int t = 0; t < EPL; t++) acc[t] *= corr;
 #pragma unroll
         for (int t = 0; t < TILE; t++) {
-            const float p = __builtin_amdgcn_exp2f(s[t] - m_new);  // 2^(-inf) = 0 for keys past the end
+            const float p = __builtin_amdgcn_exp2f(s[t] - top);  // 2^(-inf) = 0 for keys past the end
             psum += p;
             float vv[EPL];
             kv_piece<KV>(vr[t], vv);

@@ -3,6 +3,7 @@ around the kernel's tiles and splits."""
 import numpy as np
 import pytest
 
+import f64_model
 from coeus_amd import Transformer250MConfig, TransformerModelPlugin
 
 pytestmark = pytest.mark.gpu
@@ -50,3 +51,28 @@ def test_many_heads_match_prompt_pass(heads, hd, max_ctx, kv):
     for b in (0, 7, 15):
         want = model.forward(ids[b])
         assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), b
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("ctx", [130, 300, 700])
+def test_keys_that_score_minus_infinity(orc, hd, ctx):
+    """Keys 64 on, up to the last, overflow to a score of -inf against the last query: they weigh nothing, also where a wave or
+    a split has only such keys.  The others' scores are finite and far apart."""
+    H, V = 2 * hd, 60
+    kw = dict(hidden_dim=H, num_layers=1, num_heads=2, intermediate_dim=64, vocab_size=V, max_seq_len=ctx, norm_scope="token", use_bias=False)
+    oc = orc.config_from_kwargs(kw)
+    params = orc.init_seeded(oc, 9)
+    rng = np.random.default_rng(ctx)
+    table = params[:V * H].reshape(V, H)
+    table[:] = rng.standard_normal((V, H))
+    table[:, 0], table[:30, 1], table[30:, 1] = 10.0, 0.1 * table[:30, 1], -1000.0
+    first, _, rel = f64_model.offsets(oc)
+    for name, row, scale in (("wq", 0, 1e20), ("wk", 1, 2e17)):
+        w = params[first + rel[name][0]:first + rel[name][0] + H * H].reshape(H, H)
+        w[:], w[row, 0], w[row, hd] = 0, scale, scale  # the first element of each head
+    ids = np.concatenate([rng.integers(0, 30, 64), rng.integers(30, V, ctx - 65), rng.integers(0, 30, 1)]).astype(np.uint64)
+    model = TransformerModelPlugin().create_builder().build(Transformer250MConfig(**kw), parameters=params)
+    s = model.session(batch=1, max_ctx=ctx)
+    s.prefill(ids[None, :-1], want_logits=False)
+    got, want = s.decode(ids[-1:])[0], f64_model.forward_all(oc, params, ids)[-1]
+    assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()  # (f32, as above)
