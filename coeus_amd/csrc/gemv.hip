@@ -2156,15 +2156,19 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         (void)once;                                                                                                           \
         hipLaunchKernelGGL((gemv_mfma_kernel<BF16, BPV, NV, PV, KV>), mgrid, mblock, mlds, st, (const typename MfmaType<BF16>::W *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
     } while (0)
-#define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (np % 3 == 0 || np == 5) COEUS_MFMA4(BPV, NV, 3, false); else COEUS_MFMA4(BPV, NV, 4, false); } while (0)
+            // Pairs in flight: two or three, whichever asks for fewer in vain at the end of a wave's share.  Where that is the
+            // same, three for 2 - 4 rows (us for two / three: 4 rows of bf16 5120 x 32000 67.0 / 65.5, 2 of 12288 x 8192 36.5 / 35.0), two
+            // for one row (6144 x 512 7.2 / 7.4) and for 8 (6144 x 4096 13.0 / 13.5).  A norm in front fills the first trip, and
+            // three pay from the second tile on (2 rows of bf16 3072 x 4096 12.7 / 13.3, x 12288 22.4 / 20.8).  Four in flight are
+            // never faster (4 rows, us for 2 / 3 / 4: 3072 x 4096 7.1 / 6.4 / 7.1, 4096 x 4096 7.7 / 9.2 / 7.8, 10240 x 512 12.1 / 13.7 /
+            // 14.0).
+            const uint32_t by2 = (np + 1) / 2 * 2, by3 = (np + 2) / 3 * 3;
+            const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && batch > 1 && bp <= 4);
+#define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (BPV < 16 && three) COEUS_MFMA4(BPV < 16 ? BPV : 8, NV, 3, false); else COEUS_MFMA4(BPV, NV, 2, false); } while (0)
 #define COEUS_MFMA(BPV) do { if (norm == 4) { if constexpr (!BF16) COEUS_MFMA3(BPV, 4); } else if (norm == 1) COEUS_MFMA3(BPV, 1); else if (norm == 2) COEUS_MFMA3(BPV, 2); else COEUS_MFMA3(BPV, 3); } while (0)
-            constexpr int P8 = BF16 ? 2 : 4;  // (bf16, 8 rows: four pairs do not fit the registers)
             if (norm == 0 && bp <= 4) COEUS_MFMA3(4, 0);
-            else if (norm == 0 && bp == 8 && np <= 2) COEUS_MFMA4(8, 0, 2, true);
-            else if (norm == 0 && bp == 8 && np % 3 == 0) COEUS_MFMA4(8, 0, 3, false);
-            else if (norm == 0 && bp == 8) COEUS_MFMA4(8, 0, P8, false);
-            else if (norm == 0 && np <= 2) COEUS_MFMA4(16, 0, 2, true);
-            else if (norm == 0) COEUS_MFMA4(16, 0, 2, false);
+            else if (norm == 0 && bp == 8) COEUS_MFMA3(8, 0);
+            else if (norm == 0) COEUS_MFMA3(16, 0);
             else if (bp == 2) COEUS_MFMA(2);
             else if (bp == 4) COEUS_MFMA(4);
             else if (bp == 8) COEUS_MFMA(8);
