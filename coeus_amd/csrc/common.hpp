@@ -240,7 +240,7 @@ int launch_row_stats16(const float *h, uint64_t rows, uint64_t k, float2 *stats,
 int launch_gemv(const Weight &w, const void *x, uint64_t batch, const Epilogue &ep, hipStream_t st,
                 const NormFuse *nf = nullptr);
 
-// True when launch_gemv multiplies `rows` (2 - 16) rows of f32 weights on the matrix cores; short prompts take it too.
+// True when the prompt matmul of `rows` (2 - 16) rows of f32 weights is launch_gemv.
 bool gemv_takes_f32_rows(const Weight &w, uint64_t rows);
 
 // Prefill matmul on f32 activations: C[m, n] = A[m, k] . W.  Low-precision weights need

@@ -1366,7 +1366,7 @@ __global__ __launch_bounds__(256) void gemv_row_kernel(const void *__restrict__ 
 //   4096 x 22016   47 / 34     73 / 36      118 / 40      215 / 55
 //   768 x 50257    28 / 14     41 / 14       68 / 16      127 / 18
 // f32: 768 x 3072 9.0 / 4.4 at batch 8, 768 x 50257 79 / 30, 4096 x 4096 31 / 15.
-// (one row: 4.2, 8.7, 33, 18.5 there, which keeps it: a wave per row needs no sum over waves.)  The large ones are
+// (One row: 4.2, 8.7, 33, 18.5 there; where it comes here gemv_uses_mfma says.)  The large ones are
 // at 5 TB/s of weights.  A matrix with an infinite value stays there (times a piece that is zero it would be a NaN).
 //
 // The workgroup's waves take a share of k each, in pairs of 32-wide chunks: a wave request is 8 rows x 128 bytes, as
@@ -1767,27 +1767,45 @@ bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch) {
 
 // Weights whose rows are whole pairs of chunks (128 bytes), one for every wave at least, and none of whose values is infinite
 // (an activation's three bf16 may be zero).
-static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves) {
+static bool gemv_mfma_shape(const Weight &w, uint32_t waves) {
     const uint64_t ku = w.dtype == COEUS_W_BF16 ? 64 : 32;
-    // (f32, two or three rows on fewer than 64 tiles: a wave per row keeps more compute units busy, 6.7 against 7.9 us
-    // for 2 rows of 3072 x 768; four rows 8.7 against 8.1)
-    if (w.dtype == COEUS_W_F32 && batch < 4 && w.n <= 63 * 16) return false;
-    // (one row of bf16 weights: long rows few of which there are, 11008 x 4096 20.8 us there, 18.9 here, 4096 x 4096 8.6 / 7.9;
-    // and short rows many of which there are, 768 x 50257 18.5 / 13.9; between them a wave per row: 2048 x 5632 7.1 / 8.4)
-    if (batch == 1 && (w.dtype != COEUS_W_BF16 || !((w.k >= 4096 && w.n <= 4096) || (w.k <= 1024 && w.n >= 16384)))) return false;
-    return w.dtype <= COEUS_W_BF16 && !w.infinite && batch >= 1 && w.k % ku == 0 && w.k / ku >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
+    return w.dtype <= COEUS_W_BF16 && !w.infinite && w.k % ku == 0 && w.k / ku >= waves && w.k < (1ull << 31) && w.n < (1ull << 31) - 16;
+}
+// Where the matrix cores are the faster of the two (us with weights from memory: a wave per row / here).
+static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves, bool folded) {
+    if (!gemv_mfma_shape(w, waves) || batch < 1) return false;
+    const bool bf = w.dtype == COEUS_W_BF16;
+    if (batch == 1) {
+        if (!bf || folded) return false;
+        // Short rows of which there are many: 768 x 50257 18.5 / 14.0, 1024 x 16384 8.7 / 7.9.
+        if (w.k <= 1024) return w.n >= 16384;
+        // Long rows of which there are few: 4096 x 4096 9.1 / 7.9, 8192 x 512 9.5 / 8.6, 11008 x 4096 21.6 / 18.9; but 2048 x 2048 4.3 / 4.8,
+        // 4096 x 6144 11.7 / 12.4 and 6144 x 6144 16.2 / 17.7.  Shares of an uneven number of pairs ask for one in vain, which up
+        // to 5120 elements takes many rows to pay: 4608 x 512 6.3 / 6.7, x 3584 9.5 / 8.9.  Rows 32 KiB apart share their memory
+        // channels: 16384 x 3584 24.4 / 22.9, x 4096 26.2 / 28.7, 32768 x 4096 50 / 66.
+        return w.k >= 4096 && w.n <= 4096 && (w.k % 2048 == 0 || w.k > 5120 || w.n >= 2048) && (w.k % 16384 || w.n <= 3584);
+    }
+    // (A norm in front costs a wave per row more: f32, 2 rows of 768 x 768 7.4 / 5.8.  Two rows of bf16 are the exception where they
+    // are long and few: 2560 x 4096 11.0 / 11.6, x 12288 22.7 / 19.1.)
+    if (folded) return !(bf && batch == 2 && w.k > 2048 && w.n <= 4096);
+    // Two or three rows on few tiles: a wave per row keeps more compute units busy.  f32, 2 rows of 768 x 768 3.4 / 4.0,
+    // 8192 x 1024 13.6 / 16.0, 1024 x 1536 4.4 / 4.7, but 1024 x 2304 5.2 / 5.1, 2048 x 1152 6.5 / 6.2; 3 rows of 1024 x 1024 4.3 / 4.5,
+    // x 1152 4.9 / 4.6, 64 x 1024 3.1 / 2.9; bf16, 2 rows of 1024 x 256 3.2 / 3.4, but x 1280 3.5 / 3.5, 1536 x 256 4.0 / 3.8.
+    if (!bf && batch <= 3) return w.k <= 256 || (w.n > 1024 && (batch == 3 || w.k > 1024 || w.n > 2048));
+    if (bf && batch == 2) return w.k <= 256 || w.k > 1024 || w.n > 1024;
+    return true;
 }
 // Waves of a plain launch: as many as have two pairs of chunks each.
 static uint32_t gemv_mfma_waves(uint64_t pairs) { return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (pairs + 1) / 2)); }
 bool gemv_takes_f32_rows(const Weight &w, uint64_t rows) {
-    return w.dtype == COEUS_W_F32 && rows <= 16 && gemv_uses_mfma(w, rows, gemv_mfma_waves(w.k / 32));
+    return w.dtype == COEUS_W_F32 && rows >= 2 && rows <= 16 && (rows > 3 || w.n > 63 * 16) && gemv_mfma_shape(w, gemv_mfma_waves(w.k / 32));
 }
 static size_t gemv_mfma_norm_lds(const Weight &w, uint32_t bp, size_t staging) {
     const bool bf = w.dtype == COEUS_W_BF16;
     return (bf ? SplitRows::bytes(bp, w.k) : PlainRows::bytes(bp, w.k)) + std::max((size_t)16 * 16 * 128, staging);
 }
 bool gemv_can_fuse_whole_norm(const Weight &w, uint64_t batch) {
-    if (w.dtype != COEUS_W_F32 || batch < 2 || batch > 16 || !gemv_can_fuse_norm_dense(w, batch) || !gemv_uses_mfma(w, batch, 16)) return false;
+    if (w.dtype != COEUS_W_F32 || batch < 2 || batch > 16 || !gemv_can_fuse_norm_dense(w, batch) || !gemv_uses_mfma(w, batch, 16, true)) return false;
     const uint32_t bp = pad_batch(batch);
     return gemv_mfma_norm_lds(w, bp, gemv_whole_norm_lds(w.k, bp)) <= 160 * 1024;
 }
@@ -2073,9 +2091,9 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
         nf.bias || (nf.y && (!nf.h_out || nf.h_out == nf.h)))
         return fail(COEUS_INVALID_INPUT, "folded hyper-connections: bad arguments or too many streams");
     const uint32_t bp = pad_batch(batch), b = (uint32_t)batch, k = (uint32_t)w.k, nit = hyper_pairs(w.k);
-    // (the matrix-core instance lays its LDS out for two rows: one stays with a wave per weight row, also where gemv_uses_mfma
-    // takes one row of a plain launch; in front of three or four a model's step has a launch of its own)
-    const bool mf = BF16 && nit == 1 && bp == 2 && gemv_uses_mfma(w, batch, 16);
+    // (the matrix-core instance lays its LDS out for two rows: one stays with a wave per weight row, and in front of three or
+    // four a model's step has a launch of its own)
+    const bool mf = BF16 && nit == 1 && bp == 2 && gemv_uses_mfma(w, batch, 16, true);
     const size_t lds = mf ? 16 * 16 * mfma_wave_lds<true>(0) + SplitRows::bytes(bp, k) : (size_t)bp * k * 4;  // (57 KiB at most)
     const uint32_t bs = b | nf.streams << 16;
     const HyperFold *fold = (const HyperFold *)nf.fold;
@@ -2147,7 +2165,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         const uint32_t xbp = std::max(bp, 4u), xq = nf ? 0 : (xbp + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
         const size_t corners = (size_t)mw * 16 * mfma_wave_lds<BF16>(xq),
                      mlds = nf ? gemv_mfma_norm_lds(w, bp, lds) : corners;
-        if (aligned && !(nf && batch == 1) && gemv_uses_mfma(w, batch, nf ? 16 : mw) && mlds <= 160 * 1024) {
+        if (aligned && gemv_uses_mfma(w, batch, nf ? 16 : mw, nf) && mlds <= 160 * 1024) {
             const uint32_t tiles = (uint32_t)ceil_div(w.n, 16), np = (pairs + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
 #define COEUS_MFMA4(BPV, NV, PV, KV)                                                                                          \

@@ -20,9 +20,11 @@ def bound(x, w, k):
 
 
 # one pair of chunks for one wave; waves with unequal shares; shares of 1, 2, 3, 4 and more pairs; weight rows that
-# do not fill a tile; more tiles than workgroups (16 * 4096 rows)
+# do not fill a tile; more tiles than workgroups (16 * 4096 rows); both sides of the lines up to which one, two and three rows
+# stay with a wave per weight row
 @pytest.mark.parametrize("k,n", [(64, 1), (64, 16), (192, 33), (320, 50), (768, 130), (1024, 17), (2048, 70), (2112, 40), (3072, 31),
-                                 (4096, 48), (5632, 20), (11008, 18), (128, 65552), (1024, 5003)])
+                                 (4096, 48), (5632, 20), (11008, 18), (128, 65552), (1024, 5003),
+                                 (256, 1000), (1024, 1024), (1088, 1040), (1024, 2056), (4608, 33), (5184, 33), (16384, 18)])
 @pytest.mark.parametrize("batch", [1, 2, 3, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_F32])
 def test_rows_match_float64(orc, dtype, k, n, batch):
