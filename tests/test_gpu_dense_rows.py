@@ -50,6 +50,41 @@ def test_timed_matmul_is_the_one_that_runs(dtype, rows):
     assert ms.value > 0 and np.array_equal(y.to_host(), w.gemm(x))
 
 
+# A norm in front: the shortest rows that give each of 16 waves a pair of chunks, the longest whose staging fits for 2, 4, 8 and 16 rows,
+# both sides of the lengths at which the staging changes (1024, 2048), shares of up to 8 pairs, and three in flight (a share of
+# three, more than 256 tiles)
+@pytest.mark.parametrize("kind", [_lib.NORM_LAYERNORM, _lib.NORM_RMSNORM])
+@pytest.mark.parametrize("dtype,batch,k,n", [
+    (_lib.W_F32, 16, 512, 18), (_lib.W_F32, 9, 768, 34), (_lib.W_F32, 16, 864, 50), (_lib.W_F32, 8, 1024, 18), (_lib.W_F32, 5, 1056, 40),
+    (_lib.W_F32, 8, 1600, 34), (_lib.W_F32, 4, 2048, 18), (_lib.W_F32, 3, 2080, 40), (_lib.W_F32, 4, 2688, 18), (_lib.W_F32, 2, 4064, 34),
+    (_lib.W_F32, 2, 1536, 4200), (_lib.W_F32, 6, 1504, 4106), (_lib.W_BF16, 8, 1024, 34), (_lib.W_BF16, 5, 1600, 18), (_lib.W_BF16, 4, 2112, 40),
+    (_lib.W_BF16, 3, 2688, 18), (_lib.W_BF16, 2, 2048, 34), (_lib.W_BF16, 2, 2112, 4200), (_lib.W_BF16, 2, 4032, 4106)])
+def test_norm_in_front(orc, dtype, batch, k, n, kind):
+    rng = np.random.default_rng(k + n + kind)
+    w = (rng.standard_normal((k, n)) * 0.05).astype(np.float32)
+    h = (rng.standard_normal((batch, k)) * 3 + 1).astype(np.float32)
+    scale, nbias = rng.uniform(0.5, 1.5, k).astype(np.float32), rng.standard_normal(k).astype(np.float32)
+    wt, wd = Weight(dtype, w), oracle_roundtrip(orc, dtype, w).astype(np.float64)
+    x = h.astype(np.float64)
+    if kind == _lib.NORM_LAYERNORM:
+        x = x - x.mean(1, keepdims=True)
+    x = x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-5) * scale + (nbias if kind == _lib.NORM_LAYERNORM else 0)
+    pre = x @ wd
+    # f32 sums over k of the magnitudes, and the norm's own few roundings of the row
+    e = (3 * k + 40) * 2.0 ** -24 * (np.abs(x) @ np.abs(wd))
+    sd, nd = dev(scale), dev(nbias)
+    for shift, gated in ((0, False), (0, True), (1, False)):  # (rows off a 16-byte boundary take the general kernel)
+        hd, y, fused = dev(np.concatenate([np.zeros(shift, np.float32), h.ravel()])), DeviceArray((batch, n // 2 if gated else n)), C.c_int()
+        _check(_lib.load().coeus_op_norm_gemv(wt.h, hd.ptr + 4 * shift, batch, kind, sd.ptr, nd.ptr, C.c_float(1e-5), None, None,
+                                              _lib.EPI_SILU_GATE if gated else 0, y.ptr, C.byref(fused), None))
+        want, lim = pre, e
+        if gated:
+            g, u = pre[:, 0::2], pre[:, 1::2]
+            want = g / (1 + np.exp(-g)) * u
+            lim = 1.1 * (e[:, 0::2] * np.abs(u) + e[:, 1::2] * np.abs(g)) + 2.0 ** -20 * np.abs(want) + 1e-6
+        assert fused.value == 1 and (np.abs(y.to_host() - want) <= lim).all(), (shift, gated)
+
+
 @pytest.mark.parametrize("batch", [2, 5, 16])
 def test_gated_pairs_and_bias(orc, batch):
     rng = np.random.default_rng(batch)

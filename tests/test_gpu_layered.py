@@ -434,6 +434,26 @@ def test_batches_and_reused_sessions(folder, name, dtype):
     assert off(one.feed(ids[1], want=range(90))[0], want[1]) < LIMIT[dtype]
 
 
+# Steps of several sequences of models wide enough for the matrix cores, the norm behind the sublayer before folded into their matmuls:
+# both sides of the lengths at which its staging changes (1024, 2048), shares of one to five pairs of chunks, more than 256
+# tiles, a query latent whose norm is folded too, rows of one width that fit for 2, 4 and 8
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("width,ff,q_rank,batches", [(512, 40, 512, (5, 8)), (1088, 40, 1024, (2, 3, 4)), (1536, 2100, 1088, (2,)), (2112, 2100, 64, (2,))])
+def test_steps_of_wide_models(tmp_path, dtype, width, ff, q_rank, batches):
+    cfg = config(width, 90, [delta(2, 1, 16, 16, 2, ff=ff), latent(2, 16, 16, q_rank, 32, 5, ff=48)])
+    w = weights(cfg, width)
+    m = load_model(write_folder(str(tmp_path), cfg, w), weight_dtype=dtype, max_seq_len=16, max_batch=8)
+    ids = np.stack([tokens(cfg, 8, 20 + b) for b in range(max(batches))])
+    want = [L.forward(cfg, w, row) for row in ids]
+    for batch in batches:
+        s = m.session(batch=batch, max_ctx=8)
+        s.prefill(ids[:batch, :3], want_logits=False)
+        for i in range(3, 8):
+            got = s.decode(ids[:batch, i])
+            for b in range(batch):
+                assert off(got[b], want[b][i]) < 2.5 * LIMIT[dtype], (batch, i, b)
+
+
 def oracle_greedy(cfg, w, ids, n):
     ids, out, margin = list(ids), [], np.inf
     for _ in range(n):
