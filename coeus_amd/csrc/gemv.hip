@@ -1727,6 +1727,25 @@ __device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__res
     }
 }
 
+static constexpr size_t kDenseNormLdsLimit = 64 * 1024;
+// rows + scale + bias + per-wave partial sums + statistics
+static constexpr size_t gemv_dense_norm_lds(uint64_t k, uint32_t bp) { return ((size_t)(bp + 2) * k + 16 * bp + 32) * 4; }
+static constexpr size_t gemv_dense_post_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)bp * k * 4; }
+// The most pairs of chunks in a row that a folded norm over bp rows leaves room for, and of these in the share of one of 16 waves
+// (0: a wave has none).  Nothing is built for more.
+template <bool BF16>
+static constexpr uint32_t gemv_fold_row_pairs(int norm, uint32_t bp) {
+    const uint64_t ku = MfmaType<BF16>::KU;
+    uint32_t pairs = 0;
+    while ((norm == 3 ? gemv_dense_post_lds((pairs + 1) * ku, bp) : gemv_dense_norm_lds((pairs + 1) * ku, bp)) <= kDenseNormLdsLimit) pairs++;
+    return pairs;
+}
+template <bool BF16>
+static constexpr uint32_t gemv_fold_share(int norm, uint32_t bp) {
+    const uint32_t pairs = gemv_fold_row_pairs<BF16>(norm, bp);
+    return pairs < 16 ? 0 : (pairs + 15) / 16;
+}
+
 // NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
 template <bool BF16, int BP, int NORM, int PD, bool KEEP>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
@@ -1741,8 +1760,9 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType
     uint4 *corners = NORM ? (uint4 *)((char *)mlds + Rows::bytes(BP, k)) : mlds;
     mfma_rows<BF16, PD, KEEP, XQ>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
         if constexpr (NORM != 0) {
-            if (k <= 1024) stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
-            else if (k <= 2048) stage_rows_by_wave<NORM, 8>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
+            constexpr uint32_t LONGEST = gemv_fold_row_pairs<BF16>(NORM, BP) * MfmaType<BF16>::KU;
+            if (LONGEST <= 1024 || k <= 1024) stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
+            else if (LONGEST <= 2048 || k <= 2048) stage_rows_by_wave<NORM, 8>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
             else
                 stage_normed_rows<BP, NORM>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post,
                                             [&](uint32_t b, uint32_t i, float v) { xs.put(b, i, v); });
@@ -1750,10 +1770,6 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType
         }
     });
 }
-
-static const size_t kDenseNormLdsLimit = 64 * 1024;
-// rows + scale + bias + per-wave partial sums + statistics
-static size_t gemv_dense_norm_lds(uint64_t k, uint32_t bp) { return ((size_t)(bp + 2) * k + 16 * bp + 32) * 4; }
 
 // (a norm over all rows: the partial sums in f64)
 static size_t gemv_whole_norm_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)16 * bp * 4; }
@@ -1809,7 +1825,6 @@ bool gemv_can_fuse_whole_norm(const Weight &w, uint64_t batch) {
     const uint32_t bp = pad_batch(batch);
     return gemv_mfma_norm_lds(w, bp, gemv_whole_norm_lds(w.k, bp)) <= 160 * 1024;
 }
-static size_t gemv_dense_post_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)bp * k * 4; }
 bool gemv_can_fuse_post_norm(const Weight &w, uint64_t batch) {
     if (w.dtype >= COEUS_W_Q8_0 || batch < 1 || batch > 16) return false;
     return gemv_dense_post_lds(w.k, pad_batch(batch)) <= kDenseNormLdsLimit;
@@ -2183,7 +2198,13 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
             const uint32_t by2 = (np + 1) / 2 * 2, by3 = (np + 2) / 3 * 3;
             const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && batch > 1 && bp <= 4);
 #define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (BPV < 16 && three) COEUS_MFMA4(BPV < 16 ? BPV : 8, NV, 3, false); else COEUS_MFMA4(BPV, NV, 2, false); } while (0)
-#define COEUS_MFMA(BPV) do { if (norm == 4) { if constexpr (!BF16) COEUS_MFMA3(BPV, 4); } else if (norm == 1) COEUS_MFMA3(BPV, 1); else if (norm == 2) COEUS_MFMA3(BPV, 2); else COEUS_MFMA3(BPV, 3); } while (0)
+#define COEUS_MFMAN(BPV, NV)                                                                               \
+    do {                                                                                                   \
+        if constexpr (gemv_fold_share<BF16>(NV, BPV) > 2) COEUS_MFMA3(BPV, NV);                             \
+        else if constexpr (gemv_fold_share<BF16>(NV, BPV) > 0) COEUS_MFMA4(BPV, NV, 2, true);               \
+        else return fail(COEUS_INVALID_INPUT, "norm fusion needs the normalised activations to fit in LDS"); \
+    } while (0)
+#define COEUS_MFMA(BPV) do { if (norm == 4) { if constexpr (!BF16) COEUS_MFMAN(BPV, 4); } else if (norm == 1) COEUS_MFMAN(BPV, 1); else if (norm == 2) COEUS_MFMAN(BPV, 2); else COEUS_MFMAN(BPV, 3); } while (0)
             if (norm == 0 && bp <= 4) COEUS_MFMA3(4, 0);
             else if (norm == 0 && bp == 8) COEUS_MFMA3(8, 0);
             else if (norm == 0) COEUS_MFMA3(16, 0);
@@ -2192,6 +2213,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
             else if (bp == 8) COEUS_MFMA(8);
             else COEUS_MFMA(16);
 #undef COEUS_MFMA
+#undef COEUS_MFMAN
 #undef COEUS_MFMA3
 #undef COEUS_MFMA4
             COEUS_HIP(hipGetLastError());
