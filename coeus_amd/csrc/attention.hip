@@ -14,6 +14,8 @@
 //                         the per-split (max, sum, partial output) triples.
 #include "device_utils.hpp"
 
+#include <algorithm>
+
 namespace coeus {
 
 template <typename T> __device__ __forceinline__ float kv_load(const T *p);
@@ -713,21 +715,24 @@ uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t hd, uint32_
     // 128 at 500 6.4 / 7.1, 48 of 64 at 960 6.7 / 7.4.
     const uint64_t pairs = batch * heads, key_bytes = max_ctx * hd * (kv_dtype == COEUS_KV_F32 ? 4 : 2);
     if (key_bytes <= (64u << 10) || (pairs >= 64 && key_bytes <= (128u << 10))) return 1;
-    // Else as many as fill the CUs with one workgroup each, a power of two: three splits of 2048 keys (704 + 704 + 640, the
-    // wave tiles no longer line up) ran 17.6 us at batch 8 x 12 heads of 64 against 14.0 us with four.  More than 128
-    // heads stay whole (us, two splits / one of eight waves: 5 x 32 heads of 128 at 700 / 2000 / 4000 keys 14.9 / 33.0 / 63.5
-    // against 11.4 / 28.8 / 53.3; 16 x 12 of 64 at 1000 / 2000 11.3 / 19.1 against 9.3 / 17.1; 4 x 32 of 128 at 2000 24.0 / 27.4).
-    // At context 4096 with 32 heads of 128, batch 1, 8 splits 17.3 us against 17.8 with 16.
+    // More than 128 heads stay whole (us, two splits / one of eight waves: 3 x 43 heads of 64 at 560 / 1000 / 4000 keys 8.2 / 10.7 / 31.0
+    // against 6.5 / 8.1 / 26.1, of 128 12.4 / 17.8 / 58.3 against 9.8 / 14.3 / 48.1; 4 x 56 of 128 15.3 / 21.7 / 73.5 against
+    // 13.1 / 19.7 / 69.3; but 4 x 32 of 128 at 2000 24.0 / 27.4).
     if (pairs > 128) return 1;
+    // Else as many as fill the CUs with one workgroup each, a power of two: three splits of 2048 keys (704 + 704 + 640, the
+    // wave tiles no longer line up) ran 17.6 us at batch 8 x 12 heads of 64 against 14.0 us with four.
+    // At context 4096 with 32 heads of 128, batch 1, 8 splits 17.3 us against 17.8 with 16.
     uint64_t want = ceil_div(256, pairs);
     while (want & (want - 1)) want++;
-    // 256 keys per split, but 128 up to eight splits (us per launch, 256 / 128 keys: 32 heads of 128 at 520 keys 8.3 / 7.0,
-    // at 1080 9.3 / 8.3; 12 heads of 64 at 560 5.9 / 5.3; at 2025, sixteen splits against eight, 7.3 / 6.3)
-    uint64_t cap = ceil_div(max_ctx, 256);
-    const uint64_t fine = ceil_div(max_ctx, 128);
-    if (cap < 8) cap = fine < 8 ? fine : 8;
+    // 256 keys per split, but 128 up to eight splits of one workgroup per CU (us per launch, 256 / 128 keys: 32 heads of 128
+    // at 520 keys 8.3 / 7.0, at 1080 9.3 / 8.3; 12 heads of 64 at 560 5.9 / 5.3; at 2025, sixteen splits against eight, 7.3 / 6.3; beyond
+    // a workgroup per CU 48 heads of 128 at 1000 8.6 / 9.3, 8 x 12 of 128 at 640 9.8 / 10.4).  Four splits of 256 keys are as fast as eight
+    // for more than 16 heads in 16 bits (32 heads of 64 / of 128 at 1000 keys 6.4 / 6.8 and 7.7 / 8.1, but 12 of 128 6.9 / 6.6, in f32
+    // at 900 9.4 / 7.1).
+    const uint64_t most = pairs > 16 && kv_dtype != COEUS_KV_F32 && max_ctx <= 1024 ? 4 : 8;
+    const uint64_t cap = ceil_div(max_ctx, 256), fine = std::min(most, ceil_div(max_ctx, 128));
     uint64_t s = 1;
-    while (s * 2 <= want && s * 2 <= cap && s * 2 <= kAttnMaxSplits) s *= 2;
+    while (s * 2 <= want && (s * 2 <= cap || (s * 2 <= fine && s * 2 * pairs <= 256)) && s * 2 <= kAttnMaxSplits) s *= 2;
     return (uint32_t)s;
 }
 

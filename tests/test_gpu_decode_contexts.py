@@ -35,10 +35,12 @@ def test_steps_match_prompt_pass(heads, hd, max_ctx, kv):
             assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), (ctx, b)
 
 
-@pytest.mark.parametrize("heads,hd,max_ctx", [(4, 64, 1024), (4, 64, 1025), (4, 128, 512), (8, 64, 1030), (9, 64, 1500), (9, 128, 700)])
+@pytest.mark.parametrize("heads,hd,max_ctx", [(4, 64, 1024), (4, 64, 1025), (4, 128, 512), (8, 64, 1030), (9, 64, 1500), (9, 128, 700),
+                                              (2, 64, 1000), (2, 128, 1030), (3, 64, 1025), (6, 128, 640)])
 @pytest.mark.parametrize("kv", ["f32", "f16"])
 def test_many_heads_match_prompt_pass(heads, hd, max_ctx, kv):
-    # 16 sequences: 64 heads and up to 128 KiB of keys a head whole, 64 - 128 heads split beyond that, more than 128 whole
+    # 16 sequences: 64 heads and up to 128 KiB of keys a head whole, 64 - 128 heads split beyond that, more than 128 whole;
+    # 32 heads in four splits up to 1024 keys (f32: eight) and eight beyond, 48 in four, 96 in two
     cfg = Transformer250MConfig(hidden_dim=heads * hd, num_layers=1, num_heads=heads, intermediate_dim=256, vocab_size=160,
                                 max_seq_len=max_ctx, norm_scope="token", max_batch=16, kv_dtype=kv)
     model = TransformerModelPlugin().create_builder().build(cfg, seed=6)
