@@ -1377,12 +1377,16 @@ static bool gemm_uses_h256(const Weight &w, uint64_t m) {
 // and a second kernel sums them in split order (deterministic) and runs the epilogue.  At least 8
 // slices per split (the request pipeline is 3 deep), at most 16 splits, no more workgroups than CUs (one workgroup
 // fills a CU's LDS).  Each split adds a plane of m x n floats to write and read back: of the splits that fit, the one
-// with the shortest sum of 0.6 us per slice, 4.5 us for the second launch and the planes at 5.5 TB/s (us, the most
+// with the shortest sum of 0.6 us per slice of the longest share, 4.5 us for the second launch and the planes at 5.5 TB/s (us, the most
 // splits that fit / this rule: 201 rows of 4096 x 4096 34.6 / 31.5, of 768 x 3072 22.9 / 22.9; 512 rows of 768 x 3072
-// 29.5 / 24.9; 2000 rows of 768 x 2304 35.4 / 28.0).
+// 29.5 / 24.9; 2000 rows of 768 x 2304 35.4 / 28.0).  k % 64 == 0: shares are made of 64-wide slices (counted in 32s, 256 rows of
+// 2048 x 3072 got six uneven shares instead of eight even ones, 29.3 against 27.4 us; 700 of 1024 x 2048 three instead of four, 31.1 /
+// 29.2).  Over 389 launches of 24 matrices and 65 - 2000 rows, each timed with every number of splits that fits: 0.7 % above the
+// fastest one on average (most that fit 2.9 %, counted in 32s 0.9 %), 8 % at worst; 16 of them are 2 - 7 % slower than with the
+// most that fit (256 rows of 1536 x 4096 28.4 with six, 30.2 with the four of this rule).
 static uint32_t gemm_splits_wanted(const Weight &w, uint64_t m) {
     if (!gemm_uses_h256(w, m)) return 1;
-    const uint64_t tiles = ceil_div(m, TM) * ceil_div(w.n, TN), slices = w.k / TK;
+    const uint64_t tiles = ceil_div(m, TM) * ceil_div(w.n, TN), slices = w.k / TK, unit = w.k % UK == 0 ? UK / TK : 1;
     if (tiles > 128) return 1;
     uint64_t most = 256 / tiles;
     if (most > slices / 8) most = slices / 8;
@@ -1390,7 +1394,7 @@ static uint32_t gemm_splits_wanted(const Weight &w, uint64_t m) {
     uint32_t best = 1;
     double best_us = 0.6 * (double)slices;
     for (uint64_t s = 2; s <= most; s++) {
-        const double us = 0.6 * (double)ceil_div(slices, s) + 4.5 + (double)(s * m * w.n) * 8.0 / 5.5e6;
+        const double us = 0.6 * (double)(ceil_div(slices / unit, s) * unit) + 4.5 + (double)(s * m * w.n) * 8.0 / 5.5e6;
         if (us < best_us) { best_us = us; best = (uint32_t)s; }
     }
     return best;
