@@ -10,7 +10,7 @@ decode step (one new token per sequence: every linear weight streamed once, atte
 cached context).  W warm-up steps and K timed steps run as one greedy generation on the device.
 
 Prints ONE JSON line: whole-job tokens/s plus
-  roofline     - the decode matmul (gemv_quant_kernel): algorithmic bytes per launch / average
+  roofline     - the decode matmul (gemv_rows_kernel): algorithmic bytes per launch / average
                  launch duration, timed live with HIP events on the stream the kernels run on
                  (a captured graph of one step's 129 matmul launches, replayed), against 8 TB/s;
   prefill      - the prompt pass of the same run (tokens/s) and the matrix-core roofline of its
@@ -324,7 +324,7 @@ def decode_workload(name, batches, K, W, use_graph, check):
             "value": round(B * K / dt, 2), "unit": "tok/s", "ms_per_step": round(dt * 1e3 / K, 4),
             "prefill": {"tokens": int(B * prompt.shape[1]), "ms": round(prefill_s * 1e3, 2),
                         "tok_s": round(B * prompt.shape[1] / prefill_s, 1)},
-            "roofline": {"kernel": (("gemv_quad_kernel" if B <= 4 else "gemv_quant_kernel") if quant
+            "roofline": {"kernel": (("gemv_quad_kernel" if B <= 4 else "gemv_rows_kernel") if quant
                                     else "gemv_dense_kernel, gemv_row_kernel, gemv_mfma_kernel"),
                          "bound": "hbm",
                          "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -561,7 +561,7 @@ def main():
     ms, launches, alg_bytes = sess.time_decode_matmuls(reps)
     achieved = alg_bytes / (ms * 1e-3) / 1e9
     roofline = {
-        "kernel": (("gemv_quad_kernel" if B <= 4 else "gemv_quant_kernel") if cfg.weight_dtype in ("q4_0", "q8_0")
+        "kernel": (("gemv_quad_kernel" if B <= 4 else "gemv_rows_kernel") if cfg.weight_dtype in ("q4_0", "q8_0")
                    else "gemv_dense_kernel, gemv_row_kernel, gemv_mfma_kernel"),
         "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "traffic_source": None,
@@ -637,7 +637,7 @@ def main():
                 leg["roofline"]["traffic"] = json.load(f)["hbm_bytes_per_launch"]
             leg["roofline"]["traffic_source"] = f"{arel}: rocprofv3 FETCH_SIZE + WRITE_SIZE of the same command, offline"
         mms, mlaunches, mbytes = s16.time_decode_matmuls(reps)
-        leg["matmul_roofline"] = {"kernel": "gemv_quant_kernel", "bound": "hbm",
+        leg["matmul_roofline"] = {"kernel": "gemv_rows_kernel", "bound": "hbm",
                                   "achieved": round(mbytes / (mms * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS,
                                   "unit": "GB/s", "frac": round(mbytes / (mms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                                   "bytes_per_launch": mbytes // mlaunches,

@@ -6,16 +6,13 @@
 //                      wave owns four consecutive 128-k chunks, stages exactly their activations
 //                      (with or without the folded norm) into its private slice of LDS and feeds
 //                      the quants to v_mfma_f32_16x16x32_f16 as f16 subnormals.
-//   gemv_quant_kernel  the same weights for batches of 5 to 16.  One workgroup owns a tile of
-//                      16 output rows (or four); its waves take interleaved 128-k chunks (1 KiB
-//                      of Q4_0 quants = one fully coalesced 16 B/lane load per wave).  Each 32-k
-//                      block is one v_mfma_f32_16x16x32_f16 between the 16 activation rows (f16)
-//                      and the block's integers (q-8 resp. q, exact in f16); the f32 block result
-//                      is scaled by the block's f16 scale on the VALU.  Activation rows come from
-//                      LDS (staged once per workgroup) or, when they do not fit, from L2 product
-//                      by product; there a workgroup takes four tiles and a wave multiplies each
-//                      fragment with all four.  In both kernels the value used for every weight is
-//                      exactly its dequantised value q*d.
+//   gemv_rows_kernel   the same weights for batches of 5 to 16.  One workgroup owns one to six tiles
+//                      of 16 output rows; its waves take 128-k chunks (1 KiB of Q4_0 quants = one
+//                      fully coalesced 16 B/lane load per wave).  Each 32-k block is one
+//                      v_mfma_f32_16x16x32_f16 between the 16 activation rows (f16, straight from
+//                      L2 into registers) and the block's integers (q-8 resp. q, exact in f16); the
+//                      f32 block result is scaled by the block's f16 scale on the VALU.  In both
+//                      kernels the value used for every weight is exactly its dequantised value q*d.
 //   gemv_dense_kernel  f32 / bf16 weights, one wave per output row, f32 FMA on the VALU.
 //   gemv_row_kernel    one activation row behind a norm of up to 1024 elements: the row in every
 //                      wave's registers, no LDS and no barrier.
@@ -78,11 +75,7 @@ __device__ __forceinline__ half8_t unpack_q8(uint32_t lo, uint32_t hi) {
     return out;
 }
 
-// One chunk = 16 rows x 128 k.  Matrix-core roles: A = activations (row = batch entry),
-// B = weights (column = weight row), so lane (j = lane%16, ig = lane/16) ends up holding the
-// results of weight row j for batch entries 4*ig..4*ig+3, and a block's scale is ONE value per
-// lane.  Activations come from LDS when the whole reduction run fits (staged once per
-// workgroup, overlapped with the first weight loads), from global memory (L2) otherwise.
+// One chunk = 16 weight rows x 128 k, as a wave holds it.
 template <bool Q4>
 struct ChunkRegs {
     uint4 q0, q1;  // q1 only for Q8_0
@@ -106,14 +99,13 @@ __device__ __forceinline__ void load_chunk(ChunkRegs<Q4> &r, const uint4 *__rest
     r.s = make_uint2(sv.x, sv.y);
 }
 
-// How the activation block reaches the matrix cores.
-enum { X_GLOBAL = 0,  // xq read from global memory (L2) per block: no LDS needed, any size (gemv_quant_kernel)
-       X_LDS = 1,     // xq copied into LDS (once per workgroup; gemv_quad_kernel: each wave its own pieces)
-       X_LAYERNORM = 2, X_RMSNORM = 3,    // gemv_quad_kernel: f32 residual rows normalised while staged into LDS
-       X_RMSPRE = 4 };  // gemv_quad_kernel: rows that their producer stored as h * scale: times 1 / rms while staged
+// How the activation block reaches the matrix cores in gemv_quad_kernel.
+enum { X_LDS = 1,     // xq: each wave copies its own pieces into LDS
+       X_LAYERNORM = 2, X_RMSNORM = 3,    // f32 residual rows normalised while staged into LDS
+       X_RMSPRE = 4 };  // rows that their producer stored as h * scale: times 1 / rms while staged
 
 struct XArgs {
-    const uint4 *xq;      // X_GLOBAL / X_LDS
+    const uint4 *xq;      // X_LDS
     const float *h;       // X_*NORM: [batch, k]; X_RMSPRE: the rows times the norm's scale
     const float *nscale, *nbias;
     const float2 *stats;  // X_*NORM: [batch][ceil(k/16)] {sum, M2} records of h
@@ -189,243 +181,120 @@ int launch_norm_from_stats(const NormFuse &nf, uint64_t batch, uint64_t k, uint6
     return COEUS_OK;
 }
 
-// Compile-time shape of one gemv_quant_kernel variant, packed into an int:
-//   bit 0     always set
-//   bit 5     two tiles per workgroup
-//   bit 6     6 chunks in flight per wave instead of 4 (Q8_0: 3 instead of 2)
-//   bit 7     2 chunks in flight per wave instead of 4 (Q8_0: 1): short reductions, where the waves
-//             of a workgroup cover k in fewer chunks and the extra requests would be re-reads
-//   bit 8     four tiles per workgroup (activations from global memory only)
-constexpr int CFG_TPW2 = 32, CFG_PF6 = 64, CFG_PF2 = 128, CFG_TPW4 = 256;
-
-// One workgroup takes TPW tiles of 16 output rows; several workgroups share a CU, so that the
-// staging and the epilogue of one overlap with the weight stream of the others (the register
-// budget is capped to keep 6-8 waves per SIMD resident).  With TPW = 2 the activation block is
-// staged once for two tiles and both tiles' chunks are requested before either is used.
-// Activations that do not fit LDS are read from global memory (L2) product by product; there a
-// wave takes its chunks of all TPW tiles (2 or 4), so that one activation fragment (1 KiB per
-// product at 16 batch rows, against 288 bytes of Q4_0 weights) serves TPW products.
-template <bool Q4, int BP, int XMODE, int CFG>
-__global__ __launch_bounds__(1024)
-__attribute__((amdgpu_waves_per_eu((XMODE == X_GLOBAL && (CFG & (CFG_TPW2 | CFG_TPW4))) ? 4 : 6, 8)))
-void gemv_quant_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds, XArgs xa,
-                       uint32_t ngroups, uint32_t tiles, uint32_t batch, EpiArgs e) {
+// ---------------------------------------------------------------- batches of 5 to 16
+// Bound by the trips to memory that a wave makes one behind the other and, for long reductions, by the activation rows
+// that every workgroup reads from L2 (16 rows x 11008 x 2 B = 352 KB next to 99 KB of Q4_0 weights).  So nothing is staged:
+// a wave asks for the four activation fragments of its chunk and for the chunk's weights in its TPW tiles at once, 16 bytes
+// a lane each, and multiplies as they arrive; a fragment is read once per workgroup and serves TPW products.  Matrix-core
+// roles: A = activations (row = batch entry), B = weights (column = weight row), so lane (j = lane % 16, ig = lane / 16)
+// ends up with the results of weight row j for batch entries 4 ig .. 4 ig + 3, and a block's scale is ONE value per lane.
+// The waves' sums meet in LDS, added in wave order; every thread then finishes outputs of its own, whose residual and bias
+// were requested at the start.  Chains of real shapes, one job, us a launch with the launch in front (before: activations
+// staged in LDS where they fit in 48 KiB, two to six chunks a wave in flight, sums and epilogue on one wave a tile):
+//   16 rows, Q4_0: 4096 x 12288 14.2 -> 11.8, 4096 x 4096 9.2 -> 8.6, 4096 x 22016 gated 20.9 -> 16.3, 11008 x 4096 15.6 -> 14.3
+//    8 rows, Q8_0: 768 x 2304 6.8 -> 6.0, 768 x 768 7.6 -> 6.0, 768 x 3072 7.2 -> 6.5, 3072 x 768 9.1 -> 7.2, 768 x 50257 14.4 -> 12.6
+template <bool Q4, int BP, int TPW>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 8)))
+void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds, const uint4 *__restrict__ xq, uint32_t ngroups,
+                      uint32_t tiles, uint32_t batch, EpiArgs e) {
     static_assert(BP == 8 || BP == 16, "batches of up to 4 take gemv_quad_kernel");
-    static_assert(XMODE == X_GLOBAL || XMODE == X_LDS, "activations from L2 or staged in LDS");
-    constexpr int NI = 4;  // accumulator rows of a lane
-    constexpr bool XLDS = XMODE != X_GLOBAL;
-    constexpr int TPW = (CFG & CFG_TPW4) ? 4 : (CFG & CFG_TPW2) ? 2 : 1;
-    constexpr bool SHARE_X = XMODE == X_GLOBAL && TPW > 1;
-    extern __shared__ uint4 smem[];      // [x: ngroups*16*BP uint4 if XLDS][reduction]
+    extern __shared__ float rows_red[];  // [TPW][nwaves][4][64]
     const uint32_t lane = threadIdx.x & 63, nwaves = blockDim.x >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t T0 = blockIdx.x * TPW;
-    const uint32_t g = lane >> 4, xb = (lane & 15) & (BP - 1);
-    float acc[NI];
-#pragma unroll
-    for (int i = 0; i < NI; i++) acc[i] = 0.f;
+    const uint32_t T0 = blockIdx.x * TPW, j = lane & 15, ig = lane >> 4, xb = j & (BP - 1);
     const float4_t zero = {0.f, 0.f, 0.f, 0.f};
-    const uint4 *__restrict__ xq = xa.xq;
-    const uint32_t nx = ngroups * 16 * BP;  // uint4 pieces of the activation block
-    float *red = (float *)(smem + (XLDS ? nx : 0));  // [TPW][nwaves][NI][64]
-
-    // 0. the residual elements this wave will need if it runs a tile's epilogue (wave t < TPW
-    // finishes tile T0 + t): requested now, unconditionally (other waves repeat wave 0's, a
-    // missing residual reads a valid dummy), so the epilogue does not wait for a load of its own
-    constexpr bool RES_PRE = true;
-    float res_pre[NI];
+    // Output o of the workgroup = (tile, batch row, column); a thread finishes o = threadIdx.x and every blockDim.x-th behind it.
+    constexpr uint32_t OUTS = TPW * 16 * BP;
+    const bool gated = e.act == COEUS_EPI_SILU_GATE;
+    const uint32_t kvpos = (e.kv_k && !e.kv_rows_per_seq) ? *e.kv_pos : 0u;
+    float res_pre, bias_pre;  // of the first output (loads unconditional, from a valid address)
     {
-        const float *rp = e.residual ? e.residual : (const float *)ds;
-        const uint32_t Tw = min(T0 + (wave < (uint32_t)TPW ? wave : 0u), tiles - 1);
-        const uint64_t jp = (uint64_t)Tw * 16 + (lane & 15);
-#pragma unroll
-        for (int i = 0; i < NI; i++) {
-            const uint32_t b = 4 * g + i;
-            const bool ok = e.residual && b < batch && jp < e.n;
-            res_pre[i] = rp[ok ? (uint64_t)b * e.n_eff + jp : 0];
-        }
+        const uint32_t o = threadIdx.x < OUTS ? threadIdx.x : 0, b = o / 16 % BP;
+        const uint64_t col = (uint64_t)(T0 + o / (16 * BP)) * 16 + (o & 15);
+        const bool ok = e.residual && !gated && b < batch && col < e.n;
+        const float *rp = ok ? e.residual : (const float *)ds, *bp = e.bias ? e.bias : (const float *)ds;
+        res_pre = rp[ok ? (uint64_t)b * e.n_eff + col : 0];
+        bias_pre = bp[(e.bias && col < e.n) ? col : 0];
     }
-
-    // 1. activations first: a wave's loads are answered in order, and these are needed first
-    constexpr int XPT = 2;
-    uint4 xr[XPT];
-    if (XMODE == X_LDS) {
+    float acc[TPW][4];
+    uint64_t cb[TPW];
 #pragma unroll
-        for (int u = 0; u < XPT; u++) {
-            const uint32_t i = threadIdx.x + u * blockDim.x;
-            xr[u] = xq[i < nx ? i : 0];  // unconditional, from a clamped address (see step 2)
-        }
+    for (int t = 0; t < TPW; t++) {
+        cb[t] = (uint64_t)min(T0 + t, tiles - 1) * ngroups;
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[t][i] = 0.f;
     }
-    auto stage = [&]() {
-        if (XMODE == X_LDS) {
+#pragma unroll 1
+    for (uint32_t G = wave; G < ngroups; G += nwaves) {
+        uint4 xv[4];
+        ChunkRegs<Q4> r[TPW];
 #pragma unroll
-            for (int u = 0; u < XPT; u++) {
-                const uint32_t i = threadIdx.x + u * blockDim.x;
-                if (i < nx) smem[i] = xr[u];
-            }
-            for (uint32_t i = threadIdx.x + XPT * blockDim.x; i < nx; i += blockDim.x) smem[i] = xq[i];
-        }
-        if (XLDS) lds_barrier();
-    };
-
-    // 2. PF chunks (PF KiB of Q4_0 quants per wave and tile) are requested before any of them is
-    // used.  Passes in which every wave has all its chunks use unconditional loads: the compiler
-    // then knows exactly how many loads are in flight, and the staging and the first chunks are
-    // used while later ones are still on their way.  (A load under a branch makes it wait for
-    // everything.)  Only a last partial pass loads under wave-uniform branches.
-    constexpr int PF = (CFG & CFG_PF6) ? (Q4 ? 6 : 3) : (CFG & CFG_PF2) ? (Q4 ? 2 : 1) : (Q4 ? 4 : 2);
-    auto consume = [&](const ChunkRegs<Q4> &r, uint32_t G) {
-        const uint32_t qw[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, Q4 ? 0u : r.q1.x, Q4 ? 0u : r.q1.y,
-                                Q4 ? 0u : r.q1.z, Q4 ? 0u : r.q1.w};
-        union { uint2 u2; half2_t h[2]; } sc;
-        sc.u2 = r.s;
-        const float d[4] = {(float)sc.h[0].x, (float)sc.h[0].y, (float)sc.h[1].x, (float)sc.h[1].y};
+        for (int jj = 0; jj < 4; jj++) xv[jj] = xq[((G * 4 + jj) * 4 + ig) * BP + xb];
+#pragma unroll
+        for (int t = 0; t < TPW; t++) load_chunk<Q4>(r[t], qs, ds, cb[t] + G, lane);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int jj = 0; jj < 4; jj++) {
-            const uint32_t xi = ((G * 4 + jj) * 4 + g) * BP + xb;
-            union { uint4 u4; half8_t h; } xv;
-            xv.u4 = XLDS ? smem[xi] : xq[xi];
-            const half8_t wv = Q4 ? unpack_q4(qw[jj]) : unpack_q8(qw[2 * jj], qw[2 * jj + 1]);
-            const float4_t part = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv.h, wv, zero, 0, 0, 0);
+            if (TPW == 4) __builtin_amdgcn_sched_barrier(0);  // (Q8_0: without it the unpacked operands of two blocks live at once and spill)
+            union { uint4 u4; half8_t h; } x;
+            x.u4 = xv[jj];
 #pragma unroll
-            for (int i = 0; i < NI; i++) acc[i] = fmaf(d[jj], part[i], acc[i]);
-        }
-    };
-    // a tile's partial result of this wave, parked for the cross-wave sum
-    auto park = [&](int t) {
-#pragma unroll
-        for (int i = 0; i < NI; i++) {
-            red[((t * nwaves + wave) * NI + i) * 64 + lane] = acc[i];
-            acc[i] = 0.f;
-        }
-    };
-    if constexpr (SHARE_X) {
-        // a wave's chunk G of every tile, against one set of activation fragments
-        constexpr int PFS = (!Q4 && TPW == 4) ? 1 : 2;  // chunks of a tile in flight per wave
-        float accs[TPW][NI];
-        uint64_t cb[TPW];
-#pragma unroll
-        for (int t = 0; t < TPW; t++) {
-            cb[t] = (uint64_t)min(T0 + t, tiles - 1) * ngroups;
-#pragma unroll
-            for (int i = 0; i < NI; i++) accs[t][i] = 0.f;
-        }
-        auto pass = [&](uint32_t Gp, auto full) {
-            ChunkRegs<Q4> r[PFS][TPW];
-            uint4 xv[PFS][4];
-#pragma unroll
-            for (int u = 0; u < PFS; u++) {
-                const uint32_t G = Gp + u * nwaves;
-                if (decltype(full)::value || G < ngroups) {
-#pragma unroll
-                    for (int jj = 0; jj < 4; jj++) xv[u][jj] = xq[((G * 4 + jj) * 4 + g) * BP + xb];
-#pragma unroll
-                    for (int t = 0; t < TPW; t++) load_chunk<Q4>(r[u][t], qs, ds, cb[t] + G, lane);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < PFS; u++) {
-                if (decltype(full)::value || Gp + u * nwaves < ngroups) {
-#pragma unroll
-                    for (int t = 0; t < TPW; t++) {
-                        const ChunkRegs<Q4> &c = r[u][t];
-                        const uint32_t qw[8] = {c.q0.x, c.q0.y, c.q0.z, c.q0.w, Q4 ? 0u : c.q1.x, Q4 ? 0u : c.q1.y,
-                                                Q4 ? 0u : c.q1.z, Q4 ? 0u : c.q1.w};
-                        union { uint2 u2; half2_t h[2]; } sc;
-                        sc.u2 = c.s;
-                        const float d[4] = {(float)sc.h[0].x, (float)sc.h[0].y, (float)sc.h[1].x, (float)sc.h[1].y};
-#pragma unroll
-                        for (int jj = 0; jj < 4; jj++) {
-                            union { uint4 u4; half8_t h; } xf;
-                            xf.u4 = xv[u][jj];
-                            const half8_t wv = Q4 ? unpack_q4(qw[jj]) : unpack_q8(qw[2 * jj], qw[2 * jj + 1]);
-                            const float4_t part = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf.h, wv, zero, 0, 0, 0);
-#pragma unroll
-                            for (int i = 0; i < NI; i++) accs[t][i] = fmaf(d[jj], part[i], accs[t][i]);
-                        }
-                    }
-                }
-            }
-        };
-        uint32_t Gp = wave;
-        for (; Gp + (PFS - 1) * nwaves < ngroups; Gp += nwaves * PFS) pass(Gp, std::true_type{});
-        if (Gp < ngroups) pass(Gp, std::false_type{});
-#pragma unroll
-        for (int t = 0; t < TPW; t++)
-#pragma unroll
-            for (int i = 0; i < NI; i++) red[((t * nwaves + wave) * NI + i) * 64 + lane] = accs[t][i];
-    } else {
-        uint32_t G0 = wave;  // < ngroups: a workgroup never has more waves than chunks
-        {   // first pass, always with unconditional loads (a slot past the end re-reads a valid
-            // chunk and is not used)
-            ChunkRegs<Q4> r[TPW][PF];
-    #pragma unroll
             for (int t = 0; t < TPW; t++) {
-                const uint64_t cbase = (uint64_t)min(T0 + t, tiles - 1) * ngroups;
-    #pragma unroll
-                for (int u = 0; u < PF; u++)
-                    load_chunk<Q4>(r[t][u], qs, ds, cbase + min(G0 + u * nwaves, ngroups - 1), lane);
-            }
-            stage();
-    #pragma unroll
-            for (int t = 0; t < TPW; t++) {
-    #pragma unroll
-                for (int u = 0; u < PF; u++)
-                    if (G0 + u * nwaves < ngroups) consume(r[t][u], G0 + u * nwaves);
-                if (TPW > 1) park(t);  // two tiles per workgroup: the reduction takes a single pass
+                const ChunkRegs<Q4> &c = r[t];
+                const uint32_t qw[8] = {c.q0.x, c.q0.y, c.q0.z, c.q0.w, Q4 ? 0u : c.q1.x, Q4 ? 0u : c.q1.y,
+                                        Q4 ? 0u : c.q1.z, Q4 ? 0u : c.q1.w};
+                union { uint2 u2; _Float16 h[4]; } s;
+                s.u2 = c.s;
+                const half8_t wv = Q4 ? unpack_q4(qw[jj]) : unpack_q8(qw[2 * jj], qw[2 * jj + 1]);
+                const float4_t part = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.h, wv, zero, 0, 0, 0);
+                const float d = (float)s.h[jj];
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[t][i] = fmaf(d, part[i], acc[t][i]);
             }
         }
-        if (TPW == 1) {
-            const uint64_t cbase = (uint64_t)T0 * ngroups;
-            for (G0 += nwaves * PF; G0 + (PF - 1) * nwaves < ngroups; G0 += nwaves * PF) {
-                ChunkRegs<Q4> r[PF];
-    #pragma unroll
-                for (int u = 0; u < PF; u++) load_chunk<Q4>(r[u], qs, ds, cbase + G0 + u * nwaves, lane);
-    #pragma unroll
-                for (int u = 0; u < PF; u++) consume(r[u], G0 + u * nwaves);
-            }
-            if (G0 < ngroups) {  // partial last pass
-                ChunkRegs<Q4> r[PF];
-    #pragma unroll
-                for (int u = 0; u < PF; u++)
-                    if (G0 + u * nwaves < ngroups) load_chunk<Q4>(r[u], qs, ds, cbase + G0 + u * nwaves, lane);
-    #pragma unroll
-                for (int u = 0; u < PF; u++)
-                    if (G0 + u * nwaves < ngroups) consume(r[u], G0 + u * nwaves);
-            }
-        }
-
     }
-
-    // deterministic cross-wave reduction (fixed order); wave t runs the epilogue of tile T0 + t
-    uint32_t T = T0;
-    if (nwaves > 1 || TPW > 1) {
-        if (TPW == 1) park(0);  // (several tiles: parked above)
-        lds_barrier();
-        if (wave >= (uint32_t)TPW) return;
-        T = T0 + wave;
-        if (T >= tiles) return;
-        for (uint32_t w = 0; w < nwaves; w++)
 #pragma unroll
-            for (int i = 0; i < NI; i++) acc[i] += red[((wave * nwaves + w) * NI + i) * 64 + lane];
-    }
-    const uint64_t j = (uint64_t)T * 16 + (lane & 15);
-    const bool gated = e.act == COEUS_EPI_SILU_GATE;
+    for (int t = 0; t < TPW; t++)
 #pragma unroll
-    for (int i = 0; i < NI; i++) {
-        const uint32_t b = 4 * g + i;
-        // gated: weight rows (2m, 2m+1) = (gate_m, up_m) sit in neighbouring lanes
-        const float other = lane_xor1(acc[i]);
-        const bool live = b < batch && j < e.n;
+        for (int i = 0; i < 4; i++) rows_red[((t * nwaves + wave) * 4 + i) * 64 + lane] = acc[t][i];
+    lds_barrier();
+    // q|k|v of sizes that are no multiples of 16: a tile may hold columns of two parts or heads
+    const bool kv_odd = e.kv_k && ((e.kv_inner | e.kv_hd) & 15u);
+    for (uint32_t o = threadIdx.x; o < OUTS; o += nwaves * 64) {  // (whole waves: OUTS is a multiple of 64)
+        const uint32_t t = o / (16 * BP), b = o / 16 % BP, T = T0 + t;
+        const uint64_t col = (uint64_t)T * 16 + (o & 15);
         float v = 0.f;
+        for (uint32_t w = 0; w < nwaves; w++) v += rows_red[((t * nwaves + w) * 4 + (b & 3)) * 64 + (b >> 2) * 16 + (o & 15)];
+        const bool live = b < batch && col < e.n, first = o == threadIdx.x;
+        if (e.kv_k && (kv_odd || T * 16 >= e.kv_inner)) {
+            if (live) epi_store<true>(e, b, col, v, first, res_pre, !e.kv_rows_per_seq, kvpos);
+            continue;
+        }
+        if (e.bias) v += first ? bias_pre : live ? e.bias[col] : 0.f;
+        if (gated) {
+            // weight rows (2m, 2m+1) = (gate_m, up_m) sit in neighbouring lanes
+            const float up = lane_xor1(v);
+            if (live && (o & 1) == 0) {
+                const uint64_t m = col >> 1;
+                float g = fast_silu(v) * up;
+                if (e.residual) g += e.residual[(uint64_t)b * e.n_eff + m];
+                if (e.out_f32) e.out_f32[(uint64_t)b * e.n_eff + m] = g;
+                if (e.out_xq) e.out_xq[xq_index(m, b, e.bp_out)] = __float2half_rn(g);
+                if (e.out_lp) e.out_lp[(uint64_t)b * e.lp_ld + m] = f32_to_lp_bits(g, e.lp_bf16);
+            }
+            continue;
+        }
+        if (e.act == COEUS_EPI_GELU) v = fast_gelu(v);
+        if (e.residual) v += first ? res_pre : live ? e.residual[(uint64_t)b * e.n_eff + col] : 0.f;
         if (live) {
-            if (!gated) v = epi_store<true>(e, b, j, acc[i], RES_PRE, res_pre[i]);
-            else if ((lane & 1) == 0) epi_store_gated(e, b, j >> 1, acc[i], other);
+            if (e.out_f32) e.out_f32[(uint64_t)b * e.n_eff + col] = v;
+            if (e.out_xq) e.out_xq[xq_index(col, b, e.bp_out)] = __float2half_rn(v);
+            if (e.out_lp) e.out_lp[(uint64_t)b * e.lp_ld + col] = f32_to_lp_bits(v, e.lp_bf16);
         }
         if (e.stats_out) {  // uniform; never combined with the gated epilogue
-            const uint32_t left = (uint32_t)e.n - T * 16;
-            const float2 r = group16_stats(v, live, left < 16 ? left : 16u);
-            if ((lane & 15) == 0 && b < batch) e.stats_out[(uint64_t)b * e.stats_tiles + T] = r;
+            const uint32_t left = (uint32_t)e.n - T * 16;  // (a tile past the end: unused)
+            const float2 r = group16_stats(live ? v : 0.f, live, left < 16 ? left : 16u);
+            if ((o & 15) == 0 && live) e.stats_out[(uint64_t)b * e.stats_tiles + T] = r;
         }
     }
 }
@@ -793,16 +662,6 @@ void gemv_quad_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds
 
 static const size_t kXLdsLimit = 48 * 1024;
 
-// Waves per workgroup of gemv_quant_kernel: enough waves to cover the chip several times over, at
-// least 2 chunks per wave.
-static uint32_t gemv_quant_waves(const Weight &w) {
-    const uint32_t ngroups = (uint32_t)(w.k_pad / 128), tiles = (uint32_t)(w.n_pad / 16);
-    uint32_t waves = 4;
-    while (waves < 16 && (uint64_t)tiles * waves < 4096 && ngroups >= waves * 4) waves *= 2;
-    while (waves > 1 && waves > ngroups) waves /= 2;
-    return waves;
-}
-
 bool gemv_can_fuse_norm(const Weight &w, uint64_t batch) {
     if (w.dtype < COEUS_W_Q8_0 || batch < 1 || batch > 16) return false;
     const uint32_t bp = pad_batch(batch);
@@ -822,29 +681,6 @@ struct GemvLaunch {
     uint32_t ngroups, tiles, batch;
     EpiArgs e;
 };
-
-template <bool Q4, int BPV, int MODE, int CFG>
-static void gemv_launch_one(const GemvLaunch &L) {
-    hipLaunchKernelGGL((gemv_quant_kernel<Q4, BPV, MODE, CFG>), L.grid, L.block, L.lds, L.st, L.qs,
-                       L.ds, L.xa, L.ngroups, L.tiles, L.batch, L.e);
-}
-
-template <bool Q4, int BPV, int MODE>
-static bool gemv_launch_cfg(int cfg, const GemvLaunch &L) {
-    switch (cfg) {
-        case 1: gemv_launch_one<Q4, BPV, MODE, 1>(L); return true;
-        case 1 | CFG_TPW2: if constexpr (MODE == X_LDS) { gemv_launch_one<Q4, BPV, MODE, 1 | CFG_TPW2>(L); return true; } return false;
-        case 1 | CFG_TPW4: if constexpr (MODE == X_GLOBAL) { gemv_launch_one<Q4, BPV, MODE, 1 | CFG_TPW4>(L); return true; } return false;
-        case 1 | CFG_PF6: gemv_launch_one<Q4, BPV, MODE, 1 | CFG_PF6>(L); return true;
-        case 1 | CFG_PF2: gemv_launch_one<Q4, BPV, MODE, 1 | CFG_PF2>(L); return true;
-        default: return false;
-    }
-}
-
-template <bool Q4, int BPV>
-static bool gemv_launch_mode(int xmode, int cfg, const GemvLaunch &L) {
-    return xmode == X_GLOBAL ? gemv_launch_cfg<Q4, BPV, X_GLOBAL>(cfg, L) : gemv_launch_cfg<Q4, BPV, X_LDS>(cfg, L);
-}
 
 template <bool Q4, int BPV, int MODE, int QPWV, int SRECV>
 static bool quad_launch_one(const GemvLaunch &L) {
@@ -934,62 +770,61 @@ static int launch_gemv_quad(const Weight &w, const __half *xq, uint64_t batch, c
     return COEUS_OK;
 }
 
+// Batches of 5 to 16: tiles and waves of a workgroup of gemv_rows_kernel.  Every workgroup reads all activation rows, so it
+// takes as many tiles as leave about a workgroup per CU, six at most (Q8_0 four: registers), else two workgroups per CU;
+// waves as many as share the reduction in few trips.  Measured for 8 and 16 rows over 35 matrices of 768 - 5120 wide models
+// with 1 - 6 tiles and 2 - 16 waves; the choice is within 4 % of the best of them (4096 x 22016, 16 rows, Q4_0: six tiles 15.9,
+// three 17, two 17.4 us; 1536 x 8192: two 6.9, one 7.3; 768 x 50257: two tiles of three waves 12.2, one of six 17.2).
+static void gemv_rows_shape(bool q4, uint32_t ngroups, uint32_t tiles, uint32_t &tpw, uint32_t &waves) {
+    tpw = 0;
+    for (uint32_t t : {1u, 2u, 3u, 4u, 6u})
+        if (!tpw && (t < 6 || q4) && ceil_div(tiles, t) <= 256) tpw = t;
+    for (uint32_t t : {2u, 3u, 4u})
+        if (!tpw && ceil_div(tiles, t) <= 512) tpw = t;
+    const bool many = !tpw;
+    if (!tpw) tpw = ngroups <= 8 ? 2 : 4;
+    waves = (tpw == 3 || tpw == 4) ? 8 : (tpw == 1 && ngroups <= 16) ? 8 : 12;
+    if (many && ngroups <= 8) waves = (ngroups + 1) / 2;
+    waves = std::min(waves, ngroups);
+}
+
+template <bool Q4, int BP, int TPW>
+static int launch_gemv_rows(const Weight &w, const __half *xq, uint32_t batch, uint32_t waves, const EpiArgs &e, hipStream_t st) {
+    const size_t lds = (size_t)TPW * waves * 4 * 64 * 4;
+    if (lds > 48 * 1024) {
+        static const hipError_t once = hipFuncSetAttribute((const void *)gemv_rows_kernel<Q4, BP, TPW>,
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        COEUS_HIP(once);
+    }
+    const uint32_t ngroups = (uint32_t)(w.k_pad / 128), tiles = (uint32_t)(w.n_pad / 16);
+    hipLaunchKernelGGL((gemv_rows_kernel<Q4, BP, TPW>), dim3((uint32_t)ceil_div(tiles, TPW)), dim3(waves * 64), lds, st, (const uint4 *)w.data,
+                       (const uint2 *)w.scales, (const uint4 *)xq, ngroups, tiles, batch, e);
+    COEUS_HIP(hipGetLastError());
+    return COEUS_OK;
+}
+
 template <bool Q4>
 static int launch_gemv_quant(const Weight &w, const __half *xq, uint64_t batch, const EpiArgs &e,
                              hipStream_t st, const NormFuse *nf) {
     if (pad_batch(batch) <= 4) return launch_gemv_quad<Q4>(w, xq, batch, e, st, nf);
-    // batches of 5 to 16: gemv_quant_kernel on staged f16 activations (the norm is a launch of its own)
+    // batches of 5 to 16: gemv_rows_kernel on staged f16 activations (the norm is a launch of its own)
     if (nf) return fail(COEUS_INVALID_INPUT, "norm fusion is for batches of up to 4");
-    const uint32_t ngroups = (uint32_t)(w.k_pad / 128), tiles = (uint32_t)(w.n_pad / 16);
-    const uint32_t bp = pad_batch(batch), b = (uint32_t)batch;
-    uint32_t waves = gemv_quant_waves(w);
-    const size_t x_bytes = (size_t)w.k_pad * bp * 2;
-    const bool xlds = x_bytes <= kXLdsLimit;
     if (e.stats_out && e.act == COEUS_EPI_SILU_GATE)
         return fail(COEUS_INVALID_INPUT, "statistics records are not produced by the gated epilogue");
-    const int xmode = xlds ? X_LDS : X_GLOBAL;
-    XArgs xa{};
-    xa.xq = (const uint4 *)xq;
-    xa.k = (uint32_t)w.k;
-    const uint32_t pf = Q4 ? 4 : 2;
-    const bool one_pass = ngroups <= pf * waves;
-    int cfg = 1;
-    if (!one_pass && ngroups <= pf * waves * 3 / 2) {
-        cfg |= CFG_PF6;  // one pass of 6 chunks per wave instead of a full and a partial pass
-    } else if (ngroups <= (pf / 2) * waves) {
-        cfg |= CFG_PF2;  // half as many chunks per wave cover k: no requests past the end
-    }
-    // two tiles per workgroup where one pass covers the reduction and the tiles still fill the
-    // chip: the activation block is staged half as often
-    uint32_t tpw = 1;
-    if (xmode == X_GLOBAL) {
-        // activations from L2: several tiles per workgroup share every activation fragment; the
-        // waves split k finer instead, so that the chip still holds thousands of them
-        tpw = tiles >= 768 ? 4 : 1;
-        if (tpw > 1) {
-            cfg = 1 | CFG_TPW4;
-            waves = tiles / tpw < 256 ? 16 : 8;
-            while (waves > 1 && waves * 2 > ngroups) waves /= 2;
+    uint32_t tpw, waves;
+    gemv_rows_shape(Q4, (uint32_t)(w.k_pad / 128), (uint32_t)(w.n_pad / 16), tpw, waves);
+    auto with = [&](auto bp) -> int {
+        constexpr int BP = decltype(bp)::value;
+        switch (tpw) {
+            case 1: return launch_gemv_rows<Q4, BP, 1>(w, xq, (uint32_t)batch, waves, e, st);
+            case 2: return launch_gemv_rows<Q4, BP, 2>(w, xq, (uint32_t)batch, waves, e, st);
+            case 3: return launch_gemv_rows<Q4, BP, 3>(w, xq, (uint32_t)batch, waves, e, st);
+            case 4: return launch_gemv_rows<Q4, BP, 4>(w, xq, (uint32_t)batch, waves, e, st);
+            default: if constexpr (Q4) return launch_gemv_rows<Q4, BP, 6>(w, xq, (uint32_t)batch, waves, e, st);
         }
-    } else if (one_pass && waves >= 2 && tiles >= 1024 && cfg == 1) {
-        cfg |= CFG_TPW2;
-        tpw = 2;
-    }
-    const size_t red_bytes = (waves > 1 || tpw > 1) ? (size_t)tpw * waves * 4 * 64 * 4 : 0;
-    GemvLaunch L;
-    L.grid = dim3((unsigned)ceil_div(tiles, tpw));
-    L.block = dim3(waves * 64);
-    L.lds = (xmode != X_GLOBAL ? x_bytes : 0) + red_bytes;
-    L.st = st;
-    L.qs = (const uint4 *)w.data;
-    L.ds = (const uint2 *)w.scales;
-    L.xa = xa;
-    L.ngroups = ngroups; L.tiles = tiles; L.batch = b;
-    L.e = e;
-    const bool ok = bp == 8 ? gemv_launch_mode<Q4, 8>(xmode, cfg, L) : gemv_launch_mode<Q4, 16>(xmode, cfg, L);
-    if (!ok) return fail(COEUS_INVALID_INPUT, "decode matmul: no kernel variant %d for mode %d", cfg, xmode);
-    COEUS_HIP(hipGetLastError());
-    return COEUS_OK;
+        return fail(COEUS_INVALID_INPUT, "decode matmul: no kernel for %u tiles a workgroup", tpw);
+    };
+    return pad_batch(batch) == 8 ? with(std::integral_constant<int, 8>{}) : with(std::integral_constant<int, 16>{});
 }
 
 // ---------------------------------------------------------------- dense kernel (f32 / bf16)

@@ -444,9 +444,8 @@ REAL_SHAPES = [(4096, 12288, False), (4096, 4096, False), (4096, 22016, True), (
 @pytest.mark.parametrize("k,n,gated", REAL_SHAPES)
 def test_gemv_benchmark_shapes(orc, dtype, k, n, gated):
     """coeus_op_gemv (activations staged from the f16 interchange buffer): batch 1, 4, 8 and 16 take
-    the variants with 1 / 4 / 4 / 4 live accumulator rows, the (11008, 4096) matrix the one with six
-    chunks in flight per wave, batch 16 at k = 11008 the one that reads activations from L2, batch
-    16 on 768 tiles and more the one whose waves share an activation fragment among four tiles."""
+    the variants with 1 / 4 / 4 / 4 live accumulator rows; batch 8 and 16 have workgroups of one tile
+    (256 tiles of 16 outputs at most), three (768) or six (1376; Q8_0 three)."""
     wt, wdq = _seeded(dtype, k, n, 1000 + k + n)
     # the device's dequantised values are the oracle's (bit-exact), on a corner of the matrix
     w_corner = np.array([[np.float32(0.02) * np.float32(orc.lib().orc_synth_normal(1000 + k + n, l * n + j))
@@ -480,6 +479,26 @@ def test_gemv_benchmark_shapes(orc, dtype, k, n, gated):
             want = pre + res
             got = wt.gemv(dev(x), residual=dev(res))
         assert rel_err(got, want) < 2e-5, (batch, rel_err(got, want))
+
+
+# Tiles of 16 outputs at both sides of every line where a workgroup of batches of 5 to 16 takes more of them (one, two, three,
+# four, six; beyond 512 workgroups of four: two or four by k), ragged last tiles, one chunk of k and a partial last trip.
+@pytest.mark.parametrize("dtype", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("k,n", [(96, 256 * 16), (96, 256 * 16 + 2), (160, 512 * 16 - 14), (160, 513 * 16), (1184, 768 * 16),
+                                 (160, 769 * 16 - 2), (160, 1024 * 16 + 2), (160, 1536 * 16), (160, 1537 * 16), (160, 2049 * 16),
+                                 (1184, 2049 * 16 - 6)])
+def test_gemv_rows_shapes(orc, dtype, k, n):
+    wt, wdq = _seeded(dtype, k, n, k + n)
+    rng = np.random.default_rng(k + n)
+    bias = rng.standard_normal(n).astype(np.float32) * 0.1
+    for batch in (5, 16):
+        x = rng.standard_normal((batch, k)).astype(np.float32)
+        res = rng.standard_normal((batch, n)).astype(np.float32)
+        pre = _f16(x) @ wdq
+        # (sums of at most 1184 products in f32: far below the bound that the other shapes are held to)
+        assert rel_err(wt.gemv(dev(x), bias=dev(bias), residual=dev(res)), pre + bias + res) < 2e-5
+        g, u = (pre + bias)[:, 0::2], (pre + bias)[:, 1::2]
+        assert rel_err(wt.gemv(dev(x), bias=dev(bias), epilogue=_lib.EPI_SILU_GATE), g / (1 + np.exp(-g)) * u) < 2e-5
 
 
 def _norm64(h, kind, sc, bi, eps):
