@@ -8,6 +8,7 @@
 //                     quantised weights, which are expanded to f16(q * d) first).
 //     gemm_h256k64_kernel  k % 64 == 0: 256x256 tile, four waves of 128x128, 64-wide k slices
 //                          loaded straight into a ring of five LDS regions
+//     gemm_narrow_kernel   k % 64 == 0, launches of few tiles: 128 or 256 rows by 64 to 128 columns
 //     gemm_h256_kernel     k % 32 == 0: 256x256 tile, eight waves of 128x64, 32-wide slices
 //     gemm_h_kernel        any k: 128x128 tile, register-staged
 //     gemm_qskinny_kernel  up to 64 rows on quantised weights: streams the quantised blocks
@@ -402,6 +403,8 @@ __device__ __forceinline__ bool epi_vec4(const EpiArgs &e) {
     return (e.n_eff & 3) == 0 && (e.lp_ld & 3) == 0 && (e.out_f32 || e.out_lp) && !e.out_xq;
 }
 // Columns col .. col + 3 of activation row `row` (bias, cache append or activation, residual, store).
+// FAST: GELU and SiLU on the hardware's exp2 and reciprocal (1 ulp each).
+template <bool FAST = false>
 __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCols &kc, uint64_t row,
                                          uint64_t col, uint64_t n, float (&v)[4]) {
     if (vec4 && col + 3 < n) {
@@ -425,7 +428,7 @@ __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCo
         }
         if (e.act == COEUS_EPI_GELU)
 #pragma unroll
-            for (int q = 0; q < 4; q++) v[q] = gelu_tanh(v[q]);
+            for (int q = 0; q < 4; q++) v[q] = FAST ? fast_gelu(v[q]) : gelu_tanh(v[q]);
         if (e.act == COEUS_EPI_SOFTCAP)
 #pragma unroll
             for (int q = 0; q < 4; q++) v[q] = soft_cap(v[q], e.limit);
@@ -442,13 +445,14 @@ __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCo
 }
 // Gated outputs ocol .. ocol + 3 of row `row`, from the weight rows (gate, up) = raw columns
 // raw .. raw + 7 (raw = 2 ocol).
+template <bool FAST = false>
 __device__ __forceinline__ void epi_row4_gated(const EpiArgs &e, bool vec4, uint64_t row, uint64_t ocol,
                                                uint64_t raw, uint64_t n, const float (&gv)[4],
                                                const float (&uv)[4]) {
     if (vec4 && !e.bias && !e.residual && raw + 7 < n) {
         float o[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) o[q] = e.act == COEUS_EPI_CLAMP_GATE ? clamped_gate(gv[q], uv[q], e.limit) : silu(gv[q]) * uv[q];
+        for (int q = 0; q < 4; q++) o[q] = e.act == COEUS_EPI_CLAMP_GATE ? clamped_gate(gv[q], uv[q], e.limit) : (FAST ? fast_silu(gv[q]) : silu(gv[q])) * uv[q];
         epi_store4(e, row, ocol, o);
     } else {
 #pragma unroll
@@ -1363,6 +1367,227 @@ __global__ __launch_bounds__(256) void gemm_h256k64_kernel(const uint16_t *a, co
     }
 }
 
+// ---------------------------------------------------------------- few rows
+// Prompts whose 256x256 tiles do not fill the chip leave CUs without work, or split k so often that the planes cost more than the
+// products.  So smaller tiles (256 or 128 rows, 64 - 128 columns): eight waves, of which waves 0 - 3 multiply the first two
+// 16-wide k steps of every 64-wide slice and waves 4 - 7 the last two (two waves a SIMD, one's fragment reads behind the other's
+// products); wave % 4 has RB x NB blocks of 32 x 32, WM rows of waves by 4 / WM.  The two halves are added through LDS.
+// Bound by the path from L2 into LDS, which gives a CU 60 - 70 GB/s and all of them 14 - 17 TB/s: 128 (rows + columns) bytes a slice,
+// 0.34 us for 128x64 and 0.63 us for 256x96, where the products take 0.12 and 0.36.  The weights come from memory and a slice is
+// shorter than that trip: their ring in LDS is deeper than the activations', and waves 0 - 3 request the A rows, waves 4 - 7 the W
+// rows, so that neither waits for the other's (a wave's loads return in order).  Layout of a slice as in gemm_h256k64_kernel.
+// With all of a slice's fragments read before its products instead of one step ahead: 4096 x 22016 on 201 rows 73.8 us, 59.8 so.
+template <int WM, int RB, int NB>
+struct NarrowTile {
+    static constexpr int WN = 4 / WM, ROWS = WM * RB * 32, COLS = WN * NB * 32;
+    static constexpr int UA = ROWS / 32, UW = COLS / 32;  // requests of a wave and slice: 8 rows x 128 bytes each, four waves an operand
+    static constexpr int DA = ROWS == 256 ? 3 : 5, DW = ROWS == 256 ? (COLS == 128 ? 4 : COLS == 96 ? 5 : 6) : COLS == 128 ? 5 : 6;
+    static constexpr size_t ring = ((size_t)DA * ROWS + (size_t)DW * COLS) * UK * 2, tile = (size_t)ROWS * (COLS + 4) * 4, lds = ring > tile ? ring : tile;
+    static_assert(lds <= 160 * 1024, "fits the LDS of a CU");
+};
+
+__host__ __device__ constexpr int wait_vm_lds(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070; }  // vmcnt(n) lgkmcnt(0)
+
+// Requests [Q0, Q1) of a slice: 8 rows x 128 bytes each into LDS.
+template <int Q0, int Q1, int Q>
+__device__ __forceinline__ void narrow_request(const char *src, const uint32_t (&off)[Q], uint16_t *dst, uint32_t w4) {
+    typedef const __attribute__((address_space(1))) void *gptr_t;
+    typedef __attribute__((address_space(3))) void *lptr_t;
+#pragma unroll
+    for (int q = Q0; q < Q1; q++)
+        __builtin_amdgcn_global_load_lds((gptr_t)(src + off[q]), (lptr_t)(dst + (4 * q + w4) * 512), 16, 0, 0);
+}
+// Half a slice: the products of one k step on fragments already in registers, the reads of the next step's fragments between
+// them, and requests for a later slice in front (the W rows and the first half of the A rows; SECOND: the other half).  The regions read and the one written
+// are distinct (see k64_period).
+template <bool BF16, class T, int RB, int NB, bool SECOND, int Q>
+__device__ __forceinline__ void narrow_step(const uint16_t *__restrict__ ra, const uint16_t *__restrict__ rw, uint16_t *__restrict__ dst,
+                                            const char *src, const uint32_t (&off)[Q], bool takes_a, uint32_t w4, uint32_t la, uint32_t lw,
+                                            const uint4 (&af)[RB], const uint4 (&wf)[NB], uint4 (&an)[RB], uint4 (&wn)[NB],
+                                            float16_t (&acc)[RB][NB]) {
+    if (takes_a) narrow_request<SECOND ? T::UA / 2 : 0, SECOND ? T::UA : T::UA / 2>(src, off, dst, w4);
+    else if (!SECOND) narrow_request<0, T::UW>(src, off, dst, w4);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < (RB * NB > RB + NB ? RB * NB : RB + NB); i++) {
+        if (i < RB * NB) mfma_32x32x16<BF16>(wf[i / RB], af[i % RB], acc[i % RB][i / RB]);
+        if (i < RB) an[i] = k64_read(ra, la, i);
+        else if (i < RB + NB) wn[i - RB] = k64_read(rw, lw, i - RB);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+template <bool BF16, int WM, int RB, int NB>
+__global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, const uint16_t *w, uint64_t m, uint64_t n, uint64_t k, uint64_t lda,
+                                                          uint64_t ldw, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits, EpiArgs e) {
+    using T = NarrowTile<WM, RB, NB>;
+    constexpr int DA = T::DA, DW = T::DW, Q = T::UA > T::UW ? T::UA : T::UW;
+    constexpr uint32_t RA = T::ROWS * UK, RW = T::COLS * UK;  // elements of a region
+    extern __shared__ __attribute__((aligned(16))) uint16_t sm[];  // A regions 0 .. DA - 1, W regions 0 .. DW - 1
+    // Workgroups go round-robin to the 8 XCDs: each takes consecutive tiles, rows first, so that its L2 fetches a column tile's
+    // weights once (the grid is a multiple of 8).
+    const uint32_t tiles = tiles_m * tiles_n, id = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+    if (id >= tiles * splits) return;
+    const uint32_t split = id / tiles, r = id - split * tiles, tn = r / tiles_m, tm = r - tn * tiles_m;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), w4 = wave & 3, half = wave >> 2;
+    const uint32_t wrow = w4 / T::WN * RB * 32, wcol = w4 % T::WN * NB * 32;
+    const uint64_t m0 = (uint64_t)tm * T::ROWS, n0 = (uint64_t)tn * T::COLS;
+    const uint64_t nslices = k / UK, kbeg = nslices * split / splits * UK, kend = nslices * (split + 1) / splits * UK;
+    if (splits > 1) e.out_f32 += (uint64_t)split * m * e.n_eff;
+    float16_t acc[RB][NB];
+#pragma unroll
+    for (int x = 0; x < RB; x++)
+#pragma unroll
+        for (int y = 0; y < NB; y++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[x][y][i] = 0.f;
+    const bool takes_a = half == 0;
+    uint32_t off[Q];
+    {
+        const uint32_t last = (uint32_t)(takes_a ? min((uint64_t)T::ROWS - 1, m - 1 - m0) : min((uint64_t)T::COLS - 1, n - 1 - n0));
+        const uint32_t ld = (uint32_t)(takes_a ? lda : ldw) * 2;
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const uint32_t row = 8 * (4 * q + w4) + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+            off[q] = min(row, last) * ld + piece * 16;
+        }
+    }
+    const char *origin = takes_a ? (const char *)(a + m0 * lda) : (const char *)(w + n0 * ldw);
+    // slices past the end are requested as repeats of the last one (and never used): the number of loads in flight at each
+    // wait does not depend on the number of slices
+    const uint64_t klast = kend - UK;
+    auto source = [&](uint64_t kk) { return origin + 2 * (kk < klast ? kk : klast); };
+    uint32_t la[2], lw[2];
+    {
+        const uint32_t frow = lane & 31, fhf = lane >> 5, fsw = (lane >> 1) & 7;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const uint32_t slot = 8 * ((2 * (2 * half + j) + fhf) ^ fsw);
+            la[j] = (wrow + frow) * UK + slot;
+            lw[j] = (wcol + frow) * UK + slot;
+        }
+    }
+    uint16_t *const rega = sm, *const regw = sm + DA * RA;
+    uint16_t *const ring = takes_a ? rega : regw;
+    const uint32_t depth = takes_a ? DA : DW, rsize = takes_a ? RA : RW;
+    for (uint32_t j = 0; j < depth; j++) {
+        if (takes_a) narrow_request<0, T::UA>(source(kbeg + (uint64_t)j * UK), off, ring + j * RA, w4);
+        else narrow_request<0, T::UW>(source(kbeg + (uint64_t)j * UK), off, ring + j * RW, w4);
+    }
+    // every wave's loads of the next slice have landed (all but the newest `depth - 2` slices'), and it has read all of the last one
+    auto meet = [&](auto more) {
+        constexpr int D = decltype(more)::value;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        if (takes_a) __builtin_amdgcn_s_waitcnt(wait_vm_lds((DA - 2 + D) * T::UA));
+        else __builtin_amdgcn_s_waitcnt(wait_vm_lds((DW - 2 + D) * T::UW));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    uint4 af[2][RB], wf[2][NB];
+    meet(std::integral_constant<int, 1>{});  // slice 0
+#pragma unroll
+    for (int x = 0; x < RB; x++) af[0][x] = k64_read(rega, la[0], x);
+#pragma unroll
+    for (int y = 0; y < NB; y++) wf[0][y] = k64_read(regw, lw[0], y);
+    const uint32_t nsl = (uint32_t)((kend - kbeg) / UK);
+    // Slice s: the products of its first step, while the second step's fragments are read; then, when nobody reads the slice any
+    // more, those of the second, while the next slice's are read.  Slice s + depth goes into the region of slice s.
+    uint32_t ia = 0, iw = 0, io = depth - 1;  // regions of slice s; of slice s - 1, whose second half of requests is left
+    for (uint32_t s = 0; s < nsl; s++) {
+        if (s) {
+            narrow_step<BF16, T, RB, NB, true>(rega + ia * RA, regw + iw * RW, ring + io * rsize, source(kbeg + (uint64_t)(s - 1 + depth) * UK), off,
+                                               takes_a, w4, la[1], lw[1], af[0], wf[0], af[1], wf[1], acc);
+        } else {
+#pragma unroll
+            for (int x = 0; x < RB; x++) af[1][x] = k64_read(rega, la[1], x);
+#pragma unroll
+            for (int y = 0; y < NB; y++) wf[1][y] = k64_read(regw, lw[1], y);
+#pragma unroll
+            for (int i = 0; i < RB * NB; i++) mfma_32x32x16<BF16>(wf[0][i / RB], af[0][i % RB], acc[i % RB][i / RB]);
+        }
+        meet(std::integral_constant<int, 0>{});
+        uint16_t *const freed = ring + (takes_a ? ia : iw) * rsize;
+        ia = ia + 1 == DA ? 0 : ia + 1;
+        iw = iw + 1 == DW ? 0 : iw + 1;
+        io = io + 1 == depth ? 0 : io + 1;
+        narrow_step<BF16, T, RB, NB, false>(rega + ia * RA, regw + iw * RW, freed, source(kbeg + (uint64_t)(s + depth) * UK), off, takes_a, w4,
+                                            la[0], lw[0], af[1], wf[1], af[0], wf[0], acc);
+    }
+    __builtin_amdgcn_s_waitcnt(0x0070);  // the repeats have landed too
+    __syncthreads();
+    // The two halves meet in a [ROWS][COLS + 4] f32 tile; then every thread finishes four (gated: eight) columns of some rows.
+    constexpr uint32_t TS = T::COLS + 4;
+    float *tile = (float *)sm;
+    float *mine = tile + (wrow + (lane & 31)) * TS + wcol + 4 * (lane >> 5);
+    if (half == 0) {
+#pragma unroll
+        for (int x = 0; x < RB; x++)
+#pragma unroll
+            for (int y = 0; y < NB; y++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *(float4 *)(mine + x * 32 * TS + y * 32 + 8 * g) = make_float4(acc[x][y][4 * g], acc[x][y][4 * g + 1], acc[x][y][4 * g + 2], acc[x][y][4 * g + 3]);
+    }
+    __syncthreads();
+    if (half == 1) {
+#pragma unroll
+        for (int x = 0; x < RB; x++)
+#pragma unroll
+            for (int y = 0; y < NB; y++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    float4 *p = (float4 *)(mine + x * 32 * TS + y * 32 + 8 * g);
+                    const float4 o = *p;
+                    *p = make_float4(o.x + acc[x][y][4 * g], o.y + acc[x][y][4 * g + 1], o.z + acc[x][y][4 * g + 2], o.w + acc[x][y][4 * g + 3]);
+                }
+    }
+    __syncthreads();
+    const bool vec4 = epi_vec4(e);
+    const uint32_t live = (uint32_t)min((uint64_t)T::ROWS, m - m0);
+    if (!epi_gated(e.act)) {
+        constexpr uint32_t CG = T::COLS / 4, RP = 512 / CG;
+        const uint32_t c4 = tid % CG * 4;
+        if (tid >= RP * CG || n0 + c4 >= n) return;
+        const KvCols kc = epi_kv_cols(e, n0 + c4, n);
+        for (uint32_t q = tid / CG; q < live; q += RP) {
+            const float4 t = *(const float4 *)(tile + q * TS + c4);
+            float v[4] = {t.x, t.y, t.z, t.w};
+            epi_row4<true>(e, vec4, kc, m0 + q, n0 + c4, n, v);
+        }
+    } else {
+        constexpr uint32_t CG = T::COLS / 8, RP = 512 / CG;
+        const uint32_t c8 = tid % CG * 8;
+        if (tid >= RP * CG || n0 + c8 >= n) return;
+        for (uint32_t q = tid / CG; q < live; q += RP) {
+            const float4 p0 = *(const float4 *)(tile + q * TS + c8), p1 = *(const float4 *)(tile + q * TS + c8 + 4);
+            const float gv[4] = {p0.x, p0.z, p1.x, p1.z}, uv[4] = {p0.y, p0.w, p1.y, p1.w};
+            epi_row4_gated<true>(e, vec4, m0 + q, (n0 + c8) >> 1, n0 + c8, n, gv, uv);
+        }
+    }
+}
+
+template <bool BF16, int WM, int RB, int NB>
+static int launch_narrow(const uint16_t *a, const uint16_t *w, uint64_t m, uint64_t n, uint64_t k, uint64_t lda, uint64_t ldw, uint32_t splits,
+                         const EpiArgs &e, hipStream_t st) {
+    using T = NarrowTile<WM, RB, NB>;
+    static const hipError_t once = hipFuncSetAttribute((const void *)gemm_narrow_kernel<BF16, WM, RB, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    COEUS_HIP(once);
+    const uint32_t tiles_m = (uint32_t)ceil_div(m, T::ROWS), tiles_n = (uint32_t)ceil_div(n, T::COLS);
+    hipLaunchKernelGGL((gemm_narrow_kernel<BF16, WM, RB, NB>), dim3((uint32_t)round_up((uint64_t)tiles_m * tiles_n * splits, 8)), dim3(512), T::lds, st, a, w, m, n, k,
+                       lda, ldw, tiles_m, tiles_n, splits, e);
+    COEUS_HIP(hipGetLastError());
+    return COEUS_OK;
+}
+template <bool BF16>
+static int launch_narrow_plan(uint32_t rows, uint32_t cols, const uint16_t *a, const uint16_t *wp, uint64_t m, const Weight &w, uint64_t lda,
+                              uint64_t ldw, uint32_t splits, const EpiArgs &e, hipStream_t st) {
+    if (rows == 256) return cols == 128 ? launch_narrow<BF16, 2, 4, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st) : launch_narrow<BF16, 4, 2, 3>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st);
+    if (cols == 128) return launch_narrow<BF16, 2, 2, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st);
+    return cols == 96 ? launch_narrow<BF16, 4, 1, 3>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st) : launch_narrow<BF16, 4, 1, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st);
+}
+
 // Any number of rows: a short prompt leaves most of a 256-row tile empty (rows past the end are
 // clamped on the way in and not stored), and is still several times faster here than in the
 // 128x128 register-staged kernel (1B shape, 16 rows: 24.5 ms per prompt pass there).
@@ -1400,6 +1625,35 @@ static uint32_t gemm_splits_wanted(const Weight &w, uint64_t m) {
     return best;
 }
 
+// Which kernel and how many shares of k a launch of k % 64 == 0 takes: rows 0 = the 256x256 tiles.  Launches that fill more than one
+// round of those keep them.  Else the estimate below is taken for every narrow tile and number of shares, and the shortest
+// one runs if it is under 0.95 of the 256x256 kernel's: per round of 256 workgroups 3.6 us and 0.25 us per 1024 outputs of a
+// tile, per slice the tile's 128 (rows + columns) bytes at 66 GB/s a CU and 17 TB/s in all (what the path from L2 into LDS
+// gives), for several shares 5.8 us and the planes at 4.4 TB/s; 256x256: 14 us and 0.9 us a slice.  Fitted to 19 matrices of
+// 768 - 22016 with 65 - 2036 rows, every tile and number of shares timed: 1 % above the fastest on average, 13 % at worst
+// (2048 x 2048, 65 rows, 12.6 against 11.2 us).  us, 256x256 tiles / this: 201 rows of 4096 x 4096 32.8 / 21.7, of 4096 x 12288
+// 53.0 / 38.3, of 4096 x 22016 70.8 / 59.8, of 11008 x 4096 56.2 / 39.4; 512 of 768 x 3072 25.3 / 9.4, of 3072 x 768
+// 28.3 / 16.3; 1019 of 4096 x 4096 55.6 / 44.4; 2036 of 2048 x 2048 42.6 / 27.5, of 1024 x 2048 30.9 / 17.8.
+struct GemmPlan { uint32_t rows = 0, cols = 0, splits = 1; };
+static constexpr uint32_t kNarrowTiles[][2] = {{256, 128}, {256, 96}, {128, 128}, {128, 96}, {128, 64}};
+static GemmPlan gemm_plan(const Weight &w, uint64_t m, bool may_split) {
+    GemmPlan best;
+    best.splits = may_split ? gemm_splits_wanted(w, m) : 1;
+    const uint64_t tiles256 = ceil_div(m, TM) * ceil_div(w.n, TN), slices = w.k / UK;
+    if (!gemm_uses_h256(w, m) || w.k % UK || tiles256 > 256) return best;
+    auto sum_us = [&](uint64_t splits) { return splits > 1 ? 5.8 + (double)(splits * m * w.n) * 8.0 / 4.4e6 : 0.0; };
+    double best_us = 0.95 * (14.0 + 0.9 * (double)ceil_div(slices, best.splits) + sum_us(best.splits));
+    for (const auto &t : kNarrowTiles) {
+        const uint64_t tiles = ceil_div(m, t[0]) * ceil_div(w.n, t[1]);
+        for (uint64_t s = 1; s <= (may_split ? 16 : 1) && (s == 1 || (tiles * s <= 256 && slices / s >= 3)); s++) {
+            const double kb = 0.125 * (t[0] + t[1]), busy = (double)std::min<uint64_t>(256, tiles * s);
+            const double us = (double)ceil_div(tiles * s, 256) * (3.6 + 0.25 * t[0] * t[1] / 1024.0 + (double)ceil_div(slices, s) * kb * std::max(1 / 66.0, busy / 17e3)) + sum_us(s);
+            if (us < best_us) { best_us = us; best.rows = t[0]; best.cols = t[1]; best.splits = (uint32_t)s; }
+        }
+    }
+    return best;
+}
+
 // A larger launch runs its tiles in rounds of 256 (one workgroup fills a CU), and the last round
 // is rarely full: 1376 tiles are five rounds and 96 tiles, which take as long as a sixth round.
 // When that remainder is at most half a round its tiles alone are split along k (as many shares
@@ -1425,8 +1679,9 @@ uint64_t gemm_split_scratch_bytes(const Weight &w, uint64_t m) {
         return sf > 1 ? (uint64_t)sf * m * w.n * 4 : 0;
     }
     if (gemm_uses_qskinny(w, m)) return gemm_qskinny_scratch_bytes(w, m);
-    const uint32_t s = gemm_splits_wanted(w, m);
-    if (s > 1) return (uint64_t)s * m * w.n * 4;
+    const GemmPlan plan = gemm_plan(w, m, true);
+    if (plan.splits > 1) return (uint64_t)plan.splits * m * w.n * 4;
+    if (plan.rows) return 0;
     uint32_t full = 0;
     const uint32_t st = gemm_tail_splits_wanted(w, m, &full);
     if (st > 1) return (uint64_t)st * (ceil_div(m, TM) * ceil_div(w.n, TN) - full) * TM * TN * 4;
@@ -1513,9 +1768,11 @@ int launch_gemm(const Weight &w, const void *a_in, uint64_t m, const Epilogue &e
         const uint32_t tiles_m = (uint32_t)ceil_div(m, TM), tiles_n = (uint32_t)ceil_div(w.n, TN);
         // split along k (every tile, or the tiles of the last round) when the caller's scratch has
         // room for the partial products
-        uint32_t splits = gemm_splits_wanted(w, m), full_tiles = 0, tail_splits = 1;
-        if (splits > 1 && (!scr.partials || scr.partials_bytes < (uint64_t)splits * m * w.n * 4)) splits = 1;
-        if (splits == 1) {
+        GemmPlan plan = gemm_plan(w, m, true);
+        if (plan.splits > 1 && (!scr.partials || scr.partials_bytes < (uint64_t)plan.splits * m * w.n * 4)) plan = gemm_plan(w, m, false);
+        const uint32_t splits = plan.splits;
+        uint32_t full_tiles = 0, tail_splits = 1;
+        if (splits == 1 && !plan.rows) {
             tail_splits = gemm_tail_splits_wanted(w, m, &full_tiles);
             if (tail_splits > 1 && (!scr.partials || scr.partials_bytes < gemm_split_scratch_bytes(w, m)))
                 tail_splits = 1;
@@ -1534,7 +1791,10 @@ int launch_gemm(const Weight &w, const void *a_in, uint64_t m, const Epilogue &e
         const uint64_t groups = ceil_div(w.n, epi_gated(e.act) ? 8 : 4);
         if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
         for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) {
-            if (w.k % UK == 0 && bf)
+            if (plan.rows)
+                COEUS_TRY(bf ? launch_narrow_plan<true>(plan.rows, plan.cols, ap, wp, m, w, lda, ldw, splits, ke, st)
+                             : launch_narrow_plan<false>(plan.rows, plan.cols, ap, wp, m, w, lda, ldw, splits, ke, st));
+            else if (w.k % UK == 0 && bf)
                 hipLaunchKernelGGL(gemm_h256k64_kernel<true>, grid, dim3(256), lds64, st, ap, wp, m, w.n, w.k, lda, ldw, tiles_m, tiles_n, ksplits, full_tiles, tail_part, ke);
             else if (w.k % UK == 0)
                 hipLaunchKernelGGL(gemm_h256k64_kernel<false>, grid, dim3(256), lds64, st, ap, wp, m, w.n, w.k, lda, ldw, tiles_m, tiles_n, ksplits, full_tiles, tail_part, ke);
