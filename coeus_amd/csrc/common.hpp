@@ -319,6 +319,8 @@ int launch_argmax(const float *logits, uint64_t rows, uint64_t vocab, uint64_t *
 int launch_advance(uint32_t *pos, uint32_t *step, hipStream_t st);
 // dids[0 .. n) = ids (host memory, n <= 16; read before the call returns), dpos = {pos, 0}
 int launch_step_state(const uint64_t *ids, uint64_t n, uint32_t pos, uint64_t *dids, uint32_t *dpos, hipStream_t st);
+// dst[0 .. n) = ids (host memory, read before the call returns)
+int launch_upload_ids(const uint64_t *ids, uint64_t n, uint64_t *dst, hipStream_t st);
 int launch_sample(const float *logits, uint64_t rows, uint64_t vocab, const coeus_sampling &cfg,
                   uint64_t pos0, const uint32_t *pos_dev, uint64_t *out_ids, uint64_t *history,
                   uint64_t history_stride, const uint32_t *step_dev, hipStream_t st);

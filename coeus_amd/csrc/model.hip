@@ -6,7 +6,10 @@
 #include <sys/mman.h>
 #include <unistd.h>
 
+#include <atomic>
+#include <chrono>
 #include <cmath>
+#include <thread>
 
 namespace coeus {
 
@@ -44,41 +47,125 @@ static bool known_to_runtime(const void *p) {
     return false;
 }
 
+// Bound by the link to the host: few workgroups are enough to fill it, and finish the pieces nearly in order.
+__global__ __launch_bounds__(256) void copy_out_kernel(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst, uint64_t words,
+                                                       uint32_t *flags, uint32_t turn) {
+    constexpr uint32_t U = HostCopy::kPiece / 16 / 256;
+    const uint64_t quads = words / 4, pieces = (words * 4 + HostCopy::kPiece - 1) / HostCopy::kPiece;
+    for (uint64_t p = blockIdx.x; p < pieces; p += gridDim.x) {
+        const uint64_t q0 = p * (256 * U) + threadIdx.x;
+        uint4 v[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++)
+            if (q0 + 256 * u < quads) v[u] = ((const uint4 *)src)[q0 + 256 * u];
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++)
+            if (q0 + 256 * u < quads) ((uint4 *)dst)[q0 + 256 * u] = v[u];
+        if (p + 1 == pieces && threadIdx.x < (words & 3)) dst[4 * quads + threadIdx.x] = src[4 * quads + threadIdx.x];
+        __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(flags + p, turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st) {
-    const bool slots_help = bytes > 4096 && !known_to_runtime(dst);
-    if (!pin && slots_help) {
-        bool ok = hipHostMalloc((void **)&pin, kSlot * kSlots, hipHostMallocDefault) == hipSuccess;
-        for (uint64_t i = 0; i < kSlots && ok; i++) ok = hipEventCreateWithFlags(&done[i], hipEventDisableTiming) == hipSuccess;
-        if (!ok) {
-            release();
+    const bool helps = bytes > 4096 && bytes % 4 == 0 && !known_to_runtime(dst);
+    if (!pin && helps) {
+        if (hipHostMalloc((void **)&pin, 2 * kHalf + 2 * kPieces * 4, hipHostMallocCoherent) == hipSuccess) {
+            std::memset(pin + 2 * kHalf, 0, 2 * kPieces * 4);
+        } else {
+            pin = nullptr;
             (void)hipGetLastError();
         }
     }
-    if (!pin || !slots_help) {
+    if (!pin || !helps) {
         COEUS_HIP(hipMemcpyAsync(dst, src_dev, bytes, hipMemcpyDeviceToHost, st));
         COEUS_HIP(hipStreamSynchronize(st));
         return COEUS_OK;
     }
-    const uint64_t slots = ceil_div(bytes, kSlot);
-    auto size = [&](uint64_t i) { return i + 1 < slots ? kSlot : bytes - i * kSlot; };
-    auto request = [&](uint64_t i) -> hipError_t {
-        const hipError_t e = hipMemcpyAsync(pin + i % kSlots * kSlot, (const char *)src_dev + i * kSlot, size(i), hipMemcpyDeviceToHost, st);
-        return e == hipSuccess && i + 1 < slots ? hipEventRecord(done[i % kSlots], st) : e;
+    const uint64_t rounds = ceil_div(bytes, kHalf);  // round r goes through half r % 2
+    const uint32_t before = turn;
+    uint32_t *flags = (uint32_t *)(pin + 2 * kHalf);
+    auto size = [&](uint64_t r) { return std::min(kHalf, bytes - r * kHalf); };
+    auto launch = [&](uint64_t r) -> hipError_t {
+        if (++turn == 0) turn = 1;
+        hipLaunchKernelGGL(copy_out_kernel, dim3(16), dim3(256), 0, st, (const uint32_t *)((const char *)src_dev + r * kHalf),
+                           (uint32_t *)(pin + r % 2 * kHalf), size(r) / 4, flags + r % 2 * kPieces, turn);
+        return hipGetLastError();
     };
-    for (uint64_t i = 0; i < slots && i < kSlots; i++) COEUS_HIP(request(i));
-    map_pages(dst, bytes);
-    for (uint64_t i = 0; i < slots; i++) {
-        COEUS_HIP(i + 1 < slots ? hipEventSynchronize(done[i % kSlots]) : hipStreamSynchronize(st));
-        std::memcpy((char *)dst + i * kSlot, pin + i % kSlots * kSlot, size(i));
-        if (i + kSlots < slots) COEUS_HIP(request(i + kSlots));
+    auto turn_of = [&](uint64_t r) {  // (turns skip 0, which fresh flags hold)
+        const uint32_t t = before + 1 + (uint32_t)r;
+        return t > before ? t : t + 1;
+    };
+    for (uint64_t r = 0; r < rounds && r < 2; r++) COEUS_HIP(launch(r));
+    const uint32_t threads = bytes >= kThreadsFrom ? 3 : 1;
+    std::atomic<bool> stop{false};
+    std::atomic<uint64_t> copied[2] = {};  // pieces out of each half, over all rounds
+    auto arrived = [&](uint64_t r, uint64_t p) { return __atomic_load_n(flags + r % 2 * kPieces + p, __ATOMIC_ACQUIRE) == turn_of(r); };
+    auto copy = [&](uint64_t r, uint64_t p) {
+        std::memcpy((char *)dst + r * kHalf + p * kPiece, pin + r % 2 * kHalf + p * kPiece, std::min(kPiece, size(r) - p * kPiece));
+        copied[r % 2].fetch_add(1, std::memory_order_release);
+    };
+    auto share = [&](uint32_t t) {  // thread t maps its part of the pages
+        const uint64_t from = bytes * t / threads, to = bytes * (t + 1) / threads;
+        map_pages((char *)dst + from, to - from);
+    };
+    std::atomic<uint64_t> next{0};  // (with several threads they take the pieces one by one; a round has kPieces but the last)
+    auto take = [&](uint64_t &r, uint64_t &p) {
+        const uint64_t i = next.fetch_add(1, std::memory_order_relaxed);
+        r = i / kPieces;
+        p = i % kPieces;
+        return r < rounds && p * kPiece < size(r);
+    };
+    auto helper = [&](uint32_t t) {
+        share(t);
+        for (uint64_t r, p; !stop.load(std::memory_order_relaxed) && take(r, p);) {
+            while (!arrived(r, p)) {
+                if (stop.load(std::memory_order_relaxed)) return;
+                __builtin_ia32_pause();
+            }
+            copy(r, p);
+        }
+    };
+    std::thread others[2];
+    for (uint32_t t = 1; t < threads; t++) {
+        try {
+            others[t - 1] = std::thread(helper, t);
+        } catch (...) {
+            // no more threads to be had: the others take its pieces, its pages are mapped as they are written
+        }
     }
+    share(0);
+    // This thread also launches the rounds that wait for a half to be copied out.  It spins for some milliseconds, then
+    // waits in the runtime, which knows of errors.
+    hipError_t err = hipSuccess;
+    uint64_t launched = std::min<uint64_t>(rounds, 2);
+    const auto start = std::chrono::steady_clock::now();
+    auto wait = [&](auto ready, uint64_t needs) {  // needs: the rounds that `ready` is about are launched when this many are
+        for (uint32_t n = 1; !ready() && err == hipSuccess; n++) {
+            // round `launched` takes the half of round launched - 2, the last of launched / 2 rounds out of that half
+            if (launched < rounds && copied[launched % 2].load(std::memory_order_acquire) == launched / 2 * kPieces) err = launch(launched++);
+            __builtin_ia32_pause();
+            if (n % 256 || std::chrono::steady_clock::now() - start < std::chrono::milliseconds(5)) continue;
+            const bool all = launched >= needs;
+            if (err == hipSuccess) err = hipStreamSynchronize(st);
+            if (err == hipSuccess && all && needs && !ready()) err = hipErrorUnknown;  // (the launch is over and its flag is not there)
+            std::this_thread::yield();
+        }
+    };
+    for (uint64_t r, p; err == hipSuccess && take(r, p);) {
+        wait([&] { return arrived(r, p); }, r + 1);
+        if (err == hipSuccess) copy(r, p);
+    }
+    // (other threads' last pieces)
+    wait([&] { return copied[0].load(std::memory_order_acquire) + copied[1].load(std::memory_order_acquire) == ceil_div(bytes, kPiece); }, 0);
+    if (err != hipSuccess) stop.store(true);
+    for (std::thread &t : others)
+        if (t.joinable()) t.join();
+    COEUS_HIP(err);
     return COEUS_OK;
 }
 void HostCopy::release() {
-    for (hipEvent_t &e : done) {
-        if (e) (void)hipEventDestroy(e);
-        e = nullptr;
-    }
     if (pin) (void)hipHostFree(pin);
     pin = nullptr;
 }
@@ -478,7 +565,7 @@ int model_forward(Model &m, const uint64_t *ids, uint64_t seq_len, float *logits
         COEUS_TRY(state.create(*m.stack, c.weight_dtype == COEUS_W_BF16, 1, seq_len, st));
         COEUS_TRY(layered_workspace(m, m.ws, 1, seq_len, 0));
         COEUS_TRY(m.ws.logits.ensure((all_rows ? seq_len : 1) * V * 4));
-        COEUS_HIP(hipMemcpyAsync(m.ws.ids.p, ids, seq_len * 8, hipMemcpyHostToDevice, st));
+        COEUS_TRY(launch_upload_ids(ids, seq_len, (uint64_t *)m.ws.ids.p, st));
         COEUS_TRY(layered_prefill(m, m.ws, state, 1, seq_len, 0, nullptr, st));
         const int rc = finish_forward(m, seq_len, logits_out, all_rows, st);
         const hipError_t e = hipStreamSynchronize(st);  // (also on failure: the state goes away below)
@@ -492,7 +579,7 @@ int model_forward(Model &m, const uint64_t *ids, uint64_t seq_len, float *logits
     COEUS_TRY(m.tmp_k.ensure(cache_bytes));
     COEUS_TRY(m.tmp_v.ensure(cache_bytes));
     Cache cache{m.tmp_k.p, m.tmp_v.p, seq_len, 0, false};
-    COEUS_HIP(hipMemcpyAsync(m.ws.ids.p, ids, seq_len * 8, hipMemcpyHostToDevice, st));
+    COEUS_TRY(launch_upload_ids(ids, seq_len, (uint64_t *)m.ws.ids.p, st));
     COEUS_TRY(run_blocks_prefill(m, m.ws, cache, 1, seq_len, 0, st));
     COEUS_TRY(finish_forward(m, seq_len, logits_out, all_rows, st));
     COEUS_HIP(hipStreamSynchronize(st));
@@ -581,7 +668,7 @@ static int feed_rows(Session &s, const uint64_t *ids, uint64_t n, float *residua
     const uint64_t rows = s.batch * n;
     if (m.stack) COEUS_TRY(layered_workspace(m, s.ws, s.batch, n, s.pos));
     else COEUS_TRY(s.ws.ensure(m, rows, 0));
-    COEUS_HIP(hipMemcpyAsync(s.ws.ids.p, ids, rows * 8, hipMemcpyHostToDevice, st));
+    COEUS_TRY(launch_upload_ids(ids, rows, (uint64_t *)s.ws.ids.p, st));
     if (m.stack) {
         COEUS_TRY(layered_prefill(m, s.ws, s.state, s.batch, n, s.pos, residuals_out, st));
     } else {
@@ -610,7 +697,7 @@ int session_prefill(Session &s, const uint64_t *ids, uint64_t n, float *logits_o
         COEUS_TRY(launch_norm(c.norm, COEUS_SCOPE_TOKEN, last, s.batch, H, m.fin_s, m.fin_b,
                               c.layer_norm_eps, x, nullptr, 0, st));
         COEUS_TRY(logits_gemv(m, s.ws, x, s.batch, (float *)s.dlogits.p, st));
-        COEUS_TRY(m.host_copy.out(logits_out, s.dlogits.p, s.batch * V * 4, st));
+        return m.host_copy.out(logits_out, s.dlogits.p, s.batch * V * 4, st);
     }
     COEUS_HIP(hipStreamSynchronize(st));
     return COEUS_OK;

@@ -762,4 +762,22 @@ int launch_step_state(const uint64_t *ids, uint64_t n, uint32_t pos, uint64_t *d
     return COEUS_OK;
 }
 
+// Token ids of a short prompt with a kernel's arguments: a copy out of the caller's memory goes through the runtime's staging and
+// a copy kernel.
+struct PromptIds { uint64_t id[128]; };
+__global__ void prompt_ids_kernel(PromptIds a, uint32_t n, uint64_t *dst) {
+    if (threadIdx.x < n) dst[threadIdx.x] = a.id[threadIdx.x];
+}
+int launch_upload_ids(const uint64_t *ids, uint64_t n, uint64_t *dst, hipStream_t st) {
+    if (n > 128) {
+        COEUS_HIP(hipMemcpyAsync(dst, ids, n * 8, hipMemcpyHostToDevice, st));
+        return COEUS_OK;
+    }
+    PromptIds a;
+    std::memcpy(a.id, ids, n * 8);
+    hipLaunchKernelGGL(prompt_ids_kernel, dim3(1), dim3(128), 0, st, a, (uint32_t)n, dst);
+    COEUS_HIP(hipGetLastError());
+    return COEUS_OK;
+}
+
 }  // namespace coeus

@@ -58,3 +58,18 @@ def test_into_pinned_and_device_memory():
         d = DeviceArray((size,), np.float32)
         _check(call(model._h, ids.ctypes.data, n, d.ptr))
         assert np.array_equal(d.to_host(), want)
+
+
+# a 16 KiB piece and one value less or more; a half of 4 MiB and one more; two halves; 8 MiB (three threads) and one row more, and
+# an odd number of values in five rounds
+@pytest.mark.parametrize("vocab,rows", [(1365, 3), (4096, 1), (4097, 1), (1024, 1024), (1025, 1024), (2048, 1024), (2049, 1024), (4999, 877)])
+def test_pieces_halves_and_threads(vocab, rows):
+    cfg = Transformer250MConfig(hidden_dim=32, num_layers=1, num_heads=2, intermediate_dim=64, vocab_size=vocab, max_seq_len=rows,
+                                norm_scope="token")
+    model = TransformerModelPlugin().create_builder().build(cfg, seed=3)
+    lib = _lib.load()
+    for seed in (1, 2, 3):  # (the flags of one call are not the next one's)
+        ids = np.random.default_rng(seed).integers(0, vocab, rows, dtype=np.uint64)
+        d = DeviceArray((rows * vocab,), np.float32)
+        _check(lib.coeus_model_forward_all(model._h, ids.ctypes.data, rows, d.ptr))
+        assert np.array_equal(model.forward_all(ids).ravel(), d.to_host())
