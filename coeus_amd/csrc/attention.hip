@@ -688,6 +688,118 @@ __global__ __launch_bounds__(256) void attn_prefill_f32_kernel(const float *__re
                                                            o[d][4 * g + 2] * inv, o[d][4 * g + 3] * inv);
 }
 
+// The same products where 128 queries a workgroup leave CUs without one (128 rows of 12 heads: 12 workgroups): 32 queries, and the
+// four waves take the key tiles in turn, straight from memory into registers (a tile's operands are used by one wave once), each
+// with its own running maximum; their shares meet in LDS.  Bound by the chain of a wave's tiles, a quarter as long.
+template <int HD>
+__global__ __launch_bounds__(256) void attn_prefill_f32_few_kernel(const float *__restrict__ qkv, const float *__restrict__ kc,
+                                                                   const float *__restrict__ vc, uint32_t n, uint32_t heads,
+                                                                   uint32_t max_ctx, uint32_t pos0, float *__restrict__ out) {
+    constexpr int KT = 32, HH = HD / 2, NDT = HD / 32, LD = HD + 4;
+    __shared__ __attribute__((aligned(16))) float so[4][32 * LD];  // [wave][query][dim]
+    __shared__ float sm[4][32], sl[4][32];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t qi = lane & 31, hf = lane >> 5;
+    uint32_t qt, h;
+    prefill_tile_of_block(qt, h);
+    const uint32_t b = blockIdx.z, inner = heads * HD, r0 = qt * 32;
+    const uint32_t r = r0 + qi, rc = r < n ? r : n - 1;  // rows past the end repeat the last
+    const uint32_t qpos = pos0 + rc, kmax = pos0 + min(n - 1, r0 + 31), ntiles = kmax / KT + 1;
+    const float scale2 = 1.4426950408889634f / sqrtf((float)HD);  // scale * log2(e)
+    float qf[HH];
+    {
+        const float *qp = qkv + ((uint64_t)b * n + rc) * 3 * inner + h * HD + hf * HH;
+#pragma unroll
+        for (int s = 0; s < HH; s += 4) {
+            const float4 a = *(const float4 *)(qp + s);
+            qf[s] = a.x; qf[s + 1] = a.y; qf[s + 2] = a.z; qf[s + 3] = a.w;
+        }
+    }
+    const uint64_t base = ((uint64_t)b * heads + h) * max_ctx * HD;
+    const float *kb = kc + base, *vb = vc + base;
+    float16_t o[NDT];
+#pragma unroll
+    for (int d = 0; d < NDT; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[d][i] = 0.f;
+    float m = -INFINITY, l = 0.f;
+    for (uint32_t t = wave; t < ntiles; t += 4) {
+        // keys past the last one repeat it: masked below
+        float4 kr[HH / 4];
+        float vr[16][NDT];
+        const float *kp = kb + (uint64_t)min(t * KT + qi, kmax) * HD + hf * HH;
+#pragma unroll
+        for (int s = 0; s < HH / 4; s++) kr[s] = *(const float4 *)(kp + 4 * s);
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const float *vp = vb + (uint64_t)min(t * KT + 8 * (j >> 2) + 4 * hf + (j & 3), kmax) * HD + qi;
+#pragma unroll
+            for (int d = 0; d < NDT; d++) vr[j][d] = vp[d * 32];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float16_t sc;
+#pragma unroll
+        for (int i = 0; i < 16; i++) sc[i] = 0.f;
+#pragma unroll
+        for (int s = 0; s < HH / 4; s++) {
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[s].x, qf[4 * s], sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[s].y, qf[4 * s + 1], sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[s].z, qf[4 * s + 2], sc, 0, 0, 0);
+            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(kr[s].w, qf[4 * s + 3], sc, 0, 0, 0);
+        }
+        // online softmax in base 2; element i = key 8 (i / 4) + 4 hf + i % 4 of the tile
+        const uint32_t key0 = t * KT + 4 * hf;
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            sc[i] = key0 + 8 * (i >> 2) + (i & 3) > qpos ? -INFINITY : sc[i];
+            tmax = fmaxf(tmax, sc[i]);
+        }
+        const float m_new = fmaxf(m, both_halves_max(tmax) * scale2);
+        const float top = m_new == -INFINITY ? 0.f : m_new;  // (every key of this wave's tiles so far masked)
+        float psum = 0.f, pv[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            pv[i] = __builtin_amdgcn_exp2f(fmaf(sc[i], scale2, -top));
+            psum += pv[i];
+        }
+        const float corr = __builtin_amdgcn_exp2f(m - top);
+        l = l * corr + xor32_sum(psum);
+        m = m_new;
+#pragma unroll
+        for (int d = 0; d < NDT; d++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) o[d][i] *= corr;
+#pragma unroll
+        for (int j = 0; j < 16; j++)
+#pragma unroll
+            for (int d = 0; d < NDT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(vr[j][d], pv[j], o[d], 0, 0, 0);
+    }
+    if (hf == 0) { sm[wave][qi] = m; sl[wave][qi] = l; }
+#pragma unroll
+    for (int d = 0; d < NDT; d++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+            *(float4 *)(&so[wave][qi * LD + d * 32 + 8 * g + 4 * hf]) = make_float4(o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]);
+    __syncthreads();
+    // thread: four dims of query tid / (HD / 4) (and of every 1024 / HD-th behind it); wave 0 has key 0, so the maximum is finite
+    // unless every key scores -inf
+    for (uint32_t q = tid / (HD / 4); q < 32 && r0 + q < n; q += 1024 / HD) {
+        const uint32_t d4 = tid % (HD / 4) * 4;
+        float mm = fmaxf(fmaxf(sm[0][q], sm[1][q]), fmaxf(sm[2][q], sm[3][q]));
+        float lt = 0.f, a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float c = sm[w][q] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sm[w][q] - mm);
+            const float4 v = *(const float4 *)(&so[w][q * LD + d4]);
+            lt += sl[w][q] * c;
+            a0 += v.x * c; a1 += v.y * c; a2 += v.z * c; a3 += v.w * c;
+        }
+        const float inv = 1.0f / lt;
+        *(float4 *)(out + ((uint64_t)b * n + r0 + q) * inner + h * HD + d4) = make_float4(a0 * inv, a1 * inv, a2 * inv, a3 * inv);
+    }
+}
+
 int launch_kv_append(const float *qkv, void *kc, void *vc, uint32_t kv_dtype, uint64_t batch,
                      uint64_t n, uint64_t heads, uint64_t hd, uint64_t max_ctx, uint64_t pos0,
                      const uint32_t *pos_dev, hipStream_t st) {
@@ -812,7 +924,19 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
     if (lp) return fail(COEUS_INVALID_INPUT, "16-bit attention output needs the matrix-core prefill kernel");
     if (kv_dtype == COEUS_KV_F32 && n >= 16 && (hd == 64 || hd == 128) && !pos_dev && out && !out_xq) {
         const dim3 pgrid((unsigned)ceil_div(n, 128), (unsigned)heads, (unsigned)batch);
-        if (hd == 64)
+        // The kernel of 32 queries and four key shares as long as 128 queries give few workgroups (us, 128 queries / 32: 12 heads of 64
+        // at 64 / 128 / 512 / 1024 rows 7.6 / 5.0, 13.0 / 6.1, 42 / 16, 81 / 49; 32 heads of 128 at 128 / 512 / 1024 23 / 12, 79 / 43,
+        // 153 / 145); beyond, each tile of keys serves four times the queries (4 x 32 heads of 128 at 1024 355 / 591; 8 x 12
+        // of 64 at 1024 216 / 266).
+        if ((uint64_t)pgrid.x * heads * batch <= (hd == 64 ? 384 : 256)) {
+            const dim3 fgrid((unsigned)ceil_div(n, 32), (unsigned)heads, (unsigned)batch);
+            if (hd == 64)
+                hipLaunchKernelGGL(attn_prefill_f32_few_kernel<64>, fgrid, dim3(256), 0, st, qkv, (const float *)kc, (const float *)vc, (uint32_t)n,
+                                   (uint32_t)heads, (uint32_t)max_ctx, (uint32_t)pos0, out);
+            else
+                hipLaunchKernelGGL(attn_prefill_f32_few_kernel<128>, fgrid, dim3(256), 0, st, qkv, (const float *)kc, (const float *)vc, (uint32_t)n,
+                                   (uint32_t)heads, (uint32_t)max_ctx, (uint32_t)pos0, out);
+        } else if (hd == 64)
             hipLaunchKernelGGL(attn_prefill_f32_kernel<64>, pgrid, dim3(256), 0, st, qkv, (const float *)kc,
                                (const float *)vc, (uint32_t)n, (uint32_t)heads, (uint32_t)max_ctx,
                                (uint32_t)pos0, out);

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__
         // gated: columns (2c, 2c+1) hold (gate_c, up_c) and sit in neighbouring lanes
         const float other = lane_xor1(acc[i]);
         if (row >= m || col >= n) continue;
-        if (!gated) epi_store(e, row, col, acc[i]);
+        if (!gated) epi_store<true>(e, row, col, acc[i]);
         else if ((lane & 1) == 0) epi_store_gated(e, row, col >> 1, acc[i], other);
     }
 }
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float *__rest
         const uint64_t row = m0 + 8 * wave + 4 * (lane >> 5) + q;
         const float other = lane_xor1(v);
         if (row >= m || col >= n) continue;
-        if (!gated) epi_store(e, row, col, v);
+        if (!gated) epi_store<true>(e, row, col, v);
         else if ((lane & 1) == 0) epi_store_gated(e, row, col >> 1, v, other);
     }
 }
@@ -1689,6 +1689,8 @@ uint64_t gemm_split_scratch_bytes(const Weight &w, uint64_t m) {
 }
 
 bool gemm_appends_kv(const Weight &w, uint64_t m, uint64_t inner, uint64_t hd) {
+    // (f32: element by element, or by the kernel that sums a split launch's planes, four columns at a time)
+    if (w.dtype == COEUS_W_F32) return m < (1ull << 32) && w.n == 3 * inner && (inner & 3) == 0 && (hd & 3) == 0;
     // rows fit 32 bits; a lane's 4 columns stay inside one head.  (The short-prompt kernel for
     // quantised weights qualifies when it is split along k: the kernel that sums its partial
     // planes runs this same epilogue.)

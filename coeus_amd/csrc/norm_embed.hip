@@ -225,46 +225,82 @@ __global__ __launch_bounds__(1024) void norm_sequence_kernel(const float *__rest
 // second launch adds up the partials in the same order, so all of them hold the same statistics.
 // part: [2][kNormSeqMaxGroups] f64.
 constexpr uint32_t kNormSeqMaxGroups = 256;
-// PHASE 0: part[0][g], part[1][g].  PHASE 1: y.
-template <bool RMS, int PHASE>
+// PHASE 0: part[0][g], part[1][g].  PHASE 1: y.  VEC: n, chunk and hidden are multiples of 4 and the pointers of 16 bytes.
+// Bound by the trips to memory one behind the other: 16 bytes a lane, both sums in one exchange, and what phase 1 does not need
+// the statistics for requested before them (98304 elements, us a launch: 4.8 + 4.7 with single elements and two exchanges).
+template <bool RMS, int PHASE, bool VEC>
 __global__ __launch_bounds__(256) void norm_sequence_part_kernel(const float *__restrict__ x, uint64_t n,
                                                                  uint64_t chunk, uint64_t hidden,
                                                                  const float *__restrict__ scale,
                                                                  const float *__restrict__ bias,
                                                                  float eps, double *part, float *y) {
-    __shared__ double sh[16];
+    __shared__ double sh[2][4];
+    constexpr uint32_t E = VEC ? 4 : 1;
+    struct Piece { float v[E]; };
+    auto load = [](const float *p) {
+        Piece r;
+        if constexpr (VEC) {
+            const float4 t = *(const float4 *)p;
+            r.v[0] = t.x; r.v[1] = t.y; r.v[2] = t.z; r.v[3] = t.w;
+        } else {
+            r.v[0] = *p;
+        }
+        return r;
+    };
+    auto block_sums = [&](double &a, double &b) {  // over 256 threads, for all of them
+        a = wave_sum_f64(a);
+        b = wave_sum_f64(b);
+        if ((threadIdx.x & 63) == 0) { sh[0][threadIdx.x >> 6] = a; sh[1][threadIdx.x >> 6] = b; }
+        lds_barrier();
+        a = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+        b = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
+    };
     const uint32_t G = gridDim.x, g = blockIdx.x;
-    const uint64_t lo = (uint64_t)g * chunk, hi = lo + chunk < n ? lo + chunk : n;
+    const uint64_t lo = (uint64_t)g * chunk, hi = lo + chunk < n ? lo + chunk : n, first = lo + threadIdx.x * E;
     const double c = RMS ? 0.0 : (double)x[0];
     if (PHASE == 0) {
         double s1 = 0.0, s2 = 0.0;
-        for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-            const double d = (double)x[i] - c;
-            s1 += d;
-            s2 += d * d;
+        for (uint64_t i = first; i < hi; i += 256 * E) {
+            const Piece p = load(x + i);
+#pragma unroll
+            for (uint32_t u = 0; u < E; u++) {
+                const double d = (double)p.v[u] - c;
+                s1 += d;
+                s2 += d * d;
+            }
         }
-        if (!RMS) s1 = block_sum_f64(s1, sh);
-        s2 = block_sum_f64(s2, sh);
+        block_sums(s1, s2);
         if (threadIdx.x == 0) {
             part[g] = s1;
             part[kNormSeqMaxGroups + g] = s2;
         }
     } else {
         // (G <= 256 = blockDim.x: one partial per thread, summed in the same order by every workgroup)
-        double s1 = !RMS && threadIdx.x < G ? part[threadIdx.x] : 0.0;
-        double s2 = threadIdx.x < G ? part[kNormSeqMaxGroups + threadIdx.x] : 0.0;
-        if (!RMS) s1 = block_sum_f64(s1, sh);
-        s2 = block_sum_f64(s2, sh);
+        const uint32_t t = threadIdx.x < G ? threadIdx.x : G - 1;
+        double s1 = part[t], s2 = part[kNormSeqMaxGroups + t];
+        const uint64_t at = first < hi ? first : lo;
+        uint64_t col = at % hidden;  // one division; then stepped along
+        Piece p = load(x + at), sc = load(scale + col), bi = RMS ? Piece{} : load(bias + col);
+        if (threadIdx.x >= G) s1 = s2 = 0.0;
+        block_sums(s1, s2);
         const double mc = RMS ? 0.0 : s1 / (double)n;
         const float var = (float)(s2 / (double)n - mc * mc);
         const float sd = sqrtf(var + eps), meanf = (float)(c + mc);
-        uint64_t col = (lo + threadIdx.x) % hidden;  // one division; then stepped along with i
-        for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-            float v = scale[col] * (x[i] - meanf) / sd;
-            if (!RMS) v += bias[col];
-            y[i] = v;
-            col += blockDim.x;
-            while (col >= hidden) col -= hidden;
+        for (uint64_t i = first; i < hi; i += 256 * E) {
+            if (i != first) {
+                col += 256 * E;
+                while (col >= hidden) col -= hidden;
+                p = load(x + i); sc = load(scale + col);
+                if (!RMS) bi = load(bias + col);
+            }
+            Piece o;
+#pragma unroll
+            for (uint32_t u = 0; u < E; u++) {
+                o.v[u] = sc.v[u] * (p.v[u] - meanf) / sd;
+                if (!RMS) o.v[u] += bi.v[u];
+            }
+            if constexpr (VEC) *(float4 *)(y + i) = make_float4(o.v[0], o.v[1], o.v[2], o.v[3]);
+            else y[i] = o.v[0];
         }
     }
 }
@@ -285,13 +321,17 @@ int launch_norm(uint32_t kind, uint32_t scope, const float *x, uint64_t rows, ui
         if (partials && n >= 32768) {
             // at least 1024 elements per workgroup (128 x 768: 96 workgroups; with 4096 per workgroup
             // 24 CUs did the work of a launch that is all latency: 6.4 + 8.2 us)
-            const uint32_t G = (uint32_t)std::min<uint64_t>(kNormSeqMaxGroups, n / 1024);
-            const uint64_t chunk = ceil_div(n, G);
-#define COEUS_NSP(RMSV, PH)                                                                          \
-    hipLaunchKernelGGL((norm_sequence_part_kernel<RMSV, PH>), dim3(G), dim3(256), 0, st, x, n, chunk, \
+            const uint64_t chunk = round_up(ceil_div(n, std::min<uint64_t>(kNormSeqMaxGroups, n / 1024)), 4);
+            const uint32_t G = (uint32_t)ceil_div(n, chunk);
+            const bool rms = kind == COEUS_NORM_RMSNORM;
+            const bool vec = hidden % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)scale | (rms ? 0 : (uintptr_t)bias)) & 15) == 0;
+#define COEUS_NSP(RMSV, PH, V)                                                                          \
+    hipLaunchKernelGGL((norm_sequence_part_kernel<RMSV, PH, V>), dim3(G), dim3(256), 0, st, x, n, chunk, \
                        hidden, scale, bias, eps, partials, y)
-            if (kind == COEUS_NORM_RMSNORM) { COEUS_NSP(true, 0); COEUS_NSP(true, 1); }
-            else { COEUS_NSP(false, 0); COEUS_NSP(false, 1); }
+            if (rms && vec) { COEUS_NSP(true, 0, true); COEUS_NSP(true, 1, true); }
+            else if (rms) { COEUS_NSP(true, 0, false); COEUS_NSP(true, 1, false); }
+            else if (vec) { COEUS_NSP(false, 0, true); COEUS_NSP(false, 1, true); }
+            else { COEUS_NSP(false, 0, false); COEUS_NSP(false, 1, false); }
 #undef COEUS_NSP
             COEUS_HIP(hipGetLastError());
             return COEUS_OK;
