@@ -1145,6 +1145,28 @@ __device__ __forceinline__ void k64_strip_gated(const float *strip, uint32_t lan
     }
 }
 
+// The same to 16 bits straight from the accumulators: a lane holds row lane % 32 of a 32 x 32 block and, per register group g, the
+// pairs of outputs 4 g + 2 (lane / 32) and + 1.  Packed, two swaps with the lane that has the row's other outputs leave 16
+// consecutive bytes a lane, 32 a row: no trip through LDS (7B shape, 4071 rows, whole pass 51.8 -> 51.1 ms).  Rows without a
+// gate are better off through LDS, where a store covers 256 bytes of a row (1B shape with GELU 44.8 -> 45.2 ms this way).
+template <bool CLAMP, bool BF16OUT>
+__device__ __forceinline__ void k64_direct_gated(const float16_t (&t)[4], uint32_t lane, const EpiArgs &e, uint64_t row, uint64_t col0,
+                                                 uint64_t em) {
+    uint16_t *out = e.out_lp + row * e.lp_ld + (col0 >> 1) + 8 * (lane >> 5);
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+        uint32_t p[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const float g0 = t[y][4 * g], u0 = t[y][4 * g + 1], g1 = t[y][4 * g + 2], u1 = t[y][4 * g + 3];
+            const float a = CLAMP ? clamped_gate(g0, u0, e.limit) : k64_silu(g0) * u0, b = CLAMP ? clamped_gate(g1, u1, e.limit) : k64_silu(g1) * u1;
+            p[g] = (uint32_t)f32_to_lp_bits(a, BF16OUT) | ((uint32_t)f32_to_lp_bits(b, BF16OUT) << 16);
+        }
+        const auto lo = __builtin_amdgcn_permlane32_swap(p[0], p[2], false, false), hi = __builtin_amdgcn_permlane32_swap(p[1], p[3], false, false);
+        if (row < em) *(uint4 *)(out + y * 16) = make_uint4(lo[0], lo[1], hi[0], hi[1]);
+    }
+}
+
 // Which of the walks above serves a wave's block: decided once per block.
 enum : uint32_t { K64_GENERIC = 0, K64_ROWS = 1, K64_KV = 2, K64_GATED = 3 };
 // for K64_ROWS the low bits of `bits` select bias (1), residual (2), GELU (4), 16-bit output (8)
@@ -1350,6 +1372,28 @@ __global__ __launch_bounds__(256) void gemm_h256k64_kernel(const uint16_t *a, co
     uint32_t bits;
     const uint32_t kind = k64_epilogue_kind(e, vec4, en0 + wn, en, bits);
     __syncthreads();  // every wave has finished reading the operand slices
+    if (kind == K64_GATED && e.out_lp && (e.lp_ld & 7) == 0 && ((uintptr_t)e.out_lp & 15) == 0) {  // 16-byte stores
+        const bool clamp = e.act == COEUS_EPI_CLAMP_GATE;
+#pragma unroll 1
+        for (uint32_t x = 0; x < 4; x++) {
+            float16_t t[4];
+#define COEUS_T(X) { t[0] = acc[X][0]; t[1] = acc[X][1]; t[2] = acc[X][2]; t[3] = acc[X][3]; }
+            if (x == 0) COEUS_T(0)
+            else if (x == 1) COEUS_T(1)
+            else if (x == 2) COEUS_T(2)
+            else COEUS_T(3)
+#undef COEUS_T
+            const uint64_t row = em0 + wm + x * 32 + (lane & 31);
+            if (e.lp_bf16) {
+                if (clamp) k64_direct_gated<true, true>(t, lane, e, row, en0 + wn, em);
+                else k64_direct_gated<false, true>(t, lane, e, row, en0 + wn, em);
+            } else {
+                if (clamp) k64_direct_gated<true, false>(t, lane, e, row, en0 + wn, em);
+                else k64_direct_gated<false, false>(t, lane, e, row, en0 + wn, em);
+            }
+        }
+        return;
+    }
     if (kind == K64_ROWS && (bits & ~1u) == 2) {
         if (bits & 1) k64_epilogue_residual<true>(strip, acc, lane, e, em0 + wm, en0 + wn, em);
         else k64_epilogue_residual<false>(strip, acc, lane, e, em0 + wm, en0 + wn, em);
