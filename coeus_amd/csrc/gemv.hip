@@ -16,6 +16,7 @@
 //   gemv_dense_kernel  f32 / bf16 weights, one wave per output row, f32 FMA on the VALU.
 //   gemv_row_kernel    one activation row behind a norm of up to 1024 elements: the row in every
 //                      wave's registers, no LDS and no barrier.
+//   gemv_many_kernel   one plain activation row: two weight rows a wave, up to four steps of both in flight.
 //   gemv_mfma_kernel   2 - 16 activation rows on f32 / bf16 weights: 16 output rows a workgroup on
 //                      the matrix cores (bf16: the f32 activations as three bf16 each).
 #include "device_utils.hpp"
@@ -1186,6 +1187,77 @@ __global__ __launch_bounds__(256) void gemv_row_kernel(const void *__restrict__ 
     }
 }
 
+// One plain activation row, k % 8 == 0: two weight rows a wave, D steps of 512 k of both in flight next to the activations they
+// share.  Bound by the weights' stream; gemv_dense_kernel, a weight row a wave and two steps at most, reads twice the weights'
+// bytes in activations (f32 next to bf16) and leaves memory idle between its steps.  us, distinct weights in turn, there /
+// here: bf16 4096 x 22016 33.2 / 29.0, x 32000 46.3 / 40.9, x 12352 19.7 / 18.3, 2048 x 11264 11.2 / 9.0, x 2048 4.3 / 3.5,
+// 3072 x 768 4.9 / 3.6; f32 4096 x 22016 74.6 / 65.9.  The matrix cores had rows of these: 5632 x 2048 7.7 / 5.5, 11008 x 4096
+// 18.4 / 17.7, 4096 x 4096 7.5 / 7.5, 768 x 50257 13.5 / 13.4, 1024 x 16384 7.5 / 6.9.  Four rows a wave with two or three steps:
+// 29.9, 40.0, 20.1, 10.1, 4.3; eight are slower than one.
+template <bool BF16, int D>
+__global__ __launch_bounds__(256) void gemv_many_kernel(const void *__restrict__ wdata, const float *__restrict__ x, uint32_t k, EpiArgs e) {
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int R = 2, Q = BF16 ? 1 : 2;
+    const uint32_t n = (uint32_t)e.n, j0 = (blockIdx.x * 4 + wave) * R, trips = (k + 512 * D - 1) / (512 * D);
+    uint4 wv[D][R][Q];
+    float4 xv[D][2];
+    const char *row[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) row[r] = (const char *)wdata + (uint64_t)min(j0 + r, n - 1) * k * (BF16 ? 2 : 4);
+    auto request = [&](int d, uint32_t step) {  // (a lane behind the end re-reads the last 8 and does not use them)
+        const uint32_t i = min(512 * step + 8 * lane, k - 8);
+        xv[d][0] = *(const float4 *)(x + i);
+        xv[d][1] = *(const float4 *)(x + i + 4);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int q = 0; q < Q; q++) wv[d][r][q] = load_stream((const uint4 *)(row[r] + (uint64_t)i * (BF16 ? 2 : 4)) + q);
+    };
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.f;
+    auto multiply = [&](int d) {
+        const float v[8] = {xv[d][0].x, xv[d][0].y, xv[d][0].z, xv[d][0].w, xv[d][1].x, xv[d][1].y, xv[d][1].z, xv[d][1].w};
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint4 a = wv[d][r][0], c = wv[d][r][Q - 1];
+            float t[8];
+            if (BF16) {
+                const uint32_t q[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+                for (int u = 0; u < 4; u++) { t[2 * u] = __uint_as_float(q[u] << 16); t[2 * u + 1] = __uint_as_float(q[u] & 0xffff0000u); }
+            } else {
+                const uint32_t q[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+                for (int u = 0; u < 8; u++) t[u] = __uint_as_float(q[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc[r] = fmaf(t[u], v[u], acc[r]);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) request(d, d);
+    for (uint32_t i = 0; i + 1 < trips; i++) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(d);
+            __builtin_amdgcn_sched_barrier(0);
+            request(d, (i + 1) * D + d);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; d++)
+        if (512 * ((trips - 1) * D + d) + 8 * lane < k) multiply(d);
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = wave_sum(acc[r]);
+    if (epi_gated(e.act)) {
+        if (lane == 0 && j0 + 1 < n) epi_store_gated(e, 0, j0 / 2, acc[0], acc[1]);
+    } else if (lane < R && j0 + lane < n) {
+        epi_store<true>(e, 0, j0 + lane, lane ? acc[1] : acc[0]);
+    }
+}
+
 // ---------------------------------------------------------------- dense rows on the matrix cores (2 - 16 rows)
 // y[b, j] for a tile of 16 weight rows j and all b at once.  bf16 weights: v_mfma_f32_16x16x32_bf16 with the weights as
 // they are stored and every activation as the sum of three bf16 (8 mantissa bits each: x exactly), three instructions
@@ -1201,7 +1273,7 @@ __global__ __launch_bounds__(256) void gemv_row_kernel(const void *__restrict__ 
 //   4096 x 22016   47 / 34     73 / 36      118 / 40      215 / 55
 //   768 x 50257    28 / 14     41 / 14       68 / 16      127 / 18
 // f32: 768 x 3072 9.0 / 4.4 at batch 8, 768 x 50257 79 / 30, 4096 x 4096 31 / 15.
-// (One row: 4.2, 8.7, 33, 18.5 there; where it comes here gemv_uses_mfma says.)  The large ones are
+// (One row: gemv_many_kernel.)  The large ones are
 // at 5 TB/s of weights.  A matrix with an infinite value stays there (times a piece that is zero it would be a NaN).
 //
 // The workgroup's waves take a share of k each, in pairs of 32-wide chunks: a wave request is 8 rows x 128 bytes, as
@@ -1624,18 +1696,8 @@ static bool gemv_mfma_shape(const Weight &w, uint32_t waves) {
 }
 // Where the matrix cores are the faster of the two (us with weights from memory: a wave per row / here).
 static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves, bool folded) {
-    if (!gemv_mfma_shape(w, waves) || batch < 1) return false;
+    if (!gemv_mfma_shape(w, waves) || batch < 2) return false;
     const bool bf = w.dtype == COEUS_W_BF16;
-    if (batch == 1) {
-        if (!bf || folded) return false;
-        // Short rows of which there are many: 768 x 50257 18.5 / 14.0, 1024 x 16384 8.7 / 7.9.
-        if (w.k <= 1024) return w.n >= 16384;
-        // Long rows of which there are few: 4096 x 4096 9.1 / 7.9, 8192 x 512 9.5 / 8.6, 11008 x 4096 21.6 / 18.9; but 2048 x 2048 4.3 / 4.8,
-        // 4096 x 6144 11.7 / 12.4 and 6144 x 6144 16.2 / 17.7.  Shares of an uneven number of pairs ask for one in vain, which up
-        // to 5120 elements takes many rows to pay: 4608 x 512 6.3 / 6.7, x 3584 9.5 / 8.9.  Rows 32 KiB apart share their memory
-        // channels: 16384 x 3584 24.4 / 22.9, x 4096 26.2 / 28.7, 32768 x 4096 50 / 66.
-        return w.k >= 4096 && w.n <= 4096 && (w.k % 2048 == 0 || w.k > 5120 || w.n >= 2048) && (w.k % 16384 || w.n <= 3584);
-    }
     // (A norm in front costs a wave per row more: f32, 2 rows of 768 x 768 7.4 / 5.8.  Two rows of bf16 are the exception where they
     // are long and few: 2560 x 4096 11.0 / 11.6, x 12288 22.7 / 19.1.)
     if (folded) return !(bf && batch == 2 && w.k > 2048 && w.n <= 4096);
@@ -2008,6 +2070,16 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         COEUS_HIP(hipGetLastError());
         return COEUS_OK;
     }
+    // f32: a wave per row is ahead on short or few rows (768 x 768 2.8 / 3.1, x 3072 4.2 / 4.3, 3072 x 768 5.6 / 5.9, 520 x 3001 3.8 / 3.9; but
+    // 1536 x 4000 7.3 / 6.7, 2048 x 2048 6.1 / 5.3, 1024 x 8192 8.6 / 8.3).  Two steps in flight are all of up to 1024 elements.
+    if (norm == 0 && b == 1 && aligned && w.k % 8 == 0 && w.k < (1ull << 31) && w.n < (1ull << 31) - 8 &&
+        (BF16 || (w.n >= 2048 && (w.k >= 1536 || w.n >= 8192)))) {
+        const dim3 mgrid((unsigned)ceil_div(w.n, 8));
+        if (w.k <= 1024) hipLaunchKernelGGL((gemv_many_kernel<BF16, 2>), mgrid, dim3(256), 0, st, w.data, xin, (uint32_t)w.k, e);
+        else hipLaunchKernelGGL((gemv_many_kernel<BF16, 4>), mgrid, dim3(256), 0, st, w.data, xin, (uint32_t)w.k, e);
+        COEUS_HIP(hipGetLastError());
+        return COEUS_OK;
+    }
     {
         // plain: workgroups enough to fill the compute units' 16 waves;
         // a folded norm: one workgroup of 16 waves per compute unit, which stages the rows once
@@ -2026,12 +2098,12 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     } while (0)
             // Pairs in flight: two or three, whichever asks for fewer in vain at the end of a wave's share.  Where that is the
             // same, three for 2 - 4 rows (us for two / three: 4 rows of bf16 5120 x 32000 67.0 / 65.5, 2 of 12288 x 8192 36.5 / 35.0), two
-            // for one row (6144 x 512 7.2 / 7.4) and for 8 (6144 x 4096 13.0 / 13.5).  A norm in front fills the first trip, and
+            // for 8 (6144 x 4096 13.0 / 13.5).  A norm in front fills the first trip, and
             // three pay from the second tile on (2 rows of bf16 3072 x 4096 12.7 / 13.3, x 12288 22.4 / 20.8).  Four in flight are
             // never faster (4 rows, us for 2 / 3 / 4: 3072 x 4096 7.1 / 6.4 / 7.1, 4096 x 4096 7.7 / 9.2 / 7.8, 10240 x 512 12.1 / 13.7 /
             // 14.0).
             const uint32_t by2 = (np + 1) / 2 * 2, by3 = (np + 2) / 3 * 3;
-            const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && batch > 1 && bp <= 4);
+            const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && bp <= 4);
 #define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (BPV < 16 && three) COEUS_MFMA4(BPV < 16 ? BPV : 8, NV, 3, false); else COEUS_MFMA4(BPV, NV, 2, false); } while (0)
 #define COEUS_MFMAN(BPV, NV)                                                                               \
     do {                                                                                                   \
