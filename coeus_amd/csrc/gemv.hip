@@ -117,6 +117,7 @@ struct XArgs {
 // The same normalisation as a launch of its own, for batches whose activation block does not fit
 // the matmul's LDS staging: row b of h -> xq, statistics merged from the producer's records
 // (no reduction over the row).  Grid (k pieces / 256, batch); every wave merges its row's records.
+// Bound by one trip to memory behind the launch: everything is requested at once, and the wave's sums are register moves.
 template <bool RMS>
 __global__ __launch_bounds__(256) void norm_from_stats_kernel(const float *__restrict__ h,
                                                               const float2 *__restrict__ stats,
@@ -124,38 +125,52 @@ __global__ __launch_bounds__(256) void norm_from_stats_kernel(const float *__res
                                                               const float *__restrict__ nbias,
                                                               float eps, uint32_t k, uint32_t k_pad,
                                                               uint32_t bp, uint4 *__restrict__ xq) {
+    constexpr int SREC = 4;  // records a lane holds (k <= 4096); the others are read again
     const uint32_t lane = threadIdx.x & 63, b = blockIdx.y, nt = (k + 15) / 16;
     const uint32_t kp = blockIdx.x * 256 + threadIdx.x;  // piece = 8 consecutive k
-    const float2 *rec = stats + (uint64_t)b * nt;
-    float s = 0.f;
-    for (uint32_t t = lane; t < nt; t += 64) s += rec[t].x;
+    const uint32_t kk = kp * 8, kc = kk < k ? kk : 0;    // k % 8 == 0
+    const float2 *row = stats + (uint64_t)b * nt;
+    float2 rec[SREC];
+#pragma unroll
+    for (int u = 0; u < SREC; u++) rec[u] = row[min(lane + 64 * u, nt - 1)];
+    const float4 a0 = *(const float4 *)(h + (uint64_t)b * k + kc), a1 = *(const float4 *)(h + (uint64_t)b * k + kc + 4);
+    const float4 s0 = *(const float4 *)(nscale + kc), s1 = *(const float4 *)(nscale + kc + 4);
+    const float *nb = RMS ? nscale : nbias;
+    const float4 b0 = *(const float4 *)(nb + kc), b1 = *(const float4 *)(nb + kc + 4);
+    __builtin_amdgcn_sched_barrier(0);
+    auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
     const float rk = __builtin_amdgcn_rcpf((float)k);
-    const float mean = RMS ? 0.f : wave_sum(s) * rk;
-    const uint32_t tail = k & 15;
-    float q = 0.f;
-    for (uint32_t t = lane; t < nt; t += 64) {
-        const bool last = tail && t == nt - 1;
-        const float c = last ? (float)tail : 16.f;
-        const float d = rec[t].x * __builtin_amdgcn_rcpf(c) - mean;
-        q += fmaf(c * d, d, rec[t].y);
+    float mean = 0.f;
+    if (!RMS) {
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < SREC; u++) s += lane + 64 * u < nt ? rec[u].x : 0.f;
+        for (uint32_t t = lane + 64 * SREC; t < nt; t += 64) s += row[t].x;
+        mean = row_sum(s) * rk;
     }
-    const float rsd = __builtin_amdgcn_rsqf(wave_sum(q) * rk + eps);
+    const uint32_t tail = k & 15;
+    const float rc_tail = tail ? __builtin_amdgcn_rcpf((float)tail) : 0.0625f;
+    float q = 0.f;
+    auto spread = [&](const float2 &r, uint32_t t) {
+        const bool last = tail && t == nt - 1;
+        const float d = r.x * (last ? rc_tail : 0.0625f) - mean;
+        return fmaf((last ? (float)tail : 16.f) * d, d, r.y);
+    };
+#pragma unroll
+    for (int u = 0; u < SREC; u++) q += lane + 64 * u < nt ? spread(rec[u], lane + 64 * u) : 0.f;
+    for (uint32_t t = lane + 64 * SREC; t < nt; t += 64) q += spread(row[t], t);
+    const float rsd = __builtin_amdgcn_rsqf(row_sum(q) * rk + eps);
     if (kp >= k_pad / 8) return;
     uint4 o = make_uint4(0, 0, 0, 0);
-    const uint32_t kk = kp * 8;
-    if (kk < k) {  // k % 8 == 0
-        const float4 a0 = *(const float4 *)(h + (uint64_t)b * k + kk), a1 = *(const float4 *)(h + (uint64_t)b * k + kk + 4);
-        const float4 s0 = *(const float4 *)(nscale + kk), s1 = *(const float4 *)(nscale + kk + 4);
+    if (kk < k) {
         const float v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
         const float sc[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+        const float bi[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
         float y[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) y[u] = (v[u] - mean) * (sc[u] * rsd);
-        if (!RMS) {
-            const float4 b0 = *(const float4 *)(nbias + kk), b1 = *(const float4 *)(nbias + kk + 4);
-            const float bi[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-#pragma unroll
-            for (int u = 0; u < 8; u++) y[u] += bi[u];
+        for (int u = 0; u < 8; u++) {
+            y[u] = (v[u] - mean) * (sc[u] * rsd);
+            if (!RMS) y[u] += bi[u];
         }
         union { uint4 u; half2_t h2[4]; } cv;
 #pragma unroll
