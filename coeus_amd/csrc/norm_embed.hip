@@ -13,9 +13,8 @@
 namespace coeus {
 
 __device__ __forceinline__ float block_sum(float v, float *sh) {
-    // blockDim.x <= 1024; sh holds 16 floats
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-    v = wave_sum(v);
+    v = xor32_sum(xor16_sum(group_sum<16>(v)));  // (whole waves)
     __syncthreads();
     if (lane == 0) sh[wave] = v;
     __syncthreads();
@@ -373,6 +372,9 @@ int launch_norm(uint32_t kind, uint32_t scope, const float *x, uint64_t rows, ui
 
 // Norm behind a sublayer: h[row, :] += y[row, :] / rms(y[row, :]) * scale (* ls), and the 16-bit copy of
 // the new h for the next matmul.  One workgroup per row; rows of up to 8192 elements are read once.
+// VM > 0: up to 1024 VM elements, a multiple of 4; VM = 0: any width.  One row (a decode step) is bound by trips to memory: the
+// vectors and the residual row are requested with y, not behind its sum.
+template <int VM>
 __global__ __launch_bounds__(256) void norm_residual_kernel(const float *__restrict__ y, uint32_t hidden,
                                                             const float *__restrict__ scale,
                                                             const float *__restrict__ ls, float eps, float *h,
@@ -381,33 +383,40 @@ __global__ __launch_bounds__(256) void norm_residual_kernel(const float *__restr
     const uint64_t row = blockIdx.x;
     const float *yr = y + row * hidden;
     float *hr = h + row * hidden;
-    constexpr int VMAX = 8;
-    if ((hidden & 3) == 0 && hidden <= 4u * 256u * VMAX && (lp_ld & 3) == 0) {
+    if constexpr (VM > 0) {
         const uint32_t n4 = hidden / 4;
-        float4 v[VMAX];
+        float4 v[VM], sc[VM], l4[VM], o[VM];
+        const float *lp = ls ? ls : scale;
+#pragma unroll
+        for (int u = 0; u < VM; u++) {
+            const uint32_t i = min(threadIdx.x + 256 * u, n4 - 1);
+            v[u] = *(const float4 *)(yr + 4 * i);
+            sc[u] = *(const float4 *)(scale + 4 * i);
+            l4[u] = *(const float4 *)(lp + 4 * i);
+            o[u] = *(const float4 *)(hr + 4 * i);
+        }
+        __builtin_amdgcn_sched_barrier(0);
         float s2 = 0.f;
 #pragma unroll
-        for (int u = 0; u < VMAX; u++) {
-            const uint32_t i = threadIdx.x + 256 * u;
-            v[u] = i < n4 ? *(const float4 *)(yr + 4 * i) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int u = 0; u < VM; u++) {
+            if (threadIdx.x + 256 * u >= n4) v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
             s2 = fmaf(v[u].x, v[u].x, s2); s2 = fmaf(v[u].y, v[u].y, s2);
             s2 = fmaf(v[u].z, v[u].z, s2); s2 = fmaf(v[u].w, v[u].w, s2);
+            if (!ls) l4[u] = make_float4(1.f, 1.f, 1.f, 1.f);
         }
         const float rs = 1.0f / sqrtf(block_sum(s2, sh) / (float)hidden + eps);
 #pragma unroll
-        for (int u = 0; u < VMAX; u++) {
+        for (int u = 0; u < VM; u++) {
             const uint32_t i = threadIdx.x + 256 * u;
             if (i >= n4) continue;
-            const float4 sc = *(const float4 *)(scale + 4 * i);
-            const float4 l4 = ls ? *(const float4 *)(ls + 4 * i) : make_float4(1.f, 1.f, 1.f, 1.f);
-            float4 o = *(const float4 *)(hr + 4 * i);
-            o.x = fmaf(v[u].x * rs * sc.x, l4.x, o.x); o.y = fmaf(v[u].y * rs * sc.y, l4.y, o.y);
-            o.z = fmaf(v[u].z * rs * sc.z, l4.z, o.z); o.w = fmaf(v[u].w * rs * sc.w, l4.w, o.w);
-            *(float4 *)(hr + 4 * i) = o;
+            float4 r = o[u];
+            r.x = fmaf(v[u].x * rs * sc[u].x, l4[u].x, r.x); r.y = fmaf(v[u].y * rs * sc[u].y, l4[u].y, r.y);
+            r.z = fmaf(v[u].z * rs * sc[u].z, l4[u].z, r.z); r.w = fmaf(v[u].w * rs * sc[u].w, l4[u].w, r.w);
+            *(float4 *)(hr + 4 * i) = r;
             if (h_lp) {
                 uint2 p;
-                p.x = (uint32_t)f32_to_lp_bits(o.x, lp_bf16) | ((uint32_t)f32_to_lp_bits(o.y, lp_bf16) << 16);
-                p.y = (uint32_t)f32_to_lp_bits(o.z, lp_bf16) | ((uint32_t)f32_to_lp_bits(o.w, lp_bf16) << 16);
+                p.x = (uint32_t)f32_to_lp_bits(r.x, lp_bf16) | ((uint32_t)f32_to_lp_bits(r.y, lp_bf16) << 16);
+                p.y = (uint32_t)f32_to_lp_bits(r.z, lp_bf16) | ((uint32_t)f32_to_lp_bits(r.w, lp_bf16) << 16);
                 *(uint2 *)(h_lp + row * lp_ld + 4 * i) = p;
             }
         }
@@ -426,8 +435,15 @@ __global__ __launch_bounds__(256) void norm_residual_kernel(const float *__restr
 int launch_norm_residual(const float *y, uint64_t rows, uint64_t hidden, const float *scale, const float *ls,
                          float eps, float *h, hipStream_t st, const LpOut *h_lp) {
     if (rows == 0 || hidden == 0 || hidden > 0xffffffffull) return fail(COEUS_INVALID_INPUT, "bad normalisation shape");
-    hipLaunchKernelGGL(norm_residual_kernel, dim3((unsigned)rows), dim3(256), 0, st, y, (uint32_t)hidden, scale, ls,
-                       eps, h, h_lp ? (uint16_t *)h_lp->p : nullptr, h_lp ? h_lp->ld : 0, h_lp && h_lp->bf16);
+    const bool vec = (hidden & 3) == 0 && hidden <= 8192 && !(h_lp && (h_lp->ld & 3));
+#define COEUS_NRES(VM) hipLaunchKernelGGL(norm_residual_kernel<VM>, dim3((unsigned)rows), dim3(256), 0, st, y, (uint32_t)hidden, scale, ls, \
+                       eps, h, h_lp ? (uint16_t *)h_lp->p : nullptr, h_lp ? h_lp->ld : 0, h_lp && h_lp->bf16)
+    if (!vec) COEUS_NRES(0);
+    else if (hidden <= 1024) COEUS_NRES(1);
+    else if (hidden <= 2048) COEUS_NRES(2);
+    else if (hidden <= 4096) COEUS_NRES(4);
+    else COEUS_NRES(8);
+#undef COEUS_NRES
     COEUS_HIP(hipGetLastError());
     return COEUS_OK;
 }
@@ -442,13 +458,15 @@ __global__ __launch_bounds__(VM == 1 ? 1024 : 256) void hyper_kernel(float *__re
     const uint64_t row = blockIdx.x;
     const uint32_t n4 = hidden / 4, S = h.streams;
     float *xr = x + row * S * hidden;
-    float4 v[VM];
+    float4 v[VM], nw[VM];
     float s1 = 0.f;
 #pragma unroll
     for (int u = 0; u < VM; u++) {
         const uint32_t i = threadIdx.x + blockDim.x * u;
         v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        nw[u] = make_float4(1.f, 1.f, 1.f, 1.f);
         if (i >= n4) continue;
+        if (h.norm) nw[u] = *(const float4 *)(h.norm + 4 * i);  // (not behind the sums: a trip to memory less)
         float4 a[SMAX], y;
         if (h.y) y = *(const float4 *)(h.y + row * hidden + 4 * i);
 #pragma unroll
@@ -498,7 +516,7 @@ __global__ __launch_bounds__(VM == 1 ? 1024 : 256) void hyper_kernel(float *__re
     for (int u = 0; u < VM; u++) {
         const uint32_t i = threadIdx.x + blockDim.x * u;
         if (i >= n4) continue;
-        const float4 sc = h.norm ? *(const float4 *)(h.norm + 4 * i) : make_float4(1.f, 1.f, 1.f, 1.f);
+        const float4 sc = nw[u];
         const float4 o = make_float4((v[u].x - mean) * rs * sc.x, (v[u].y - mean) * rs * sc.y, (v[u].z - mean) * rs * sc.z,
                                      (v[u].w - mean) * rs * sc.w);
         if (out) *(float4 *)(out + row * hidden + 4 * i) = o;
