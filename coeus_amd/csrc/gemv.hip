@@ -292,7 +292,7 @@ void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds
             const float up = lane_xor1(v);
             if (live && (o & 1) == 0) {
                 const uint64_t m = col >> 1;
-                float g = fast_silu(v) * up;
+                float g = silu_f32(v) * up;
                 if (e.residual) g += e.residual[(uint64_t)b * e.n_eff + m];
                 if (e.out_f32) e.out_f32[(uint64_t)b * e.n_eff + m] = g;
                 if (e.out_xq) e.out_xq[xq_index(m, b, e.bp_out)] = __float2half_rn(g);
@@ -300,7 +300,7 @@ void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds
             }
             continue;
         }
-        if (e.act == COEUS_EPI_GELU) v = fast_gelu(v);
+        if (e.act == COEUS_EPI_GELU) v = gelu_f32(v);
         if (e.residual) v += first ? res_pre : live ? e.residual[(uint64_t)b * e.n_eff + col] : 0.f;
         if (live) {
             if (e.out_f32) e.out_f32[(uint64_t)b * e.n_eff + col] = v;
