@@ -403,8 +403,8 @@ __device__ __forceinline__ bool epi_vec4(const EpiArgs &e) {
     return (e.n_eff & 3) == 0 && (e.lp_ld & 3) == 0 && (e.out_f32 || e.out_lp) && !e.out_xq;
 }
 // Columns col .. col + 3 of activation row `row` (bias, cache append or activation, residual, store).
-// FAST: GELU and SiLU on the hardware's exp2 and reciprocal (1 ulp each).
-template <bool FAST = false>
+// OWN: GELU and SiLU by times_sigmoid, no further off than the math library forms.
+template <bool OWN = false>
 __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCols &kc, uint64_t row,
                                          uint64_t col, uint64_t n, float (&v)[4]) {
     if (vec4 && col + 3 < n) {
@@ -428,7 +428,7 @@ __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCo
         }
         if (e.act == COEUS_EPI_GELU)
 #pragma unroll
-            for (int q = 0; q < 4; q++) v[q] = FAST ? fast_gelu(v[q]) : gelu_tanh(v[q]);
+            for (int q = 0; q < 4; q++) v[q] = OWN ? gelu_f32(v[q]) : gelu_tanh(v[q]);
         if (e.act == COEUS_EPI_SOFTCAP)
 #pragma unroll
             for (int q = 0; q < 4; q++) v[q] = soft_cap(v[q], e.limit);
@@ -445,14 +445,14 @@ __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCo
 }
 // Gated outputs ocol .. ocol + 3 of row `row`, from the weight rows (gate, up) = raw columns
 // raw .. raw + 7 (raw = 2 ocol).
-template <bool FAST = false>
+template <bool OWN = false>
 __device__ __forceinline__ void epi_row4_gated(const EpiArgs &e, bool vec4, uint64_t row, uint64_t ocol,
                                                uint64_t raw, uint64_t n, const float (&gv)[4],
                                                const float (&uv)[4]) {
     if (vec4 && !e.bias && !e.residual && raw + 7 < n) {
         float o[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) o[q] = e.act == COEUS_EPI_CLAMP_GATE ? clamped_gate(gv[q], uv[q], e.limit) : (FAST ? fast_silu(gv[q]) : silu(gv[q])) * uv[q];
+        for (int q = 0; q < 4; q++) o[q] = e.act == COEUS_EPI_CLAMP_GATE ? clamped_gate(gv[q], uv[q], e.limit) : (OWN ? silu_f32(gv[q]) : silu(gv[q])) * uv[q];
         epi_store4(e, row, ocol, o);
     } else {
 #pragma unroll

@@ -58,3 +58,10 @@ def _silu_and_gelu(dtype, k, rows, call, f16_weights=False):
 @pytest.mark.parametrize("rows", [5, 8, 16])
 def test_decode_rows_on_quantised_weights(dtype, rows):
     _silu_and_gelu(dtype, 64, rows, "gemv")
+
+
+# tiles of 128 rows by 64 columns; few slices of k, and many
+@pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_Q8_0])
+@pytest.mark.parametrize("k,rows", [(64, 65), (64, 300), (4096, 100)])
+def test_prompts_of_few_tiles(dtype, k, rows):
+    _silu_and_gelu(dtype, k, rows, "gemm", f16_weights=dtype == _lib.W_Q8_0)
