@@ -1426,6 +1426,9 @@ struct NarrowTile {
     static constexpr int WN = 4 / WM, ROWS = WM * RB * 32, COLS = WN * NB * 32;
     static constexpr int UA = ROWS / 32, UW = COLS / 32;  // requests of a wave and slice: 8 rows x 128 bytes each, four waves an operand
     static constexpr int DA = ROWS == 256 ? 3 : 5, DW = ROWS == 256 ? (COLS == 128 ? 4 : COLS == 96 ? 5 : 6) : COLS == 128 ? 5 : 6;
+    // Sums can begin again after some slices (a wave of eight blocks has no registers for that), see GemmPlan.
+    static constexpr bool AGAIN = RB * NB <= 6;
+    static constexpr int TRB = AGAIN ? RB : 1, TNB = AGAIN ? NB : 1;
     static constexpr size_t ring = ((size_t)DA * ROWS + (size_t)DW * COLS) * UK * 2, tile = (size_t)ROWS * (COLS + 4) * 4, lds = ring > tile ? ring : tile;
     static_assert(lds <= 160 * 1024, "fits the LDS of a CU");
 };
@@ -1463,7 +1466,7 @@ __device__ __forceinline__ void narrow_step(const uint16_t *__restrict__ ra, con
 
 template <bool BF16, int WM, int RB, int NB>
 __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, const uint16_t *w, uint64_t m, uint64_t n, uint64_t k, uint64_t lda,
-                                                          uint64_t ldw, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits, EpiArgs e) {
+                                                          uint64_t ldw, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits, uint32_t period, EpiArgs e) {
     using T = NarrowTile<WM, RB, NB>;
     constexpr int DA = T::DA, DW = T::DW, Q = T::UA > T::UW ? T::UA : T::UW;
     constexpr uint32_t RA = T::ROWS * UK, RW = T::COLS * UK;  // elements of a region
@@ -1486,6 +1489,11 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
         for (int y = 0; y < NB; y++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[x][y][i] = 0.f;
+    float16_t total[T::TRB][T::TNB];  // of the slices before the present ones
+#pragma unroll
+    for (int x = 0; x < T::TRB; x++)
+#pragma unroll
+        for (int y = 0; y < T::TNB; y++) total[x][y] = acc[x][y];
     const bool takes_a = half == 0;
     uint32_t off[Q];
     {
@@ -1539,6 +1547,7 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
     // Slice s: the products of its first step, while the second step's fragments are read; then, when nobody reads the slice any
     // more, those of the second, while the next slice's are read.  Slice s + depth goes into the region of slice s.
     uint32_t ia = 0, iw = 0, io = depth - 1;  // regions of slice s; of slice s - 1, whose second half of requests is left
+    uint32_t until = period - 1;  // the slice behind which sums begin again
     for (uint32_t s = 0; s < nsl; s++) {
         if (s) {
             narrow_step<BF16, T, RB, NB, true>(rega + ia * RA, regw + iw * RW, ring + io * rsize, source(kbeg + (uint64_t)(s - 1 + depth) * UK), off,
@@ -1558,6 +1567,27 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
         io = io + 1 == depth ? 0 : io + 1;
         narrow_step<BF16, T, RB, NB, false>(rega + ia * RA, regw + iw * RW, freed, source(kbeg + (uint64_t)(s + depth) * UK), off, takes_a, w4,
                                             la[0], lw[0], af[1], wf[1], af[0], wf[0], acc);
+        if constexpr (T::AGAIN) {
+            if (s == until) {
+                until += period;
+#pragma unroll
+                for (int x = 0; x < RB; x++)
+#pragma unroll
+                    for (int y = 0; y < NB; y++)
+#pragma unroll
+                        for (int i = 0; i < 16; i++) { total[x][y][i] += acc[x][y][i]; acc[x][y][i] = 0.f; }
+            }
+        }
+    }
+    if constexpr (T::AGAIN) {
+        if (period <= nsl) {
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+#pragma unroll
+                for (int y = 0; y < NB; y++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[x][y][i] += total[x][y][i];
+        }
     }
     __builtin_amdgcn_s_waitcnt(0x0070);  // the repeats have landed too
     __syncthreads();
@@ -1614,22 +1644,22 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
 
 template <bool BF16, int WM, int RB, int NB>
 static int launch_narrow(const uint16_t *a, const uint16_t *w, uint64_t m, uint64_t n, uint64_t k, uint64_t lda, uint64_t ldw, uint32_t splits,
-                         const EpiArgs &e, hipStream_t st) {
+                         uint32_t period, const EpiArgs &e, hipStream_t st) {
     using T = NarrowTile<WM, RB, NB>;
     static const hipError_t once = hipFuncSetAttribute((const void *)gemm_narrow_kernel<BF16, WM, RB, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     COEUS_HIP(once);
     const uint32_t tiles_m = (uint32_t)ceil_div(m, T::ROWS), tiles_n = (uint32_t)ceil_div(n, T::COLS);
     hipLaunchKernelGGL((gemm_narrow_kernel<BF16, WM, RB, NB>), dim3((uint32_t)round_up((uint64_t)tiles_m * tiles_n * splits, 8)), dim3(512), T::lds, st, a, w, m, n, k,
-                       lda, ldw, tiles_m, tiles_n, splits, e);
+                       lda, ldw, tiles_m, tiles_n, splits, period, e);
     COEUS_HIP(hipGetLastError());
     return COEUS_OK;
 }
 template <bool BF16>
 static int launch_narrow_plan(uint32_t rows, uint32_t cols, const uint16_t *a, const uint16_t *wp, uint64_t m, const Weight &w, uint64_t lda,
-                              uint64_t ldw, uint32_t splits, const EpiArgs &e, hipStream_t st) {
-    if (rows == 256) return cols == 128 ? launch_narrow<BF16, 2, 4, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st) : launch_narrow<BF16, 4, 2, 3>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st);
-    if (cols == 128) return launch_narrow<BF16, 2, 2, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st);
-    return cols == 96 ? launch_narrow<BF16, 4, 1, 3>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st) : launch_narrow<BF16, 4, 1, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, e, st);
+                              uint64_t ldw, uint32_t splits, uint32_t period, const EpiArgs &e, hipStream_t st) {
+    if (rows == 256) return cols == 128 ? launch_narrow<BF16, 2, 4, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, period, e, st) : launch_narrow<BF16, 4, 2, 3>(a, wp, m, w.n, w.k, lda, ldw, splits, period, e, st);
+    if (cols == 128) return launch_narrow<BF16, 2, 2, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, period, e, st);
+    return cols == 96 ? launch_narrow<BF16, 4, 1, 3>(a, wp, m, w.n, w.k, lda, ldw, splits, period, e, st) : launch_narrow<BF16, 4, 1, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, period, e, st);
 }
 
 // Any number of rows: a short prompt leaves most of a 256-row tile empty (rows past the end are
@@ -1678,7 +1708,13 @@ static uint32_t gemm_splits_wanted(const Weight &w, uint64_t m) {
 // (2048 x 2048, 65 rows, 12.6 against 11.2 us).  us, 256x256 tiles / this: 201 rows of 4096 x 4096 32.8 / 21.7, of 4096 x 12288
 // 53.0 / 38.3, of 4096 x 22016 70.8 / 59.8, of 11008 x 4096 56.2 / 39.4; 512 of 768 x 3072 25.3 / 9.4, of 3072 x 768
 // 28.3 / 16.3; 1019 of 4096 x 4096 55.6 / 44.4; 2036 of 2048 x 2048 42.6 / 27.5, of 1024 x 2048 30.9 / 17.8.
-struct GemmPlan { uint32_t rows = 0, cols = 0, splits = 1; };
+// Roundings: a result is the end of a chain of k / 16 sums in the 256x256 tiles, of k / 32 here, divided by the shares, and of the
+// shares' sum.  Few shares of a long k were up to twice as far from 64 bits as the tiles whose place they take.  So sums begin again every
+// `period` slices, as seldom as makes the chain no longer than theirs; 256x128 has no registers for that and is taken where its
+// shares are at least half as many.  bf16, root mean square error in 1e-8 of the result's, 256x256 tiles / without that / so, and us without / with:
+// 700 rows of 5632 x 2048 15.9 / 32.3 / 15.7, 31.1 / 32.8; 300 of 4096 x 4096 13.7 / 27.1 / 13.3, 25.4 / 25.7; 201 of 4096 x 4096
+// 13.6 / 18.8 / 13.3, 20.4 / 20.6; 512 of 768 x 768 9.3 / 11.0 / 8.3, 8.2 / 8.7; 65 of 2048 x 8192 10.2 / 18.5 / 9.8, 14.6 / 15.5.
+struct GemmPlan { uint32_t rows = 0, cols = 0, splits = 1, period = ~0u; };
 static constexpr uint32_t kNarrowTiles[][2] = {{256, 128}, {256, 96}, {128, 128}, {128, 96}, {128, 64}};
 static GemmPlan gemm_plan(const Weight &w, uint64_t m, bool may_split) {
     GemmPlan best;
@@ -1686,14 +1722,24 @@ static GemmPlan gemm_plan(const Weight &w, uint64_t m, bool may_split) {
     const uint64_t tiles256 = ceil_div(m, TM) * ceil_div(w.n, TN), slices = w.k / UK;
     if (!gemm_uses_h256(w, m) || w.k % UK || tiles256 > 256) return best;
     auto sum_us = [&](uint64_t splits) { return splits > 1 ? 5.8 + (double)(splits * m * w.n) * 8.0 / 4.4e6 : 0.0; };
-    double best_us = 0.95 * (14.0 + 0.9 * (double)ceil_div(slices, best.splits) + sum_us(best.splits));
+    const uint64_t shares = best.splits;
+    double best_us = 0.95 * (14.0 + 0.9 * (double)ceil_div(slices, shares) + sum_us(shares));
     for (const auto &t : kNarrowTiles) {
         const uint64_t tiles = ceil_div(m, t[0]) * ceil_div(w.n, t[1]);
         for (uint64_t s = 1; s <= (may_split ? 16 : 1) && (s == 1 || (tiles * s <= 256 && slices / s >= 3)); s++) {
+            if (t[0] * t[1] == 256 * 128 && 2 * s < shares) continue;
             const double kb = 0.125 * (t[0] + t[1]), busy = (double)std::min<uint64_t>(256, tiles * s);
             const double us = (double)ceil_div(tiles * s, 256) * (3.6 + 0.25 * t[0] * t[1] / 1024.0 + (double)ceil_div(slices, s) * kb * std::max(1 / 66.0, busy / 17e3)) + sum_us(s);
             if (us < best_us) { best_us = us; best.rows = t[0]; best.cols = t[1]; best.splits = (uint32_t)s; }
         }
+    }
+    if (best.rows && best.rows * best.cols < 256 * 128) {
+        auto planes = [](uint64_t s) { return s > 1 ? s : 0; };
+        const uint64_t share = ceil_div(slices, best.splits), most = 4 * ceil_div(slices, shares) + planes(shares);
+        auto chain = [&](uint64_t parts) { return ceil_div(2 * share, parts) + parts + planes(best.splits); };
+        uint64_t parts = 1;
+        while (chain(parts) > most && chain(parts + 1) < chain(parts)) parts++;
+        if (parts > 1) best.period = (uint32_t)ceil_div(share, parts);
     }
     return best;
 }
@@ -1838,8 +1884,8 @@ int launch_gemm(const Weight &w, const void *a_in, uint64_t m, const Epilogue &e
         if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
         for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) {
             if (plan.rows)
-                COEUS_TRY(bf ? launch_narrow_plan<true>(plan.rows, plan.cols, ap, wp, m, w, lda, ldw, splits, ke, st)
-                             : launch_narrow_plan<false>(plan.rows, plan.cols, ap, wp, m, w, lda, ldw, splits, ke, st));
+                COEUS_TRY(bf ? launch_narrow_plan<true>(plan.rows, plan.cols, ap, wp, m, w, lda, ldw, splits, plan.period, ke, st)
+                             : launch_narrow_plan<false>(plan.rows, plan.cols, ap, wp, m, w, lda, ldw, splits, plan.period, ke, st));
             else if (w.k % UK == 0 && bf)
                 hipLaunchKernelGGL(gemm_h256k64_kernel<true>, grid, dim3(256), lds64, st, ap, wp, m, w.n, w.k, lda, ldw, tiles_m, tiles_n, ksplits, full_tiles, tail_part, ke);
             else if (w.k % UK == 0)

@@ -22,3 +22,16 @@ def test_decode_rows_on_quantised_weights(dtype, k, n, limit, rows):
     x = np.random.default_rng(k).standard_normal((rows, k)).astype(np.float32)
     want = x.astype(np.float16).astype(np.float64) @ wt.dequantize().astype(np.float64)
     assert _rms(wt.gemv(dev(x)), want) <= limit
+
+
+# Limits: 256x256 tiles with the shares of k that they take there (8, 8, 8, 3, 8, 5), one sum per 16 of k, and 2 % for other inputs
+@pytest.mark.parametrize("dtype,m,k,n,limit", [(_lib.W_BF16, 700, 5632, 2048, 1.62e-7), (_lib.W_BF16, 300, 4096, 4096, 1.40e-7), (_lib.W_BF16, 201, 2048, 2048, 1.04e-7),
+                                               (_lib.W_BF16, 512, 768, 768, 9.45e-8), (_lib.W_Q8_0, 300, 4096, 4096, 1.59e-7), (_lib.W_BF16, 65, 4096, 12288, 1.72e-7)])
+def test_prompts_of_few_tiles(orc, dtype, m, k, n, limit):
+    wt = Weight(dtype, seed=5, shape=(k, n))
+    a = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+    rows = np.arange(0, m, m // 24)
+    ar, wd = a[rows], wt.dequantize()
+    ar, wd = (orc.bf16_round(ar), wd) if dtype == _lib.W_BF16 else (ar.astype(np.float16), wd.astype(np.float16))
+    want = ar.astype(np.float64) @ wd.astype(np.float64)
+    assert _rms(wt.gemm(dev(a))[rows], want) <= limit
