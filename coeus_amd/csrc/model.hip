@@ -9,6 +9,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <thread>
 
 namespace coeus {
@@ -117,8 +118,25 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
         p = i % kPieces;
         return r < rounds && p * kPiece < size(r);
     };
+    // Every thread spins for some milliseconds.  After that the calling one waits in the runtime, which knows of errors, and the others
+    // sleep until it has seen the first piece: a long pass keeps no core busy with its results.
+    const auto start = std::chrono::steady_clock::now();
+    auto long_since = [&] { return std::chrono::steady_clock::now() - start >= std::chrono::milliseconds(5); };
+    std::mutex mu;
+    std::condition_variable first_seen;
+    std::atomic<bool> seen{false};
+    auto wake = [&](std::atomic<bool> &what) {
+        { std::lock_guard<std::mutex> lock(mu); what.store(true); }
+        first_seen.notify_all();
+    };
     auto helper = [&](uint32_t t) {
         share(t);
+        for (uint32_t n = 1; !seen.load() && !stop.load(); n++) {
+            __builtin_ia32_pause();
+            if (n % 256 || !long_since()) continue;
+            std::unique_lock<std::mutex> lock(mu);
+            first_seen.wait(lock, [&] { return seen.load() || stop.load(); });
+        }
         for (uint64_t r, p; !stop.load(std::memory_order_relaxed) && take(r, p);) {
             while (!arrived(r, p)) {
                 if (stop.load(std::memory_order_relaxed)) return;
@@ -136,17 +154,15 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
         }
     }
     share(0);
-    // This thread also launches the rounds that wait for a half to be copied out.  It spins for some milliseconds, then
-    // waits in the runtime, which knows of errors.
+    // This thread also launches the rounds that wait for a half to be copied out.
     hipError_t err = hipSuccess;
     uint64_t launched = std::min<uint64_t>(rounds, 2);
-    const auto start = std::chrono::steady_clock::now();
     auto wait = [&](auto ready, uint64_t needs) {  // needs: the rounds that `ready` is about are launched when this many are
         for (uint32_t n = 1; !ready() && err == hipSuccess; n++) {
             // round `launched` takes the half of round launched - 2, the last of launched / 2 rounds out of that half
             if (launched < rounds && copied[launched % 2].load(std::memory_order_acquire) == launched / 2 * kPieces) err = launch(launched++);
             __builtin_ia32_pause();
-            if (n % 256 || std::chrono::steady_clock::now() - start < std::chrono::milliseconds(5)) continue;
+            if (n % 256 || !long_since()) continue;
             const bool all = launched >= needs;
             if (err == hipSuccess) err = hipStreamSynchronize(st);
             if (err == hipSuccess && all && needs && !ready()) err = hipErrorUnknown;  // (the launch is over and its flag is not there)
@@ -155,11 +171,13 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
     };
     for (uint64_t r, p; err == hipSuccess && take(r, p);) {
         wait([&] { return arrived(r, p); }, r + 1);
-        if (err == hipSuccess) copy(r, p);
+        if (err != hipSuccess) break;
+        if (threads > 1 && !seen.load(std::memory_order_relaxed)) wake(seen);
+        copy(r, p);
     }
     // (other threads' last pieces)
     wait([&] { return copied[0].load(std::memory_order_acquire) + copied[1].load(std::memory_order_acquire) == ceil_div(bytes, kPiece); }, 0);
-    if (err != hipSuccess) stop.store(true);
+    if (err != hipSuccess) wake(stop);
     for (std::thread &t : others)
         if (t.joinable()) t.join();
     COEUS_HIP(err);

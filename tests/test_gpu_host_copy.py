@@ -1,6 +1,8 @@
 """Logits on their way to the caller: sizes around the pinned slots (1 MiB, four of them) and results that start in the
 middle of a page, against the same rows fetched one at a time."""
 import ctypes as C
+import resource
+import time
 
 import numpy as np
 import pytest
@@ -73,3 +75,25 @@ def test_pieces_halves_and_threads(vocab, rows):
         d = DeviceArray((rows * vocab,), np.float32)
         _check(lib.coeus_model_forward_all(model._h, ids.ctypes.data, rows, d.ptr))
         assert np.array_equal(model.forward_all(ids).ravel(), d.to_host())
+
+
+def test_long_pass_keeps_no_core_busy():
+    """Results large enough for three threads behind a pass of some 100 ms: the two others sleep.  The calling thread may spin for all
+    of it in the runtime (1.0 of the pass), the others for 5 ms each and their share of the copy; without sleep 3.0 in all."""
+    cfg = Transformer250MConfig(hidden_dim=2048, num_layers=48, num_heads=16, intermediate_dim=8192, vocab_size=1100, max_seq_len=2048,
+                                norm_scope="token")
+    model = TransformerModelPlugin().create_builder().build(cfg, seed=3)
+    ids = np.random.default_rng(5).integers(0, 1100, 2048, dtype=np.uint64)
+    d = DeviceArray((2048 * 1100,), np.float32)
+    _check(_lib.load().coeus_model_forward_all(model._h, ids.ctypes.data, 2048, d.ptr))
+    out = d.to_host().reshape(2048, 1100)
+    assert out.nbytes > 8 << 20  # (three rounds through two halves)
+    used, took = [], []
+    for _ in range(3):
+        r, t = resource.getrusage(resource.RUSAGE_SELF), time.perf_counter()
+        assert np.array_equal(model.forward_all(ids), out)
+        took.append(time.perf_counter() - t)
+        e = resource.getrusage(resource.RUSAGE_SELF)
+        used.append(e.ru_utime + e.ru_stime - r.ru_utime - r.ru_stime)
+    assert min(took) > 0.06, took  # (else the pass is too short to tell)
+    assert min(u / t for u, t in zip(used, took)) < 1.8, (used, took)
