@@ -617,6 +617,10 @@ int coeus_op_attention(const float *qkv_dev, uint64_t rows, uint64_t num_heads, 
     COEUS_GUARD_END
 }
 
+uint32_t coeus_plan_attention_f32(uint64_t batch, uint64_t rows, uint64_t cached, uint64_t num_heads, uint64_t head_dim) {
+    return attn_prefill_f32_queries(batch, rows, cached, num_heads, head_dim);
+}
+
 static int check_attention_decode_args(const float *qkv_dev, const void *k, const void *v, uint32_t kv_dtype,
                                        uint64_t batch, uint64_t heads, uint64_t hd, uint64_t max_ctx,
                                        uint64_t ctx, uint32_t *nsplit, uint32_t merge, const float *out_dev) {

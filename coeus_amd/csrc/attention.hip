@@ -819,6 +819,20 @@ bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype) {
     return n >= 16 && (hd == 64 || hd == 128) && kv_dtype != COEUS_KV_F32;
 }
 
+// Queries of a workgroup of f32 prompt attention: 32, with four key shares, while 128 queries give few workgroups.  us, 128 queries / 32:
+// heads of 64, up to 384 workgroups: 12 heads at 64 / 128 / 512 / 1024 rows 7.6 / 5.0, 13.0 / 6.1, 42 / 16, 81 / 49; 48 at 1024 1.28x as
+// fast; 192 at 80 and 256 rows 10.7 / 11.1 and 32.4 / 33.1.  Beyond neither is ahead throughout: 8 x 12 heads at 1024 (768 workgroups)
+// 216 / 266, at 1500 406 / 338, at 2048 822 / 793, at 3000 1327 / 1250, at 4096 3202 / 2582.
+// Heads of 128 hold 68 KB of shares a workgroup, which a short walk over the keys does not pay for once every CU has one: 128 workgroups, or
+// 256 from 768 rows on.  32 heads at 64 / 512 / 1024 rows 1.27, 1.67, 1.10x as fast, 128 at 128 28.4 / 26.1, 64 at 256 0.75 of the
+// time; but 64 at 512 82 / 92, 128 at 129 / 256 28.1 / 30.4 and 45.6 / 60.8, 256 at 33 / 128 13.7 / 17.4 and 28.4 / 42.7; 32 at 1500 225 / 293, 4 x 32
+// at 1024 355 / 591.  One tile of keys leaves three waves without work: 17 / 32 rows of 32 heads 8.0 / 8.8 and 8.2 / 9.5.
+uint32_t attn_prefill_f32_queries(uint64_t batch, uint64_t n, uint64_t pos0, uint64_t heads, uint64_t hd) {
+    if (n < 16 || (hd != 64 && hd != 128)) return 4;  // (attn_generic_kernel)
+    const uint64_t wgs = ceil_div(n, 128) * heads * batch;
+    return (hd == 64 ? wgs <= 384 : pos0 + n > 32 && wgs <= (n >= 768 ? 256 : 128)) ? 32 : 128;
+}
+
 uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t hd, uint32_t kv_dtype, uint64_t max_ctx) {
     // More than one split costs its records' two trips through memory, 1.5 - 2 us.  So one split where a head's keys fit
     // the requests of one workgroup: 64 KiB of them (512 keys of 64 in 16 bits), and 128 KiB with at least 64 workgroups
@@ -922,13 +936,9 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
         return COEUS_OK;
     }
     if (lp) return fail(COEUS_INVALID_INPUT, "16-bit attention output needs the matrix-core prefill kernel");
-    if (kv_dtype == COEUS_KV_F32 && n >= 16 && (hd == 64 || hd == 128) && !pos_dev && out && !out_xq) {
+    if (kv_dtype == COEUS_KV_F32 && attn_prefill_f32_queries(batch, n, pos0, heads, hd) > 4 && !pos_dev && out && !out_xq) {
         const dim3 pgrid((unsigned)ceil_div(n, 128), (unsigned)heads, (unsigned)batch);
-        // The kernel of 32 queries and four key shares as long as 128 queries give few workgroups (us, 128 queries / 32: 12 heads of 64
-        // at 64 / 128 / 512 / 1024 rows 7.6 / 5.0, 13.0 / 6.1, 42 / 16, 81 / 49; 32 heads of 128 at 128 / 512 / 1024 23 / 12, 79 / 43,
-        // 153 / 145); beyond, each tile of keys serves four times the queries (4 x 32 heads of 128 at 1024 355 / 591; 8 x 12
-        // of 64 at 1024 216 / 266).
-        if ((uint64_t)pgrid.x * heads * batch <= (hd == 64 ? 384 : 256)) {
+        if (attn_prefill_f32_queries(batch, n, pos0, heads, hd) == 32) {
             const dim3 fgrid((unsigned)ceil_div(n, 32), (unsigned)heads, (unsigned)batch);
             if (hd == 64)
                 hipLaunchKernelGGL(attn_prefill_f32_few_kernel<64>, fgrid, dim3(256), 0, st, qkv, (const float *)kc, (const float *)vc, (uint32_t)n,

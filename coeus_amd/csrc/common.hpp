@@ -331,6 +331,7 @@ int launch_kv_append(const float *qkv, void *kc, void *vc, uint32_t kv_dtype, ui
 uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t hd, uint32_t kv_dtype, uint64_t max_ctx);
 // True when n new rows per sequence take the matrix-core prefill kernel (which can write 16-bit
 // output rows) rather than the generic one.
+uint32_t attn_prefill_f32_queries(uint64_t batch, uint64_t n, uint64_t pos0, uint64_t heads, uint64_t hd);
 bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype);
 // Attention of n new rows per sequence (positions pos..pos+n-1) against the cache.
 // part_scratch: [batch*heads*nsplit*(head_dim+2)] f32 for the split decode kernel (nullable);
