@@ -57,6 +57,11 @@ class CLatentShape(C.Structure):
     _fields_ = [(f, C.c_uint64) for f in ("heads", "dim", "vdim", "q_rank", "kv_rank", "window")] + [("scale", C.c_float)]
 
 
+class CMatmulPlan(C.Structure):
+    _fields_ = [("kernel", C.c_char_p), ("tile_rows", C.c_uint32), ("tile_cols", C.c_uint32), ("waves", C.c_uint32), ("shares", C.c_uint32),
+                ("tail_shares", C.c_uint32)]
+
+
 class CHyperStep(C.Structure):
     _fields_ = ([("streams", C.c_uint64)] + [(f, C.c_void_p) for f in ("y_dev", "mix_dev", "out_dev", "in_dev", "norm_dev")] +
                 [("mult", C.c_float), ("eps", C.c_float)])
@@ -160,6 +165,7 @@ SIGNATURES = {
                                      _vp]),
     "coeus_op_gemm": (C.c_int, [_vp, _vp, _u64, _vp, _vp, _u32, _vp, _vp]),
     "coeus_op_matmul_limited": (C.c_int, [_vp, _vp, _u64, C.c_int, _u32, _f32, _vp, _vp]),
+    "coeus_plan_matmul": (C.c_int, [_u32, _u64, _u64, _u64, C.c_int, C.POINTER(CMatmulPlan)]),
     "coeus_op_gemm_timed": (C.c_int, [_vp, _vp, _u64, _u32, _vp, _u32, _vp, _vp]),
     "coeus_op_norm": (C.c_int, [_u32, _u32, _vp, _u64, _u64, _vp, _vp, _f32, _vp, _vp]),
     "coeus_op_embed": (C.c_int, [_vp, _vp, _vp, _u64, _u64, _u64, _vp, _vp]),

@@ -522,6 +522,17 @@ int coeus_op_matmul_limited(const coeus_weight *w, const float *x_dev, uint64_t 
     COEUS_GUARD_END
 }
 
+int coeus_plan_matmul(uint32_t dtype, uint64_t k_in, uint64_t n_out, uint64_t rows, int prompt, coeus_matmul_plan *out) {
+    COEUS_GUARD_BEGIN
+    if (!out) return fail(COEUS_INVALID_INPUT, "null pointer argument");
+    if (rows == 0 || (!prompt && rows > 16)) return fail(COEUS_INVALID_INPUT, "matmul of %llu rows", (unsigned long long)rows);
+    Weight w;
+    COEUS_TRY(weight_shape(w, dtype, k_in, n_out));
+    *out = prompt ? gemm_launch_plan(w, rows) : gemv_plan(w, rows);
+    return COEUS_OK;
+    COEUS_GUARD_END
+}
+
 int coeus_op_gemm_timed(const coeus_weight *w, const float *a_dev, uint64_t m, uint32_t epilogue,
                         float *c_dev, uint32_t reps, float *ms_out, void *stream) {
     COEUS_GUARD_BEGIN

@@ -96,6 +96,7 @@ struct Weight {
     // has 288 GB).  Saves re-expanding every weight on every prompt pass.
     mutable __half *expanded = nullptr;
 };
+int weight_shape(Weight &w, uint32_t dtype, uint64_t k, uint64_t n);  // sizes alone, no memory
 int weight_alloc(Weight &w, uint32_t dtype, uint64_t k, uint64_t n);
 void weight_free(Weight &w);
 
@@ -265,8 +266,13 @@ struct GemmScratch {
 // Bytes of GemmScratch::partials that launch_gemm would use for this weight on m rows (0: it would
 // not split).
 uint64_t gemm_split_scratch_bytes(const Weight &w, uint64_t m);
+// The launch that plain rows get, as the launchers decide it (coeus_plan_matmul): the decode matmul, and the prompt matmul with room for
+// its partial products.
+coeus_matmul_plan gemv_plan(const Weight &w, uint64_t batch);
+coeus_matmul_plan gemm_launch_plan(const Weight &w, uint64_t m);
 // Short prompts on quantised weights: the matmul that streams the quantised blocks (gemv.hip).
 struct EpiArgs;
+uint32_t qskinny_splits(const Weight &w);
 bool gemm_uses_qskinny(const Weight &w, uint64_t m);
 uint64_t gemm_qskinny_scratch_bytes(const Weight &w, uint64_t m);
 int launch_gemm_qskinny(const Weight &w, const uint16_t *a, uint64_t lda, uint64_t m, const EpiArgs &e,

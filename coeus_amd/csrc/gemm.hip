@@ -1778,6 +1778,21 @@ uint64_t gemm_split_scratch_bytes(const Weight &w, uint64_t m) {
     return 0;
 }
 
+coeus_matmul_plan gemm_launch_plan(const Weight &w, uint64_t m) {
+    if (w.dtype == COEUS_W_F32) {
+        if (gemv_takes_f32_rows(w, m)) return gemv_plan(w, m);
+        if (gemm_f32_is_small(w, m)) return {"gemm_f32_small_kernel", SM, SN, 4, gemm_f32_splits_wanted(w, m), 1};
+        return {"gemm_f32_kernel", BM, BN, 4, 1, 1};
+    }
+    if (gemm_uses_qskinny(w, m)) return {"gemm_qskinny_kernel", 64, 0, 4, qskinny_splits(w), 1};
+    if (!gemm_uses_h256(w, m)) return {"gemm_h_kernel", HM, HN, 4, 1, 1};
+    const GemmPlan plan = gemm_plan(w, m, true);
+    if (plan.rows) return {"gemm_narrow_kernel", plan.rows, plan.cols, 8, plan.splits, 1};
+    uint32_t full = 0;
+    const uint32_t tail = plan.splits == 1 ? gemm_tail_splits_wanted(w, m, &full) : 1;
+    return {w.k % UK == 0 ? "gemm_h256k64_kernel" : "gemm_h256_kernel", TM, TN, w.k % UK == 0 ? 4u : 8u, plan.splits, tail};
+}
+
 bool gemm_appends_kv(const Weight &w, uint64_t m, uint64_t inner, uint64_t hd) {
     // (f32: element by element, or by the kernel that sums a split launch's planes, four columns at a time)
     if (w.dtype == COEUS_W_F32) return m < (1ull << 32) && w.n == 3 * inner && (inner & 3) == 0 && (hd & 3) == 0;

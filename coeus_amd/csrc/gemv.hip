@@ -801,10 +801,19 @@ static int launch_gemv_quad(const Weight &w, const __half *xq, uint64_t batch, c
 // waves as many as share the reduction in few trips.  Measured for 8 and 16 rows over 35 matrices of 768 - 5120 wide models
 // with 1 - 6 tiles and 2 - 16 waves; the choice is within 4 % of the best of them (4096 x 22016, 16 rows, Q4_0: six tiles 15.9,
 // three 17, two 17.4 us; 1536 x 8192: two 6.9, one 7.3; 768 x 50257: two tiles of three waves 12.2, one of six 17.2).
+// Few chunks (k <= 512) are few waves, and the outputs of several tiles are more than these finish at once: one tile, a wave per chunk, as long
+// as the activations are next to nothing, else two; six tiles only from nine chunks on.  Q4_0, 16 rows, us with as many tiles as above / so: 64 x
+// 16400 12.9 / 6.3, x 100000 10.5 / 9.9, 256 x 16400 10.2 / 6.3, x 33000 9.6 / 8.1, 512 x 16400 8.8 / 6.8, x 50257 10.9 / 10.2, 768 x 16400
+// 9.3 / 8.0.  400 sizes with 1 - 6 tiles and 1 - 16 waves: 1.3 % above the best of them on average.
 static void gemv_rows_shape(bool q4, uint32_t ngroups, uint32_t tiles, uint32_t &tpw, uint32_t &waves) {
+    if (ngroups <= 4 && tiles > 256) {
+        tpw = ngroups == 1 || tiles <= (ngroups == 2 ? 2048 : 1536) ? 1 : 2;
+        waves = ngroups;
+        return;
+    }
     tpw = 0;
     for (uint32_t t : {1u, 2u, 3u, 4u, 6u})
-        if (!tpw && (t < 6 || q4) && ceil_div(tiles, t) <= 256) tpw = t;
+        if (!tpw && (t < 6 || (q4 && ngroups > 8)) && ceil_div(tiles, t) <= 256) tpw = t;
     for (uint32_t t : {2u, 3u, 4u})
         if (!tpw && ceil_div(tiles, t) <= 512) tpw = t;
     const bool many = !tpw;
@@ -2059,6 +2068,22 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
     return COEUS_OK;
 }
 
+// f32: a wave per row is ahead on short or few rows (768 x 768 2.8 / 3.1, x 3072 4.2 / 4.3, 3072 x 768 5.6 / 5.9, 520 x 3001 3.8 / 3.9; but
+// 1536 x 4000 7.3 / 6.7, 2048 x 2048 6.1 / 5.3, 1024 x 8192 8.6 / 8.3).  Two steps in flight are all of up to 1024 elements.
+static bool gemv_takes_many(const Weight &w, uint64_t batch) {
+    return batch == 1 && w.dtype <= COEUS_W_BF16 && w.k % 8 == 0 && w.k < (1ull << 31) && w.n < (1ull << 31) - 8 &&
+           (w.dtype == COEUS_W_BF16 || (w.n >= 2048 && (w.k >= 1536 || w.n >= 8192)));
+}
+
+// Plain rows on the matrix cores: waves of a workgroup, LDS, and whether they go there.
+struct MfmaPlain { bool runs; uint32_t waves; size_t lds; };
+template <bool BF16>
+static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
+    const uint32_t waves = gemv_mfma_waves(std::min<uint64_t>(w.k / MfmaType<BF16>::KU, 1u << 20)), xbp = std::max(pad_batch(batch), 4u);
+    const size_t lds = (size_t)waves * 16 * mfma_wave_lds<BF16>((xbp + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS);
+    return {gemv_uses_mfma(w, batch, waves, false) && lds <= 160 * 1024, waves, lds};
+}
+
 template <bool BF16>
 static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, const EpiArgs &e,
                              hipStream_t st, const NormFuse *nf) {
@@ -2095,10 +2120,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         COEUS_HIP(hipGetLastError());
         return COEUS_OK;
     }
-    // f32: a wave per row is ahead on short or few rows (768 x 768 2.8 / 3.1, x 3072 4.2 / 4.3, 3072 x 768 5.6 / 5.9, 520 x 3001 3.8 / 3.9; but
-    // 1536 x 4000 7.3 / 6.7, 2048 x 2048 6.1 / 5.3, 1024 x 8192 8.6 / 8.3).  Two steps in flight are all of up to 1024 elements.
-    if (norm == 0 && b == 1 && aligned && w.k % 8 == 0 && w.k < (1ull << 31) && w.n < (1ull << 31) - 8 &&
-        (BF16 || (w.n >= 2048 && (w.k >= 1536 || w.n >= 8192)))) {
+    if (norm == 0 && aligned && gemv_takes_many(w, batch)) {
         const dim3 mgrid((unsigned)ceil_div(w.n, 8));
         if (w.k <= 1024) hipLaunchKernelGGL((gemv_many_kernel<BF16, 2>), mgrid, dim3(256), 0, st, w.data, xin, (uint32_t)w.k, e);
         else hipLaunchKernelGGL((gemv_many_kernel<BF16, 4>), mgrid, dim3(256), 0, st, w.data, xin, (uint32_t)w.k, e);
@@ -2108,11 +2130,11 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     {
         // plain: workgroups enough to fill the compute units' 16 waves;
         // a folded norm: one workgroup of 16 waves per compute unit, which stages the rows once
-        const uint32_t pairs = (uint32_t)std::min<uint64_t>(w.k / MfmaType<BF16>::KU, 1u << 20), mw = nf ? 16u : gemv_mfma_waves(pairs);
-        const uint32_t xbp = std::max(bp, 4u), xq = nf ? 0 : (xbp + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
-        const size_t corners = (size_t)mw * 16 * mfma_wave_lds<BF16>(xq),
-                     mlds = nf ? gemv_mfma_norm_lds(w, bp, lds) : corners;
-        if (aligned && gemv_uses_mfma(w, batch, nf ? 16 : mw, nf) && mlds <= 160 * 1024) {
+        const uint32_t pairs = (uint32_t)std::min<uint64_t>(w.k / MfmaType<BF16>::KU, 1u << 20);
+        const MfmaPlain plain = gemv_mfma_plain<BF16>(w, batch);
+        const uint32_t mw = nf ? 16u : plain.waves;
+        const size_t mlds = nf ? gemv_mfma_norm_lds(w, bp, lds) : plain.lds;
+        if (aligned && (nf ? gemv_uses_mfma(w, batch, 16, true) && mlds <= 160 * 1024 : plain.runs)) {
             const uint32_t tiles = (uint32_t)ceil_div(w.n, 16), np = (pairs + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
 #define COEUS_MFMA4(BPV, NV, PV, KV)                                                                                          \
@@ -2168,6 +2190,20 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
 #undef COEUS_GEMVD2
     COEUS_HIP(hipGetLastError());
     return COEUS_OK;
+}
+
+coeus_matmul_plan gemv_plan(const Weight &w, uint64_t batch) {
+    const uint32_t bp = pad_batch(batch);
+    if (w.dtype >= COEUS_W_Q8_0) {
+        if (bp <= 4) return {"gemv_quad_kernel", bp, 16, 0, 1, 1};
+        uint32_t tpw, waves;
+        gemv_rows_shape(w.dtype == COEUS_W_Q4_0, (uint32_t)(w.k_pad / 128), (uint32_t)(w.n_pad / 16), tpw, waves);
+        return {"gemv_rows_kernel", bp, 16 * tpw, waves, 1, 1};
+    }
+    if (gemv_takes_many(w, batch)) return {"gemv_many_kernel", 1, 8, 4, 1, 1};
+    const MfmaPlain mp = w.dtype == COEUS_W_BF16 ? gemv_mfma_plain<true>(w, batch) : gemv_mfma_plain<false>(w, batch);
+    if (mp.runs) return {"gemv_mfma_kernel", bp, 16, mp.waves, 1, 1};
+    return {"gemv_dense_kernel", bp, 4, 4, 1, 1};
 }
 
 int launch_gemv(const Weight &w, const void *x, uint64_t batch, const Epilogue &ep, hipStream_t st,
@@ -2337,7 +2373,7 @@ static uint32_t qskinny_gpw(const Weight &w) {
     const uint32_t wgs = (tiles + 7) / 8;
     return wgs * ((ngroups + 3) / 4) >= 512 ? 4 : 2;
 }
-static uint32_t qskinny_splits(const Weight &w) {
+uint32_t qskinny_splits(const Weight &w) {
     const uint32_t ngroups = (uint32_t)(w.k_pad / 128), gpw = qskinny_gpw(w);
     return (ngroups + gpw - 1) / gpw;
 }

@@ -306,7 +306,7 @@ int launch_f32_to_16(const float *src, void *dst, uint64_t rows, uint64_t k, uin
 }
 
 // ---------------------------------------------------------------- host side
-int weight_alloc(Weight &w, uint32_t dtype, uint64_t k, uint64_t n) {
+int weight_shape(Weight &w, uint32_t dtype, uint64_t k, uint64_t n) {
     if (dtype > COEUS_W_Q4_0) return fail(COEUS_INVALID_INPUT, "unknown weight dtype %u", dtype);
     if (k == 0 || n == 0) return fail(COEUS_INVALID_INPUT, "empty weight %llu x %llu",
                                       (unsigned long long)k, (unsigned long long)n);
@@ -314,19 +314,23 @@ int weight_alloc(Weight &w, uint32_t dtype, uint64_t k, uint64_t n) {
     w.dtype = dtype;
     w.k = k;
     w.n = n;
+    const bool quant = dtype != COEUS_W_F32 && dtype != COEUS_W_BF16;
+    if (quant && k % 32 != 0)
+        return fail(COEUS_INVALID_INPUT,
+                    "quantised weights need an input dimension divisible by 32, got %llu",
+                    (unsigned long long)k);
+    w.k_pad = quant ? round_up(k, 128) : k;
+    w.n_pad = quant ? round_up(n, 16) : n;
+    return COEUS_OK;
+}
+
+int weight_alloc(Weight &w, uint32_t dtype, uint64_t k, uint64_t n) {
+    COEUS_TRY(weight_shape(w, dtype, k, n));
     if (dtype == COEUS_W_F32 || dtype == COEUS_W_BF16) {
-        w.k_pad = k;
-        w.n_pad = n;
         w.bytes = k * n * (dtype == COEUS_W_F32 ? 4 : 2);
         COEUS_HIP(hipMalloc(&w.data, w.bytes));
         return COEUS_OK;
     }
-    if (k % 32 != 0)
-        return fail(COEUS_INVALID_INPUT,
-                    "quantised weights need an input dimension divisible by 32, got %llu",
-                    (unsigned long long)k);
-    w.k_pad = round_up(k, 128);
-    w.n_pad = round_up(n, 16);
     const uint64_t elems = w.k_pad * w.n_pad;
     const uint64_t qbytes = dtype == COEUS_W_Q4_0 ? elems / 2 : elems;
     const uint64_t sbytes = elems / 32 * 2;

@@ -344,6 +344,14 @@ int coeus_op_gemm(const coeus_weight *w, const float *a_dev, uint64_t m, const f
  * and bf16 weights.  prompt 0: the decode matmul (rows <= 16), else the prefill matmul. */
 int coeus_op_matmul_limited(const coeus_weight *w, const float *x_dev, uint64_t rows, int prompt, uint32_t epilogue,
                             float limit, float *y_dev, void *stream);
+/* The launch that a matmul of plain rows gets (no counterpart in the reference; for profiles and tests, no device is touched): `rows` of
+ * the decode matmul (prompt 0), or of the prompt matmul with room for its partial products.  tile_rows x tile_cols outputs a
+ * workgroup, waves of a workgroup, shares of k (tail_shares: of the tiles of a launch's last round). */
+typedef struct coeus_matmul_plan {
+    const char *kernel;
+    uint32_t tile_rows, tile_cols, waves, shares, tail_shares;
+} coeus_matmul_plan;
+int coeus_plan_matmul(uint32_t dtype, uint64_t k_in, uint64_t n_out, uint64_t rows, int prompt, coeus_matmul_plan *out);
 /* Measurement variant of coeus_op_gemm (no reference counterpart; used by the benchmark's
  * matrix-core roofline): runs the staging conversions and one untimed matmul, then launches the
  * matmul kernel `reps` times between two events on `stream` and returns the elapsed

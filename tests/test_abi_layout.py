@@ -197,7 +197,8 @@ def test_rust_extern_declarations_match_the_header():
 def test_layered_structs_match_the_header(tmp_path):
     pairs = [(_lib.CLoadOptions, "coeus_load_options"), (_lib.CDeltaShape, "coeus_delta_shape"), (_lib.CDeltaWeights, "coeus_delta_weights"),
              (_lib.CLatentShape, "coeus_latent_shape"), (_lib.CHyperStep, "coeus_hyper_step"), (_lib.CMemoryShape, "coeus_memory_shape"),
-             (_lib.CMemoryWeights, "coeus_memory_weights"), (_lib.CSharedKvShape, "coeus_shared_kv_shape")]
+             (_lib.CMemoryWeights, "coeus_memory_weights"), (_lib.CSharedKvShape, "coeus_shared_kv_shape"),
+             (_lib.CMatmulPlan, "coeus_matmul_plan")]
     lines = ['#include <stddef.h>', '#include <stdio.h>', '#include "coeus.h"', 'int main(void) {']
     for cls, name in pairs:
         lines.append(f'  printf("{name} %zu\\n", sizeof({name}));')

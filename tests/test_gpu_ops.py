@@ -486,7 +486,9 @@ def test_gemv_benchmark_shapes(orc, dtype, k, n, gated):
 @pytest.mark.parametrize("dtype", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("k,n", [(96, 256 * 16), (96, 256 * 16 + 2), (160, 512 * 16 - 14), (160, 513 * 16), (1184, 768 * 16),
                                  (160, 769 * 16 - 2), (160, 1024 * 16 + 2), (160, 1536 * 16), (160, 1537 * 16), (160, 2049 * 16),
-                                 (1184, 2049 * 16 - 6)])
+                                 (1184, 2049 * 16 - 6),
+                                 # (two to four chunks: a tile up to 2048 and 1536 of them, then two; from nine chunks on up to six)
+                                 (256, 2048 * 16), (256, 2049 * 16 - 2), (512, 1536 * 16), (352, 1537 * 16 - 14), (1024, 1025 * 16), (1056, 1025 * 16 - 2)])
 def test_gemv_rows_shapes(orc, dtype, k, n):
     wt, wdq = _seeded(dtype, k, n, k + n)
     rng = np.random.default_rng(k + n)

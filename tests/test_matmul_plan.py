@@ -1,0 +1,35 @@
+"""Which kernel, tiles and shares a matmul gets at both sides of the lines of its rules (no device is touched)."""
+import ctypes as C
+
+import pytest
+
+from coeus_amd import _lib
+
+
+def plan(dtype, k, n, rows, prompt=0):
+    p = _lib.CMatmulPlan()
+    assert _lib.load().coeus_plan_matmul(dtype, k, n, rows, prompt, C.byref(p)) == 0
+    return p
+
+
+def test_what_no_weight_can_be_is_refused():
+    p, call = _lib.CMatmulPlan(), _lib.load().coeus_plan_matmul
+    for dtype, k, n, rows, prompt in [(9, 64, 64, 1, 0), (0, 0, 64, 1, 0), (0, 64, 0, 1, 0), (3, 48, 64, 1, 0), (0, 64, 64, 0, 0), (0, 64, 64, 17, 0), (0, 64, 64, 0, 1)]:
+        assert call(dtype, k, n, rows, prompt, C.byref(p)) != 0
+    assert call(0, 64, 64, 1, 0, None) != 0
+
+
+# Few chunks of 128: a tile of 16 outputs or two a workgroup, a wave per chunk (six tiles of one wave were 12.9 us at 64 x 16400 and 16 rows, one is 6.3)
+@pytest.mark.parametrize("dtype,k,n,outputs,waves", [
+    (_lib.W_Q4_0, 64, 4096, 16, 1), (_lib.W_Q4_0, 64, 16400, 16, 1), (_lib.W_Q8_0, 128, 100000, 16, 1), (_lib.W_Q4_0, 256, 16400, 16, 2), (_lib.W_Q4_0, 256, 32768, 16, 2),
+    (_lib.W_Q4_0, 256, 32784, 32, 2), (_lib.W_Q8_0, 384, 24576, 16, 3), (_lib.W_Q8_0, 512, 24592, 32, 4), (_lib.W_Q4_0, 512, 8192, 16, 4), (_lib.W_Q4_0, 768, 16400, 48, 6),
+    (_lib.W_Q4_0, 1024, 16400, 48, 8), (_lib.W_Q4_0, 1152, 16400, 96, 9), (_lib.W_Q4_0, 4096, 22016, 96, 12), (_lib.W_Q8_0, 4096, 22016, 48, 8), (_lib.W_Q8_0, 768, 50257, 32, 3),
+    (_lib.W_Q8_0, 768, 768, 16, 6), (_lib.W_Q4_0, 11008, 4096, 16, 12)])
+@pytest.mark.parametrize("rows", [5, 16])
+def test_decode_rows_on_quantised_weights(dtype, k, n, outputs, waves, rows):
+    p = plan(dtype, k, n, rows)
+    assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_rows_kernel", outputs, waves)
+
+
+def test_decode_batches_of_up_to_four_on_quantised_weights():
+    assert all(plan(d, 768, 2304, b).kernel == b"gemv_quad_kernel" for d in (_lib.W_Q8_0, _lib.W_Q4_0) for b in (1, 2, 3, 4))
