@@ -1307,7 +1307,7 @@ __global__ __launch_bounds__(256) void gemv_many_kernel(const void *__restrict__
 //   4096 x 22016   47 / 34     73 / 36      118 / 40      215 / 55
 //   768 x 50257    28 / 14     41 / 14       68 / 16      127 / 18
 // f32: 768 x 3072 9.0 / 4.4 at batch 8, 768 x 50257 79 / 30, 4096 x 4096 31 / 15.
-// (One row: gemv_many_kernel.)  The large ones are
+// (One row: 4.2, 8.7, 33, 18.5 there; where it comes here gemv_uses_mfma says.)  The large ones are
 // at 5 TB/s of weights.  A matrix with an infinite value stays there (times a piece that is zero it would be a NaN).
 //
 // The workgroup's waves take a share of k each, in pairs of 32-wide chunks: a wave request is 8 rows x 128 bytes, as
@@ -1730,8 +1730,12 @@ static bool gemv_mfma_shape(const Weight &w, uint32_t waves) {
 }
 // Where the matrix cores are the faster of the two (us with weights from memory: a wave per row / here).
 static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves, bool folded) {
-    if (!gemv_mfma_shape(w, waves) || batch < 2) return false;
+    if (!gemv_mfma_shape(w, waves) || batch < 1) return false;
     const bool bf = w.dtype == COEUS_W_BF16;
+    // One row (two weight rows a wave / here): short rows of which there are many (256 x 16384 5.0 / 4.4, x 100000 18.3 / 11.1, 512 x 50257 12.6 / 10.8;
+    // but 512 x 12000 0.89 of the time, 576 x 50257 0.89), and long ones a little beyond the 2048 that give every compute unit one
+    // workgroup (11008 x 3072 17.7 / 16.8, 14336 x 3072 20.6 / 19.0; x 2048 0.74 of the time, x 3584 the same, 8192 x 3072 the same).
+    if (batch == 1) return bf && !folded && (w.k <= 512 ? w.n >= 16384 : w.k >= 10240 && w.n > 2048 && w.n <= 3328);
     // (A norm in front costs a wave per row more: f32, 2 rows of 768 x 768 7.4 / 5.8.  Two rows of bf16 are the exception where they
     // are long and few: 2560 x 4096 11.0 / 11.6, x 12288 22.7 / 19.1.)
     if (folded) return !(bf && batch == 2 && w.k > 2048 && w.n <= 4096);
@@ -2068,11 +2072,18 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
     return COEUS_OK;
 }
 
-// f32: a wave per row is ahead on short or few rows (768 x 768 2.8 / 3.1, x 3072 4.2 / 4.3, 3072 x 768 5.6 / 5.9, 520 x 3001 3.8 / 3.9; but
-// 1536 x 4000 7.3 / 6.7, 2048 x 2048 6.1 / 5.3, 1024 x 8192 8.6 / 8.3).  Two steps in flight are all of up to 1024 elements.
+// One plain row: two weight rows a wave where that is the faster form (us, the other one / here).
+// f32, against a wave per row: ahead from 1536 of k and 2048 rows on, and from 1032 and 8192, but not a little beyond the 2048 rows that give
+// every compute unit one workgroup (2048 x 2048 6.1 / 5.3, 4096 x 3328 0.93 of the time, 1088 x 8192 0.93; 2304 rows of 1536 - 8192 1.04 - 1.11,
+// 3072 1.03 - 1.09); short rows only where there are very many (768 x 50257 0.97, x 32000 0.98; 640 x 11008 1.05, 512 x 16384 1.05, 1024 x
+// 11008 1.06).  bf16: all that the matrix cores do not take (gemv_uses_mfma), but rows 32 KiB apart, which share their memory channels,
+// are a wave's each between 4096 and 6144 of them (16384 x 4608 1.07, 32768 x 4608 1.14; x 6144 1.00, x 8192 0.86).
 static bool gemv_takes_many(const Weight &w, uint64_t batch) {
-    return batch == 1 && w.dtype <= COEUS_W_BF16 && w.k % 8 == 0 && w.k < (1ull << 31) && w.n < (1ull << 31) - 8 &&
-           (w.dtype == COEUS_W_BF16 || (w.n >= 2048 && (w.k >= 1536 || w.n >= 8192)));
+    if (batch != 1 || w.dtype > COEUS_W_BF16 || w.k % 8 || w.k >= (1ull << 31) || w.n >= (1ull << 31) - 8) return false;
+    if (w.dtype == COEUS_W_BF16)
+        return !gemv_uses_mfma(w, 1, gemv_mfma_waves(w.k / MfmaType<true>::KU), false) && !(w.k % 16384 == 0 && w.n > 4096 && w.n < 6144);
+    if (w.k >= 1536) return w.n == 2048 || w.n > 3200;
+    return w.k > 1024 ? w.n >= 8192 : w.k > 512 && w.k < 1024 && w.n >= 20000;
 }
 
 // Plain rows on the matrix cores: waves of a workgroup, LDS, and whether they go there.
@@ -2145,12 +2156,12 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     } while (0)
             // Pairs in flight: two or three, whichever asks for fewer in vain at the end of a wave's share.  Where that is the
             // same, three for 2 - 4 rows (us for two / three: 4 rows of bf16 5120 x 32000 67.0 / 65.5, 2 of 12288 x 8192 36.5 / 35.0), two
-            // for 8 (6144 x 4096 13.0 / 13.5).  A norm in front fills the first trip, and
+            // for one row (6144 x 512 7.2 / 7.4) and for 8 (6144 x 4096 13.0 / 13.5).  A norm in front fills the first trip, and
             // three pay from the second tile on (2 rows of bf16 3072 x 4096 12.7 / 13.3, x 12288 22.4 / 20.8).  Four in flight are
             // never faster (4 rows, us for 2 / 3 / 4: 3072 x 4096 7.1 / 6.4 / 7.1, 4096 x 4096 7.7 / 9.2 / 7.8, 10240 x 512 12.1 / 13.7 /
             // 14.0).
             const uint32_t by2 = (np + 1) / 2 * 2, by3 = (np + 2) / 3 * 3;
-            const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && bp <= 4);
+            const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && batch > 1 && bp <= 4);
 #define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (BPV < 16 && three) COEUS_MFMA4(BPV < 16 ? BPV : 8, NV, 3, false); else COEUS_MFMA4(BPV, NV, 2, false); } while (0)
 #define COEUS_MFMAN(BPV, NV)                                                                               \
     do {                                                                                                   \

@@ -33,3 +33,18 @@ def test_decode_rows_on_quantised_weights(dtype, k, n, outputs, waves, rows):
 
 def test_decode_batches_of_up_to_four_on_quantised_weights():
     assert all(plan(d, 768, 2304, b).kernel == b"gemv_quad_kernel" for d in (_lib.W_Q8_0, _lib.W_Q4_0) for b in (1, 2, 3, 4))
+
+
+# One row: where two weight rows a wave were slower than what there was before (bf16 64 x 128000 2.98 times, 512 x 50257 1.16; f32 3072 x 2304 1.10)
+@pytest.mark.parametrize("dtype,k,n,kernel", [
+    (_lib.W_BF16, 64, 16384, b"gemv_mfma_kernel"), (_lib.W_BF16, 512, 50257, b"gemv_mfma_kernel"), (_lib.W_BF16, 512, 16383, b"gemv_many_kernel"),
+    (_lib.W_BF16, 576, 50257, b"gemv_many_kernel"), (_lib.W_BF16, 520, 50257, b"gemv_many_kernel"), (_lib.W_BF16, 200, 50257, b"gemv_many_kernel"),
+    (_lib.W_BF16, 11008, 3072, b"gemv_mfma_kernel"), (_lib.W_BF16, 11008, 2048, b"gemv_many_kernel"), (_lib.W_BF16, 11008, 4096, b"gemv_many_kernel"),
+    (_lib.W_BF16, 8192, 3072, b"gemv_many_kernel"), (_lib.W_BF16, 16384, 4608, b"gemv_dense_kernel"), (_lib.W_BF16, 16384, 6144, b"gemv_many_kernel"),
+    (_lib.W_BF16, 16384, 4096, b"gemv_many_kernel"), (_lib.W_BF16, 770, 770, b"gemv_dense_kernel"), (_lib.W_BF16, 768, 50257, b"gemv_many_kernel"),
+    (_lib.W_F32, 3072, 2304, b"gemv_dense_kernel"), (_lib.W_F32, 3072, 2048, b"gemv_many_kernel"), (_lib.W_F32, 1536, 3201, b"gemv_many_kernel"),
+    (_lib.W_F32, 1536, 3200, b"gemv_dense_kernel"), (_lib.W_F32, 1032, 8192, b"gemv_many_kernel"), (_lib.W_F32, 1024, 50257, b"gemv_dense_kernel"),
+    (_lib.W_F32, 768, 50257, b"gemv_many_kernel"), (_lib.W_F32, 768, 11008, b"gemv_dense_kernel"), (_lib.W_F32, 512, 50257, b"gemv_dense_kernel"),
+    (_lib.W_F32, 768, 3072, b"gemv_dense_kernel"), (_lib.W_F32, 3072, 768, b"gemv_dense_kernel")])
+def test_decode_of_one_row(dtype, k, n, kernel):
+    assert plan(dtype, k, n, 1).kernel == kernel
