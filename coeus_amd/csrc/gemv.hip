@@ -2077,11 +2077,13 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
 // every compute unit one workgroup (2048 x 2048 6.1 / 5.3, 4096 x 3328 0.93 of the time, 1088 x 8192 0.93; 2304 rows of 1536 - 8192 1.04 - 1.11,
 // 3072 1.03 - 1.09); short rows only where there are very many (768 x 50257 0.97, x 32000 0.98; 640 x 11008 1.05, 512 x 16384 1.05, 1024 x
 // 11008 1.06).  bf16: all that the matrix cores do not take (gemv_uses_mfma), but rows 32 KiB apart, which share their memory channels,
-// are a wave's each between 4096 and 6144 of them (16384 x 4608 1.07, 32768 x 4608 1.14; x 6144 1.00, x 8192 0.86).
+// are a wave's each between 4096 and 6144 of them (16384 x 4608 1.07, 32768 x 4608 1.14; x 6144 1.00, x 8192 0.86), and so are few
+// rows of exactly one step of 512 (x 300 1.10, x 768 1.11, x 1024 1.06, x 3000 0.97; 448 x 768 0.96).
 static bool gemv_takes_many(const Weight &w, uint64_t batch) {
     if (batch != 1 || w.dtype > COEUS_W_BF16 || w.k % 8 || w.k >= (1ull << 31) || w.n >= (1ull << 31) - 8) return false;
     if (w.dtype == COEUS_W_BF16)
-        return !gemv_uses_mfma(w, 1, gemv_mfma_waves(w.k / MfmaType<true>::KU), false) && !(w.k % 16384 == 0 && w.n > 4096 && w.n < 6144);
+        return !gemv_uses_mfma(w, 1, gemv_mfma_waves(w.k / MfmaType<true>::KU), false) && !(w.k % 16384 == 0 && w.n > 4096 && w.n < 6144) &&
+               !(w.k == 512 && w.n < 2048);
     if (w.k >= 1536) return w.n == 2048 || w.n > 3200;
     return w.k > 1024 ? w.n >= 8192 : w.k > 512 && w.k < 1024 && w.n >= 20000;
 }

@@ -42,6 +42,7 @@ def test_decode_batches_of_up_to_four_on_quantised_weights():
     (_lib.W_BF16, 11008, 3072, b"gemv_mfma_kernel"), (_lib.W_BF16, 11008, 2048, b"gemv_many_kernel"), (_lib.W_BF16, 11008, 4096, b"gemv_many_kernel"),
     (_lib.W_BF16, 8192, 3072, b"gemv_many_kernel"), (_lib.W_BF16, 16384, 4608, b"gemv_dense_kernel"), (_lib.W_BF16, 16384, 6144, b"gemv_many_kernel"),
     (_lib.W_BF16, 16384, 4096, b"gemv_many_kernel"), (_lib.W_BF16, 770, 770, b"gemv_dense_kernel"), (_lib.W_BF16, 768, 50257, b"gemv_many_kernel"),
+    (_lib.W_BF16, 512, 768, b"gemv_dense_kernel"), (_lib.W_BF16, 512, 2048, b"gemv_many_kernel"), (_lib.W_BF16, 448, 768, b"gemv_many_kernel"),
     (_lib.W_F32, 3072, 2304, b"gemv_dense_kernel"), (_lib.W_F32, 3072, 2048, b"gemv_many_kernel"), (_lib.W_F32, 1536, 3201, b"gemv_many_kernel"),
     (_lib.W_F32, 1536, 3200, b"gemv_dense_kernel"), (_lib.W_F32, 1032, 8192, b"gemv_many_kernel"), (_lib.W_F32, 1024, 50257, b"gemv_dense_kernel"),
     (_lib.W_F32, 768, 50257, b"gemv_many_kernel"), (_lib.W_F32, 768, 11008, b"gemv_dense_kernel"), (_lib.W_F32, 512, 50257, b"gemv_dense_kernel"),
