@@ -43,7 +43,7 @@ __device__ __forceinline__ float4 f32_piece(const float *__restrict__ base, uint
     return v;
 }
 
-template <bool VEC>
+template <bool VEC, bool KV>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__ a,
                                                        const float *__restrict__ w, uint64_t m,
                                                        uint64_t n, uint64_t k, EpiArgs e) {
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__
         // gated: columns (2c, 2c+1) hold (gate_c, up_c) and sit in neighbouring lanes
         const float other = lane_xor1(acc[i]);
         if (row >= m || col >= n) continue;
-        if (!gated) epi_store<true>(e, row, col, acc[i]);
+        if (!gated) epi_store<KV>(e, row, col, acc[i]);
         else if ((lane & 1) == 0) epi_store_gated(e, row, col >> 1, acc[i], other);
     }
 }
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__
 constexpr int SM = 32, SN = 32, F32S_AHEAD = 6;
 struct F32SliceS { float4 a, w; };
 
-template <bool VEC>
+template <bool VEC, bool KV>
 __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float *__restrict__ a,
                                                              const float *__restrict__ w, uint64_t m,
                                                              uint64_t n, uint64_t k, uint32_t splits, EpiArgs e) {
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float *__rest
         const uint64_t row = m0 + 8 * wave + 4 * (lane >> 5) + q;
         const float other = lane_xor1(v);
         if (row >= m || col >= n) continue;
-        if (!gated) epi_store<true>(e, row, col, v);
+        if (!gated) epi_store<KV>(e, row, col, v);
         else if ((lane & 1) == 0) epi_store_gated(e, row, col >> 1, v, other);
     }
 }
@@ -254,14 +254,16 @@ static int launch_gemm_f32(const Weight &w, const float *a, uint64_t m, const Ep
     const uint64_t groups = ceil_div(w.n, epi_gated(e.act) ? 8 : 4);
     if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
     for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) {
-        if (small && (w.k & 3) == 0)
-            hipLaunchKernelGGL(gemm_f32_small_kernel<true>, sgrid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, splits, ke);
-        else if (small)
-            hipLaunchKernelGGL(gemm_f32_small_kernel<false>, sgrid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, splits, ke);
-        else if ((w.k & 3) == 0)
-            hipLaunchKernelGGL(gemm_f32_kernel<true>, grid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, e);
-        else
-            hipLaunchKernelGGL(gemm_f32_kernel<false>, grid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, e);
+        // (KV: cache rows; their code in every epilogue costs launches of 128 rows 2 - 3 %, 768 x 768 9.4 -> 9.6 us)
+#define COEUS_F32(VECV, KVV)                                                                                                                        \
+    do {                                                                                                                                            \
+        if (small) hipLaunchKernelGGL((gemm_f32_small_kernel<VECV, KVV>), sgrid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, splits, ke); \
+        else hipLaunchKernelGGL((gemm_f32_kernel<VECV, KVV>), grid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, e);                      \
+    } while (0)
+        if ((w.k & 3) == 0) { if (ke.kv_k) COEUS_F32(true, true); else COEUS_F32(true, false); }
+        else if (ke.kv_k) COEUS_F32(false, true);
+        else COEUS_F32(false, false);
+#undef COEUS_F32
         if (splits > 1)
             hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)ceil_div(m * groups, 256)), dim3(256), 0, st,
                                (const float *)scr.partials, splits, m, w.n, e);
