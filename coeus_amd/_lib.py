@@ -165,6 +165,7 @@ SIGNATURES = {
                                      _vp]),
     "coeus_op_gemm": (C.c_int, [_vp, _vp, _u64, _vp, _vp, _u32, _vp, _vp]),
     "coeus_op_matmul_limited": (C.c_int, [_vp, _vp, _u64, C.c_int, _u32, _f32, _vp, _vp]),
+    "coeus_op_gemm16": (C.c_int, [_vp, _vp, _u64, _u32, _f32, C.c_int, _u64, _vp, _vp]),
     "coeus_plan_matmul": (C.c_int, [_u32, _u64, _u64, _u64, C.c_int, C.POINTER(CMatmulPlan)]),
     "coeus_op_gemm_timed": (C.c_int, [_vp, _vp, _u64, _u32, _vp, _u32, _vp, _vp]),
     "coeus_op_norm": (C.c_int, [_u32, _u32, _vp, _u64, _u64, _vp, _vp, _f32, _vp, _vp]),

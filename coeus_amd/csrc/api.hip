@@ -522,6 +522,22 @@ int coeus_op_matmul_limited(const coeus_weight *w, const float *x_dev, uint64_t 
     COEUS_GUARD_END
 }
 
+int coeus_op_gemm16(const coeus_weight *w, const float *a_dev, uint64_t m, uint32_t epilogue, float limit, int bf16, uint64_t ld, void *c_dev,
+                    void *stream) {
+    COEUS_GUARD_BEGIN
+    if (!w || !a_dev || !c_dev) return fail(COEUS_INVALID_INPUT, "null pointer argument");
+    Epilogue e;
+    if (epilogue > COEUS_EPI_SILU_GATE) {
+        COEUS_TRY(limited_epilogue(epilogue, limit, nullptr, e));
+    } else {
+        e.act = epilogue;
+    }
+    if (ld < (epi_gated(epilogue) ? w->w.n / 2 : w->w.n)) return fail(COEUS_INVALID_INPUT, "rows of %llu values do not hold the outputs", (unsigned long long)ld);
+    e.out_lp = LpOut{c_dev, ld, bf16 != 0};
+    return run_gemm(w->w, a_dev, m, e, (hipStream_t)stream);
+    COEUS_GUARD_END
+}
+
 int coeus_plan_matmul(uint32_t dtype, uint64_t k_in, uint64_t n_out, uint64_t rows, int prompt, coeus_matmul_plan *out) {
     COEUS_GUARD_BEGIN
     if (!out) return fail(COEUS_INVALID_INPUT, "null pointer argument");

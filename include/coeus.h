@@ -344,6 +344,10 @@ int coeus_op_gemm(const coeus_weight *w, const float *a_dev, uint64_t m, const f
  * and bf16 weights.  prompt 0: the decode matmul (rows <= 16), else the prefill matmul. */
 int coeus_op_matmul_limited(const coeus_weight *w, const float *x_dev, uint64_t rows, int prompt, uint32_t epilogue,
                             float limit, float *y_dev, void *stream);
+/* The prompt matmul with 16-bit outputs, as a prompt pass hands them to the next matmul: c_dev rows of `ld` bf16 (bf16 != 0) or f16 values,
+ * any epilogue (limit: those that have one). */
+int coeus_op_gemm16(const coeus_weight *w, const float *a_dev, uint64_t m, uint32_t epilogue, float limit, int bf16, uint64_t ld, void *c_dev,
+                    void *stream);
 /* The launch that a matmul of plain rows gets (no counterpart in the reference; for profiles and tests, no device is touched): `rows` of
  * the decode matmul (prompt 0), or of the prompt matmul with room for its partial products.  tile_rows x tile_cols outputs a
  * workgroup, waves of a workgroup, shares of k (tail_shares: of the tiles of a launch's last round). */

@@ -179,8 +179,8 @@ def test_gemm_gelu_fast_epilogue_walks(orc, dtype):
 @pytest.mark.parametrize("m,k,n", [(70, 1024, 334), (300, 2048, 520), (16, 4096, 256)])
 def test_gemm_split_along_k(orc, dtype, m, k, n):
     """Few output tiles and a long k: the 16-bit matmul runs as several workgroups per tile over
-    shares of k plus a kernel that sums the partial products and applies the epilogue (here 4, 8
-    and 16 shares; 334 and 520 columns end inside a tile, 334 is not a multiple of 4).  Plain,
+    shares of k plus a kernel that sums the partial products and applies the epilogue (tiles of 128x64, here 1, 8
+    and 16 shares; 334 and 520 columns end inside a tile, 334 is not a multiple of 4; 256x256 tiles: test_gpu_large_tiles.py).  Plain,
     bias + GELU + residual, and gated epilogues against float64 on the rounded operands.  The f32
     matmul splits its 32x32-tile launches from 1536 elements of k (here 5 and 8 shares; the first
     shape runs unsplit)."""
@@ -214,10 +214,9 @@ def test_gemm_split_along_k(orc, dtype, m, k, n):
 @pytest.mark.parametrize("dtype", ["bf16", "q8_0"])
 @pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 576])
 def test_gemm_slice_pipeline_boundaries(orc, dtype, k):
-    """The 16-bit matmul for k % 64 == 0 keeps three slices of A rows and two of W rows in LDS and
-    changes its schedule with the number of 64-wide slices (1, 2, 3: nothing left to request; from 4
-    on the steady-state period runs).  300 rows and 392 columns end inside the second tiles, no
-    launch here is split along k.  Plain, bias + GELU + residual, and gated epilogues against
+    """The 16-bit matmul of few tiles for k % 64 == 0 (128x64 here) keeps five slices of A rows and six of W rows in LDS: fewer
+    64-wide slices than that, as many, more.  300 rows and 392 columns end inside the last tiles, no
+    launch here is split along k (256x256 tiles: test_gpu_large_tiles.py).  Plain, bias + GELU + residual, and gated epilogues against
     float64 on the rounded operands."""
     m, n = 300, 392
     rng = np.random.default_rng(k + 5)

@@ -109,7 +109,8 @@ def clamped(z, limit):
 @pytest.mark.parametrize("wd", [_lib.W_F32, _lib.W_BF16])
 @pytest.mark.parametrize("rows,k,n,prompt", [(1, 96, 64, 0), (3, 130, 34, 0), (16, 64, 130, 0), (2, 2048, 512, 0), (1, 64, 130, 1),
                                              (5, 96, 34, 1), (70, 130, 200, 1), (150, 128, 512, 1), (600, 256, 1024, 1), (1100, 64, 2816, 1),
-                                             (2048, 512, 2048, 1), (300, 1024, 384, 1)])
+                                             (2048, 512, 2048, 1), (300, 1024, 384, 1),
+                                             (4400, 64, 4400, 1)])  # (256x256 tiles; the others of k % 64 == 0 are smaller ones)
 def test_limited_epilogues(epi, wd, rows, k, n, prompt):
     rng = np.random.default_rng(rows + n)
     x = bf16_round(rng.normal(size=(rows, k)))  # (a bf16 prompt matmul rounds its activations)

@@ -49,3 +49,24 @@ def test_decode_batches_of_up_to_four_on_quantised_weights():
     (_lib.W_F32, 768, 3072, b"gemv_dense_kernel"), (_lib.W_F32, 3072, 768, b"gemv_dense_kernel")])
 def test_decode_of_one_row(dtype, k, n, kernel):
     assert plan(dtype, k, n, 1).kernel == kernel
+
+
+# Prompts: the shapes that test_gpu_narrow_gemm.py, test_gpu_sum_error.py and test_gpu_large_tiles.py multiply reach all five small tiles, shares of k on
+# small and on large ones, and one workgroup a large tile
+@pytest.mark.parametrize("m,k,n,kernel,rows,cols,shared", [
+    (65, 64, 128, b"gemm_narrow_kernel", 128, 64, False), (512, 3072, 768, b"gemm_narrow_kernel", 128, 64, True), (201, 4096, 4098, b"gemm_narrow_kernel", 128, 128, True),
+    (257, 1024, 7000, b"gemm_narrow_kernel", 128, 96, False), (201, 1024, 22016, b"gemm_narrow_kernel", 256, 96, False), (2036, 4096, 2560, b"gemm_narrow_kernel", 256, 96, False),
+    (700, 2048, 8192, b"gemm_narrow_kernel", 256, 128, False), (300, 11008, 4096, b"gemm_h256k64_kernel", 256, 256, True), (5000, 64, 5100, b"gemm_h256k64_kernel", 256, 256, False),
+    (17, 96, 512, b"gemm_h256_kernel", 256, 256, False), (300, 90, 512, b"gemm_h_kernel", 128, 128, False)])
+def test_prompts(m, k, n, kernel, rows, cols, shared):
+    p = plan(_lib.W_BF16, k, n, m, 1)
+    assert (p.kernel, p.tile_rows, p.tile_cols, p.shares > 1) == (kernel, rows, cols, shared)
+    if k % 32 == 0:
+        assert plan(_lib.W_Q8_0, k, n, max(m, 65), 1).kernel == plan(_lib.W_BF16, k, n, max(m, 65), 1).kernel
+
+
+def test_other_prompts():
+    assert plan(_lib.W_Q4_0, 4096, 4096, 64, 1).kernel == b"gemm_qskinny_kernel" and plan(_lib.W_Q4_0, 4096, 4096, 65, 1).kernel == b"gemm_narrow_kernel"
+    assert plan(_lib.W_Q4_0, 4096, 22016, 4071, 1).tail_shares == 2 and plan(_lib.W_BF16, 512, 4090, 4100, 1).tail_shares == 2
+    assert plan(_lib.W_F32, 768, 768, 5, 1).kernel == b"gemv_mfma_kernel" and plan(_lib.W_F32, 768, 768, 128, 1).kernel == b"gemm_f32_small_kernel"
+    assert plan(_lib.W_F32, 3072, 768, 128, 1).shares == 8 and plan(_lib.W_F32, 768, 50257, 128, 1).kernel == b"gemm_f32_kernel"
