@@ -171,6 +171,8 @@ def prefill_report(cfg, batch, n_prompt, prefill_s, weight_dtype=None):
         _check(lib.coeus_op_gemm_timed(h, a.ptr, rows, 2 if gated else 1, c.ptr, reps, C.byref(ms), None))
         best = min(best, ms.value)
     lib.coeus_weight_destroy(h)
+    plan = _lib.CMatmulPlan()
+    _check(lib.coeus_plan_matmul(wdt, k, n, rows, 1, C.byref(plan)))
     tflops = 2.0 * rows * n * k * reps / (best * 1e-3) / 1e12
     traffic, traffic_source = _prefill_traffic(cfg, rows, n, k) if wname == cfg.weight_dtype else (None, None)
     f32 = wname == "f32"
@@ -178,7 +180,7 @@ def prefill_report(cfg, batch, n_prompt, prefill_s, weight_dtype=None):
     return {
         "tokens": rows, "ms": round(prefill_s * 1e3, 2), "tok_s": round(rows / prefill_s, 1),
         "roofline": {
-            "kernel": "gemm_f32_kernel" if f32 else "gemm_h256k64_kernel", "bound": "mfma",
+            "kernel": plan.kernel.decode(), "bound": "mfma",
             "achieved": round(tflops, 1), "peak": peak, "unit": "TFLOP/s",
             "frac": round(tflops / peak, 4), "traffic": traffic, "traffic_source": traffic_source,
             "shape": {"m": rows, "n": n, "k": k}, "us_per_launch": round(best * 1e3 / reps, 1),

@@ -114,8 +114,8 @@ struct XArgs {
     uint32_t k;           // logical reduction length
 };
 
-// The same normalisation as a launch of its own, for batches whose activation block does not fit
-// the matmul's LDS staging: row b of h -> xq, statistics merged from the producer's records
+// The same normalisation as a launch of its own, for all batches of 5 to 16 (and of up to 4 whose rows do not fit
+// gemv_quad_kernel's LDS): row b of h -> xq, statistics merged from the producer's records
 // (no reduction over the row).  Grid (k pieces / 256, batch); every wave merges its row's records.
 // Bound by one trip to memory behind the launch: everything is requested at once, and the wave's sums are register moves.
 template <bool RMS>

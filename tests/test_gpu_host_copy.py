@@ -1,5 +1,5 @@
-"""Logits on their way to the caller: sizes around the pinned slots (1 MiB, four of them) and results that start in the
-middle of a page, against the same rows fetched one at a time."""
+"""Logits on their way to the caller: sizes around the pieces (16 KiB) and halves (4 MiB, two of them) of the pinned memory that they go through, and
+results that start in the middle of a page, against the same rows fetched one at a time."""
 import ctypes as C
 import resource
 import time
@@ -14,7 +14,7 @@ from coeus_amd.plugin import _check
 pytestmark = pytest.mark.gpu
 
 
-# 4 * vocab bytes a row: 4096 in all; one slot, and one value more; four slots; nine and a bit
+# 4 * vocab bytes a row: 4096 in all (the runtime's copy) and one row more; 1 MiB and one value a row more; one half; three rounds through the halves, three threads
 @pytest.mark.parametrize("vocab,rows", [(512, 2), (1024, 256), (1025, 256), (4096, 256), (9001, 270), (513, 2)])
 def test_every_row_arrives(vocab, rows):
     cfg = Transformer250MConfig(hidden_dim=32, num_layers=1, num_heads=2, intermediate_dim=64, vocab_size=vocab, max_seq_len=rows,
@@ -26,7 +26,8 @@ def test_every_row_arrives(vocab, rows):
     _check(_lib.load().coeus_model_forward_all(model._h, ids.ctypes.data, rows, buf.ctypes.data + 17 * 4))
     assert np.array_equal(buf[17:17 + rows * vocab].reshape(rows, vocab), want)
     assert (buf[:17] == 7.0).all() and (buf[17 + rows * vocab:] == 7.0).all()
-    per = (1 << 20) // (4 * vocab)  # rows of a slot
+    # rows on both sides of every MiB: of pieces' and halves' ends
+    per = (1 << 20) // (4 * vocab)
     for r in sorted({0, rows - 1, *[i for k in range(1, 11) for i in (per * k - 1, per * k, per * k + 1) if 0 <= i < rows]}):
         one = model.forward(ids[:r + 1])  # per-token norms: a row does not see what follows it
         assert np.abs(one - want[r]).max() <= 2e-5 * np.abs(want[r]).max(), r
@@ -38,7 +39,7 @@ def test_every_row_arrives(vocab, rows):
 
 
 def test_into_pinned_and_device_memory():
-    """Results that the caller wants in pinned memory (26 slots' worth, and less than a slot), or on the device."""
+    """Results that the caller wants in pinned memory (seven halves' worth, and a few pieces), or on the device."""
     vocab, rows = 50257, 128
     cfg = Transformer250MConfig(hidden_dim=32, num_layers=1, num_heads=2, intermediate_dim=64, vocab_size=vocab, max_seq_len=rows,
                                 norm_scope="token")
