@@ -405,7 +405,9 @@ __device__ __forceinline__ bool epi_vec4(const EpiArgs &e) {
     return (e.n_eff & 3) == 0 && (e.lp_ld & 3) == 0 && (e.out_f32 || e.out_lp) && !e.out_xq;
 }
 // Columns col .. col + 3 of activation row `row` (bias, cache append or activation, residual, store).
-// OWN: GELU and SiLU by times_sigmoid, no further off than the math library forms.
+// OWN: GELU and SiLU by times_sigmoid where the caller sees f32 results (no further off than the math library's forms), else on the
+// hardware's exp2 and reciprocal: at most 17 of 2^-24 off, where the rounding to f16 takes 2^12 of them (root mean square error of a gate to f16 2.0794e-4
+// either way; 512 rows of 768 x 3072 with GELU 10.6 us by times_sigmoid, 9.7 on the hardware's).
 template <bool OWN = false>
 __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCols &kc, uint64_t row,
                                          uint64_t col, uint64_t n, float (&v)[4]) {
@@ -430,7 +432,7 @@ __device__ __forceinline__ void epi_row4(const EpiArgs &e, bool vec4, const KvCo
         }
         if (e.act == COEUS_EPI_GELU)
 #pragma unroll
-            for (int q = 0; q < 4; q++) v[q] = OWN ? gelu_f32(v[q]) : gelu_tanh(v[q]);
+            for (int q = 0; q < 4; q++) v[q] = !OWN ? gelu_tanh(v[q]) : e.out_f32 ? gelu_f32(v[q]) : fast_gelu(v[q]);
         if (e.act == COEUS_EPI_SOFTCAP)
 #pragma unroll
             for (int q = 0; q < 4; q++) v[q] = soft_cap(v[q], e.limit);
@@ -454,7 +456,7 @@ __device__ __forceinline__ void epi_row4_gated(const EpiArgs &e, bool vec4, uint
     if (vec4 && !e.bias && !e.residual && raw + 7 < n) {
         float o[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) o[q] = e.act == COEUS_EPI_CLAMP_GATE ? clamped_gate(gv[q], uv[q], e.limit) : (OWN ? silu_f32(gv[q]) : silu(gv[q])) * uv[q];
+        for (int q = 0; q < 4; q++) o[q] = e.act == COEUS_EPI_CLAMP_GATE ? clamped_gate(gv[q], uv[q], e.limit) : (!OWN ? silu(gv[q]) : e.out_f32 ? silu_f32(gv[q]) : fast_silu(gv[q])) * uv[q];
         epi_store4(e, row, ocol, o);
     } else {
 #pragma unroll
@@ -1428,9 +1430,6 @@ struct NarrowTile {
     static constexpr int WN = 4 / WM, ROWS = WM * RB * 32, COLS = WN * NB * 32;
     static constexpr int UA = ROWS / 32, UW = COLS / 32;  // requests of a wave and slice: 8 rows x 128 bytes each, four waves an operand
     static constexpr int DA = ROWS == 256 ? 3 : 5, DW = ROWS == 256 ? (COLS == 128 ? 4 : COLS == 96 ? 5 : 6) : COLS == 128 ? 5 : 6;
-    // Sums can begin again after some slices (a wave of eight blocks has no registers for that), see GemmPlan.
-    static constexpr bool AGAIN = RB * NB <= 6;
-    static constexpr int TRB = AGAIN ? RB : 1, TNB = AGAIN ? NB : 1;
     static constexpr size_t ring = ((size_t)DA * ROWS + (size_t)DW * COLS) * UK * 2, tile = (size_t)ROWS * (COLS + 4) * 4, lds = ring > tile ? ring : tile;
     static_assert(lds <= 160 * 1024, "fits the LDS of a CU");
 };
@@ -1466,7 +1465,8 @@ __device__ __forceinline__ void narrow_step(const uint16_t *__restrict__ ra, con
     }
 }
 
-template <bool BF16, int WM, int RB, int NB>
+// AGAIN: sums begin again every `period` slices, see GemmPlan (a wave of eight blocks has no registers for that).
+template <bool BF16, int WM, int RB, int NB, bool AGAIN>
 __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, const uint16_t *w, uint64_t m, uint64_t n, uint64_t k, uint64_t lda,
                                                           uint64_t ldw, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits, uint32_t period, EpiArgs e) {
     using T = NarrowTile<WM, RB, NB>;
@@ -1491,11 +1491,11 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
         for (int y = 0; y < NB; y++)
 #pragma unroll
             for (int i = 0; i < 16; i++) acc[x][y][i] = 0.f;
-    float16_t total[T::TRB][T::TNB];  // of the slices before the present ones
+    float16_t total[AGAIN ? RB : 1][AGAIN ? NB : 1];  // of the slices before the present ones
 #pragma unroll
-    for (int x = 0; x < T::TRB; x++)
+    for (int x = 0; x < (AGAIN ? RB : 1); x++)
 #pragma unroll
-        for (int y = 0; y < T::TNB; y++) total[x][y] = acc[x][y];
+        for (int y = 0; y < (AGAIN ? NB : 1); y++) total[x][y] = acc[x][y];
     const bool takes_a = half == 0;
     uint32_t off[Q];
     {
@@ -1569,7 +1569,7 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
         io = io + 1 == depth ? 0 : io + 1;
         narrow_step<BF16, T, RB, NB, false>(rega + ia * RA, regw + iw * RW, freed, source(kbeg + (uint64_t)(s + depth) * UK), off, takes_a, w4,
                                             la[0], lw[0], af[1], wf[1], af[0], wf[0], acc);
-        if constexpr (T::AGAIN) {
+        if constexpr (AGAIN) {
             if (s == until) {
                 until += period;
 #pragma unroll
@@ -1581,15 +1581,13 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
             }
         }
     }
-    if constexpr (T::AGAIN) {
-        if (period <= nsl) {
+    if constexpr (AGAIN) {
 #pragma unroll
-            for (int x = 0; x < RB; x++)
+        for (int x = 0; x < RB; x++)
 #pragma unroll
-                for (int y = 0; y < NB; y++)
+            for (int y = 0; y < NB; y++)
 #pragma unroll
-                    for (int i = 0; i < 16; i++) acc[x][y][i] += total[x][y][i];
-        }
+                for (int i = 0; i < 16; i++) acc[x][y][i] += total[x][y][i];
     }
     __builtin_amdgcn_s_waitcnt(0x0070);  // the repeats have landed too
     __syncthreads();
@@ -1644,15 +1642,17 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
     }
 }
 
-template <bool BF16, int WM, int RB, int NB>
+template <bool BF16, int WM, int RB, int NB, bool AGAIN = false>
 static int launch_narrow(const uint16_t *a, const uint16_t *w, uint64_t m, uint64_t n, uint64_t k, uint64_t lda, uint64_t ldw, uint32_t splits,
                          uint32_t period, const EpiArgs &e, hipStream_t st) {
+    if constexpr (!AGAIN && RB * NB < 8)
+        if (period != ~0u) return launch_narrow<BF16, WM, RB, NB, true>(a, w, m, n, k, lda, ldw, splits, period, e, st);
     using T = NarrowTile<WM, RB, NB>;
-    static const hipError_t once = hipFuncSetAttribute((const void *)gemm_narrow_kernel<BF16, WM, RB, NB>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    static const hipError_t once = hipFuncSetAttribute((const void *)gemm_narrow_kernel<BF16, WM, RB, NB, AGAIN>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     COEUS_HIP(once);
     const uint32_t tiles_m = (uint32_t)ceil_div(m, T::ROWS), tiles_n = (uint32_t)ceil_div(n, T::COLS);
-    hipLaunchKernelGGL((gemm_narrow_kernel<BF16, WM, RB, NB>), dim3((uint32_t)round_up((uint64_t)tiles_m * tiles_n * splits, 8)), dim3(512), T::lds, st, a, w, m, n, k,
-                       lda, ldw, tiles_m, tiles_n, splits, period, e);
+    hipLaunchKernelGGL((gemm_narrow_kernel<BF16, WM, RB, NB, AGAIN>), dim3((uint32_t)round_up((uint64_t)tiles_m * tiles_n * splits, 8)), dim3(512), T::lds, st, a, w, m, n,
+                       k, lda, ldw, tiles_m, tiles_n, splits, period, e);
     COEUS_HIP(hipGetLastError());
     return COEUS_OK;
 }
