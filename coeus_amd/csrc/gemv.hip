@@ -988,13 +988,98 @@ __device__ __forceinline__ void stage_normed_rows(float *xn, const float *__rest
     }
 }
 
-template <bool BF16, int BP, int NORM>
-__global__ __launch_bounds__(1024) void gemv_dense_kernel(const void *__restrict__ wdata,
+// One plain activation row, k % 8 == 0: R weight rows a wave, D steps of 512 k of each in flight next to the activations they
+// share.  Bound by the weights' stream, and where that is short by the trips to memory a wave makes one behind the other.
+// Two rows (gemv_many_kernel) against one with two steps at most (gemv_dense_kernel's general form), which reads twice the weights'
+// bytes in activations (f32 next to bf16) and leaves memory idle between its steps, us, distinct weights in turn, there /
+// here: bf16 4096 x 22016 33.2 / 29.0, x 32000 46.3 / 40.9, x 12352 19.7 / 18.3, 2048 x 11264 11.2 / 9.0, x 2048 4.3 / 3.5;
+// f32 4096 x 22016 74.6 / 65.9.  The matrix cores had rows of these: 5632 x 2048 7.7 / 5.5, 11008 x 4096
+// 18.4 / 17.7, 4096 x 4096 7.5 / 7.5, 768 x 50257 13.5 / 13.4, 1024 x 16384 7.5 / 6.9.  Four rows a wave with two or three steps:
+// 29.9, 40.0, 20.1, 10.1, 4.3; eight are slower than one.
+// One row with D steps (gemv_dense_kernel's D) where up to 1024 rows leave compute units without a workgroup of two, against what they
+// had: f32 3072 x 768 5.76 / 4.85, 8192 x 1024 11.9 / 9.0, 768 x 3072 4.43 / 4.11, 4096 x 3072 13.3 / 12.8; bf16 3072 x 768 3.81 / 3.39,
+// 11008 x 1024 8.3 / 6.9.  A row over two or four waves that meet in LDS: 5.07, 10.1 and 3.49, 7.1 at best.
+template <bool BF16, int D, int R>
+__device__ __forceinline__ void one_row(const void *__restrict__ wdata, const float *__restrict__ x, uint32_t k, const EpiArgs &e) {
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int Q = BF16 ? 1 : 2;
+    const uint32_t n = (uint32_t)e.n, j0 = (blockIdx.x * 4 + wave) * R, trips = (k + 512 * D - 1) / (512 * D);
+    uint4 wv[D][R][Q];
+    float4 xv[D][2];
+    const char *row[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) row[r] = (const char *)wdata + (uint64_t)min(j0 + r, n - 1) * k * (BF16 ? 2 : 4);
+    auto request = [&](int d, uint32_t step) {  // (a lane behind the end re-reads the last 8 and does not use them)
+        const uint32_t i = min(512 * step + 8 * lane, k - 8);
+        xv[d][0] = *(const float4 *)(x + i);
+        xv[d][1] = *(const float4 *)(x + i + 4);
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int q = 0; q < Q; q++) wv[d][r][q] = load_stream((const uint4 *)(row[r] + (uint64_t)i * (BF16 ? 2 : 4)) + q);
+    };
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = 0.f;
+    auto multiply = [&](int d) {
+        const float v[8] = {xv[d][0].x, xv[d][0].y, xv[d][0].z, xv[d][0].w, xv[d][1].x, xv[d][1].y, xv[d][1].z, xv[d][1].w};
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint4 a = wv[d][r][0], c = wv[d][r][Q - 1];
+            float t[8];
+            if (BF16) {
+                const uint32_t q[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+                for (int u = 0; u < 4; u++) { t[2 * u] = __uint_as_float(q[u] << 16); t[2 * u + 1] = __uint_as_float(q[u] & 0xffff0000u); }
+            } else {
+                const uint32_t q[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+#pragma unroll
+                for (int u = 0; u < 8; u++) t[u] = __uint_as_float(q[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc[r] = fmaf(t[u], v[u], acc[r]);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) request(d, d);
+    for (uint32_t i = 0; i + 1 < trips; i++) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(d);
+            __builtin_amdgcn_sched_barrier(0);
+            request(d, (i + 1) * D + d);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; d++)
+        if (512 * ((trips - 1) * D + d) + 8 * lane < k) multiply(d);
+#pragma unroll
+    for (int r = 0; r < R; r++) acc[r] = wave_sum(acc[r]);
+    if (epi_gated(e.act)) {
+        if (lane == 0 && j0 + 1 < n) epi_store_gated(e, 0, j0 / 2, acc[0], acc[R - 1]);  // (R == 2)
+    } else if (lane < R && j0 + lane < n) {
+        epi_store<true>(e, 0, j0 + lane, lane ? acc[R - 1] : acc[0]);
+    }
+}
+
+template <bool BF16, int D>
+__global__ __launch_bounds__(256) void gemv_many_kernel(const void *__restrict__ wdata, const float *__restrict__ x, uint32_t k, EpiArgs e) {
+    one_row<BF16, D, 2>(wdata, x, k, e);
+}
+
+// D > 0: one plain row, k % 8 == 0, 16-byte pointers, no gate: the code above with a weight row a wave
+template <bool BF16, int BP, int NORM, int D = 0>
+__global__ __launch_bounds__(D ? 256 : 1024) void gemv_dense_kernel(const void *__restrict__ wdata,
                                                           const float *__restrict__ x, uint64_t k,
                                                           uint32_t batch, EpiArgs e,
                                                           const float *__restrict__ nscale,
                                                           const float *__restrict__ nbias, float eps,
                                                           uint64_t ldx, PostNorm post) {
+    if constexpr (D > 0) {
+        one_row<BF16, D, 1>(wdata, x, (uint32_t)k, e);
+        return;
+    }
     extern __shared__ float xn[];  // NORM: [BP][k] rows, [2][k] scale and bias, partial sums, statistics
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
     const uint64_t j = (uint64_t)blockIdx.x * nwaves + wave;
@@ -1218,77 +1303,6 @@ __global__ __launch_bounds__(256) void gemv_row_kernel(const void *__restrict__ 
         for (int r = 1; r < R; r++)
             if (lane == (uint32_t)r) t = acc[r];
         if (lane < R && j0 + lane < n) epi_store<true>(e, 0, j0 + lane, t);
-    }
-}
-
-// One plain activation row, k % 8 == 0: two weight rows a wave, D steps of 512 k of both in flight next to the activations they
-// share.  Bound by the weights' stream; gemv_dense_kernel, a weight row a wave and two steps at most, reads twice the weights'
-// bytes in activations (f32 next to bf16) and leaves memory idle between its steps.  us, distinct weights in turn, there /
-// here: bf16 4096 x 22016 33.2 / 29.0, x 32000 46.3 / 40.9, x 12352 19.7 / 18.3, 2048 x 11264 11.2 / 9.0, x 2048 4.3 / 3.5,
-// 3072 x 768 4.9 / 3.6; f32 4096 x 22016 74.6 / 65.9.  The matrix cores had rows of these: 5632 x 2048 7.7 / 5.5, 11008 x 4096
-// 18.4 / 17.7, 4096 x 4096 7.5 / 7.5, 768 x 50257 13.5 / 13.4, 1024 x 16384 7.5 / 6.9.  Four rows a wave with two or three steps:
-// 29.9, 40.0, 20.1, 10.1, 4.3; eight are slower than one.
-template <bool BF16, int D>
-__global__ __launch_bounds__(256) void gemv_many_kernel(const void *__restrict__ wdata, const float *__restrict__ x, uint32_t k, EpiArgs e) {
-    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    constexpr int R = 2, Q = BF16 ? 1 : 2;
-    const uint32_t n = (uint32_t)e.n, j0 = (blockIdx.x * 4 + wave) * R, trips = (k + 512 * D - 1) / (512 * D);
-    uint4 wv[D][R][Q];
-    float4 xv[D][2];
-    const char *row[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) row[r] = (const char *)wdata + (uint64_t)min(j0 + r, n - 1) * k * (BF16 ? 2 : 4);
-    auto request = [&](int d, uint32_t step) {  // (a lane behind the end re-reads the last 8 and does not use them)
-        const uint32_t i = min(512 * step + 8 * lane, k - 8);
-        xv[d][0] = *(const float4 *)(x + i);
-        xv[d][1] = *(const float4 *)(x + i + 4);
-#pragma unroll
-        for (int r = 0; r < R; r++)
-#pragma unroll
-            for (int q = 0; q < Q; q++) wv[d][r][q] = load_stream((const uint4 *)(row[r] + (uint64_t)i * (BF16 ? 2 : 4)) + q);
-    };
-    float acc[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) acc[r] = 0.f;
-    auto multiply = [&](int d) {
-        const float v[8] = {xv[d][0].x, xv[d][0].y, xv[d][0].z, xv[d][0].w, xv[d][1].x, xv[d][1].y, xv[d][1].z, xv[d][1].w};
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            const uint4 a = wv[d][r][0], c = wv[d][r][Q - 1];
-            float t[8];
-            if (BF16) {
-                const uint32_t q[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-                for (int u = 0; u < 4; u++) { t[2 * u] = __uint_as_float(q[u] << 16); t[2 * u + 1] = __uint_as_float(q[u] & 0xffff0000u); }
-            } else {
-                const uint32_t q[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
-#pragma unroll
-                for (int u = 0; u < 8; u++) t[u] = __uint_as_float(q[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < 8; u++) acc[r] = fmaf(t[u], v[u], acc[r]);
-        }
-    };
-#pragma unroll
-    for (int d = 0; d < D; d++) request(d, d);
-    for (uint32_t i = 0; i + 1 < trips; i++) {
-#pragma unroll
-        for (int d = 0; d < D; d++) {
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(d);
-            __builtin_amdgcn_sched_barrier(0);
-            request(d, (i + 1) * D + d);
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < D; d++)
-        if (512 * ((trips - 1) * D + d) + 8 * lane < k) multiply(d);
-#pragma unroll
-    for (int r = 0; r < R; r++) acc[r] = wave_sum(acc[r]);
-    if (epi_gated(e.act)) {
-        if (lane == 0 && j0 + 1 < n) epi_store_gated(e, 0, j0 / 2, acc[0], acc[1]);
-    } else if (lane < R && j0 + lane < n) {
-        epi_store<true>(e, 0, j0 + lane, lane ? acc[1] : acc[0]);
     }
 }
 
@@ -2078,14 +2092,29 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
 // 3072 1.03 - 1.09); short rows only where there are very many (768 x 50257 0.97, x 32000 0.98; 640 x 11008 1.05, 512 x 16384 1.05, 1024 x
 // 11008 1.06).  bf16: all that the matrix cores do not take (gemv_uses_mfma), but rows 32 KiB apart, which share their memory channels,
 // are a wave's each between 4096 and 6144 of them (16384 x 4608 1.07, 32768 x 4608 1.14; x 6144 1.00, x 8192 0.86), and so are few
-// rows of exactly one step of 512 (x 300 1.10, x 768 1.11, x 1024 1.06, x 3000 0.97; 448 x 768 0.96).
-static bool gemv_takes_many(const Weight &w, uint64_t batch) {
+// rows of exactly one step of 512 (x 300 1.10, x 768 1.11, x 1024 1.06, x 3000 0.97; 448 x 768 0.96), and up to 1024 of more than two steps
+// (1032 x 1030 0.99, x 768 0.98 of the time with a wave per row, 2048 x 1024 0.92, 11008 x 1024 0.80, but 1536 x 1536 1.07).
+static bool gemv_takes_many(const Weight &w, uint64_t batch, bool gated = false) {
     if (batch != 1 || w.dtype > COEUS_W_BF16 || w.k % 8 || w.k >= (1ull << 31) || w.n >= (1ull << 31) - 8) return false;
     if (w.dtype == COEUS_W_BF16)
         return !gemv_uses_mfma(w, 1, gemv_mfma_waves(w.k / MfmaType<true>::KU), false) && !(w.k % 16384 == 0 && w.n > 4096 && w.n < 6144) &&
-               !(w.k == 512 && w.n < 2048);
+               !(w.k == 512 && w.n < 2048) && (gated || w.k <= 1024 || w.n > 1024);
     if (w.k >= 1536) return w.n == 2048 || w.n > 3200;
     return w.k > 1024 ? w.n >= 8192 : w.k > 512 && w.k < 1024 && w.n >= 20000;
+}
+
+// One plain row of the others: steps in flight of a weight row a wave (0: the general form, for gates, whose pairs it holds in two waves,
+// and lengths that are no multiple of 8).  f32 (us with 2 / 3 / 4 / 6): two where a workgroup a CU and less is all there is (8192 x 1024 8.98 /
+// 9.18 / 9.04 / 9.43, 16384 x 768 15.1 / - / 15.6), else three or four, whichever asks for fewer steps in vain (4096 x 3072 13.1 / 13.3 / 12.8 /
+// 14.7, 3072 x 3072 10.8 / 10.6 / 10.9 / 10.9).  bf16: four, or six where they are fewer trips with no more in vain (3072 x 768 3.99 / 3.50 / 3.53 / 3.39,
+// 8192 x 1024 6.70 / 5.79 / 5.18 / 5.40); rows 32 KiB apart stay with the general form (16384 x 4608 30.8, two steps of these 34.2, four 32.7).
+static uint32_t gemv_one_row_steps(const Weight &w, uint64_t batch, bool gated) {
+    if (batch != 1 || w.dtype > COEUS_W_BF16 || w.k % 8 || w.k >= (1ull << 31) || w.n >= (1ull << 31) - 8 || gated) return 0;
+    const uint64_t steps = ceil_div(w.k, 512);
+    if (steps <= 2) return (uint32_t)steps;
+    auto slots = [&](uint64_t d) { return ceil_div(steps, d) * d; };
+    if (w.dtype == COEUS_W_F32) return w.n <= 1024 ? 2 : slots(3) < slots(4) ? 3 : 4;
+    return w.n > 1024 ? 0 : slots(6) <= slots(4) && steps % 4 ? 6 : 4;
 }
 
 // Plain rows on the matrix cores: waves of a workgroup, LDS, and whether they go there.
@@ -2133,7 +2162,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         COEUS_HIP(hipGetLastError());
         return COEUS_OK;
     }
-    if (norm == 0 && aligned && gemv_takes_many(w, batch)) {
+    if (norm == 0 && aligned && gemv_takes_many(w, batch, epi_gated(e.act))) {
         const dim3 mgrid((unsigned)ceil_div(w.n, 8));
         if (w.k <= 1024) hipLaunchKernelGGL((gemv_many_kernel<BF16, 2>), mgrid, dim3(256), 0, st, w.data, xin, (uint32_t)w.k, e);
         else hipLaunchKernelGGL((gemv_many_kernel<BF16, 4>), mgrid, dim3(256), 0, st, w.data, xin, (uint32_t)w.k, e);
@@ -2186,6 +2215,17 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
             COEUS_HIP(hipGetLastError());
             return COEUS_OK;
         }
+    }
+    if (const uint32_t steps = norm == 0 && aligned ? gemv_one_row_steps(w, batch, epi_gated(e.act)) : 0) {
+#define COEUS_ONE(DV) hipLaunchKernelGGL((gemv_dense_kernel<BF16, 1, 0, DV>), grid, block, 0, st, w.data, xin, w.k, b, e, ns, nb, eps, ldx, post)
+        if (steps == 1) COEUS_ONE(1);
+        else if (steps == 2) COEUS_ONE(2);
+        else if (steps == 3) COEUS_ONE(3);
+        else if (steps == 4) COEUS_ONE(4);
+        else COEUS_ONE(6);
+#undef COEUS_ONE
+        COEUS_HIP(hipGetLastError());
+        return COEUS_OK;
     }
     if (norm == 4) return fail(COEUS_INVALID_INPUT, "a folded norm over all rows needs its vectors on 16-byte boundaries");
 #define COEUS_GEMVD2(BPV, NV) \

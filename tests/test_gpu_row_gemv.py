@@ -34,3 +34,10 @@ def test_matches_float64(orc, dtype, k, n, gated):
         got, want = wt.gemv(dev(x), bias=dev(bias), residual=dev(res)), pre + res
         e = e + 2.0 ** -23 * np.abs(want)
     assert (np.abs(got - want) <= e).all()
+
+
+# A weight row a wave: one, two, three, four and six steps in flight, with shares that end inside a step and inside a trip, both sides of 1024 rows
+@pytest.mark.parametrize("dtype", [_lib.W_F32, _lib.W_BF16])
+@pytest.mark.parametrize("k,n", [(512, 768), (776, 3), (1288, 1030), (1544, 1024), (2560, 1025), (2568, 5), (3072, 1024), (3080, 1001), (4608, 6), (5640, 1023), (16384, 4097)])
+def test_a_weight_row_a_wave(orc, dtype, k, n):
+    test_matches_float64(orc, dtype, k, n, False)

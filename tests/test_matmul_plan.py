@@ -51,6 +51,13 @@ def test_decode_of_one_row(dtype, k, n, kernel):
     assert plan(dtype, k, n, 1).kernel == kernel
 
 
+# Up to 1024 rows of more than two steps: a wave each (bf16 11008 x 1024 8.3 us with two rows a wave, 6.9 so)
+@pytest.mark.parametrize("k,n,kernel", [(1024, 1024, b"gemv_many_kernel"), (1032, 1024, b"gemv_dense_kernel"), (1032, 1025, b"gemv_many_kernel"),
+                                        (11008, 1024, b"gemv_dense_kernel"), (11008, 1025, b"gemv_many_kernel")])
+def test_few_long_rows_of_bf16(k, n, kernel):
+    assert plan(_lib.W_BF16, k, n, 1).kernel == kernel
+
+
 # Prompts: the shapes that test_gpu_narrow_gemm.py, test_gpu_sum_error.py and test_gpu_large_tiles.py multiply reach all five small tiles, shares of k on
 # small and on large ones, and one workgroup a large tile
 @pytest.mark.parametrize("m,k,n,kernel,rows,cols,shared", [
