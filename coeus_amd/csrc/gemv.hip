@@ -1329,6 +1329,13 @@ __global__ __launch_bounds__(256) void gemv_row_kernel(const void *__restrict__ 
 // lane: 8 consecutive k of one row).  Loaded the way they are multiplied (16 rows x 64 bytes, neighbouring lanes in
 // different rows) the same weights take a third longer: 4096 x 22016 at batch 4 in 51 against 40 us.  The activations
 // travel likewise.  PD pairs are in flight per wave across the ends of tiles; the waves' partial tiles meet in LDS.
+//
+// Few outputs are few tiles of 16, and a compute unit brings in 50 GB/s alone (f32 3072 x 768: 48 tiles, 257 KB each of weights and
+// activations).  Up to eight activation rows leave half of the sixteen columns unused, up to four three quarters, so the lines of a tile can be
+// TS parts of k of 16 / TS weight rows and the columns the activations of the same parts: of the product, part i's lines meet part i's
+// columns in the blocks on the diagonal, and those are added.  Twice or four times the workgroups for the same instructions.  us, tiles of 16 /
+// in parts: f32, 4 rows of 3072 x 768 8.3 / 5.1, 8192 x 1024 16.7 / 9.2, 768 x 768 4.4 / 3.4, 8 of 3072 x 768 8.8 / 6.5; bf16, 4 of 3072 x 768
+// 5.7 / 4.7, 8192 x 1024 10.1 / 7.1, 5632 x 2048 10.1 / 8.0, 8 of 2048 x 1024 5.4 / 4.9.
 
 // Two values -> their three bf16, a pair of upper halves per piece.  What is left of an infinity is zero (its own
 // difference would be a NaN).
@@ -1354,6 +1361,7 @@ __device__ __forceinline__ Split2 split2(float a, float b) {
 // k % 64 == 0 and at least one pair of chunks per wave.
 // KEEP: a wave's share of k is at most PD pairs, and its split activations stay in registers from tile to tile.
 // lds: mfma_wave_lds(XQ) uint4 per wave.
+// TS: parts of k (XQ > 0 only, requests for sixteen rows: the columns).
 // (Rows 16 bytes longer than k: at a multiple of 256 bytes apart they would share their banks.)
 struct SplitRows {  // bf16 weights: three pieces
     uint16_t *p;
@@ -1420,7 +1428,7 @@ template <> struct MfmaType<false> {
 // uint4 of a wave's corner: 16 weight rows x 128 bytes; per request of x its rows' KU values in pieces
 template <bool BF16>
 static constexpr uint32_t mfma_wave_lds(int xq) { return 128 + (BF16 ? 96 : 64) * xq; }
-template <bool BF16, int PD, bool KEEP, int XQ, class Stage>
+template <bool BF16, int PD, bool KEEP, int XQ, int TS, class Stage>
 __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
                                           uint32_t n, uint32_t batch, uint32_t nw, uint32_t grid, const EpiArgs &e, uint4 *lds,
                                           const typename MfmaType<BF16>::Rows &xs, Stage stage) {
@@ -1430,17 +1438,22 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
     constexpr uint32_t KU = MT::KU, EPP = KU / 8;  // k per pair, elements per 16-byte piece
     constexpr int XR = MT::XROWS, XN = XQ ? XQ : 1;
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t c = lane & 15, g = lane >> 4, cb = min(c, batch - 1);
-    const uint32_t pairs = k / KU, pb = pairs * wave / nw, np = pairs * (wave + 1) / nw - pb, groups = (np + PD - 1) / PD;
-    const uint32_t tiles = (n + 15) / 16;
+    static_assert(TS == 1 || XQ == 16 / XR, "parts of k need all sixteen columns");
+    constexpr uint32_t R = 16 / TS;  // weight rows of a tile, activation rows of a part
+    const uint32_t c = lane & 15, g = lane >> 4, cb = TS > 1 ? c : min(c, batch - 1);
+    const uint32_t pairs = k / (KU * TS), pb = pairs * wave / nw, np = pairs * (wave + 1) / nw - pb, groups = (np + PD - 1) / PD;
+    const uint32_t tiles = (n + R - 1) / R;
     uint4 *wl = lds + wave * mfma_wave_lds<BF16>(XQ), *xl = wl + 128;
     // (a pair behind the wave's share is the share's last one again: no branches around the requests)
-    auto pair_at = [&](uint32_t i) { return min(i, np - 1) * KU; };
+    auto pair_at = [&](uint32_t i) { return min(i, np - 1) * (KU * TS); };
     struct WRows { const W *p[2]; };
     auto tile_rows = [&](uint32_t tile) {
         WRows r;
 #pragma unroll
-        for (int q = 0; q < 2; q++) r.p[q] = w + (uint64_t)min(tile * 16 + 8 * q + (lane >> 3), n - 1) * k + pb * KU + (lane & 7) * EPP;
+        for (int q = 0; q < 2; q++) {
+            const uint32_t line = 8 * q + (lane >> 3);
+            r.p[q] = w + (uint64_t)min(tile * R + (TS > 1 ? line % R : line), n - 1) * k + (TS > 1 ? pb * TS + line / R : pb) * KU + (lane & 7) * EPP;
+        }
         return r;
     };
     const float *xr[XN];
@@ -1488,7 +1501,10 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
     if (XQ) {
         constexpr uint32_t LPR = 64 / XR;  // lanes per row
 #pragma unroll
-        for (int q = 0; q < XQ; q++) xr[q] = x + (uint64_t)min(XR * q + lane / LPR, batch - 1) * k + pb * KU + (lane % LPR) * 4;
+        for (int q = 0; q < XQ; q++) {
+            const uint32_t line = XR * q + lane / LPR;
+            xr[q] = x + (uint64_t)min(TS > 1 ? line % R : line, batch - 1) * k + (TS > 1 ? pb * TS + line / R : pb) * KU + (lane % LPR) * 4;
+        }
     }
     uint32_t tile = blockIdx.x, gi = 0;
     WRows wp = tile_rows(tile);
@@ -1517,7 +1533,10 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
             __builtin_amdgcn_wave_barrier();
         }
     }
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    // (every second pair adds up in accumulators of its own, f32's halves of one too: few waves' sums are no longer than many's)
+    // (not shares of two pairs, and not where sixteen rows of bf16 leave no registers)
+    constexpr int AS = KEEP || (BF16 && XQ == 4 && TS == 1) ? 1 : 2, AH = KEEP || BF16 ? 1 : 2;
+    float4_t acc[AS][AH] = {};
     auto group = [&](uint32_t i0, const WRows &next, uint32_t n0, auto request) {
 #pragma unroll
         for (int s = 0; s < PD; s++) {
@@ -1534,8 +1553,9 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const uint4 wf = wl[c * 8 + ((4 * h + g) ^ (c >> 1))];
-                    if constexpr (KEEP) acc = MT::mul(wf, kept[s][h], acc);
-                    else acc = MT::mul(wf, x_get(i0 + s, h), acc);
+                    float4_t &sum = acc[s % AS][h % AH];
+                    if constexpr (KEEP) sum = MT::mul(wf, kept[s][h], sum);
+                    else sum = MT::mul(wf, x_get(i0 + s, h), sum);
                 }
             }
             __builtin_amdgcn_wave_barrier();
@@ -1552,21 +1572,24 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
             group(gi * PD, wp, 0, [] { return false; });
         }
         if (ends) {
-            // lane (c, g) holds outputs 16 tile + 4 g .. + 3 of row c; a wave's corner of LDS is free
-            if (c < batch) *(float4_t *)(wl + lane) = acc;
-            acc = float4_t{0.f, 0.f, 0.f, 0.f};
+            // lane (c, g) holds lines 4 g .. + 3 of column c; a wave's corner of LDS is free
+            if (TS > 1 || c < batch) *(float4_t *)(wl + lane) = AS == 1 ? acc[0][0] : BF16 ? acc[0][0] + acc[AS - 1][0] : (acc[0][0] + acc[0][AH - 1]) + (acc[AS - 1][0] + acc[AS - 1][AH - 1]);
+#pragma unroll
+            for (int i = 0; i < AS * AH; i++) acc[i / AH][i % AH] = float4_t{0.f, 0.f, 0.f, 0.f};
             lds_barrier();
-            const uint32_t row = tile * 16 + c;
+            const uint32_t row = tile * R + c;
             for (uint32_t b = wave; b < batch; b += nw) {
-                // lane (c, g) adds output c of every fourth wave
+                // lane (c, g) adds line c of every fourth wave, in the column of its part
                 float sum = 0.f;
                 for (uint32_t v = g; v < nw; v += 4)
-                    sum += ((const float *)(lds + v * mfma_wave_lds<BF16>(XQ) + (c >> 2) * 16 + b))[c & 3];
+                    sum += ((const float *)(lds + v * mfma_wave_lds<BF16>(XQ) + (c >> 2) * 16 + (TS > 1 ? c / R * R : 0) + b))[c & 3];
                 sum = xor32_sum(xor16_sum(sum));
+                if (TS == 4) sum += dpp_f32<DPP_ROW_ROR4>(sum);
+                if (TS >= 2) sum += dpp_f32<DPP_ROW_ROR8>(sum);
                 if (epi_gated(e.act)) {
                     const float up = lane_xor1(sum);
-                    if (g == 0 && (c & 1) == 0 && row + 1 < n) epi_store_gated(e, b, row / 2, sum, up);
-                } else if (g == 0 && row < n) {
+                    if (g == 0 && (TS == 1 || c < R) && (c & 1) == 0 && row + 1 < n) epi_store_gated(e, b, row / 2, sum, up);
+                } else if (g == 0 && (TS == 1 || c < R) && row < n) {
                     epi_store<true>(e, b, row, sum);
                 }
             }
@@ -1702,18 +1725,18 @@ static constexpr uint32_t gemv_fold_share(int norm, uint32_t bp) {
 }
 
 // NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
-template <bool BF16, int BP, int NORM, int PD, bool KEEP>
+template <bool BF16, int BP, int NORM, int PD, bool KEEP, int TS = 1>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
                                                          uint32_t n, uint32_t batch, uint32_t waves, uint32_t grid, EpiArgs e,
                                                          const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
                                                          uint64_t ldx, PostNorm post) {
     extern __shared__ uint4 mlds[];
     typedef typename MfmaType<BF16>::Rows Rows;
-    constexpr int XQ = NORM ? 0 : (BP + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
+    constexpr int XQ = NORM ? 0 : ((TS > 1 ? 16 : BP) + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
     // a folded norm: the split rows first; what its staging needs lies where the corners will be
     const Rows xs{(decltype(Rows::p))mlds, k, (uint32_t)BP};
     uint4 *corners = NORM ? (uint4 *)((char *)mlds + Rows::bytes(BP, k)) : mlds;
-    mfma_rows<BF16, PD, KEEP, XQ>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
+    mfma_rows<BF16, PD, KEEP, XQ, TS>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
         if constexpr (NORM != 0) {
             constexpr uint32_t LONGEST = gemv_fold_row_pairs<BF16>(NORM, BP) * MfmaType<BF16>::KU;
             if (LONGEST <= 1024 || k <= 1024) stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
@@ -1756,7 +1779,8 @@ static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves, bool
     // Two or three rows on few tiles: a wave per row keeps more compute units busy.  f32, 2 rows of 768 x 768 3.4 / 4.0,
     // 8192 x 1024 13.6 / 16.0, 1024 x 1536 4.4 / 4.7, but 1024 x 2304 5.2 / 5.1, 2048 x 1152 6.5 / 6.2; 3 rows of 1024 x 1024 4.3 / 4.5,
     // x 1152 4.9 / 4.6, 64 x 1024 3.1 / 2.9; bf16, 2 rows of 1024 x 256 3.2 / 3.4, but x 1280 3.5 / 3.5, 1536 x 256 4.0 / 3.8.
-    if (!bf && batch <= 3) return w.k <= 256 || (w.n > 1024 && (batch == 3 || w.k > 1024 || w.n > 2048));
+    // Long rows there are dealt in parts of k (3 rows of 8192 x 1024 16.4 / 9.0).
+    if (!bf && batch <= 3) return w.k <= 256 || (w.n <= 1024 && w.k >= 4096 && w.k % 128 == 0) || (w.n > 1024 && (batch == 3 || w.k > 1024 || w.n > 2048));
     if (bf && batch == 2) return w.k <= 256 || w.k > 1024 || w.n > 1024;
     return true;
 }
@@ -1962,7 +1986,7 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
     };
     if constexpr (MF) {
         __builtin_amdgcn_sched_barrier(0);
-        mfma_rows<true, 2, true, 0>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
+        mfma_rows<true, 2, true, 0, 1>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
             __builtin_amdgcn_sched_barrier(0);
             normalise();
         });
@@ -2117,13 +2141,48 @@ static uint32_t gemv_one_row_steps(const Weight &w, uint64_t batch, bool gated) 
     return w.n > 1024 ? 0 : slots(6) <= slots(4) && steps % 4 ? 6 : 4;
 }
 
-// Plain rows on the matrix cores: waves of a workgroup, LDS, and whether they go there.
-struct MfmaPlain { bool runs; uint32_t waves; size_t lds; };
+// Plain rows on the matrix cores: whether they go there, parts of k that a tile's sixteen lines are dealt to, waves of a workgroup, LDS.
+// Parts: as many as leave at most a workgroup per CU, four up to 1024 outputs, two up to 2048; bf16 from lengths on at which a tile's trip
+// is long enough to halve (us, one / two / four parts: 4 rows of 768 x 768 3.5 / 4.0 / 3.7, 1024 x 1024 3.9 / 3.9 / 3.8, 2048 x 2048 4.7 / 4.9 / 5.2, 4096 x 2048
+// 7.6 / 6.8 / 7.1, and four where the shares are two pairs that stay in registers, 5632 x 2048 10.1 / 8.7 / 8.0; 8 rows of 1024 x 1024 4.2 / 4.2, 2048 x
+// 2048 5.6 / 5.2).  Beyond 4096 outputs a CU takes several tiles, and smaller ones even out their number: from 4096 of k on, as long as a wave's share
+// is two pairs (4 rows of bf16 4096 x 4608 12.7 / - / 10.5, x 12352 24.2 / 20.8 / 20.3, f32 4096 x 4608 20.9 / 17.7 / 17.6; but bf16 4096 x 4096 8.4 / 10.4 /
+// 10.0, 8 rows of 6144 x 8192 24.6 / 32.1).
+// Waves: eight of four pairs and more rather than sixteen, two workgroups a CU, one of which asks while the other adds up (us, 16 / 8: 4 rows of bf16
+// 2048 x 6176 8.4 / 7.4, x 2048 5.1 / 4.7, 8 of 2048 x 8192 10.4 / 9.7, but x 11264 12.4 / 13.3, 16 of 2048 x 1024 6.5 / 7.0; f32, 4 of 768 x 3072 4.9 / 4.5,
+// 1024 x 3600 6.1 / 5.3); four of f32 where there are several tiles a CU (16 / 8 / 4: 1024 x 4608 8.3 / 7.3 / 6.6, 2048 x 8192 15.0 / 13.8 / 13.7); three pairs of
+// bf16 a wave where that comes out even, asked for at once (768 x 2304, two / three: 3.83 / 3.60; - x 10272 5.65 / 5.84).
+struct MfmaPlain { bool runs; uint32_t parts, waves; size_t lds; };
 template <bool BF16>
 static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
-    const uint32_t waves = gemv_mfma_waves(std::min<uint64_t>(w.k / MfmaType<BF16>::KU, 1u << 20)), xbp = std::max(pad_batch(batch), 4u);
-    const size_t lds = (size_t)waves * 16 * mfma_wave_lds<BF16>((xbp + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS);
-    return {gemv_uses_mfma(w, batch, waves, false) && lds <= 160 * 1024, waves, lds};
+    const uint32_t xbp = std::max(pad_batch(batch), 4u), most = 16 / xbp;  // (a part needs columns for all rows)
+    auto fits = [&](uint32_t parts) { return parts <= most && w.k % (MfmaType<BF16>::KU * parts) == 0; };
+    uint32_t parts = 1;
+    if (BF16) {
+        if (w.n <= 1024 && w.k >= 1024 && fits(4)) parts = 4;
+        else if (w.n <= 2048 && w.k > 4096 && w.k <= 8192 && fits(4)) parts = 4;
+        else if (w.n > 4096 && w.k >= 4096 && w.k <= 8192 && fits(4)) parts = 4;
+        else if (((w.n <= 2048 && w.k >= (xbp == 8 || w.n <= 1024 ? 2048 : 4096)) || (w.n > 4096 && w.k == 4096)) && fits(2)) parts = 2;
+    } else {
+        if ((w.n <= 1024 || (w.n > 4096 && w.k >= 4096)) && fits(4)) parts = 4;
+        else if ((w.n <= 2048 || (w.n > 4096 && w.k >= 4096)) && fits(2)) parts = 2;
+    }
+    const uint64_t pairs = std::min<uint64_t>(w.k / (MfmaType<BF16>::KU * parts), 1u << 20);
+    uint32_t waves = gemv_mfma_waves(pairs);
+    if (BF16) {
+        if (parts > 1 && pairs > 32) waves = 8;
+        if (parts == 1 && xbp == 4 && pairs % 3 == 0 && pairs >= 9 && pairs <= 24 && w.n <= 8192) waves = (uint32_t)std::max<uint64_t>(waves / 2, pairs / 3);
+        else if (parts == 1 && (xbp == 4 || (xbp == 8 && w.n > 4096 && w.n <= 8192)) && pairs % 8 == 0) waves = std::min(waves, 8u);
+    } else if (xbp < 16 || w.n > 4096) {
+        const uint64_t four = std::max<uint64_t>(4, ceil_div(pairs, 4));
+        if (parts == 1) waves = w.n > 4096 ? 4 : (uint32_t)std::min<uint64_t>(8, four);
+        else if (parts == 2) waves = pairs >= 128 ? 16 : (uint32_t)std::min<uint64_t>(8, four);
+        else waves = (uint32_t)std::min<uint64_t>(16, four);
+        waves = (uint32_t)std::min<uint64_t>(waves, std::max<uint64_t>(1, pairs));
+    }
+    const uint32_t rows = parts > 1 ? 16 : xbp;
+    const size_t lds = (size_t)waves * 16 * mfma_wave_lds<BF16>((rows + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS);
+    return {gemv_uses_mfma(w, batch, waves, false) && lds <= 160 * 1024, parts, waves, lds};
 }
 
 template <bool BF16>
@@ -2177,14 +2236,15 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         const uint32_t mw = nf ? 16u : plain.waves;
         const size_t mlds = nf ? gemv_mfma_norm_lds(w, bp, lds) : plain.lds;
         if (aligned && (nf ? gemv_uses_mfma(w, batch, 16, true) && mlds <= 160 * 1024 : plain.runs)) {
-            const uint32_t tiles = (uint32_t)ceil_div(w.n, 16), np = (pairs + mw - 1) / mw;
+            const uint32_t parts = nf ? 1u : plain.parts, tiles = (uint32_t)ceil_div(w.n, 16 / parts), np = (pairs / parts + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
-#define COEUS_MFMA4(BPV, NV, PV, KV)                                                                                          \
+#define COEUS_MFMA5(BPV, NV, PV, KV, TV)                                                                                      \
     do {                                                                                                                      \
-        static const bool once = [] { (void)hipFuncSetAttribute((const void *)gemv_mfma_kernel<BF16, BPV, NV, PV, KV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); return true; }(); \
+        static const bool once = [] { (void)hipFuncSetAttribute((const void *)gemv_mfma_kernel<BF16, BPV, NV, PV, KV, TV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); return true; }(); \
         (void)once;                                                                                                           \
-        hipLaunchKernelGGL((gemv_mfma_kernel<BF16, BPV, NV, PV, KV>), mgrid, mblock, mlds, st, (const typename MfmaType<BF16>::W *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
+        hipLaunchKernelGGL((gemv_mfma_kernel<BF16, BPV, NV, PV, KV, TV>), mgrid, mblock, mlds, st, (const typename MfmaType<BF16>::W *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
     } while (0)
+#define COEUS_MFMA4(BPV, NV, PV, KV) COEUS_MFMA5(BPV, NV, PV, KV, 1)
             // Pairs in flight: two or three, whichever asks for fewer in vain at the end of a wave's share.  Where that is the
             // same, three for 2 - 4 rows (us for two / three: 4 rows of bf16 5120 x 32000 67.0 / 65.5, 2 of 12288 x 8192 36.5 / 35.0), two
             // for one row (6144 x 512 7.2 / 7.4) and for 8 (6144 x 4096 13.0 / 13.5).  A norm in front fills the first trip, and
@@ -2193,6 +2253,8 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
             // 14.0).
             const uint32_t by2 = (np + 1) / 2 * 2, by3 = (np + 2) / 3 * 3;
             const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && batch > 1 && bp <= 4);
+            // (sixteen lines of bf16 ask for sixteen rows of activations: three pairs of them spill)
+#define COEUS_MFMAP(TV) do { if (np <= 2) COEUS_MFMA5(16 / TV, 0, 2, true, TV); else if (!BF16 && three) COEUS_MFMA5(16 / TV, 0, (BF16 ? 2 : 3), false, TV); else COEUS_MFMA5(16 / TV, 0, 2, false, TV); } while (0)
 #define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (BPV < 16 && three) COEUS_MFMA4(BPV < 16 ? BPV : 8, NV, 3, false); else COEUS_MFMA4(BPV, NV, 2, false); } while (0)
 #define COEUS_MFMAN(BPV, NV)                                                                               \
     do {                                                                                                   \
@@ -2201,7 +2263,9 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         else return fail(COEUS_INVALID_INPUT, "norm fusion needs the normalised activations to fit in LDS"); \
     } while (0)
 #define COEUS_MFMA(BPV) do { if (norm == 4) { if constexpr (!BF16) COEUS_MFMAN(BPV, 4); } else if (norm == 1) COEUS_MFMAN(BPV, 1); else if (norm == 2) COEUS_MFMAN(BPV, 2); else COEUS_MFMAN(BPV, 3); } while (0)
-            if (norm == 0 && bp <= 4) COEUS_MFMA3(4, 0);
+            if (norm == 0 && parts == 4) COEUS_MFMAP(4);
+            else if (norm == 0 && parts == 2) COEUS_MFMAP(2);
+            else if (norm == 0 && bp <= 4) COEUS_MFMA3(4, 0);
             else if (norm == 0 && bp == 8) COEUS_MFMA3(8, 0);
             else if (norm == 0) COEUS_MFMA3(16, 0);
             else if (bp == 2) COEUS_MFMA(2);
@@ -2212,6 +2276,8 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
 #undef COEUS_MFMAN
 #undef COEUS_MFMA3
 #undef COEUS_MFMA4
+#undef COEUS_MFMA5
+#undef COEUS_MFMAP
             COEUS_HIP(hipGetLastError());
             return COEUS_OK;
         }
@@ -2255,7 +2321,7 @@ coeus_matmul_plan gemv_plan(const Weight &w, uint64_t batch) {
     }
     if (gemv_takes_many(w, batch)) return {"gemv_many_kernel", 1, 8, 4, 1, 1};
     const MfmaPlain mp = w.dtype == COEUS_W_BF16 ? gemv_mfma_plain<true>(w, batch) : gemv_mfma_plain<false>(w, batch);
-    if (mp.runs) return {"gemv_mfma_kernel", bp, 16, mp.waves, 1, 1};
+    if (mp.runs) return {"gemv_mfma_kernel", bp, 16 / mp.parts, mp.waves, 1, 1};
     return {"gemv_dense_kernel", bp, 4, 4, 1, 1};
 }
 

@@ -40,6 +40,26 @@ def test_rows_match_float64(orc, dtype, k, n, batch):
         assert (np.abs(wt.gemm(dev(x)) - want) <= bound(x, wd, k)).all()
 
 
+# Tiles of 4 and 8 weight rows whose lines are parts of k: tiles that end inside the matrix, one pair a wave, shares of one, two and more pairs,
+# several tiles a workgroup, gated pairs, and one more row of weights or 64 of k than the rule allows
+@pytest.mark.parametrize("k,n", [(128, 5), (768, 6), (1024, 1022), (1280, 1024), (2816, 1030), (3072, 7), (4096, 4098), (5632, 2046), (6144, 4100), (8192, 1026), (4160, 1000)])
+@pytest.mark.parametrize("batch", [2, 3, 4, 5, 8])
+@pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_F32])
+def test_parts_of_k(orc, dtype, k, n, batch):
+    rng = np.random.default_rng(k + 31 * n + batch)
+    w = (rng.standard_normal((k, n)) * 0.02).astype(np.float32)
+    x = (rng.standard_normal((batch, k)) * np.exp2(rng.integers(-20, 20, (batch, k)))).astype(np.float32)
+    wt, wd = Weight(dtype, w), oracle_roundtrip(orc, dtype, w).astype(np.float64)
+    assert (np.abs(wt.gemv(dev(x)) - x.astype(np.float64) @ wd) <= bound(x, wd, k)).all()
+    if n % 2 == 0:
+        x = rng.standard_normal((batch, k)).astype(np.float32)
+        pre, e = x.astype(np.float64) @ wd, bound(x, wd, k)
+        g, u = pre[:, 0::2], pre[:, 1::2]
+        want = g / (1 + np.exp(-g)) * u
+        lim = 1.1 * (e[:, 0::2] * np.abs(u) + e[:, 1::2] * np.abs(g)) + 2.0 ** -20 * np.abs(want) + 1e-6
+        assert (np.abs(wt.gemv(dev(x), epilogue=_lib.EPI_SILU_GATE) - want) <= lim).all()
+
+
 @pytest.mark.parametrize("dtype,rows", [(_lib.W_F32, 2), (_lib.W_F32, 5), (_lib.W_F32, 16), (_lib.W_F32, 17), (_lib.W_BF16, 5)])
 def test_timed_matmul_is_the_one_that_runs(dtype, rows):
     """What the repeated, timed launches leave is the bits of the plain call: the same kernel, in the same order of sums."""
