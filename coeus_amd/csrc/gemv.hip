@@ -1615,10 +1615,15 @@ __device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__res
     auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
     // (Sums in f64 next to a long row and its scale would spill.  Rows that long are at most eight, so that the last wave,
     // which has none, brings the scale into LDS.)
-    constexpr bool SCALE_LDS = NORM == 4 && VM == 8;
+    constexpr bool SCALE_LDS = NORM == 4 && VM == 8, BIAS = (NORM == 1 || NORM == 4) && VM == 4;  // (the bias of a short row comes with it)
     float *gs = sh + 64;
-    float4_t v[VM], g[SCALE_LDS ? 1 : VM];
+    float4_t v[VM], g[SCALE_LDS ? 1 : VM], bias[BIAS ? VM : 1];
     if (on) {
+        if constexpr (BIAS) {
+            const float *nb = nbias ? nbias : nscale;
+#pragma unroll
+            for (int u = 0; u < VM; u++) bias[u] = *(const float4_t *)(nb + 4 * min(lane + 64 * u, n4 - 1));
+        }
 #pragma unroll
         for (int u = 0; u < VM; u++) v[u] = *(const float4_t *)(row + 4 * min(lane + 64 * u, n4 - 1));
         if constexpr (!SCALE_LDS) {
@@ -1632,37 +1637,31 @@ __device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__res
     }
     float mean = 0.f, rs;
     if constexpr (NORM == 4) {
-        // Whole slice: sums in f64 (as norm_sequence_kernel's, which serves the longer prompts).
+        // Whole slice: sums of x - x[0] and of its square in f64, one trip through LDS (norm_sequence_part_kernel's, which serves the
+        // longer prompts).
         double *shd = (double *)sh, sum = 0.0, sq = 0.0;
-        if (on) {
-#pragma unroll
-            for (int u = 0; u < VM; u++) {
-                if (lane + 64 * u < n4) sum += ((double)v[u][0] + v[u][1]) + ((double)v[u][2] + v[u][3]);
-                __builtin_amdgcn_sched_barrier(0);  // (converted all at once, the row spills)
-            }
-            sum = wave_sum_f64(sum);
-            if (lane == 0) shd[b] = sum;
-        }
-        __syncthreads();
-        const double inv = inv_count(k * batch), m = wave_sum_f64(lane < batch ? shd[lane] : 0.0) * inv;
+        const double ref = x[0];
         if (on) {
 #pragma unroll
             for (int u = 0; u < VM; u++) {
                 if (lane + 64 * u < n4)
 #pragma unroll
                     for (int t = 0; t < 4; t++) {
-                        const double d = v[u][t] - m;
+                        const double d = v[u][t] - ref;
+                        sum += d;
                         sq = fma(d, d, sq);
                     }
-                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_sched_barrier(0);  // (converted all at once, the row spills)
             }
+            sum = wave_sum_f64(sum);
             sq = wave_sum_f64(sq);
-            if (lane == 0) shd[16 + b] = sq;
+            if (lane == 0) { shd[b] = sum; shd[16 + b] = sq; }
         }
         __syncthreads();
         if (!on) return;
-        mean = (float)m;
-        rs = whole_norm_rs(wave_sum_f64(lane < batch ? shd[16 + lane] : 0.0) * inv, eps);
+        const double inv = inv_count(k * batch), off = wave_sum_f64(lane < batch ? shd[lane] : 0.0) * inv;
+        mean = (float)(ref + off);
+        rs = whole_norm_rs(fma(-off, off, wave_sum_f64(lane < batch ? shd[16 + lane] : 0.0) * inv), eps);
     } else {
         if (!on) return;
         if (NORM == 1) {
@@ -1697,7 +1696,8 @@ __device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__res
             if (blockIdx.x == 0) *(float4_t *)(post.h_out + (uint64_t)b * k + i) = o;
         } else {
             float4_t bi = {0.f, 0.f, 0.f, 0.f};
-            if (NORM != 2 && nbias) bi = *(const float4_t *)(nbias + i);
+            if constexpr (BIAS) { if (nbias) bi = bias[u]; }
+            else if (NORM != 2 && nbias) bi = *(const float4_t *)(nbias + i);
 #pragma unroll
             for (int t = 0; t < 4; t++) o[t] = gu[t] * (v[u][t] - mean) * rs + bi[t];
         }
@@ -1787,7 +1787,7 @@ static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves, bool
 // Waves of a plain launch: as many as have two pairs of chunks each.
 static uint32_t gemv_mfma_waves(uint64_t pairs) { return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, (pairs + 1) / 2)); }
 bool gemv_takes_f32_rows(const Weight &w, uint64_t rows) {
-    return w.dtype == COEUS_W_F32 && rows >= 2 && rows <= 16 && (rows > 3 || w.n > 63 * 16) && gemv_mfma_shape(w, gemv_mfma_waves(w.k / 32));
+    return w.dtype == COEUS_W_F32 && rows >= 2 && rows <= 16 && gemv_mfma_shape(w, gemv_mfma_waves(w.k / 32));
 }
 static size_t gemv_mfma_norm_lds(const Weight &w, uint32_t bp, size_t staging) {
     const bool bf = w.dtype == COEUS_W_BF16;

@@ -99,3 +99,24 @@ def test_whole_slice_far_from_zero(orc, hidden, rows):
     # a mean that is off by one f32 step (6e-5 of values that spread by 0.5) moves every normalised value by 1.2e-4;
     # f32 sums of the matmuls: a few 1e-7
     assert np.abs(model.forward_all(ids) - want).max() <= 5e-6 * np.abs(want).max()
+
+
+# Attention of 1 - 15 new rows per sequence, a workgroup per row and head: alone, behind cached keys on both sides of one trip of the waves (64 and 128
+# keys of 64 in f32 and 16 bits, 32 and 64 of 128) and of many
+@pytest.mark.parametrize("heads,hd", [(2, 64), (3, 128)])
+@pytest.mark.parametrize("kv", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("first,n,batch", [(0, 1, 2), (0, 2, 1), (0, 15, 3), (17, 15, 1), (18, 15, 2), (50, 14, 1), (58, 7, 1), (114, 14, 2), (115, 14, 1), (300, 9, 1)])
+def test_few_rows_behind_cached_keys(orc, heads, hd, kv, first, n, batch):
+    kw = dict(hidden_dim=heads * hd, num_layers=2, num_heads=heads, intermediate_dim=4 * hd, vocab_size=130, max_seq_len=first + n, norm_scope="token")
+    oc = orc.config_from_kwargs(kw)
+    params = orc.init_seeded(oc, n)
+    model = TransformerModelPlugin().create_builder().build(Transformer250MConfig(**kw, kv_dtype=kv, max_batch=3), parameters=params)
+    ids = np.random.default_rng(n + hd).integers(0, 130, (batch, first + n), dtype=np.uint64)
+    s = model.session(batch=batch, max_ctx=first + n)
+    if first:
+        s.prefill(ids[:, :first], want_logits=False)
+    got = s.prefill(ids[:, first:])
+    tol = {"f32": 2e-5, "bf16": 2e-2, "f16": 3e-3}[kv]  # (f32 sums over two layers; keys and values of 2^-9 and 2^-12 each)
+    for b in range(batch):
+        want = f64_model.forward_all(oc, params, ids[b])[-1]
+        assert np.abs(got[b] - want).max() <= tol * np.abs(want).max(), b
