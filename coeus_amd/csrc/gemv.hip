@@ -1396,11 +1396,12 @@ struct PlainRows {  // f32 weights
 // four 16x16x4 products per 16-byte piece.
 template <bool BF16> struct MfmaType;
 template <> struct MfmaType<true> {
+    struct Frag { uint4 p[3]; };
+    static __device__ __forceinline__ void mul(const uint4 &, const Frag &, float4_t &, float4_t &) {}  // (f32 only)
     typedef uint16_t W;
     typedef SplitRows Rows;
     static constexpr uint32_t KU = 64;
     static constexpr int PIECES = 3, XROWS = 4;  // rows of x that a wave request covers
-    struct Frag { uint4 p[3]; };
     static __device__ __forceinline__ float4_t mul(const uint4 &w, const Frag &x, float4_t acc) {
         union { uint4 u; bf16x8_t v; } uw, ux;
         uw.u = w;
@@ -1423,6 +1424,15 @@ template <> struct MfmaType<false> {
         uw.u = w;
         ux.u = x.p[0];
         return mfma4(uw.v, ux.v, acc);
+    }
+    static __device__ __forceinline__ void mul(const uint4 &w, const Frag &x, float4_t &a, float4_t &b) {
+        union { uint4 u; float4_t v; } uw, ux;
+        uw.u = w;
+        ux.u = x.p[0];
+        a = __builtin_amdgcn_mfma_f32_16x16x4f32(uw.v[0], ux.v[0], a, 0, 0, 0);
+        b = __builtin_amdgcn_mfma_f32_16x16x4f32(uw.v[1], ux.v[1], b, 0, 0, 0);
+        a = __builtin_amdgcn_mfma_f32_16x16x4f32(uw.v[2], ux.v[2], a, 0, 0, 0);
+        b = __builtin_amdgcn_mfma_f32_16x16x4f32(uw.v[3], ux.v[3], b, 0, 0, 0);
     }
 };
 // uint4 of a wave's corner: 16 weight rows x 128 bytes; per request of x its rows' KU values in pieces
@@ -1533,10 +1543,17 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
             __builtin_amdgcn_wave_barrier();
         }
     }
-    // (every second pair adds up in accumulators of its own, f32's halves of one too: few waves' sums are no longer than many's)
-    // (not shares of two pairs, and not where sixteen rows of bf16 leave no registers)
-    constexpr int AS = KEEP || (BF16 && XQ == 4 && TS == 1) ? 1 : 2, AH = KEEP || BF16 ? 1 : 2;
+    // Every second pair adds up in accumulators of its own, f32's halves of one too, so that few waves' sums are no longer than many's: not
+    // shares of two pairs, and not where sixteen rows of bf16 leave no registers.  f32 in four parts: the quarters of both pairs, which
+    // makes two or three rows as exact as a wave per row (768 x 768, error to that form's 1.04 with halves, 0.94 so; 1.6 with one).
+    constexpr int AS = (KEEP && (BF16 || TS < 4)) || (BF16 && XQ == 4 && TS == 1) ? 1 : 2, AH = (KEEP && TS < 4) || BF16 ? 1 : KEEP ? 4 : 2;
     float4_t acc[AS][AH] = {};
+    auto total = [&]() {
+        float4_t t[AS];
+#pragma unroll
+        for (int s = 0; s < AS; s++) t[s] = AH == 4 ? (acc[s][0] + acc[s][AH / 4]) + (acc[s][AH / 2] + acc[s][AH - 1]) : AH == 2 ? acc[s][0] + acc[s][AH - 1] : acc[s][0];
+        return AS == 2 ? t[0] + t[AS - 1] : t[0];
+    };
     auto group = [&](uint32_t i0, const WRows &next, uint32_t n0, auto request) {
 #pragma unroll
         for (int s = 0; s < PD; s++) {
@@ -1554,7 +1571,8 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
                 for (int h = 0; h < 2; h++) {
                     const uint4 wf = wl[c * 8 + ((4 * h + g) ^ (c >> 1))];
                     float4_t &sum = acc[s % AS][h % AH];
-                    if constexpr (KEEP) sum = MT::mul(wf, kept[s][h], sum);
+                    if constexpr (AH == 4) MT::mul(wf, kept[s][h], acc[s][2 * h], acc[s][2 * h + 1]);
+                    else if constexpr (KEEP) sum = MT::mul(wf, kept[s][h], sum);
                     else sum = MT::mul(wf, x_get(i0 + s, h), sum);
                 }
             }
@@ -1573,7 +1591,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
         }
         if (ends) {
             // lane (c, g) holds lines 4 g .. + 3 of column c; a wave's corner of LDS is free
-            if (TS > 1 || c < batch) *(float4_t *)(wl + lane) = AS == 1 ? acc[0][0] : BF16 ? acc[0][0] + acc[AS - 1][0] : (acc[0][0] + acc[0][AH - 1]) + (acc[AS - 1][0] + acc[AS - 1][AH - 1]);
+            if (TS > 1 || c < batch) *(float4_t *)(wl + lane) = total();
 #pragma unroll
             for (int i = 0; i < AS * AH; i++) acc[i / AH][i % AH] = float4_t{0.f, 0.f, 0.f, 0.f};
             lds_barrier();
@@ -1776,11 +1794,11 @@ static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves, bool
     // (A norm in front costs a wave per row more: f32, 2 rows of 768 x 768 7.4 / 5.8.  Two rows of bf16 are the exception where they
     // are long and few: 2560 x 4096 11.0 / 11.6, x 12288 22.7 / 19.1.)
     if (folded) return !(bf && batch == 2 && w.k > 2048 && w.n <= 4096);
-    // Two or three rows on few tiles: a wave per row keeps more compute units busy.  f32, 2 rows of 768 x 768 3.4 / 4.0,
-    // 8192 x 1024 13.6 / 16.0, 1024 x 1536 4.4 / 4.7, but 1024 x 2304 5.2 / 5.1, 2048 x 1152 6.5 / 6.2; 3 rows of 1024 x 1024 4.3 / 4.5,
-    // x 1152 4.9 / 4.6, 64 x 1024 3.1 / 2.9; bf16, 2 rows of 1024 x 256 3.2 / 3.4, but x 1280 3.5 / 3.5, 1536 x 256 4.0 / 3.8.
-    // Long rows there are dealt in parts of k (3 rows of 8192 x 1024 16.4 / 9.0).
-    if (!bf && batch <= 3) return w.k <= 256 || (w.n <= 1024 && w.k >= 4096 && w.k % 128 == 0) || (w.n > 1024 && (batch == 3 || w.k > 1024 || w.n > 2048));
+    // Two or three rows on few tiles: a wave per row keeps more compute units busy, unless the tiles are dealt in parts of k (f32 up to 1024 outputs, with
+    // sums as near to 64 bits: 3 rows of 768 x 768 4.3 / 3.6, 8192 x 1024 16.6 / 8.6).  f32, 2 rows of
+    // 1024 x 1536 4.4 / 4.7, but 1024 x 2304 5.2 / 5.1, 2048 x 1152 6.5 / 6.2; 3 rows of 1024 x
+    // 1152 4.9 / 4.6; bf16, 2 rows of 1024 x 256 3.2 / 3.4, but x 1280 3.5 / 3.5, 1536 x 256 4.0 / 3.8.
+    if (!bf && batch <= 3) return w.k <= 256 || (w.n <= 1024 ? w.k % 128 == 0 : batch == 3 || w.k > 1024 || w.n > 2048);
     if (bf && batch == 2) return w.k <= 256 || w.k > 1024 || w.n > 1024;
     return true;
 }
@@ -2163,7 +2181,7 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
         else if (w.n <= 2048 && w.k > 4096 && w.k <= 8192 && fits(4)) parts = 4;
         else if (w.n > 4096 && w.k >= 4096 && w.k <= 8192 && fits(4)) parts = 4;
         else if (((w.n <= 2048 && w.k >= (xbp == 8 || w.n <= 1024 ? 2048 : 4096)) || (w.n > 4096 && w.k == 4096)) && fits(2)) parts = 2;
-    } else {
+    } else if (w.k >= 256) {
         if ((w.n <= 1024 || (w.n > 4096 && w.k >= 4096)) && fits(4)) parts = 4;
         else if ((w.n <= 2048 || (w.n > 4096 && w.k >= 4096)) && fits(2)) parts = 2;
     }
@@ -2177,7 +2195,7 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
         const uint64_t four = std::max<uint64_t>(4, ceil_div(pairs, 4));
         if (parts == 1) waves = w.n > 4096 ? 4 : (uint32_t)std::min<uint64_t>(8, four);
         else if (parts == 2) waves = pairs >= 128 ? 16 : (uint32_t)std::min<uint64_t>(8, four);
-        else waves = (uint32_t)std::min<uint64_t>(16, four);
+        else waves = (uint32_t)(pairs <= 12 ? std::max<uint64_t>(4, ceil_div(pairs, 2)) : std::min<uint64_t>(16, four));
         waves = (uint32_t)std::min<uint64_t>(waves, std::max<uint64_t>(1, pairs));
     }
     const uint32_t rows = parts > 1 ? 16 : xbp;

@@ -58,11 +58,10 @@ def test_few_long_rows_of_bf16(k, n, kernel):
     assert plan(_lib.W_BF16, k, n, 1).kernel == kernel
 
 
-# Several rows on few outputs: tiles of 4 or 8 weight rows, sixteen lines of parts of k (f32 3072 x 768, 4 rows 8.3 us with tiles of 16, 5.1 so); f32 of two
-# or three rows stay with a wave per row up to 1024 outputs of less than 4096
+# Several rows on few outputs: tiles of 4 or 8 weight rows, sixteen lines of parts of k (f32 3072 x 768, 4 rows 8.3 us with tiles of 16, 5.1 so)
 @pytest.mark.parametrize("dtype,k,n,rows,cols,waves", [
     (_lib.W_F32, 768, 768, 4, 4, 4), (_lib.W_F32, 3072, 768, 4, 4, 6), (_lib.W_F32, 3072, 768, 5, 8, 8), (_lib.W_F32, 3072, 768, 9, 16, 16), (_lib.W_F32, 8192, 1024, 4, 4, 16),
-    (_lib.W_F32, 8192, 2048, 8, 8, 16), (_lib.W_F32, 2048, 2048, 2, 8, 8), (_lib.W_F32, 2048, 2049, 4, 16, 8), (_lib.W_F32, 1024, 4608, 4, 16, 4), (_lib.W_F32, 4096, 1024, 3, 4, 8),
+    (_lib.W_F32, 8192, 2048, 8, 8, 16), (_lib.W_F32, 2048, 2048, 2, 8, 8), (_lib.W_F32, 2048, 2049, 4, 16, 8), (_lib.W_F32, 1024, 4608, 4, 16, 4), (_lib.W_F32, 4096, 1024, 3, 4, 8), (_lib.W_F32, 768, 768, 2, 4, 4), (_lib.W_F32, 1536, 1024, 3, 4, 6), (_lib.W_F32, 128, 768, 2, 16, 4),
     (_lib.W_F32, 96, 700, 4, 16, 3), (_lib.W_BF16, 768, 768, 4, 16, 4), (_lib.W_BF16, 1024, 1024, 4, 4, 2), (_lib.W_BF16, 1024, 1024, 5, 16, 8), (_lib.W_BF16, 3072, 768, 4, 4, 6),
     (_lib.W_BF16, 3072, 768, 8, 8, 12), (_lib.W_BF16, 5632, 2048, 4, 4, 11), (_lib.W_BF16, 5632, 2048, 5, 8, 8), (_lib.W_BF16, 4096, 2048, 4, 8, 16), (_lib.W_BF16, 2048, 10272, 4, 16, 8),
     (_lib.W_BF16, 4096, 12352, 4, 4, 8), (_lib.W_BF16, 4096, 12352, 5, 8, 16), (_lib.W_BF16, 8192, 8192, 4, 4, 16), (_lib.W_BF16, 8192, 8192, 8, 16, 8), (_lib.W_BF16, 11008, 4096, 4, 16, 16),
