@@ -175,7 +175,7 @@ struct Epilogue {
     // [rows][ceil(n/16)] for the norm folded into the next matmul (see NormFuse::stats)
     float2 *stats_out = nullptr;
     // ... and, for a root-mean-square norm, the stored values times that norm's scale (NormFuse::g):
-    // g_out[row * n + j] = value * g_scale[j].  Batches of up to 4 (gemv_quad_kernel) only.
+    // g_out[row * n + j] = value * g_scale[j].  Batches of up to 4 only (gemv_quad_kernel, whatever the size).
     const float *g_scale = nullptr;
     float *g_out = nullptr;
     LpOut out_lp;                    // prefill matmul: 16-bit copy of the output (out_f32 nullable then)
@@ -214,6 +214,7 @@ struct NormFuse {
 // True when launch_gemv can take `nf` for this weight and batch (quantised weights whose whole
 // activation block fits in LDS).
 bool gemv_can_fuse_norm(const Weight &w, uint64_t batch);
+bool gemv_norm_apart(const Weight &w, uint64_t batch);  // it can, and a launch of its own is faster
 // The same for f32 / bf16 weights (the normalised block [batch, k] f32 has to fit in LDS; the
 // statistics are computed inside the launch, NormFuse::stats is not used).
 bool gemv_can_fuse_norm_dense(const Weight &w, uint64_t batch);

@@ -1,12 +1,12 @@
 // Decode matmul: y[b, :] = x[b, :] . W for b < batch <= 16 (math::matmul, MT:50-74, with
 // m = batch), the HBM-bound kernel of token generation.
 //
-//   gemv_quad_kernel   Q8_0 / Q4_0 weights in MFMA-native tiles, batches of up to 4 (the kernel of
-//                      single-sequence generation): one workgroup per tile of 16 output rows, a
+//   gemv_quad_kernel   Q8_0 / Q4_0 weights in MFMA-native tiles, batches of 1 and 2 and some of 3 and 4 (the
+//                      kernel of single-sequence generation): one workgroup per tile of 16 output rows, a
 //                      wave owns four consecutive 128-k chunks, stages exactly their activations
 //                      (with or without the folded norm) into its private slice of LDS and feeds
 //                      the quants to v_mfma_f32_16x16x32_f16 as f16 subnormals.
-//   gemv_rows_kernel   the same weights for batches of 5 to 16.  One workgroup owns one to six tiles
+//   gemv_rows_kernel   the same weights for batches of 3 to 16.  One workgroup owns one to six tiles
 //                      of 16 output rows; its waves take 128-k chunks (1 KiB of Q4_0 quants = one
 //                      fully coalesced 16 B/lane load per wave).  Each 32-k block is one
 //                      v_mfma_f32_16x16x32_f16 between the 16 activation rows (f16, straight from
@@ -114,8 +114,8 @@ struct XArgs {
     uint32_t k;           // logical reduction length
 };
 
-// The same normalisation as a launch of its own, for all batches of 5 to 16 (and of up to 4 whose rows do not fit
-// gemv_quad_kernel's LDS): row b of h -> xq, statistics merged from the producer's records
+// The same normalisation as a launch of its own, for all batches of 5 to 16 (and of 3 and 4 on wide rows, and of up to 4
+// whose rows do not fit gemv_quad_kernel's LDS): row b of h -> xq, statistics merged from the producer's records
 // (no reduction over the row).  Grid (k pieces / 256, batch); every wave merges its row's records.
 // Bound by one trip to memory behind the launch: everything is requested at once, and the wave's sums are register moves.
 template <bool RMS>
@@ -197,7 +197,7 @@ int launch_norm_from_stats(const NormFuse &nf, uint64_t batch, uint64_t k, uint6
     return COEUS_OK;
 }
 
-// ---------------------------------------------------------------- batches of 5 to 16
+// ---------------------------------------------------------------- batches of 3 to 16
 // Bound by the trips to memory that a wave makes one behind the other and, for long reductions, by the activation rows
 // that every workgroup reads from L2 (16 rows x 11008 x 2 B = 352 KB next to 99 KB of Q4_0 weights).  So nothing is staged:
 // a wave asks for the four activation fragments of its chunk and for the chunk's weights in its TPW tiles at once, 16 bytes
@@ -211,11 +211,15 @@ int launch_norm_from_stats(const NormFuse &nf, uint64_t batch, uint64_t k, uint6
 // staged in LDS where they fit in 48 KiB, two to six chunks a wave in flight, sums and epilogue on one wave a tile):
 //   16 rows, Q4_0: 4096 x 12288 14.2 -> 11.8, 4096 x 4096 9.2 -> 8.6, 4096 x 22016 gated 20.9 -> 16.3, 11008 x 4096 15.6 -> 14.3
 //    8 rows, Q8_0: 768 x 2304 6.8 -> 6.0, 768 x 768 7.6 -> 6.0, 768 x 3072 7.2 -> 6.5, 3072 x 768 9.1 -> 7.2, 768 x 50257 14.4 -> 12.6
+// 3 and 4 rows (before: gemv_quad_kernel, whose offset term costs every row as much as the products do, and whose sums cancel it: error
+// against 64 bits 2.3e-6 of the result for Q4_0 and 2-7e-7 for Q8_0, 6e-8 - 1.1e-7 so), 4 rows, Q4_0: 4096 x 22016 20.6 -> 15.2, 11008 x 4096
+// 15.1 -> 12.5, 8192 x 2048 10.3 -> 9.5, 2048 x 8192 7.8 -> 6.9, 2048 x 32000 15.2 -> 12.7; Q8_0: 11008 x 4096 16.3 -> 14.1, 4096 x 12288 15.1
+// -> 13.8.  Two chunks of a wave in flight instead of one changed nothing (11008 x 4096 12.2 and 13.0, 8192 x 2048 9.2 and 9.5 us).
 template <bool Q4, int BP, int TPW>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds, const uint4 *__restrict__ xq, uint32_t ngroups,
                       uint32_t tiles, uint32_t batch, EpiArgs e) {
-    static_assert(BP == 8 || BP == 16, "batches of up to 4 take gemv_quad_kernel");
+    static_assert(BP == 4 || BP == 8 || BP == 16, "batch padded to 4, 8 or 16");
     extern __shared__ float rows_red[];  // [TPW][nwaves][4][64]
     const uint32_t lane = threadIdx.x & 63, nwaves = blockDim.x >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -326,7 +330,7 @@ void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds
 }
 
 // ---------------------------------------------------------------- quad kernel (batches of up to 4)
-// The decode matmul for batch <= 4, where a launch is a transient: the whole matrix (10-70 MB) is
+// The decode matmul for batches of 1 and 2, and of 3 and 4 where gemv_takes_rows says no, where a launch is a transient: the whole matrix (10-70 MB) is
 // requested within the first microsecond and the kernel ends when the last line has arrived, so
 // what counts is that every wave asks for its weights at once, that as few other bytes as possible
 // go through the CU's memory pipeline, and that little is left to do after the last line.  A wave
@@ -697,6 +701,12 @@ bool gemv_can_fuse_norm(const Weight &w, uint64_t batch) {
            (bp < 4 || w.k <= 16u * 64u * 4u);
 }
 
+// Batches of 3 and 4, the norm as a launch of its own in front of gemv_rows_kernel instead of folded into gemv_quad_kernel, whose
+// four rows every workgroup normalises again.  Decode steps of 4 sequences, ms for 24 - 32 of them, folded / apart: 1B (2048 wide, 24 layers)
+// Q4_0 45.6 / 43.6 with the prompt, 7B (4096) 48.75 / 44.2 with the prompt; 12 layers of 1536 Q4_0 15.3 / 14.4, Q8_0 15.2 / 14.8, of 1024
+// Q4_0 13.3 / 13.2, Q8_0 13.3 / 13.2 (no difference), of 768 Q8_0 11.5 / 12.1.
+bool gemv_norm_apart(const Weight &w, uint64_t batch) { return w.dtype >= COEUS_W_Q8_0 && batch > 2 && w.k >= 1536; }
+
 struct GemvLaunch {
     dim3 grid, block;
     size_t lds;
@@ -739,7 +749,7 @@ static bool quad_launch_bp(int xmode, uint32_t qpw, uint32_t srec, const GemvLau
     return false;
 }
 
-// Batches of up to 4: gemv_quad_kernel, one workgroup per tile of 16 rows.  A wave takes quads of
+// Batches of up to 4 that gemv_takes_rows leaves: gemv_quad_kernel, one workgroup per tile of 16 rows.  A wave takes quads of
 // four chunks; with a folded norm one quad per wave and as many waves as the reduction has quads;
 // plain activations: one or two quads in flight per wave, several passes when 16 waves do not cover
 // k that way.
@@ -796,7 +806,18 @@ static int launch_gemv_quad(const Weight &w, const __half *xq, uint64_t batch, c
     return COEUS_OK;
 }
 
-// Batches of 5 to 16: tiles and waves of a workgroup of gemv_rows_kernel.  Every workgroup reads all activation rows, so it
+// Batches of 3 and 4, rows as they are: gemv_rows_kernel or gemv_quad_kernel.  Over 185 sizes (512 - 14336 by 256 - 32000; 3 and 4 rows
+// alike) the former took, as a share of the latter's time: Q4_0 0.67 - 0.98 everywhere; Q8_0 0.79 - 0.95 on more than 256 tiles (a workgroup
+// takes several) and 0.87 - 0.94 up to k = 1024, 2560 - 3072 0.90 - 0.95, beyond 8192 (several passes of the quads) 0.83 - 0.98, but
+// 1.0 at 1536 and 2048 and 1.01 - 1.10 at 4096 - 8192 on up to 256 tiles, where the quads are one pass of 8 - 16 waves and the launch is a
+// single trip.  Narrow rows (k < 1024) belong to models whose norms stay folded, and stay with that kernel.
+static bool gemv_takes_rows(const Weight &w, uint64_t batch) {
+    if (batch > 4) return true;
+    if (batch < 3 || w.k < 1024) return false;
+    return w.dtype == COEUS_W_Q4_0 || w.n_pad / 16 > 256 || w.k <= 1024 || (w.k > 2048 && w.k <= 3072) || w.k > 8192;
+}
+
+// Batches of 3 to 16: tiles and waves of a workgroup of gemv_rows_kernel.  Every workgroup reads all activation rows, so it
 // takes as many tiles as leave about a workgroup per CU, six at most (Q8_0 four: registers), else two workgroups per CU;
 // waves as many as share the reduction in few trips.  Measured for 8 and 16 rows over 35 matrices of 768 - 5120 wide models
 // with 1 - 6 tiles and 2 - 16 waves; the choice is within 4 % of the best of them (4096 x 22016, 16 rows, Q4_0: six tiles 15.9,
@@ -804,7 +825,8 @@ static int launch_gemv_quad(const Weight &w, const __half *xq, uint64_t batch, c
 // Few chunks (k <= 512) are few waves, and the outputs of several tiles are more than these finish at once: one tile, a wave per chunk, as long
 // as the activations are next to nothing, else two; six tiles only from nine chunks on.  Q4_0, 16 rows, us with as many tiles as above / so: 64 x
 // 16400 12.9 / 6.3, x 100000 10.5 / 9.9, 256 x 16400 10.2 / 6.3, x 33000 9.6 / 8.1, 512 x 16400 8.8 / 6.8, x 50257 10.9 / 10.2, 768 x 16400
-// 9.3 / 8.0.  400 sizes with 1 - 6 tiles and 1 - 16 waves: 1.3 % above the best of them on average.
+// 9.3 / 8.0.  400 sizes with 1 - 6 tiles and 1 - 16 waves: 1.3 % above the best of them on average.  (4 rows, 22 sizes: within 3 % of the
+// best too, 4096 x 12288 Q4_0 7 %.)
 static void gemv_rows_shape(bool q4, uint32_t ngroups, uint32_t tiles, uint32_t &tpw, uint32_t &waves) {
     if (ngroups <= 4 && tiles > 256) {
         tpw = ngroups == 1 || tiles <= (ngroups == 2 ? 2048 : 1536) ? 1 : 2;
@@ -841,8 +863,9 @@ static int launch_gemv_rows(const Weight &w, const __half *xq, uint32_t batch, u
 template <bool Q4>
 static int launch_gemv_quant(const Weight &w, const __half *xq, uint64_t batch, const EpiArgs &e,
                              hipStream_t st, const NormFuse *nf) {
-    if (pad_batch(batch) <= 4) return launch_gemv_quad<Q4>(w, xq, batch, e, st, nf);
-    // batches of 5 to 16: gemv_rows_kernel on staged f16 activations (the norm is a launch of its own)
+    // (a folded norm and a pre-scaled copy of the output are gemv_quad_kernel's)
+    if (pad_batch(batch) <= 4 && (nf || e.g_out || !gemv_takes_rows(w, batch))) return launch_gemv_quad<Q4>(w, xq, batch, e, st, nf);
+    // gemv_rows_kernel on staged f16 activations (the norm is a launch of its own)
     if (nf) return fail(COEUS_INVALID_INPUT, "norm fusion is for batches of up to 4");
     if (e.stats_out && e.act == COEUS_EPI_SILU_GATE)
         return fail(COEUS_INVALID_INPUT, "statistics records are not produced by the gated epilogue");
@@ -859,7 +882,11 @@ static int launch_gemv_quant(const Weight &w, const __half *xq, uint64_t batch, 
         }
         return fail(COEUS_INVALID_INPUT, "decode matmul: no kernel for %u tiles a workgroup", tpw);
     };
-    return pad_batch(batch) == 8 ? with(std::integral_constant<int, 8>{}) : with(std::integral_constant<int, 16>{});
+    switch (pad_batch(batch)) {
+        case 4: return with(std::integral_constant<int, 4>{});
+        case 8: return with(std::integral_constant<int, 8>{});
+        default: return with(std::integral_constant<int, 16>{});
+    }
 }
 
 // ---------------------------------------------------------------- dense kernel (f32 / bf16)
@@ -2332,7 +2359,7 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
 coeus_matmul_plan gemv_plan(const Weight &w, uint64_t batch) {
     const uint32_t bp = pad_batch(batch);
     if (w.dtype >= COEUS_W_Q8_0) {
-        if (bp <= 4) return {"gemv_quad_kernel", bp, 16, 0, 1, 1};
+        if (!gemv_takes_rows(w, batch)) return {"gemv_quad_kernel", bp, 16, 0, 1, 1};
         uint32_t tpw, waves;
         gemv_rows_shape(w.dtype == COEUS_W_Q4_0, (uint32_t)(w.k_pad / 128), (uint32_t)(w.n_pad / 16), tpw, waves);
         return {"gemv_rows_kernel", bp, 16 * tpw, waves, 1, 1};

@@ -786,7 +786,7 @@ static int enqueue_decode_step(Session &s, hipStream_t st, int only = STEP_ALL,
     // Root-mean-square norms folded into the next matmul: the producers of h also store
     // h * scale of the norm that follows (Epilogue::g_out), which is what that matmul stages.
     const bool gpath = stats && c.norm == COEUS_NORM_RMSNORM && gemv_can_fuse_norm(m.layers[0].qkv, B) &&
-                       gemv_can_fuse_norm(m.layers[0].up, B) && gemv_can_fuse_norm(m.out, B);
+                       gemv_can_fuse_norm(m.layers[0].up, B) && gemv_can_fuse_norm(m.out, B) && !gemv_norm_apart(m.out, B);
     float *xq_g = gpath ? (float *)s.xq_g.p : nullptr;
     if (m.stack) {
         if (!matmuls_only)
@@ -805,7 +805,7 @@ static int enqueue_decode_step(Session &s, hipStream_t st, int only = STEP_ALL,
     auto normed_gemv = [&](const Weight &w, const float *ns, const float *nb, const Epilogue &e) -> int {
         if (!with_matmuls) return COEUS_OK;
         n_launch++;
-        if (quant && s.fuse && gemv_can_fuse_norm(w, B)) {
+        if (quant && s.fuse && gemv_can_fuse_norm(w, B) && !gemv_norm_apart(w, B)) {
             NormFuse nf;
             nf.h = h; nf.scale = ns; nf.bias = nb; nf.eps = c.layer_norm_eps; nf.kind = c.norm;
             nf.stats = stats;

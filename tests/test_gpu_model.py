@@ -286,6 +286,32 @@ def test_session_large_batches_against_oracle(orc, B, wd, kv, norm, gated):
     model.close()
 
 
+@pytest.mark.parametrize("wd,norm,gated", [("q4_0", "layernorm", False), ("q4_0", "rmsnorm", True), ("q8_0", "rmsnorm", False), ("q8_0", "layernorm", True)])
+@pytest.mark.parametrize("B", [3, 4])
+def test_session_of_few_wide_sequences_against_oracle(orc, B, wd, norm, gated):
+    """Batches of 3 and 4 on rows of 1536 and more: the norms are launches of their own and the matmuls the kernel of batches of 5
+    to 16; q|k|v goes into the cache, records and the residual through its epilogue.  Same bars as the larger batches."""
+    cfg = small(hidden_dim=1536, num_heads=3, head_dim=64, intermediate_dim=320, num_layers=2, norm_scope="token", weight_dtype=wd, kv_dtype="f16",
+                norm=norm, activation="silu_gated" if gated else "gelu", use_bias=not gated, max_batch=4)
+    oc = orc_cfg(orc, cfg)
+    params = orc.init_seeded(oc, 700 + B)
+    pq = orc.apply_weight_dtype(oc, params)
+    n, steps = 5, 3
+    ids = orc.synth_ids(701 + B, cfg.vocab_size, B * (n + steps)).reshape(B, n + steps)
+    model = build(cfg, params)
+    sb = model.session(batch=B, max_ctx=40)
+    lb = [sb.prefill(ids[:, :n])] + [sb.decode(ids[:, n + t]) for t in range(steps)]
+    for b in range(B):
+        want = orc.forward(oc, pq, ids[b], all_rows=True)[2]
+        s1 = model.session(batch=1, max_ctx=40)
+        l1 = [s1.prefill(ids[b, :n])] + [s1.decode(ids[b, n + t:n + t + 1]) for t in range(steps)]
+        s1.close()
+        for t in range(steps + 1):
+            assert rel_err(lb[t][b], want[n - 1 + t]) < 2e-2 and rel_err(lb[t][b], l1[t][0]) < 2e-3, (b, t)
+    sb.close()
+    model.close()
+
+
 @pytest.mark.parametrize("heads,hd,wd,kv", [(2, 128, "q4_0", "f16"), (2, 128, "bf16", "bf16"),
                                             (4, 64, "q8_0", "bf16"), (4, 64, "f32", "f16")])
 def test_decode_attention_many_splits_against_oracle(orc, heads, hd, wd, kv):

@@ -502,6 +502,25 @@ def test_gemv_rows_shapes(orc, dtype, k, n):
         assert rel_err(wt.gemv(dev(x), bias=dev(bias), epilogue=_lib.EPI_SILU_GATE), g / (1 + np.exp(-g)) * u) < 2e-5
 
 
+# Batches of 3 and 4 on the same kernel: ragged and single tiles, every number of tiles a workgroup takes, a partial last chunk, more chunks than
+# waves.  The quants and f16 activations enter exactly, so what is left is the rounding of f32 sums: a wave adds up ceil(k / 128 / waves) x 4 block
+# results of 32 products, then up to 12 waves in fours: below 2^-24 (32 + 4 x 8 + 8) of the sum of absolute products.
+@pytest.mark.parametrize("dtype", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("k,n", [(1024, 18), (1024, 4098), (1056, 513 * 16 - 14), (2080, 768 * 16 + 2), (2560, 1025 * 16 - 2), (8224, 130), (1152, 2049 * 16)])
+def test_three_and_four_rows(orc, dtype, k, n):
+    wt, wdq = _seeded(dtype, k, n, k + n)
+    rng = np.random.default_rng(k + n)
+    bias = rng.standard_normal(n).astype(np.float32) * 0.1
+    for batch in (3, 4):
+        x = rng.standard_normal((batch, k)).astype(np.float32)
+        res = rng.standard_normal((batch, n)).astype(np.float32)
+        pre, mag = _f16(x) @ wdq, np.abs(_f16(x)) @ np.abs(wdq)
+        lim = 2.0 ** -24 * ((32 + 4 * 8 + 8) * mag + 4 * (np.abs(pre) + np.abs(bias) + np.abs(res)))
+        assert (np.abs(wt.gemv(dev(x), bias=dev(bias), residual=dev(res)) - (pre + bias + res)) <= lim).all(), batch
+        g, u = (pre + bias)[:, 0::2], (pre + bias)[:, 1::2]
+        assert rel_err(wt.gemv(dev(x), bias=dev(bias), epilogue=_lib.EPI_SILU_GATE), g / (1 + np.exp(-g)) * u) < 2e-5
+
+
 def _norm64(h, kind, sc, bi, eps):
     h = h.astype(np.float64)
     if kind == _lib.NORM_RMSNORM:
