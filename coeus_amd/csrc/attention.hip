@@ -16,6 +16,7 @@
 #include "device_utils.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace coeus {
 
@@ -149,67 +150,80 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
     // one hardware exponential per key instead of expf's range reduction (this wave's sixteen keys
     // are evaluated after its last line has arrived, on the launch's tail)
     const float scale = 1.4426950408889634f / sqrtf((float)HD);
-    float m = -INFINITY, l = 0.f, acc[EPL];
+    float m, l, acc[EPL];
+    auto walk = [&](auto masked) {
+        m = -INFINITY;
+        l = 0.f;
 #pragma unroll
-    for (int t = 0; t < EPL; t++) acc[t] = 0.f;
+        for (int t = 0; t < EPL; t++) acc[t] = 0.f;
 
-    // each wave takes tiles of TILE*KPL keys, interleaved over the NW waves
-    for (uint32_t t0 = k_begin + wave * TILE * KPL; t0 < k_end; t0 += NW * TILE * KPL) {
-        // keys and values are requested together: the values do not depend on the scores, and
-        // asking for them only after the scores exposed the memory latency a second time
-        // Every load is unconditional, keys past the end re-reading the last one (their scores
-        // are masked below, so their probabilities are zero): with loads under a branch the
-        // compiler waits for all 32 before the first dot product, without it the scores start
-        // when the first keys arrive.  Keys and values are read once per step: non-temporal loads
-        // stream them faster (7B shape, context 4096, per step: batch 1 1.762 -> 1.752 ms, batch 4
-        // 4.12 -> 3.93, batch 16 7.6-7.9 -> 7.5, the batch-16 launch 177 -> 167 us; 1B shape batch
-        // 4 1.27 -> 1.17 ms; 250M Q8_0 batch 8 0.604 -> 0.566 ms).
-        uint4 kr[TILE], vr[TILE];
+        // each wave takes tiles of TILE*KPL keys, interleaved over the NW waves
+        for (uint32_t t0 = k_begin + wave * TILE * KPL; t0 < k_end; t0 += NW * TILE * KPL) {
+            // keys and values are requested together: the values do not depend on the scores, and
+            // asking for them only after the scores exposed the memory latency a second time
+            // Every load is unconditional, keys past the end re-reading the last one (their scores
+            // are masked below, so their probabilities are zero): with loads under a branch the
+            // compiler waits for all 32 before the first dot product, without it the scores start
+            // when the first keys arrive.  Keys and values are read once per step: non-temporal loads
+            // stream them faster (7B shape, context 4096, per step: batch 1 1.762 -> 1.752 ms, batch 4
+            // 4.12 -> 3.93, batch 16 7.6-7.9 -> 7.5, the batch-16 launch 177 -> 167 us; 1B shape batch
+            // 4 1.27 -> 1.17 ms; 250M Q8_0 batch 8 0.604 -> 0.566 ms).
+            uint4 kr[TILE], vr[TILE];
 #pragma unroll
-        for (int t = 0; t < TILE; t++) {
-            const uint32_t key = min(t0 + t * KPL + ksub, k_end - 1);
-            kr[t] = load_stream(k4 + (uint64_t)key * CPK + piece);
+            for (int t = 0; t < TILE; t++) {
+                const uint32_t key = min(t0 + t * KPL + ksub, k_end - 1);
+                kr[t] = load_stream(k4 + (uint64_t)key * CPK + piece);
+            }
+#pragma unroll
+            for (int t = 0; t < TILE; t++) {
+                const uint32_t key = min(t0 + t * KPL + ksub, k_end - 1);
+                vr[t] = load_stream(v4 + (uint64_t)key * CPK + piece);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // all 32 requests go out before anything is computed
+            float s[TILE], tmax = -INFINITY;
+#pragma unroll
+            for (int t = 0; t < TILE; t++) {
+                float kv[EPL], dot = 0.f;
+                kv_piece<KV>(kr[t], kv);
+#pragma unroll
+                for (int u = 0; u < EPL; u++) dot = fmaf(q[u], kv[u], dot);
+                // sum the CPK pieces of a key (the lanes of one key are an aligned group)
+                dot = group_sum<CPK == 32 ? 16 : CPK>(dot);
+                if (CPK == 32) dot = xor16_sum(dot);
+                const uint32_t key = t0 + t * KPL + ksub;
+                s[t] = key < k_end ? dot * scale : -INFINITY;
+                tmax = fmaxf(tmax, s[t]);
+            }
+            const float m_new = fmaxf(m, wave_max(tmax));
+            // (keys whose scores are all -inf weigh nothing: -inf - -inf would make a NaN of a wave's share)
+            const float top = m_new == -INFINITY ? 0.f : m_new;
+            const float corr = __builtin_amdgcn_exp2f(m - top);
+            float psum = 0.f;
+#pragma unroll
+            for (int t = 0; t < EPL; t++) acc[t] *= corr;
+#pragma unroll
+            for (int t = 0; t < TILE; t++) {
+                const float p = __builtin_amdgcn_exp2f(s[t] - top);  // 2^(-inf) = 0 for keys past the end
+                psum += p;
+                float vv[EPL];
+                if (decltype(masked)::value && t0 + t * KPL + ksub >= k_end) vr[t] = make_uint4(0u, 0u, 0u, 0u);
+                kv_piece<KV>(vr[t], vv);
+#pragma unroll
+                for (int u = 0; u < EPL; u++) acc[u] = fmaf(p, vv[u], acc[u]);
+            }
+            // every lane of a key holds the same p: count each key once
+            l = l * corr + wave_sum(psum) * (1.0f / CPK);
+            m = m_new;
         }
+    };
+    walk(std::false_type{});
+    // The lanes behind the last key weigh its values with zero, which makes a NaN of an infinite one: a wave that ends with a NaN walks again
+    // and clears what such lanes hold.  Clearing it always costs 4 % (decode launches of 12 - 32 heads, 255 - 4095 keys, geometric mean of 14,
+    // us before / always / so: 32 heads of 128 at 255 keys 6.30 / 6.78 / 6.34, 4 x 16 of 64 at 2072 10.95 / 11.54 / 10.98).
+    float odd = acc[0];
 #pragma unroll
-        for (int t = 0; t < TILE; t++) {
-            const uint32_t key = min(t0 + t * KPL + ksub, k_end - 1);
-            vr[t] = load_stream(v4 + (uint64_t)key * CPK + piece);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // all 32 requests go out before anything is computed
-        float s[TILE], tmax = -INFINITY;
-#pragma unroll
-        for (int t = 0; t < TILE; t++) {
-            float kv[EPL], dot = 0.f;
-            kv_piece<KV>(kr[t], kv);
-#pragma unroll
-            for (int u = 0; u < EPL; u++) dot = fmaf(q[u], kv[u], dot);
-            // sum the CPK pieces of a key (the lanes of one key are an aligned group)
-            dot = group_sum<CPK == 32 ? 16 : CPK>(dot);
-            if (CPK == 32) dot = xor16_sum(dot);
-            const uint32_t key = t0 + t * KPL + ksub;
-            s[t] = key < k_end ? dot * scale : -INFINITY;
-            tmax = fmaxf(tmax, s[t]);
-        }
-        const float m_new = fmaxf(m, wave_max(tmax));
-        // (keys whose scores are all -inf weigh nothing: -inf - -inf would make a NaN of a wave's share)
-        const float top = m_new == -INFINITY ? 0.f : m_new;
-        const float corr = __builtin_amdgcn_exp2f(m - top);
-        float psum = 0.f;
-#pragma unroll
-        for (int t = 0; t < EPL; t++) acc[t] *= corr;
-#pragma unroll
-        for (int t = 0; t < TILE; t++) {
-            const float p = __builtin_amdgcn_exp2f(s[t] - top);  // 2^(-inf) = 0 for keys past the end
-            psum += p;
-            float vv[EPL];
-            kv_piece<KV>(vr[t], vv);
-#pragma unroll
-            for (int u = 0; u < EPL; u++) acc[u] = fmaf(p, vv[u], acc[u]);
-        }
-        // every lane of a key holds the same p: count each key once
-        l = l * corr + wave_sum(psum) * (1.0f / CPK);
-        m = m_new;
-    }
+    for (int t = 1; t < EPL; t++) odd += acc[t];
+    if (__any(odd != odd)) walk(std::true_type{});
     // fold the KPL key-subsets of the wave: lanes with equal piece hold partial sums
 #pragma unroll
     for (int t = 0; t < EPL; t++) {

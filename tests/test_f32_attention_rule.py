@@ -97,3 +97,46 @@ def test_sequences_and_earlier_keys(orc, heads, hd, n, first):
         want = f64_model.forward_all(oc, params, ids[b])[[first + r for r in rows]]
         # (as in the other tests of f32 prompts: sums of up to 4 hd terms, a few roundings of 2^-24 each)
         assert np.abs(got[b] - want).max() <= 2e-5 * np.abs(want).max(), b
+
+
+# 1 - 15 rows, a workgroup per row and head: the lanes behind a row's last key read that key again
+@gpu
+@pytest.mark.parametrize("rows", [1, 2, 5, 15])
+@pytest.mark.parametrize("heads,hd", [(3, 64), (2, 128)])
+def test_few_rows_of_infinite_values_and_scores(rows, heads, hd):
+    """An infinite value is an infinity (or, with its opposite, no number) in that dimension of the rows that see it, and nothing elsewhere; scores
+    of -inf weigh nothing, +inf and NaN make the rows that see them NaN."""
+    rng = np.random.default_rng(rows + hd)
+    inner = heads * hd
+    clean = rng.standard_normal((rows, 3 * inner)).astype(np.float32)
+    clean[:, :inner:hd] = 1e20
+    clean[:, inner:2 * inner:hd] = 0
+    cases = []
+    for j in range(rows):
+        values = clean.copy()
+        values[j, 2 * inner::hd] = np.inf
+        values[j, 2 * inner + hd - 1::hd] = -np.inf
+        if j + 1 < rows:
+            values[j + 1, 2 * inner + 3::hd] = -np.inf
+            values[j, 2 * inner + 3::hd] = np.inf
+        cases.append(values)
+        for score in (-1e30, 1e30, np.nan):
+            scores = clean.copy()
+            scores[j, inner:2 * inner:hd] = score
+            cases.append(scores)
+    for i, qkv in enumerate(cases):
+        out = _attention(qkv, heads, hd)
+        for h in range(heads):
+            # (as f32 has them: 1e50 is infinite, and what a key weighs that nobody may see is no factor)
+            want, got = np.full((rows, hd), np.nan), out[:, h * hd:(h + 1) * hd]
+            for r in range(rows):
+                with np.errstate(over="ignore", invalid="ignore"):
+                    q, k, v = (qkv[:r + 1, at * inner + h * hd:at * inner + (h + 1) * hd].astype(np.float64) for at in range(3))
+                    s = (q[r] * k).sum(-1) / np.sqrt(hd)
+                    s = np.where(np.abs(s) > 3.5e38, np.copysign(np.inf, s), s)
+                    p = np.exp(s - s.max())
+                    want[r] = (p[:, None] * v).sum(0) / p.sum()
+            odd = ~np.isfinite(want)
+            assert np.array_equal(got[odd], want[odd].astype(np.float32), equal_nan=True), (i, h)
+            # sums of hd products and of up to 15 probabilities, exp2 to 1 ulp of arguments below 16
+            assert odd.all() or np.abs(got - want)[~odd].max() <= 1e-5 * np.abs(want[~odd]).max(), (i, h)

@@ -691,6 +691,36 @@ def test_attention_decode_large_cache(orc, hd, bf16):
             assert err < 1e-5, (ctx, nsplit, err)
 
 
+@pytest.mark.parametrize("hd,bf16", [(128, False), (64, True)])
+@pytest.mark.parametrize("ctx", [1, 5, 65, 300, 1024])
+def test_attention_decode_infinite_last_value(orc, hd, bf16, ctx):
+    """An infinite value of the last key, which lanes behind the end of a context read again: an infinity in its dimension, nothing elsewhere."""
+    lib = _lib.load()
+    heads, max_ctx = 3, 1024
+    rng = np.random.default_rng(hd + ctx)
+    qkv = rng.standard_normal((1, 3 * heads * hd)).astype(np.float32)
+    K = rng.standard_normal((heads, max_ctx, hd)).astype(np.float32)
+    V = rng.standard_normal((heads, max_ctx, hd)).astype(np.float32)
+    kbits, k64 = _to16(K, bf16, orc)
+    vbits, v64 = _to16(V, bf16, orc)
+    q64 = qkv[0, :heads * hd].astype(np.float64).reshape(heads, hd)
+    s = np.einsum("hd,hcd->hc", q64, k64[:, :ctx]) / np.sqrt(hd)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = np.einsum("hc,hcd->hd", p / p.sum(-1, keepdims=True), v64[:, :ctx])
+    want[:, 0], want[:, hd - 1] = np.inf, -np.inf
+    inf = np.uint16(0x7F80 if bf16 else 0x7C00)
+    vbits[:, ctx - 1, 0], vbits[:, ctx - 1, hd - 1] = inf, inf | 0x8000
+    dq, dk, dv, out = dev(qkv), dev(kbits), dev(vbits), DeviceArray((heads, hd), np.float32)
+    finite = np.isfinite(want)
+    for nsplit in (0, 1, 2, 8, 32):
+        for merge in (_lib.MERGE_IN_KERNEL, _lib.MERGE_SEPARATE):
+            _check(lib.coeus_op_attention_decode(dq.ptr, dk.ptr, dv.ptr, _lib.KV_BF16 if bf16 else _lib.KV_F16, 1, heads, hd, max_ctx, ctx, nsplit,
+                                                 merge, out.ptr, None))
+            got = out.to_host()
+            assert np.array_equal(got[~finite], want[~finite].astype(np.float32)), (nsplit, merge)
+            assert rel_err(got[finite], want[finite]) < 1e-5, (nsplit, merge)  # (as with a split context above)
+
+
 def test_attention_decode_argument_errors():
     lib = _lib.load()
     from coeus_amd.plugin import ProcessingError
