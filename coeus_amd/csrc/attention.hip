@@ -836,7 +836,10 @@ bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype) {
     return n >= 16 && (hd == 64 || hd == 128) && kv_dtype != COEUS_KV_F32;
 }
 
-// Queries of a workgroup of f32 prompt attention: 32, with four key shares, while 128 queries give few workgroups.  us, 128 queries / 32:
+// Prompts of fewer than 16 rows with a workgroup per row and head (attn_decode_kernel's ROWS form; grid.z holds the sequences).
+static bool attn_rows_apart(uint64_t batch, uint64_t n, uint64_t hd) { return n < 16 && (hd == 64 || hd == 128) && batch <= 65535; }
+
+// Queries of a workgroup of f32 prompt attention: one up to 15 rows; then 32, with four key shares, while 128 queries give few workgroups.  us, 128 queries / 32:
 // heads of 64, up to 384 workgroups: 12 heads at 64 / 128 / 512 / 1024 rows 7.6 / 5.0, 13.0 / 6.1, 42 / 16, 81 / 49; 48 at 1024 1.28x as
 // fast; 192 at 80 and 256 rows 10.7 / 11.1 and 32.4 / 33.1.  Beyond neither is ahead throughout: 8 x 12 heads at 1024 (768 workgroups)
 // 216 / 266, at 1500 406 / 338, at 2048 822 / 793, at 3000 1327 / 1250, at 4096 3202 / 2582.
@@ -845,6 +848,7 @@ bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype) {
 // time; but 64 at 512 82 / 92, 128 at 129 / 256 28.1 / 30.4 and 45.6 / 60.8, 256 at 33 / 128 13.7 / 17.4 and 28.4 / 42.7; 32 at 1500 225 / 293, 4 x 32
 // at 1024 355 / 591.  One tile of keys leaves three waves without work: 17 / 32 rows of 32 heads 8.0 / 8.8 and 8.2 / 9.5.
 uint32_t attn_prefill_f32_queries(uint64_t batch, uint64_t n, uint64_t pos0, uint64_t heads, uint64_t hd) {
+    if (attn_rows_apart(batch, n, hd)) return 1;
     if (n < 16 || (hd != 64 && hd != 128)) return 4;  // (attn_generic_kernel)
     const uint64_t wgs = ceil_div(n, 128) * heads * batch;
     return (hd == 64 ? wgs <= 384 : pos0 + n > 32 && wgs <= (n >= 768 ? 256 : 128)) ? 32 : 128;
@@ -977,7 +981,7 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
     // Fewer than 16 rows: a workgroup per row and head, as in a decode step whose keys stay in one piece.  Bound by the launch and one trip to
     // memory behind the queries'; attn_generic_kernel's lanes walk a key each, dimension by dimension (5 rows x 12 heads of 64, f32: 5.3 us,
     // 3.3 here).
-    if (n < 16 && (hd == 64 || hd == 128) && batch <= 65535 && pos0 + n <= max_ctx) {
+    if (attn_rows_apart(batch, n, hd)) {
         const dim3 rgrid((unsigned)n, (unsigned)heads, (unsigned)batch);
         const uint32_t kpl = 64 / ((uint32_t)hd / (kv_dtype == COEUS_KV_F32 ? 4 : 8));
         const bool few = !pos_dev && pos0 + n <= 16 * kpl;

@@ -383,7 +383,7 @@ int coeus_op_embed(const float *table_dev, const float *pe_dev, const uint64_t *
 int coeus_op_attention(const float *qkv_dev, uint64_t rows, uint64_t num_heads, uint64_t head_dim,
                        float *out_dev, void *stream);
 /* Queries that a workgroup of f32 prompt attention takes (no counterpart in the reference; for profiles and tests, no device is touched):
- * `rows` new tokens of `batch` sequences behind `cached` others.  32 or 128; 4: the kernel for any size of head. */
+ * `rows` new tokens of `batch` sequences behind `cached` others.  1 (up to 15 rows), 32 or 128; 4: the kernel for any size of head. */
 uint32_t coeus_plan_attention_f32(uint64_t batch, uint64_t rows, uint64_t cached, uint64_t num_heads, uint64_t head_dim);
 /* The attention of ONE new token per sequence (the decode step's MT:219-278: the query row
  * against every cached key, row softmax, P.V) over a caller-owned 16-bit cache

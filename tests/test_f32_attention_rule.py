@@ -1,4 +1,4 @@
-"""f32 prompt attention on both sides of every line between its two kernels (32 queries a workgroup, or 128): float64, several sequences, keys
+"""f32 prompt attention on both sides of every line between its kernels (a query a workgroup, 32, or 128): float64, several sequences, keys
 before the prompt, and scores that are infinite or no number."""
 import numpy as np
 import pytest
@@ -18,7 +18,7 @@ gpu = pytest.mark.gpu
     (1, 16, 0, 32, 128, 128), (1, 32, 0, 1, 128, 128), (8, 32, 0, 32, 128, 128), (1, 33, 0, 32, 128, 32), (1, 17, 16, 32, 128, 32), (1, 17, 15, 32, 128, 128),
     (1, 128, 0, 256, 128, 128), (2, 128, 0, 128, 128, 128), (1, 256, 0, 128, 128, 128), (1, 512, 0, 64, 128, 128), (1, 128, 0, 128, 128, 32), (1, 512, 0, 32, 128, 32),
     (1, 768, 0, 32, 128, 32), (1, 1024, 0, 32, 128, 32), (1, 767, 0, 32, 128, 128), (1, 1025, 0, 32, 128, 128), (1, 16, 0, 12, 64, 32), (1, 4096, 0, 12, 64, 32),
-    (8, 512, 0, 12, 64, 32), (8, 513, 0, 12, 64, 128), (1, 15, 0, 12, 64, 4), (1, 40, 0, 4, 96, 4)])
+    (8, 512, 0, 12, 64, 32), (8, 513, 0, 12, 64, 128), (1, 15, 0, 12, 64, 1), (8, 1, 900, 32, 128, 1), (1, 15, 0, 4, 96, 4), (1, 40, 0, 4, 96, 4)])
 def test_plan(batch, rows, cached, heads, hd, queries):
     assert _lib.load().coeus_plan_attention_f32(batch, rows, cached, heads, hd) == queries
 
