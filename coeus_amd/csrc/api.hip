@@ -410,7 +410,7 @@ int coeus_op_norm_gemv(const coeus_weight *w, const float *h_dev, uint64_t batch
     NormFuse nf;
     nf.h = h_dev; nf.scale = scale_dev; nf.bias = bias_norm_dev; nf.eps = eps; nf.kind = norm_kind;
     const bool quant = W.dtype >= COEUS_W_Q8_0;
-    const bool fused = quant ? gemv_can_fuse_norm(W, batch) : gemv_can_fuse_norm_dense(W, batch);
+    const bool fused = quant ? gemv_can_fuse_norm(W, batch) && !gemv_norm_apart(W, batch) : gemv_can_fuse_norm_dense(W, batch);
     if (fused_out) *fused_out = fused ? 1 : 0;
     DeviceBuf stats, x;
     int rc = COEUS_OK;

@@ -327,7 +327,8 @@ int coeus_op_gemv(const coeus_weight *w, const float *x_dev, uint64_t batch, con
  * normalisation of its input rows (math::layer_norm per row, MT:105-128, or a root-mean-square
  * norm; scale_dev / bias_norm_dev [k_in]) folded into the kernel's activation staging, which is
  * how a decode step runs the q|k|v, FFN-up and logits projections (MT:469, 488, 906 followed by
- * MT:50-74).  Shapes whose rows do not fit the staging run the norm as a launch of its own.
+ * MT:50-74).  Shapes whose rows do not fit the staging run the norm as a launch of its own, and so do, as in a
+ * decode step, three and four rows of quantised weights from 1536 elements on.
  * h_dev [batch, k_in] f32; *fused_out (nullable) reports whether the folded form ran.
  * Unlike the other operators this call does more than enqueue: it allocates device memory for the
  * row statistics (or the normalised rows), with quantised weights it overwrites the weight's

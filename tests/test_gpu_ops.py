@@ -554,8 +554,8 @@ def _norm_gemv(wt, h, kind, sc, bi, eps, n_eff, epilogue=0, residual=None):
     (800, 520, False, "ln"),       # k = 32 (mod 128): the last group of blocks is a padded one
 ])
 def test_norm_gemv_benchmark_shapes(orc, dtype, k, n, gated, kind):
-    """coeus_op_norm_gemv: the norm folded into the decode matmul's staging (batch 1, 2 and 4: one,
-    two and four pieces per lane where the width asks for it), and as its own launch for batch 8 and
+    """coeus_op_norm_gemv: the norm folded into the decode matmul's staging (batch 1, 2 and narrow 4: one,
+    two and four pieces per lane where the width asks for it), and as its own launch for wide 4, 8 and
     16, against a float64 norm -> f16 rounding -> float64 product on the oracle-dequantised
     weights.  The f32 norm arithmetic may round an activation to the neighbouring f16 value, so
     the bar is 1e-4 here (an indexing error is O(1))."""
@@ -577,10 +577,27 @@ def test_norm_gemv_benchmark_shapes(orc, dtype, k, n, gated, kind):
         else:
             want = pre + res
             got, fused = _norm_gemv(wt, h, nk, sc, bi, 1e-5, n_eff, 0, res)
-        # (folded for up to 4 rows whose f16 block fits 48 KiB, four rows only up to k = 4096)
-        want_fused = batch <= 4 and k * batch <= 24576 and (batch <= 2 or k <= 4096)
+        # (folded for one and two rows whose f16 block fits 48 KiB, three and four rows only below k = 1536)
+        want_fused = batch <= 4 and k * batch <= 24576 and (batch <= 2 or k < 1536)
         assert fused == (1 if want_fused else 0), (batch, fused)
         assert rel_err(got, want) < 1e-4, (batch, fused, rel_err(got, want))
+
+
+# the last width that folds, and the first whose rows are normalised apart; Q8_0 multiplies the latter with either kernel
+@pytest.mark.parametrize("k,n", [(1504, 2048), (1536, 2048), (1536, 4112), (4096, 1024)])
+@pytest.mark.parametrize("dtype", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("kind", ["ln", "rms"])
+@pytest.mark.parametrize("batch", [3, 4])
+def test_norm_gemv_three_and_four_rows(orc, dtype, k, n, kind, batch):
+    wt, wdq = _seeded(dtype, k, n, 500 + k + n)
+    rng = np.random.default_rng(k + n + batch)
+    sc = (1.0 + 0.1 * rng.standard_normal(k)).astype(np.float32)
+    bi = (0.1 * rng.standard_normal(k)).astype(np.float32) if kind == "ln" else None
+    nk = _lib.NORM_LAYERNORM if kind == "ln" else _lib.NORM_RMSNORM
+    h = (rng.standard_normal((batch, k)) * 1.5 + 0.3).astype(np.float32)
+    want = _f16(_norm64(h, nk, sc.astype(np.float64), None if bi is None else bi.astype(np.float64), 1e-5)) @ wdq
+    got, fused = _norm_gemv(wt, h, nk, sc, bi, 1e-5, n)
+    assert fused == (k < 1536) and rel_err(got, want) < 1e-4  # (as above)
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
