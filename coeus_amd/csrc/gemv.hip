@@ -2190,18 +2190,37 @@ static uint32_t gemv_one_row_steps(const Weight &w, uint64_t batch, bool gated) 
 // Parts: as many as leave at most a workgroup per CU, four up to 1024 outputs, two up to 2048; bf16 from lengths on at which a tile's trip
 // is long enough to halve (us, one / two / four parts: 4 rows of 768 x 768 3.5 / 4.0 / 3.7, 1024 x 1024 3.9 / 3.9 / 3.8, 2048 x 2048 4.7 / 4.9 / 5.2, 4096 x 2048
 // 7.6 / 6.8 / 7.1, and four where the shares are two pairs that stay in registers, 5632 x 2048 10.1 / 8.7 / 8.0; 8 rows of 1024 x 1024 4.2 / 4.2, 2048 x
-// 2048 5.6 / 5.2).  Beyond 4096 outputs a CU takes several tiles, and smaller ones even out their number: from 4096 of k on, as long as a wave's share
-// is two pairs (4 rows of bf16 4096 x 4608 12.7 / - / 10.5, x 12352 24.2 / 20.8 / 20.3, f32 4096 x 4608 20.9 / 17.7 / 17.6; but bf16 4096 x 4096 8.4 / 10.4 /
-// 10.0, 8 rows of 6144 x 8192 24.6 / 32.1).
+// 2048 5.6 / 5.2).  Beyond 4096 outputs a CU takes several tiles, and smaller ones even out their number: bf16 from 4096 of k on, as long as a wave's
+// share is two pairs (4 rows 4096 x 4608 12.7 / - / 10.5, x 12352 24.2 / 20.8 / 20.3; but 4096 x 4096 8.4 / 10.4 / 10.0, 8 rows of 6144 x 8192 24.6 / 32.1).
+// f32 from 4096 on up to 5120 outputs, whose tiles of 16 leave the second round of workgroups nearly empty, if the waves' shares come out even, and
+// wherever rows are 32 KiB apart (us, one part with sixteen waves / with eight / parts: 4 rows of 5632 x 5000 27.1 / 25.7 / 23.9, 8 of 8192 x 8192 50.7 / 62.2 /
+// 50.4; but 4 of 5632 x 8192 30.5 / 29.3 / 36.8, 8704 x 8192 44.9 / 44.1 / 67.3, 11008 x 8192 60.2 / 62.3 / 71.2, 9216 x 4112 in uneven shares 39.3 / 39.0 / 40.1;
+// 4096 x 9000 31.3 / 27.7 / 26.7 is the exception).
 // Waves: eight of four pairs and more rather than sixteen, two workgroups a CU, one of which asks while the other adds up (us, 16 / 8: 4 rows of bf16
 // 2048 x 6176 8.4 / 7.4, x 2048 5.1 / 4.7, 8 of 2048 x 8192 10.4 / 9.7, but x 11264 12.4 / 13.3, 16 of 2048 x 1024 6.5 / 7.0; f32, 4 of 768 x 3072 4.9 / 4.5,
-// 1024 x 3600 6.1 / 5.3); four of f32 where there are several tiles a CU (16 / 8 / 4: 1024 x 4608 8.3 / 7.3 / 6.6, 2048 x 8192 15.0 / 13.8 / 13.7); three pairs of
+// 1024 x 3600 6.1 / 5.3); four of f32 where there are several tiles a CU and rows are short of 4096 (16 / 8 / 4: 1024 x 4608 8.3 / 7.3 / 6.6, 2048 x 8192 15.0 / 13.8 /
+// 13.7; but 4 rows of 8224 x 8192 48.1 / 46.2 / 60.1, 16 of 4096 x 8192 26.5 / 24.6 / 30.4) or 32 KiB apart (16 of 16384 x 4112 101 / 88 / 82); twelve of 256 pairs, where
+// eight begin 4 KiB apart in rows 32 KiB apart and share their memory channels (4 rows of f32 8192 x 4096, 16 / 8 / 12: 27.4 / 30.0 / 24.0); three pairs of
 // bf16 a wave where that comes out even, asked for at once (768 x 2304, two / three: 3.83 / 3.60; - x 10272 5.65 / 5.84).
 struct MfmaPlain { bool runs; uint32_t parts, waves; size_t lds; };
 template <bool BF16>
 static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
     const uint32_t xbp = std::max(pad_batch(batch), 4u), most = 16 / xbp;  // (a part needs columns for all rows)
     auto fits = [&](uint32_t parts) { return parts <= most && w.k % (MfmaType<BF16>::KU * parts) == 0; };
+    // f32: waves for that many parts; whether they ask for little in vain, two or three pairs at once
+    auto f32_waves = [&](uint32_t parts) {
+        const uint64_t pairs = std::min<uint64_t>(w.k / (MfmaType<false>::KU * parts), 1u << 20), four = std::max<uint64_t>(4, ceil_div(pairs, 4));
+        uint64_t waves = gemv_mfma_waves(pairs);
+        if (parts == 4) waves = pairs <= 12 ? std::max<uint64_t>(4, ceil_div(pairs, 2)) : std::min<uint64_t>(16, four);
+        else if (parts == 2) waves = pairs >= 128 ? 16 : std::min<uint64_t>(8, four);
+        else if (w.n > 4096) waves = pairs < 128 || pairs % 256 == 0 ? 4 : 8;
+        else if (xbp < 16) waves = pairs == 256 ? 12 : std::min<uint64_t>(8, four);
+        return (uint32_t)std::min<uint64_t>(waves, std::max<uint64_t>(1, pairs));
+    };
+    auto even = [&](uint32_t parts) {
+        const uint64_t pairs = w.k / (MfmaType<false>::KU * parts), waves = f32_waves(parts), np = ceil_div(pairs, waves);
+        return 4 * std::min(ceil_div(np, 2) * 2, ceil_div(np, 3) * 3) * waves <= 5 * pairs;
+    };
     uint32_t parts = 1;
     if (BF16) {
         if (w.n <= 1024 && w.k >= 1024 && fits(4)) parts = 4;
@@ -2209,8 +2228,9 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
         else if (w.n > 4096 && w.k >= 4096 && w.k <= 8192 && fits(4)) parts = 4;
         else if (((w.n <= 2048 && w.k >= (xbp == 8 || w.n <= 1024 ? 2048 : 4096)) || (w.n > 4096 && w.k == 4096)) && fits(2)) parts = 2;
     } else if (w.k >= 256) {
-        if ((w.n <= 1024 || (w.n > 4096 && w.k >= 4096)) && fits(4)) parts = 4;
-        else if ((w.n <= 2048 || (w.n > 4096 && w.k >= 4096)) && fits(2)) parts = 2;
+        auto wide = [&](uint32_t p) { return w.n > 4096 && w.k >= 4096 && (w.k % 8192 == 0 || (w.n <= 5120 && even(p))); };
+        if (fits(4) && (w.n <= 1024 || wide(4))) parts = 4;
+        else if (fits(2) && (w.n <= 2048 || wide(2))) parts = 2;
     }
     const uint64_t pairs = std::min<uint64_t>(w.k / (MfmaType<BF16>::KU * parts), 1u << 20);
     uint32_t waves = gemv_mfma_waves(pairs);
@@ -2218,12 +2238,8 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
         if (parts > 1 && pairs > 32) waves = 8;
         if (parts == 1 && xbp == 4 && pairs % 3 == 0 && pairs >= 9 && pairs <= 24 && w.n <= 8192) waves = (uint32_t)std::max<uint64_t>(waves / 2, pairs / 3);
         else if (parts == 1 && (xbp == 4 || (xbp == 8 && w.n > 4096 && w.n <= 8192)) && pairs % 8 == 0) waves = std::min(waves, 8u);
-    } else if (xbp < 16 || w.n > 4096) {
-        const uint64_t four = std::max<uint64_t>(4, ceil_div(pairs, 4));
-        if (parts == 1) waves = w.n > 4096 ? 4 : (uint32_t)std::min<uint64_t>(8, four);
-        else if (parts == 2) waves = pairs >= 128 ? 16 : (uint32_t)std::min<uint64_t>(8, four);
-        else waves = (uint32_t)(pairs <= 12 ? std::max<uint64_t>(4, ceil_div(pairs, 2)) : std::min<uint64_t>(16, four));
-        waves = (uint32_t)std::min<uint64_t>(waves, std::max<uint64_t>(1, pairs));
+    } else {
+        waves = f32_waves(parts);
     }
     const uint32_t rows = parts > 1 ? 16 : xbp;
     const size_t lds = (size_t)waves * 16 * mfma_wave_lds<BF16>((rows + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS);

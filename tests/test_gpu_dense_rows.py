@@ -60,6 +60,17 @@ def test_parts_of_k(orc, dtype, k, n, batch):
         assert (np.abs(wt.gemv(dev(x), epilogue=_lib.EPI_SILU_GATE) - want) <= lim).all()
 
 
+# Long rows in shares that differ by a pair: eight waves of several tiles a workgroup, twelve where rows are 32 KiB apart
+@pytest.mark.parametrize("dtype,k,n", [(_lib.W_F32, 4128, 5130), (_lib.W_F32, 8192, 2070)])
+@pytest.mark.parametrize("batch", [2, 4, 8, 16])
+def test_waves_of_long_rows(orc, dtype, k, n, batch):
+    rng = np.random.default_rng(k + batch)
+    w = (rng.standard_normal((k, n), np.float32) * np.float32(0.02))
+    x = (rng.standard_normal((batch, k)) * np.exp2(rng.integers(-20, 20, (batch, k)))).astype(np.float32)
+    wt, wd = Weight(dtype, w), oracle_roundtrip(orc, dtype, w).astype(np.float64)
+    assert (np.abs(wt.gemv(dev(x)) - x.astype(np.float64) @ wd) <= bound(x, wd, k)).all()
+
+
 @pytest.mark.parametrize("dtype,rows", [(_lib.W_F32, 2), (_lib.W_F32, 5), (_lib.W_F32, 16), (_lib.W_F32, 17), (_lib.W_BF16, 5)])
 def test_timed_matmul_is_the_one_that_runs(dtype, rows):
     """What the repeated, timed launches leave is the bits of the plain call: the same kernel, in the same order of sums."""

@@ -81,6 +81,18 @@ def test_several_rows_on_dense_weights(dtype, k, n, rows, cols, waves):
     assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", cols, waves)
 
 
+# f32 beyond 4096 outputs, where parts of k or four waves were slower than tiles of 16 with sixteen: us, sixteen / parts or four / now: 4 rows of 8704 x 8192
+# 44.9 / 67.3 / 44.1, 8224 x 8192 48.1 / 60.1 / 46.2, 5632 x 8192 30.5 / 36.8 / 29.3, 16 of 4096 x 8192 26.5 / 30.4 / 24.6; and 256 pairs: 4 rows of 8192 x 4096 with sixteen,
+# eight and twelve waves 27.4 / 30.0 / 24.0
+@pytest.mark.parametrize("k,n,rows,cols,waves", [
+    (8704, 8192, 4, 16, 8), (8704, 8192, 2, 16, 8), (8224, 8192, 4, 16, 8), (5632, 8192, 8, 16, 8), (4096, 8192, 16, 16, 8), (4096, 5121, 4, 16, 8), (4096, 5120, 4, 4, 8),
+    (5632, 5000, 4, 4, 11), (8704, 4112, 4, 8, 16), (9216, 4112, 4, 8, 16), (8192, 8192, 8, 8, 16), (8192, 8192, 4, 4, 16), (16384, 4112, 16, 16, 4), (4064, 8192, 16, 16, 4),
+    (2048, 8192, 4, 16, 4), (8192, 4096, 4, 16, 12), (8192, 4096, 8, 16, 12), (8192, 4096, 16, 16, 16), (8224, 4096, 4, 16, 8)])
+def test_wide_rows_of_f32(k, n, rows, cols, waves):
+    p = plan(_lib.W_F32, k, n, rows)
+    assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", cols, waves)
+
+
 # Prompts: the shapes that test_gpu_narrow_gemm.py, test_gpu_sum_error.py and test_gpu_large_tiles.py multiply reach all five small tiles, shares of k on
 # small and on large ones, and one workgroup a large tile
 @pytest.mark.parametrize("m,k,n,kernel,rows,cols,shared", [
