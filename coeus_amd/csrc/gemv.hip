@@ -1816,7 +1816,8 @@ static bool gemv_uses_mfma(const Weight &w, uint64_t batch, uint32_t waves, bool
     const bool bf = w.dtype == COEUS_W_BF16;
     // One row (two weight rows a wave / here): short rows of which there are many (256 x 16384 5.0 / 4.4, x 100000 18.3 / 11.1, 512 x 50257 12.6 / 10.8;
     // but 512 x 12000 0.89 of the time, 576 x 50257 0.89), and long ones a little beyond the 2048 that give every compute unit one
-    // workgroup (11008 x 3072 17.7 / 16.8, 14336 x 3072 20.6 / 19.0; x 2048 0.74 of the time, x 3584 the same, 8192 x 3072 the same).
+    // workgroup (11008 x 3072 17.7 / 16.8, 14336 x 3072 20.6 / 19.0 with sixteen waves, 0.94 and 0.96 of that with eight; x 2048 0.74 of the time, x 3584 the
+    // same, 8192 x 3072 the same).
     if (batch == 1) return bf && !folded && (w.k <= 512 ? w.n >= 16384 : w.k >= 10240 && w.n > 2048 && w.n <= 3328);
     // (A norm in front costs a wave per row more: f32, 2 rows of 768 x 768 7.4 / 5.8.  Two rows of bf16 are the exception where they
     // are long and few: 2560 x 4096 11.0 / 11.6, x 12288 22.7 / 19.1.)
@@ -2196,12 +2197,15 @@ static uint32_t gemv_one_row_steps(const Weight &w, uint64_t batch, bool gated) 
 // wherever rows are 32 KiB apart (us, one part with sixteen waves / with eight / parts: 4 rows of 5632 x 5000 27.1 / 25.7 / 23.9, 8 of 8192 x 8192 50.7 / 62.2 /
 // 50.4; but 4 of 5632 x 8192 30.5 / 29.3 / 36.8, 8704 x 8192 44.9 / 44.1 / 67.3, 11008 x 8192 60.2 / 62.3 / 71.2, 9216 x 4112 in uneven shares 39.3 / 39.0 / 40.1;
 // 4096 x 9000 31.3 / 27.7 / 26.7 is the exception).
-// Waves: eight of four pairs and more rather than sixteen, two workgroups a CU, one of which asks while the other adds up (us, 16 / 8: 4 rows of bf16
-// 2048 x 6176 8.4 / 7.4, x 2048 5.1 / 4.7, 8 of 2048 x 8192 10.4 / 9.7, but x 11264 12.4 / 13.3, 16 of 2048 x 1024 6.5 / 7.0; f32, 4 of 768 x 3072 4.9 / 4.5,
-// 1024 x 3600 6.1 / 5.3); four of f32 where there are several tiles a CU and rows are short of 4096 (16 / 8 / 4: 1024 x 4608 8.3 / 7.3 / 6.6, 2048 x 8192 15.0 / 13.8 /
-// 13.7; but 4 rows of 8224 x 8192 48.1 / 46.2 / 60.1, 16 of 4096 x 8192 26.5 / 24.6 / 30.4) or 32 KiB apart (16 of 16384 x 4112 101 / 88 / 82); twelve of 256 pairs, where
-// eight begin 4 KiB apart in rows 32 KiB apart and share their memory channels (4 rows of f32 8192 x 4096, 16 / 8 / 12: 27.4 / 30.0 / 24.0); three pairs of
-// bf16 a wave where that comes out even, asked for at once (768 x 2304, two / three: 3.83 / 3.60; - x 10272 5.65 / 5.84).
+// Waves of one part, up to eight rows of bf16: eight rather than sixteen from 33 pairs on, two workgroups a CU, one of which asks while the other adds up (us,
+// 16 / 8: 4 rows of 4224 x 4096 9.2 / 7.9, 11008 x 4112 28.0 / 25.5, one of 11008 x 3072 14.9 / 14.0, 8 of 2112 x 12352 21.2 / 15.7, 4608 x 9000 25.9 / 21.7; 10240 and
+// 12288 - 24576 long 0.96 - 1.02 of the time; sixteen rows are not faster, 2048 x 1024 6.5 / 7.0).  Of 32 pairs, two for each of sixteen waves that stay in
+// registers, as long as outputs are few (4 rows of 2048 x 6176 7.9 / 7.0, x 11264 0.93 of the time, x 12352 11.6 / 12.4; 8 of x 8192 0.90, x 9000 1.04, x 12352 1.12); of
+// fewer as many as have two, or three where that comes out even, asked for at once (4 rows of 768 x 2304, two / three: 3.83 / 3.60; - x 10272 5.65 / 5.84, 1536 x 12352
+// 8.5 / 10.7, 8 of 1536 x 5000 6.4 / 7.1).  Twelve of 256 pairs, where eight begin 4 KiB apart in rows 32 KiB apart and share their memory channels (16 / 8 / 12: 4 rows of
+// bf16 16384 x 3600 22.6 / 26.2 / 22.4, f32 8192 x 4096 27.4 / 30.0 / 24.0).
+// f32: eight (16 / 8: 4 rows of 768 x 3072 4.9 / 4.5, 1024 x 3600 6.1 / 5.3); four where there are several tiles a CU and rows are short of 4096 (16 / 8 / 4: 1024 x 4608 8.3 /
+// 7.3 / 6.6, 2048 x 8192 15.0 / 13.8 / 13.7; but 4 rows of 8224 x 8192 48.1 / 46.2 / 60.1, 16 of 4096 x 8192 26.5 / 24.6 / 30.4) or 32 KiB apart (16 of 16384 x 4112 101 / 88 / 82).
 struct MfmaPlain { bool runs; uint32_t parts, waves; size_t lds; };
 template <bool BF16>
 static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
@@ -2235,9 +2239,9 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
     const uint64_t pairs = std::min<uint64_t>(w.k / (MfmaType<BF16>::KU * parts), 1u << 20);
     uint32_t waves = gemv_mfma_waves(pairs);
     if (BF16) {
-        if (parts > 1 && pairs > 32) waves = 8;
-        if (parts == 1 && xbp == 4 && pairs % 3 == 0 && pairs >= 9 && pairs <= 24 && w.n <= 8192) waves = (uint32_t)std::max<uint64_t>(waves / 2, pairs / 3);
-        else if (parts == 1 && (xbp == 4 || (xbp == 8 && w.n > 4096 && w.n <= 8192)) && pairs % 8 == 0) waves = std::min(waves, 8u);
+        if (parts > 1) waves = pairs > 32 ? 8 : waves;
+        else if (xbp == 4 && pairs % 3 == 0 && pairs >= 9 && pairs <= 24 && w.n <= 8192) waves = (uint32_t)std::max<uint64_t>(waves / 2, pairs / 3);
+        else if (xbp <= 8 && (pairs > 32 || (pairs == 32 && w.n <= (xbp == 4 ? 12288 : 8192)))) waves = pairs == 256 ? 12 : 8;
     } else {
         waves = f32_waves(parts);
     }

@@ -74,7 +74,7 @@ def test_few_long_rows_of_bf16(k, n, kernel):
     (_lib.W_F32, 8192, 2048, 8, 8, 16), (_lib.W_F32, 2048, 2048, 2, 8, 8), (_lib.W_F32, 2048, 2049, 4, 16, 8), (_lib.W_F32, 1024, 4608, 4, 16, 4), (_lib.W_F32, 4096, 1024, 3, 4, 8), (_lib.W_F32, 768, 768, 2, 4, 4), (_lib.W_F32, 1536, 1024, 3, 4, 6), (_lib.W_F32, 128, 768, 2, 16, 4),
     (_lib.W_F32, 96, 700, 4, 16, 3), (_lib.W_BF16, 768, 768, 4, 16, 4), (_lib.W_BF16, 1024, 1024, 4, 4, 2), (_lib.W_BF16, 1024, 1024, 5, 16, 8), (_lib.W_BF16, 3072, 768, 4, 4, 6),
     (_lib.W_BF16, 3072, 768, 8, 8, 12), (_lib.W_BF16, 5632, 2048, 4, 4, 11), (_lib.W_BF16, 5632, 2048, 5, 8, 8), (_lib.W_BF16, 4096, 2048, 4, 8, 16), (_lib.W_BF16, 2048, 10272, 4, 16, 8),
-    (_lib.W_BF16, 4096, 12352, 4, 4, 8), (_lib.W_BF16, 4096, 12352, 5, 8, 16), (_lib.W_BF16, 8192, 8192, 4, 4, 16), (_lib.W_BF16, 8192, 8192, 8, 16, 8), (_lib.W_BF16, 11008, 4096, 4, 16, 16),
+    (_lib.W_BF16, 4096, 12352, 4, 4, 8), (_lib.W_BF16, 4096, 12352, 5, 8, 16), (_lib.W_BF16, 8192, 8192, 4, 4, 16), (_lib.W_BF16, 8192, 8192, 8, 16, 8), (_lib.W_BF16, 11008, 4096, 4, 16, 8),
     (_lib.W_BF16, 3072, 768, 16, 16, 16)])
 def test_several_rows_on_dense_weights(dtype, k, n, rows, cols, waves):
     p = plan(dtype, k, n, rows)
@@ -91,6 +91,18 @@ def test_several_rows_on_dense_weights(dtype, k, n, rows, cols, waves):
 def test_wide_rows_of_f32(k, n, rows, cols, waves):
     p = plan(_lib.W_F32, k, n, rows)
     assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", cols, waves)
+
+
+# bf16, waves by pairs a wave: eight waves of three pairs were slower than twelve of two (4 rows of 1536 x 12352 10.7 us and 8.5, 8 of 1536 x 5000 7.1 and 6.4), eight of 32
+# where sixteen keep two in registers (4 of 2048 x 12352 12.4 and 11.6), eight that begin 4 KiB apart (4 of 16384 x 3600 26.2, with twelve 22.4); sixteen of 33 and more
+# (8 of 2112 x 12352 21.2, with eight 15.7)
+@pytest.mark.parametrize("k,n,rows,waves", [
+    (1536, 12352, 4, 12), (1536, 5000, 8, 12), (1536, 8192, 4, 8), (2048, 12288, 4, 8), (2048, 12304, 4, 16), (2048, 12352, 2, 16), (2048, 4096, 8, 8), (2048, 8192, 5, 8),
+    (2048, 8208, 8, 16), (2112, 12352, 8, 8), (2112, 12352, 16, 16), (4224, 4096, 4, 8), (16384, 3600, 4, 12), (16384, 6176, 8, 12), (16384, 3072, 1, 12), (11008, 3072, 1, 8),
+    (11264, 3072, 1, 8), (32768, 3072, 8, 8), (11008, 4096, 16, 16)])
+def test_waves_of_bf16_rows(k, n, rows, waves):
+    p = plan(_lib.W_BF16, k, n, rows)
+    assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", 16, waves)
 
 
 # Prompts: the shapes that test_gpu_narrow_gemm.py, test_gpu_sum_error.py and test_gpu_large_tiles.py multiply reach all five small tiles, shares of k on
