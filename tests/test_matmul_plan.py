@@ -93,6 +93,15 @@ def test_wide_rows_of_f32(k, n, rows, cols, waves):
     assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", cols, waves)
 
 
+# f32, short rows of very many outputs: four waves a workgroup took 1.14 times as long as those that have two pairs each (128 x 50257, 2 - 16 rows)
+@pytest.mark.parametrize("k,n,rows,waves", [
+    (96, 28747, 4, 2), (128, 50257, 2, 2), (128, 50257, 16, 2), (320, 28747, 8, 5), (512, 50257, 4, 8), (128, 20001, 4, 2), (128, 20000, 4, 4), (544, 50257, 4, 4),
+    (320, 8192, 4, 4)])
+def test_short_rows_of_f32(k, n, rows, waves):
+    p = plan(_lib.W_F32, k, n, rows)
+    assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", 16, waves)
+
+
 # bf16, waves by pairs a wave: eight waves of three pairs were slower than twelve of two (4 rows of 1536 x 12352 10.7 us and 8.5, 8 of 1536 x 5000 7.1 and 6.4), eight of 32
 # where sixteen keep two in registers (4 of 2048 x 12352 12.4 and 11.6), eight that begin 4 KiB apart (4 of 16384 x 3600 26.2, with twelve 22.4); sixteen of 33 and more
 # (8 of 2112 x 12352 21.2, with eight 15.7)
