@@ -2206,8 +2206,8 @@ static uint32_t gemv_one_row_steps(const Weight &w, uint64_t batch, bool gated) 
 // bf16 16384 x 3600 22.6 / 26.2 / 22.4, f32 8192 x 4096 27.4 / 30.0 / 24.0).
 // f32: eight (16 / 8: 4 rows of 768 x 3072 4.9 / 4.5, 1024 x 3600 6.1 / 5.3); four where there are several tiles a CU and rows are short of 4096 (16 / 8 / 4: 1024 x 4608 8.3 /
 // 7.3 / 6.6, 2048 x 8192 15.0 / 13.8 / 13.7; but 4 rows of 8224 x 8192 48.1 / 46.2 / 60.1, 16 of 4096 x 8192 26.5 / 24.6 / 30.4) or 32 KiB apart (16 of 16384 x 4112 101 / 88 / 82).  Very many outputs of rows
-// up to 512 long want as many waves as have two pairs in registers (time with four over that, mean of 2 - 16 rows: 128 x 50257 1.14, x 28747 1.11, 320 x 50257 1.12, 512 x
-// 50257 1.04, but 20000 outputs of 64 - 512 0.98 and 576 x 50257 0.92).
+// 96 to 512 long want as many waves as have two pairs in registers (time with four over that, mean of 2 - 16 rows: 128 x 50257 1.14, x 28747 1.11, 320 x 50257 1.12, 512 x
+// 50257 1.04, but 20000 outputs of 96 - 512 0.98, 576 x 50257 0.92, 64 x 28747 0.93).
 struct MfmaPlain { bool runs; uint32_t parts, waves; size_t lds; };
 template <bool BF16>
 static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
@@ -2219,7 +2219,7 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
         uint64_t waves = gemv_mfma_waves(pairs);
         if (parts == 4) waves = pairs <= 12 ? std::max<uint64_t>(4, ceil_div(pairs, 2)) : std::min<uint64_t>(16, four);
         else if (parts == 2) waves = pairs >= 128 ? 16 : std::min<uint64_t>(8, four);
-        else if (w.n > 4096) waves = pairs <= 16 && w.n > 20000 ? waves : pairs < 128 || pairs % 256 == 0 ? 4 : 8;
+        else if (w.n > 4096) waves = pairs > 2 && pairs <= 16 && w.n > 20000 ? waves : pairs < 128 || pairs % 256 == 0 ? 4 : 8;
         else if (xbp < 16) waves = pairs == 256 ? 12 : std::min<uint64_t>(8, four);
         return (uint32_t)std::min<uint64_t>(waves, std::max<uint64_t>(1, pairs));
     };

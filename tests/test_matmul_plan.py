@@ -96,7 +96,7 @@ def test_wide_rows_of_f32(k, n, rows, cols, waves):
 # f32, short rows of very many outputs: four waves a workgroup took 1.14 times as long as those that have two pairs each (128 x 50257, 2 - 16 rows)
 @pytest.mark.parametrize("k,n,rows,waves", [
     (96, 28747, 4, 2), (128, 50257, 2, 2), (128, 50257, 16, 2), (320, 28747, 8, 5), (512, 50257, 4, 8), (128, 20001, 4, 2), (128, 20000, 4, 4), (544, 50257, 4, 4),
-    (320, 8192, 4, 4)])
+    (320, 8192, 4, 4), (64, 28747, 8, 2)])
 def test_short_rows_of_f32(k, n, rows, waves):
     p = plan(_lib.W_F32, k, n, rows)
     assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", 16, waves)
