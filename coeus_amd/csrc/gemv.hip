@@ -1571,9 +1571,10 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
         }
     }
     // Every second pair adds up in accumulators of its own, f32's halves of one too, so that few waves' sums are no longer than many's: not
-    // shares of two pairs, and not where sixteen rows of bf16 leave no registers.  f32 in four parts: the quarters of both pairs, which
+    // shares of two pairs, unless of bf16 in two parts (8 rows of 2560 x 12352, whose waves would have one sum of twice the products they have
+    // in one part: error to 64 bits 1.1e-7 in one part, 1.24e-7 with one sum, 9.9e-8 so), and not where sixteen rows of bf16 leave no registers.  f32 in four parts: the quarters of both pairs, which
     // makes two or three rows as exact as a wave per row (768 x 768, error to that form's 1.04 with halves, 0.94 so; 1.6 with one).
-    constexpr int AS = (KEEP && (BF16 || TS < 4)) || (BF16 && XQ == 4 && TS == 1) ? 1 : 2, AH = (KEEP && TS < 4) || BF16 ? 1 : KEEP ? 4 : 2;
+    constexpr int AS = (KEEP && (BF16 ? TS != 2 : TS < 4)) || (BF16 && XQ == 4 && TS == 1) ? 1 : 2, AH = (KEEP && TS < 4) || BF16 ? 1 : KEEP ? 4 : 2;
     float4_t acc[AS][AH] = {};
     auto total = [&]() {
         float4_t t[AS];
@@ -2191,8 +2192,10 @@ static uint32_t gemv_one_row_steps(const Weight &w, uint64_t batch, bool gated) 
 // Parts: as many as leave at most a workgroup per CU, four up to 1024 outputs, two up to 2048; bf16 from lengths on at which a tile's trip
 // is long enough to halve (us, one / two / four parts: 4 rows of 768 x 768 3.5 / 4.0 / 3.7, 1024 x 1024 3.9 / 3.9 / 3.8, 2048 x 2048 4.7 / 4.9 / 5.2, 4096 x 2048
 // 7.6 / 6.8 / 7.1, and four where the shares are two pairs that stay in registers, 5632 x 2048 10.1 / 8.7 / 8.0; 8 rows of 1024 x 1024 4.2 / 4.2, 2048 x
-// 2048 5.6 / 5.2).  Beyond 4096 outputs a CU takes several tiles, and smaller ones even out their number: bf16 from 4096 of k on, as long as a wave's
-// share is two pairs (4 rows 4096 x 4608 12.7 / - / 10.5, x 12352 24.2 / 20.8 / 20.3; but 4096 x 4096 8.4 / 10.4 / 10.0, 8 rows of 6144 x 8192 24.6 / 32.1).
+// 2048 5.6 / 5.2).  Beyond 4096 outputs a CU takes several tiles, and smaller ones even out their number: bf16 where that brings a wave's
+// share down to two pairs, which stay in registers: up to 4 rows from 4096 of k to 8192 (4096 x 4608 12.7 / - / 10.5, x 12352 24.2 / 20.8 / 20.3; but 4096 x 4096 8.4 / 10.4 /
+// 10.0), 8 rows beyond 2048 to 4096 (one / two: 2560 x 8192 13.0 / 10.8, x 12352 20.4 / 14.2, 3584 x 4608 13.3 / 11.0, x 22016 37.2 / 27.6, 4096 x 12352 24.8 / 20.4; 2048 x 12352 12.7 /
+// 12.3 with shares that are two pairs already; longer ones are not, 4224 x 8192 17.0 / 24.1, 4608 x 12352 28.5 / 37.8, 6144 x 8192 22.2 / 29.9).
 // f32 from 4096 on up to 5120 outputs, whose tiles of 16 leave the second round of workgroups nearly empty, if the waves' shares come out even, and
 // wherever rows are 32 KiB apart (us, one part with sixteen waves / with eight / parts: 4 rows of 5632 x 5000 27.1 / 25.7 / 23.9, 8 of 8192 x 8192 50.7 / 62.2 /
 // 50.4; but 4 of 5632 x 8192 30.5 / 29.3 / 36.8, 8704 x 8192 44.9 / 44.1 / 67.3, 11008 x 8192 60.2 / 62.3 / 71.2, 9216 x 4112 in uneven shares 39.3 / 39.0 / 40.1;
@@ -2232,7 +2235,7 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
         if (w.n <= 1024 && w.k >= 1024 && fits(4)) parts = 4;
         else if (w.n <= 2048 && w.k > 4096 && w.k <= 8192 && fits(4)) parts = 4;
         else if (w.n > 4096 && w.k >= 4096 && w.k <= 8192 && fits(4)) parts = 4;
-        else if (((w.n <= 2048 && w.k >= (xbp == 8 || w.n <= 1024 ? 2048 : 4096)) || (w.n > 4096 && w.k == 4096)) && fits(2)) parts = 2;
+        else if (((w.n <= 2048 && w.k >= (xbp == 8 || w.n <= 1024 ? 2048 : 4096)) || (w.n > 4096 && w.k > 2048 && w.k <= 4096 && xbp == 8)) && fits(2)) parts = 2;
     } else if (w.k >= 256) {
         auto wide = [&](uint32_t p) { return w.n > 4096 && w.k >= 4096 && (w.k % 8192 == 0 || (w.n <= 5120 && even(p))); };
         if (fits(4) && (w.n <= 1024 || wide(4))) parts = 4;

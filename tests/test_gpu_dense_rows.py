@@ -42,7 +42,7 @@ def test_rows_match_float64(orc, dtype, k, n, batch):
 
 # Tiles of 4 and 8 weight rows whose lines are parts of k: tiles that end inside the matrix, one pair a wave, shares of one, two and more pairs,
 # several tiles a workgroup, gated pairs, and one more row of weights or 64 of k than the rule allows
-@pytest.mark.parametrize("k,n", [(128, 5), (768, 6), (1024, 1022), (1280, 1024), (2816, 1030), (3072, 7), (4096, 4098), (5632, 2046), (6144, 4100), (8192, 1026), (4160, 1000)])
+@pytest.mark.parametrize("k,n", [(128, 5), (768, 6), (1024, 1022), (1280, 1024), (2816, 1030), (3072, 7), (4096, 4098), (5632, 2046), (6144, 4100), (8192, 1026), (4160, 1000), (2176, 4102), (2560, 8210)])
 @pytest.mark.parametrize("batch", [2, 3, 4, 5, 8])
 @pytest.mark.parametrize("dtype", [_lib.W_BF16, _lib.W_F32])
 def test_parts_of_k(orc, dtype, k, n, batch):

@@ -93,6 +93,15 @@ def test_wide_rows_of_f32(k, n, rows, cols, waves):
     assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", cols, waves)
 
 
+# bf16, 5 - 8 rows beyond 4096 outputs: two parts of k where the waves' shares are two pairs then (2560 x 12352 20.4 us in one part, 14.2 in two; 4224 x 8192 17.0 and 24.1)
+@pytest.mark.parametrize("k,n,rows,cols,waves", [
+    (2048, 8192, 8, 16, 8), (2176, 4098, 8, 8, 9), (2560, 12352, 5, 8, 10), (3584, 22016, 8, 8, 14), (3968, 4097, 8, 8, 16), (4096, 12352, 8, 8, 16), (2112, 12352, 8, 16, 8),
+    (4160, 8192, 8, 16, 8), (4224, 8192, 8, 16, 8), (2560, 4096, 8, 16, 8), (2560, 12352, 9, 16, 16)])
+def test_two_parts_of_eight_rows(k, n, rows, cols, waves):
+    p = plan(_lib.W_BF16, k, n, rows)
+    assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", cols, waves)
+
+
 # f32, short rows of very many outputs: four waves a workgroup took 1.14 times as long as those that have two pairs each (128 x 50257, 2 - 16 rows)
 @pytest.mark.parametrize("k,n,rows,waves", [
     (96, 28747, 4, 2), (128, 50257, 2, 2), (128, 50257, 16, 2), (320, 28747, 8, 5), (512, 50257, 4, 8), (128, 20001, 4, 2), (128, 20000, 4, 4), (544, 50257, 4, 4),
