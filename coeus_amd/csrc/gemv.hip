@@ -808,13 +808,14 @@ static int launch_gemv_quad(const Weight &w, const __half *xq, uint64_t batch, c
 
 // Batches of 3 and 4, rows as they are: gemv_rows_kernel or gemv_quad_kernel.  Over 185 sizes (512 - 14336 by 256 - 32000; 3 and 4 rows
 // alike) the former took, as a share of the latter's time: Q4_0 0.67 - 0.98 everywhere; Q8_0 0.79 - 0.95 on more than 256 tiles (a workgroup
-// takes several) and 0.87 - 0.94 up to k = 1024, 2560 - 3072 0.90 - 0.95, beyond 8192 (several passes of the quads) 0.83 - 0.98, but
-// 1.0 at 1536 and 2048 and 1.01 - 1.10 at 4096 - 8192 on up to 256 tiles, where the quads are one pass of 8 - 16 waves and the launch is a
-// single trip.  Narrow rows (k < 1024) belong to models whose norms stay folded, and stay with that kernel.
+// takes several), and on up to 256 tiles by the waves that the quads, 512 of k each, are: two and a little over 0.92 - 0.99 (1024 0.92 - 0.95, 1056 - 1152 0.95 - 0.99),
+// three and four 0.98 - 1.03 (1280 - 2048), five and six 0.87 - 0.95 (2080 - 3072; 3104 0.95, 3584 0.98 and stay), eight to sixteen in one pass, a launch
+// that is a single trip, 0.97 - 1.10 (4096 - 8192), several passes 0.73 - 0.98 (beyond 8192).  Narrow rows (k < 1024) belong to models whose norms
+// stay folded, and stay with that kernel.
 static bool gemv_takes_rows(const Weight &w, uint64_t batch) {
     if (batch > 4) return true;
     if (batch < 3 || w.k < 1024) return false;
-    return w.dtype == COEUS_W_Q4_0 || w.n_pad / 16 > 256 || w.k <= 1024 || (w.k > 2048 && w.k <= 3072) || w.k > 8192;
+    return w.dtype == COEUS_W_Q4_0 || w.n_pad / 16 > 256 || w.k <= 1152 || (w.k > 2048 && w.k <= 3072) || w.k > 8192;
 }
 
 // Batches of 3 to 16: tiles and waves of a workgroup of gemv_rows_kernel.  Every workgroup reads all activation rows, so it

@@ -506,7 +506,7 @@ def test_gemv_rows_shapes(orc, dtype, k, n):
 # waves.  The quants and f16 activations enter exactly, so what is left is the rounding of f32 sums: a wave adds up ceil(k / 128 / waves) x 4 block
 # results of 32 products, then up to 12 waves in fours: below 2^-24 (32 + 4 x 8 + 8) of the sum of absolute products.
 @pytest.mark.parametrize("dtype", ["q4_0", "q8_0"])
-@pytest.mark.parametrize("k,n", [(1024, 18), (1024, 4098), (1056, 513 * 16 - 14), (2080, 768 * 16 + 2), (2560, 1025 * 16 - 2), (8224, 130), (1152, 2049 * 16)])
+@pytest.mark.parametrize("k,n", [(1024, 18), (1024, 4098), (1056, 513 * 16 - 14), (2080, 768 * 16 + 2), (2560, 1025 * 16 - 2), (8224, 130), (1152, 2049 * 16), (1120, 70)])
 def test_three_and_four_rows(orc, dtype, k, n):
     wt, wdq = _seeded(dtype, k, n, k + n)
     rng = np.random.default_rng(k + n)
