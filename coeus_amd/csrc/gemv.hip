@@ -1084,11 +1084,13 @@ __device__ __forceinline__ void one_row(const void *__restrict__ wdata, const fl
         if (512 * ((trips - 1) * D + d) + 8 * lane < k) multiply(d);
 #pragma unroll
     for (int r = 0; r < R; r++) acc[r] = wave_sum(acc[r]);
-    if (epi_gated(e.act)) {
-        if (lane == 0 && j0 + 1 < n) epi_store_gated(e, 0, j0 / 2, acc[0], acc[R - 1]);  // (R == 2)
-    } else if (lane < R && j0 + lane < n) {
-        epi_store<true>(e, 0, j0 + lane, lane ? acc[R - 1] : acc[0]);
+    if constexpr (R == 2) {
+        if (epi_gated(e.act)) {
+            if (lane == 0 && j0 + 1 < n) epi_store_gated(e, 0, j0 / 2, acc[0], acc[1]);
+            return;
+        }
     }
+    if (lane < R && j0 + lane < n) epi_store<true>(e, 0, j0 + lane, lane ? acc[R - 1] : acc[0]);
 }
 
 template <bool BF16, int D>
@@ -1424,12 +1426,11 @@ struct PlainRows {  // f32 weights
 // four 16x16x4 products per 16-byte piece.
 template <bool BF16> struct MfmaType;
 template <> struct MfmaType<true> {
-    struct Frag { uint4 p[3]; };
-    static __device__ __forceinline__ void mul(const uint4 &, const Frag &, float4_t &, float4_t &) {}  // (f32 only)
     typedef uint16_t W;
     typedef SplitRows Rows;
     static constexpr uint32_t KU = 64;
     static constexpr int PIECES = 3, XROWS = 4;  // rows of x that a wave request covers
+    struct Frag { uint4 p[3]; };
     static __device__ __forceinline__ float4_t mul(const uint4 &w, const Frag &x, float4_t acc) {
         union { uint4 u; bf16x8_t v; } uw, ux;
         uw.u = w;
@@ -2175,8 +2176,8 @@ static bool gemv_takes_many(const Weight &w, uint64_t batch, bool gated = false)
     return w.k > 1024 ? w.n >= 8192 : w.k > 512 && w.k < 1024 && w.n >= 20000;
 }
 
-// One plain row of the others: steps in flight of a weight row a wave (0: the general form, for gates, whose pairs it holds in two waves,
-// and lengths that are no multiple of 8).  f32 (us with 2 / 3 / 4 / 6): two where a workgroup a CU and less is all there is (8192 x 1024 8.98 /
+// One plain row of the others: steps in flight of a weight row a wave (f32 1 - 4, bf16 1, 4 or 6: gemv_takes_many has bf16 rows of two steps; 0: the
+// general form, for gates, whose pairs it holds in two waves, and lengths that are no multiple of 8).  f32 (us with 2 / 3 / 4 / 6): two where a workgroup a CU and less is all there is (8192 x 1024 8.98 /
 // 9.18 / 9.04 / 9.43, 16384 x 768 15.1 / - / 15.6), else three or four, whichever asks for fewer steps in vain (4096 x 3072 13.1 / 13.3 / 12.8 /
 // 14.7, 3072 x 3072 10.8 / 10.6 / 10.9 / 10.9).  bf16: four, or six where they are fewer trips with no more in vain (3072 x 768 3.99 / 3.50 / 3.53 / 3.39,
 // 8192 x 1024 6.70 / 5.79 / 5.18 / 5.40); rows 32 KiB apart stay with the general form (16384 x 4608 30.8, two steps of these 34.2, four 32.7).
@@ -2356,10 +2357,10 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     if (const uint32_t steps = norm == 0 && aligned ? gemv_one_row_steps(w, batch, epi_gated(e.act)) : 0) {
 #define COEUS_ONE(DV) hipLaunchKernelGGL((gemv_dense_kernel<BF16, 1, 0, DV>), grid, block, 0, st, w.data, xin, w.k, b, e, ns, nb, eps, ldx, post)
         if (steps == 1) COEUS_ONE(1);
-        else if (steps == 2) COEUS_ONE(2);
-        else if (steps == 3) COEUS_ONE(3);
         else if (steps == 4) COEUS_ONE(4);
-        else COEUS_ONE(6);
+        else if constexpr (BF16) COEUS_ONE(6);
+        else if (steps == 2) COEUS_ONE(2);
+        else COEUS_ONE(3);
 #undef COEUS_ONE
         COEUS_HIP(hipGetLastError());
         return COEUS_OK;
