@@ -10,7 +10,7 @@ decode step (one new token per sequence: every linear weight streamed once, atte
 cached context).  W warm-up steps and K timed steps run as one greedy generation on the device.
 
 Prints ONE JSON line: whole-job tokens/s plus
-  roofline     - the decode matmul (gemv_rows_kernel): algorithmic bytes per launch / average
+  roofline     - the decode matmul (gemv_quad_kernel): algorithmic bytes per launch / average
                  launch duration, timed live with HIP events on the stream the kernels run on
                  (a captured graph of one step's 129 matmul launches, replayed), against 8 TB/s;
   prefill      - the prompt pass of the same run (tokens/s) and the matrix-core roofline of its
@@ -303,6 +303,18 @@ def check_outputs(model, sess, prompt, out, tok0, tok, W, K, ctx, bar=2e-2):
 
 
 # ---------------------------------------------------------------- the other benchmark configurations
+def decode_matmul_kernels(cfg, B):
+    """The kernels of a decode step's matmuls."""
+    if cfg.weight_dtype not in ("q4_0", "q8_0"):
+        return "gemv_many_kernel, gemv_dense_kernel, gemv_row_kernel, gemv_mfma_kernel"
+    if B <= 2:
+        return "gemv_quad_kernel"
+    # three and four sequences: norms in front of narrow matrices, rows below 1024 and some Q8_0 sizes stay with the former
+    if B <= 4 and not (cfg.weight_dtype == "q4_0" and cfg.hidden_dim >= 1536):
+        return "gemv_quad_kernel, gemv_rows_kernel"
+    return "gemv_rows_kernel"
+
+
 def decode_workload(name, batches, K, W, use_graph, check):
     """One of the smaller decode configurations, measured like the headline one: prompt pass, W
     warm-up steps, K timed greedy steps on the device, the decode matmul's roofline from a replayed
@@ -315,7 +327,6 @@ def decode_workload(name, batches, K, W, use_graph, check):
     ctx = wl["ctx"]
     model = TransformerModelPlugin().create_builder().build(cfg, seed=0xC0E05)
     rng = np.random.default_rng(0xC0E06)
-    quant = cfg.weight_dtype in ("q4_0", "q8_0")
     legs = []
     for B in batches:
         sess, prompt, out, dt, prefill_s, tok0, tok = run_decode(model, cfg, B, K, W, ctx, use_graph, rng, True)
@@ -326,9 +337,7 @@ def decode_workload(name, batches, K, W, use_graph, check):
             "value": round(B * K / dt, 2), "unit": "tok/s", "ms_per_step": round(dt * 1e3 / K, 4),
             "prefill": {"tokens": int(B * prompt.shape[1]), "ms": round(prefill_s * 1e3, 2),
                         "tok_s": round(B * prompt.shape[1] / prefill_s, 1)},
-            "roofline": {"kernel": (("gemv_quad_kernel" if B <= (2 if cfg.hidden_dim >= 1536 else 4) else "gemv_rows_kernel") if quant
-                                    else "gemv_many_kernel, gemv_dense_kernel, gemv_row_kernel, gemv_mfma_kernel"),
-                         "bound": "hbm",
+            "roofline": {"kernel": decode_matmul_kernels(cfg, B), "bound": "hbm",
                          "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": None,
                          "bytes_per_launch": alg_bytes // launches, "us_per_launch": round(ms * 1e3 / launches, 3),
@@ -563,8 +572,7 @@ def main():
     ms, launches, alg_bytes = sess.time_decode_matmuls(reps)
     achieved = alg_bytes / (ms * 1e-3) / 1e9
     roofline = {
-        "kernel": (("gemv_quad_kernel" if B <= (2 if cfg.hidden_dim >= 1536 else 4) else "gemv_rows_kernel") if cfg.weight_dtype in ("q4_0", "q8_0")
-                   else "gemv_many_kernel, gemv_dense_kernel, gemv_row_kernel, gemv_mfma_kernel"),
+        "kernel": decode_matmul_kernels(cfg, B),
         "bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "traffic_source": None,
         "bytes_per_launch": alg_bytes // launches, "us_per_launch": round(ms * 1e3 / launches, 3),
