@@ -13,7 +13,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("k,n", [(8, 1), (64, 3), (504, 18), (512, 4), (520, 37), (768, 8195), (1024, 2306), (1032, 7), (1536, 2048), (2048, 2050),
                                  (2056, 9), (4096, 66), (4104, 2049), (5632, 130), (11008, 33),
                                  # (where other kernels take the row: the matrix cores, a wave per row)
-                                 (64, 16390), (512, 16384), (10240, 2054), (1536, 2306), (768, 20002), (1032, 8194)])
+                                 (64, 16390), (512, 16384), (10240, 2054), (1536, 2306), (768, 20002), (1032, 8194),
+                                 # two weight rows a wave again
+                                 (520, 32002), (1544, 16386), (2056, 16386), (3080, 2042)])
 @pytest.mark.parametrize("gated", [False, True])
 def test_matches_float64(orc, dtype, k, n, gated):
     if gated:
