@@ -2166,14 +2166,14 @@ static int launch_gemv_hyper(const Weight &w, uint64_t batch, const EpiArgs &e, 
 // short ones of very many (768 x 50257 0.99, x 32000 1.00, x 22016 1.03; 1032 x 8192 - 50257 1.06 - 1.09).  Gated pairs, against the general form
 // that holds them in two waves: from 1536 of k on beyond 3200 rows, from 1032 and 8192, and up to the 2048 that give every compute unit one workgroup, but not a little beyond
 // these (1536 - 8192 x 1500 - 2048 0.85 - 1.01, x 2304 1.05 - 1.12, x 3600 0.90 - 0.97, x 22016 0.85 - 0.93, x 1024 1.01 - 1.08).  bf16: all that the matrix cores do not take (gemv_uses_mfma), but rows 32 KiB apart, which share their memory channels,
-// are a wave's each between 4096 and 6144 of them (16384 x 4608 1.07, 32768 x 4608 1.14; x 6144 1.00, x 8192 0.86), and so are few
-// rows of exactly one step of 512 (x 300 1.10, x 768 1.11, x 1024 1.06, x 3000 0.97; 448 x 768 0.96), and up to 1024 of more than two steps
-// (1032 x 1030 0.99, x 768 0.98 of the time with a wave per row, 2048 x 1024 0.92, 11008 x 1024 0.80, but 1536 x 1536 1.07).
+// are a wave's each between 4096 and 6144 of them (16384 x 4608 1.07, 32768 x 4608 1.14; x 6144 1.00, x 8192 0.86), and so are up
+// to 8192 rows of one step, without a gate (64 - 512 x 128 - 8192 1.02 of the time in the mean, x 10000 - 16000 0.94; gated pairs of one step 0.85 - 0.97), and up to 1024 of
+// more than two steps (1032 x 1030 0.99, x 768 0.98 of the time with a wave per row, 2048 x 1024 0.92, 11008 x 1024 0.80, but 1536 x 1536 1.07).
 static bool gemv_takes_many(const Weight &w, uint64_t batch, bool gated = false) {
     if (batch != 1 || w.dtype > COEUS_W_BF16 || w.k % 8 || w.k >= (1ull << 31) || w.n >= (1ull << 31) - 8) return false;
     if (w.dtype == COEUS_W_BF16)
         return !gemv_uses_mfma(w, 1, gemv_mfma_waves(w.k / MfmaType<true>::KU), false) && !(w.k % 16384 == 0 && w.n > 4096 && w.n < 6144) &&
-               !(w.k == 512 && w.n < 2048) && (gated || w.k <= 1024 || w.n > 1024);
+               (gated || w.k > 512 || w.n > 8192) && (gated || w.k <= 1024 || w.n > 1024);
     if (w.k >= 1536 && gated) return (w.n > 1024 && w.n <= 2048) || w.n > 3200;
     if (w.k >= 1536) return w.k >= 2048 && w.k % 4096 && (w.n >= 16384 || 12 * round_up(w.n, 2048) <= 13 * w.n);
     return w.k > 1024 ? gated && w.n >= 8192 : w.k > 512 && w.k < 1024 && w.n >= (gated ? 20000 : 32001);

@@ -54,7 +54,7 @@ def test_three_and_four_rows_on_quantised_weights(dtype, k, n, rows):
     (_lib.W_BF16, 11008, 3072, b"gemv_mfma_kernel"), (_lib.W_BF16, 11008, 2048, b"gemv_many_kernel"), (_lib.W_BF16, 11008, 4096, b"gemv_many_kernel"),
     (_lib.W_BF16, 8192, 3072, b"gemv_many_kernel"), (_lib.W_BF16, 16384, 4608, b"gemv_dense_kernel"), (_lib.W_BF16, 16384, 6144, b"gemv_many_kernel"),
     (_lib.W_BF16, 16384, 4096, b"gemv_many_kernel"), (_lib.W_BF16, 770, 770, b"gemv_dense_kernel"), (_lib.W_BF16, 768, 50257, b"gemv_many_kernel"),
-    (_lib.W_BF16, 512, 768, b"gemv_dense_kernel"), (_lib.W_BF16, 512, 2048, b"gemv_many_kernel"), (_lib.W_BF16, 448, 768, b"gemv_many_kernel"),
+    (_lib.W_BF16, 512, 768, b"gemv_dense_kernel"), (_lib.W_BF16, 448, 8192, b"gemv_dense_kernel"), (_lib.W_BF16, 512, 8193, b"gemv_many_kernel"), (_lib.W_BF16, 520, 768, b"gemv_many_kernel"),
     (_lib.W_F32, 3072, 2304, b"gemv_dense_kernel"), (_lib.W_F32, 3072, 2048, b"gemv_many_kernel"), (_lib.W_F32, 1536, 3201, b"gemv_dense_kernel"),
     (_lib.W_F32, 3072, 1900, b"gemv_many_kernel"), (_lib.W_F32, 3072, 1890, b"gemv_dense_kernel"), (_lib.W_F32, 3072, 3600, b"gemv_dense_kernel"), (_lib.W_F32, 3072, 4090, b"gemv_many_kernel"),
     (_lib.W_F32, 2048, 9216, b"gemv_dense_kernel"), (_lib.W_F32, 2048, 17408, b"gemv_many_kernel"), (_lib.W_F32, 4096, 22016, b"gemv_dense_kernel"), (_lib.W_F32, 768, 32000, b"gemv_dense_kernel"),
