@@ -2210,8 +2210,9 @@ static uint32_t gemv_one_row_steps(const Weight &w, uint64_t batch, bool gated) 
 // 12288 - 24576 long 0.96 - 1.02 of the time; sixteen rows are not faster, 2048 x 1024 6.5 / 7.0).  Of 32 pairs, two for each of sixteen waves that stay in
 // registers, as long as outputs are few (4 rows of 2048 x 6176 7.9 / 7.0, x 11264 0.93 of the time, x 12352 11.6 / 12.4; 8 of x 8192 0.90, x 9000 1.04, x 12352 1.12); of
 // fewer as many as have two, or three where that comes out even, asked for at once (4 rows of 768 x 2304, two / three: 3.83 / 3.60; - x 10272 5.65 / 5.84, 1536 x 12352
-// 8.5 / 10.7, 8 of 1536 x 5000 6.4 / 7.1).  Twelve of 256 pairs, where eight begin 4 KiB apart in rows 32 KiB apart and share their memory channels (16 / 8 / 12: 4 rows of
-// bf16 16384 x 3600 22.6 / 26.2 / 22.4, f32 8192 x 4096 27.4 / 30.0 / 24.0).
+// 8.5 / 10.7, 8 of 1536 x 5000 6.4 / 7.1).  Twelve of a multiple of 256 pairs, where eight begin a multiple of 4 KiB apart in rows a multiple of 32 KiB apart and share
+// their memory channels (16 / 8 / 12: 4 rows of bf16 16384 x 3600 22.6 / 26.2 / 22.4, f32 8192 x 4096 27.4 / 30.0 / 24.0; 512 pairs x 2064 - 6176 0.85 - 1.02 of the time with eight, 768
+// 0.92 - 0.98; 252 and 260 pairs 1.00 - 1.05).
 // f32: eight (16 / 8: 4 rows of 768 x 3072 4.9 / 4.5, 1024 x 3600 6.1 / 5.3); four where there are several tiles a CU and rows are short of 4096 (16 / 8 / 4: 1024 x 4608 8.3 /
 // 7.3 / 6.6, 2048 x 8192 15.0 / 13.8 / 13.7; but 4 rows of 8224 x 8192 48.1 / 46.2 / 60.1, 16 of 4096 x 8192 26.5 / 24.6 / 30.4) or 32 KiB apart (16 of 16384 x 4112 101 / 88 / 82).  Very many outputs of rows
 // 96 to 512 long want as many waves as have two pairs in registers (time with four over that, mean of 2 - 16 rows: 128 x 50257 1.14, x 28747 1.11, 320 x 50257 1.12, 512 x
@@ -2228,7 +2229,7 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
         if (parts == 4) waves = pairs <= 12 ? std::max<uint64_t>(4, ceil_div(pairs, 2)) : std::min<uint64_t>(16, four);
         else if (parts == 2) waves = pairs >= 128 ? 16 : std::min<uint64_t>(8, four);
         else if (w.n > 4096) waves = pairs > 2 && pairs <= 16 && w.n > 20000 ? waves : pairs < 128 || pairs % 256 == 0 ? 4 : 8;
-        else if (xbp < 16) waves = pairs == 256 ? 12 : std::min<uint64_t>(8, four);
+        else if (xbp < 16) waves = pairs % 256 == 0 ? 12 : std::min<uint64_t>(8, four);
         return (uint32_t)std::min<uint64_t>(waves, std::max<uint64_t>(1, pairs));
     };
     auto even = [&](uint32_t parts) {
@@ -2251,7 +2252,7 @@ static MfmaPlain gemv_mfma_plain(const Weight &w, uint64_t batch) {
     if (BF16) {
         if (parts > 1) waves = pairs > 32 ? 8 : waves;
         else if (xbp == 4 && pairs % 3 == 0 && pairs >= 9 && pairs <= 24 && w.n <= 8192) waves = (uint32_t)std::max<uint64_t>(waves / 2, pairs / 3);
-        else if (xbp <= 8 && (pairs > 32 || (pairs == 32 && w.n <= (xbp == 4 ? 12288 : 8192)))) waves = pairs == 256 ? 12 : 8;
+        else if (xbp <= 8 && (pairs > 32 || (pairs == 32 && w.n <= (xbp == 4 ? 12288 : 8192)))) waves = pairs % 256 == 0 ? 12 : 8;
     } else {
         waves = f32_waves(parts);
     }

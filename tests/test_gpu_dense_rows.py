@@ -61,7 +61,7 @@ def test_parts_of_k(orc, dtype, k, n, batch):
 
 
 # Long rows in shares that differ by a pair: eight waves of several tiles a workgroup, twelve where rows are 32 KiB apart
-@pytest.mark.parametrize("dtype,k,n", [(_lib.W_F32, 4128, 5130), (_lib.W_F32, 8192, 2070), (_lib.W_BF16, 2112, 5130), (_lib.W_BF16, 16384, 2070)])
+@pytest.mark.parametrize("dtype,k,n", [(_lib.W_F32, 4128, 5130), (_lib.W_F32, 8192, 2070), (_lib.W_BF16, 2112, 5130), (_lib.W_BF16, 16384, 2070), (_lib.W_F32, 16384, 2050)])
 @pytest.mark.parametrize("batch", [1, 2, 4, 8, 16])
 def test_waves_of_long_rows(orc, dtype, k, n, batch):
     rng = np.random.default_rng(k + batch)

@@ -91,7 +91,7 @@ def test_several_rows_on_dense_weights(dtype, k, n, rows, cols, waves):
 @pytest.mark.parametrize("k,n,rows,cols,waves", [
     (8704, 8192, 4, 16, 8), (8704, 8192, 2, 16, 8), (8224, 8192, 4, 16, 8), (5632, 8192, 8, 16, 8), (4096, 8192, 16, 16, 8), (4096, 5121, 4, 16, 8), (4096, 5120, 4, 4, 8),
     (5632, 5000, 4, 4, 11), (8704, 4112, 4, 8, 16), (9216, 4112, 4, 8, 16), (8192, 8192, 8, 8, 16), (8192, 8192, 4, 4, 16), (16384, 4112, 16, 16, 4), (4064, 8192, 16, 16, 4),
-    (2048, 8192, 4, 16, 4), (8192, 4096, 4, 16, 12), (8192, 4096, 8, 16, 12), (8192, 4096, 16, 16, 16), (8224, 4096, 4, 16, 8)])
+    (2048, 8192, 4, 16, 4), (8192, 4096, 4, 16, 12), (8192, 4096, 8, 16, 12), (8192, 4096, 16, 16, 16), (16384, 4096, 4, 16, 12), (12288, 4096, 4, 16, 8), (8224, 4096, 4, 16, 8)])
 def test_wide_rows_of_f32(k, n, rows, cols, waves):
     p = plan(_lib.W_F32, k, n, rows)
     assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", cols, waves)
@@ -121,7 +121,7 @@ def test_short_rows_of_f32(k, n, rows, waves):
 @pytest.mark.parametrize("k,n,rows,waves", [
     (1536, 12352, 4, 12), (1536, 5000, 8, 12), (1536, 8192, 4, 8), (2048, 12288, 4, 8), (2048, 12304, 4, 16), (2048, 12352, 2, 16), (2048, 4096, 8, 8), (2048, 8192, 5, 8),
     (2048, 8208, 8, 16), (2112, 12352, 8, 8), (2112, 12352, 16, 16), (4224, 4096, 4, 8), (16384, 3600, 4, 12), (16384, 6176, 8, 12), (16384, 3072, 1, 12), (11008, 3072, 1, 8),
-    (11264, 3072, 1, 8), (32768, 3072, 8, 8), (11008, 4096, 16, 16)])
+    (11264, 3072, 1, 8), (32768, 3072, 8, 12), (24576, 3072, 8, 8), (11008, 4096, 16, 16)])
 def test_waves_of_bf16_rows(k, n, rows, waves):
     p = plan(_lib.W_BF16, k, n, rows)
     assert (p.kernel, p.tile_cols, p.waves) == (b"gemv_mfma_kernel", 16, waves)
