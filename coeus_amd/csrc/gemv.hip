@@ -1391,7 +1391,7 @@ __device__ __forceinline__ Split2 split2(float a, float b) {
 // k % 64 == 0 and at least one pair of chunks per wave.
 // KEEP: a wave's share of k is at most PD pairs, and its split activations stay in registers from tile to tile.
 // lds: mfma_wave_lds(XQ) uint4 per wave.
-// TS: parts of k (XQ > 0 only, requests for sixteen rows: the columns).
+// TS: parts of k (XQ > 0 only, requests for sixteen rows: the columns).  FOLD: sums of bf16 in groups (f32's always are).
 // (Rows 16 bytes longer than k: at a multiple of 256 bytes apart they would share their banks.)
 struct SplitRows {  // bf16 weights: three pieces
     uint16_t *p;
@@ -1467,7 +1467,7 @@ template <> struct MfmaType<false> {
 // uint4 of a wave's corner: 16 weight rows x 128 bytes; per request of x its rows' KU values in pieces
 template <bool BF16>
 static constexpr uint32_t mfma_wave_lds(int xq) { return 128 + (BF16 ? 96 : 64) * xq; }
-template <bool BF16, int PD, bool KEEP, int XQ, int TS, class Stage>
+template <bool BF16, int PD, bool KEEP, int XQ, int TS, bool FOLD, class Stage>
 __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
                                           uint32_t n, uint32_t batch, uint32_t nw, uint32_t grid, const EpiArgs &e, uint4 *lds,
                                           const typename MfmaType<BF16>::Rows &xs, Stage stage) {
@@ -1577,7 +1577,16 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
     // in one part: error to 64 bits 1.1e-7 in one part, 1.24e-7 with one sum, 9.9e-8 so), and not where sixteen rows of bf16 leave no registers.  f32 in four parts: the quarters of both pairs, which
     // makes two or three rows as exact as a wave per row (768 x 768, error to that form's 1.04 with halves, 0.94 so; 1.6 with one).
     constexpr int AS = (KEEP && (BF16 ? TS != 2 : TS < 4)) || (BF16 && XQ == 4 && TS == 1) ? 1 : 2, AH = (KEEP && TS < 4) || BF16 ? 1 : KEEP ? 4 : 2;
-    float4_t acc[AS][AH] = {};
+    // What a group of PD pairs adds up to starts anew with the next one and joins the sum of the groups, so that the chains of eight waves are no
+    // longer than those of sixteen (error to 64 bits, 8 rows of bf16 11008 x 4096 with sixteen waves / eight / so: 2.0e-7 / 2.9e-7 / 1.3e-7, 4 of f32 5632 x 8192 in parts of
+    // k / eight waves / so: 1.3e-7 / 2.5e-7 / 1.2e-7; 324 launches, time: f32 0.998, bf16 1.003).  bf16 only for more than four pairs a wave (2048 x 2048, 4 rows, 1.02
+    // otherwise) and not where sixteen columns leave no registers.
+    static_assert(!FOLD || (BF16 && !KEEP && XQ < 4), "sums in groups: bf16, several groups, registers left");
+    float4_t acc[AS][AH] = {}, sum_of_groups = {};
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < AS * AH; i++) acc[i / AH][i % AH] = float4_t{0.f, 0.f, 0.f, 0.f};
+    };
     auto total = [&]() {
         float4_t t[AS];
 #pragma unroll
@@ -1585,6 +1594,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
         return AS == 2 ? t[0] + t[AS - 1] : t[0];
     };
     auto group = [&](uint32_t i0, const WRows &next, uint32_t n0, auto request) {
+        if (!BF16) clear();
 #pragma unroll
         for (int s = 0; s < PD; s++) {
             // (LDS serves a wave's stores and loads in order: nothing here waits for another wave)
@@ -1596,7 +1606,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
                 w_request(s, next, n0 + s);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (i0 + s < np) {
+            if ((!BF16 && s == 0) || i0 + s < np) {
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const uint4 wf = wl[c * 8 + ((4 * h + g) ^ (c >> 1))];
@@ -1608,6 +1618,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
             }
             __builtin_amdgcn_wave_barrier();
         }
+        if (!BF16) sum_of_groups = KEEP ? total() : sum_of_groups + total();
     };
     for (;;) {
         const bool ends = gi + 1 == groups;
@@ -1619,11 +1630,15 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
         } else {
             group(gi * PD, wp, 0, [] { return false; });
         }
+        if (FOLD && !ends) {
+            sum_of_groups += total();
+            clear();
+        }
         if (ends) {
             // lane (c, g) holds lines 4 g .. + 3 of column c; a wave's corner of LDS is free
-            if (TS > 1 || c < batch) *(float4_t *)(wl + lane) = total();
-#pragma unroll
-            for (int i = 0; i < AS * AH; i++) acc[i / AH][i % AH] = float4_t{0.f, 0.f, 0.f, 0.f};
+            if (TS > 1 || c < batch) *(float4_t *)(wl + lane) = !BF16 ? sum_of_groups : FOLD ? sum_of_groups + total() : total();
+            if (BF16) clear();
+            sum_of_groups = float4_t{0.f, 0.f, 0.f, 0.f};
             lds_barrier();
             const uint32_t row = tile * R + c;
             for (uint32_t b = wave; b < batch; b += nw) {
@@ -1773,7 +1788,7 @@ static constexpr uint32_t gemv_fold_share(int norm, uint32_t bp) {
 }
 
 // NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
-template <bool BF16, int BP, int NORM, int PD, bool KEEP, int TS = 1>
+template <bool BF16, int BP, int NORM, int PD, bool KEEP, int TS = 1, bool FOLD = false>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
                                                          uint32_t n, uint32_t batch, uint32_t waves, uint32_t grid, EpiArgs e,
                                                          const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
@@ -1784,7 +1799,7 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType
     // a folded norm: the split rows first; what its staging needs lies where the corners will be
     const Rows xs{(decltype(Rows::p))mlds, k, (uint32_t)BP};
     uint4 *corners = NORM ? (uint4 *)((char *)mlds + Rows::bytes(BP, k)) : mlds;
-    mfma_rows<BF16, PD, KEEP, XQ, TS>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
+    mfma_rows<BF16, PD, KEEP, XQ, TS, FOLD>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
         if constexpr (NORM != 0) {
             constexpr uint32_t LONGEST = gemv_fold_row_pairs<BF16>(NORM, BP) * MfmaType<BF16>::KU;
             if (LONGEST <= 1024 || k <= 1024) stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
@@ -2035,7 +2050,7 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
     };
     if constexpr (MF) {
         __builtin_amdgcn_sched_barrier(0);
-        mfma_rows<true, 2, true, 0, 1>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
+        mfma_rows<true, 2, true, 0, 1, false>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
             __builtin_amdgcn_sched_barrier(0);
             normalise();
         });
@@ -2314,12 +2329,13 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
         if (aligned && (nf ? gemv_uses_mfma(w, batch, 16, true) && mlds <= 160 * 1024 : plain.runs)) {
             const uint32_t parts = nf ? 1u : plain.parts, tiles = (uint32_t)ceil_div(w.n, 16 / parts), np = (pairs / parts + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
-#define COEUS_MFMA5(BPV, NV, PV, KV, TV)                                                                                      \
+#define COEUS_MFMA6(BPV, NV, PV, KV, TV, FV)                                                                                  \
     do {                                                                                                                      \
-        static const bool once = [] { (void)hipFuncSetAttribute((const void *)gemv_mfma_kernel<BF16, BPV, NV, PV, KV, TV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); return true; }(); \
+        static const bool once = [] { (void)hipFuncSetAttribute((const void *)gemv_mfma_kernel<BF16, BPV, NV, PV, KV, TV, FV>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); return true; }(); \
         (void)once;                                                                                                           \
-        hipLaunchKernelGGL((gemv_mfma_kernel<BF16, BPV, NV, PV, KV, TV>), mgrid, mblock, mlds, st, (const typename MfmaType<BF16>::W *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
+        hipLaunchKernelGGL((gemv_mfma_kernel<BF16, BPV, NV, PV, KV, TV, FV>), mgrid, mblock, mlds, st, (const typename MfmaType<BF16>::W *)w.data, xin, (uint32_t)w.k, (uint32_t)w.n, b, mw, mgrid.x, e, ns, nb, eps, ldx, post); \
     } while (0)
+#define COEUS_MFMA5(BPV, NV, PV, KV, TV) COEUS_MFMA6(BPV, NV, PV, KV, TV, false)
 #define COEUS_MFMA4(BPV, NV, PV, KV) COEUS_MFMA5(BPV, NV, PV, KV, 1)
             // Pairs in flight: two or three, whichever asks for fewer in vain at the end of a wave's share.  Where that is the
             // same, three for 2 - 4 rows (us for two / three: 4 rows of bf16 5120 x 32000 67.0 / 65.5, 2 of 12288 x 8192 36.5 / 35.0), two
@@ -2331,7 +2347,8 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
             const bool three = norm ? by3 < by2 && tiles > 256 : by3 < by2 || (by3 == by2 && batch > 1 && bp <= 4);
             // (sixteen lines of bf16 ask for sixteen rows of activations: three pairs of them spill)
 #define COEUS_MFMAP(TV) do { if (np <= 2) COEUS_MFMA5(16 / TV, 0, 2, true, TV); else if (!BF16 && three) COEUS_MFMA5(16 / TV, 0, (BF16 ? 2 : 3), false, TV); else COEUS_MFMA5(16 / TV, 0, 2, false, TV); } while (0)
-#define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (BPV < 16 && three) COEUS_MFMA4(BPV < 16 ? BPV : 8, NV, 3, false); else COEUS_MFMA4(BPV, NV, 2, false); } while (0)
+#define COEUS_MFMAL(BPV, NV, FV) do { if (BPV < 16 && three) COEUS_MFMA6(BPV < 16 ? BPV : 8, NV, 3, false, 1, FV); else COEUS_MFMA6(BPV, NV, 2, false, 1, FV); } while (0)
+#define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (pairs > 4 * mw) COEUS_MFMAL(BPV, NV, (BF16 && NV == 0 && BPV < 16)); else COEUS_MFMAL(BPV, NV, false); } while (0)
 #define COEUS_MFMAN(BPV, NV)                                                                               \
     do {                                                                                                   \
         if constexpr (gemv_fold_share<BF16>(NV, BPV) > 2) COEUS_MFMA3(BPV, NV);                             \
@@ -2351,8 +2368,10 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
 #undef COEUS_MFMA
 #undef COEUS_MFMAN
 #undef COEUS_MFMA3
+#undef COEUS_MFMAL
 #undef COEUS_MFMA4
 #undef COEUS_MFMA5
+#undef COEUS_MFMA6
 #undef COEUS_MFMAP
             COEUS_HIP(hipGetLastError());
             return COEUS_OK;

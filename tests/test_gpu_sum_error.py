@@ -36,3 +36,14 @@ def test_prompts_of_few_tiles(orc, dtype, m, k, n, limit):
     ar, wd = (orc.bf16_round(ar), wd) if dtype == _lib.W_BF16 else (ar.astype(np.float16), wd.astype(np.float16))
     want = ar.astype(np.float64) @ wd.astype(np.float64)
     assert _rms(wt.gemm(dev(a))[rows], want) <= limit
+
+
+# Limits: waves of bf16 rows sixteen a workgroup, of f32 rows in four parts of k, chains from a wave's first pair to its last, and 2 % for other inputs
+@pytest.mark.parametrize("dtype,k,n,rows,limit", [(_lib.W_BF16, 11008, 4096, 8, 2.08e-7), (_lib.W_BF16, 4224, 6176, 8, 1.32e-7), (_lib.W_BF16, 4096, 4096, 8, 1.30e-7),
+                                                  (_lib.W_BF16, 2816, 4096, 4, 1.17e-7), (_lib.W_BF16, 2560, 12352, 8, 1.12e-7), (_lib.W_F32, 5632, 8192, 4, 1.29e-7),
+                                                  (_lib.W_F32, 4096, 8192, 8, 1.62e-7)])
+def test_decode_rows_on_dense_weights(dtype, k, n, rows, limit):
+    wt = Weight(dtype, seed=3, shape=(k, n))
+    x = np.random.default_rng(k).standard_normal((rows, k)).astype(np.float32)
+    want = x.astype(np.float64) @ wt.dequantize().astype(np.float64)
+    assert _rms(wt.gemv(dev(x)), want) <= limit
