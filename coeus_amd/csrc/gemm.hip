@@ -1,8 +1,8 @@
 // Prefill matmul: C[m, n] = A[m, k] . W (math::matmul, MT:50-74) on the matrix cores.
 //
-//   gemm_f32_kernel   f32 weights [n][k]: v_mfma_f32_32x32x2_f32 (full f32 products and
-//                     accumulation), 64x64 workgroup tile, 32-wide k slices staged in LDS, three
-//                     slices requested ahead.
+//   f32 weights [n][k]: v_mfma_f32_32x32x2_f32 (full f32 products and accumulation)
+//     gemm_f32_small_kernel, gemm_f32_kernel  k % 4 == 0: tiles of 32 to 128 rows, slices of k loaded straight into a ring of LDS regions
+//     gemm_f32_any_small_kernel, gemm_f32_any_kernel  any k: 32x32 and 64x64 tiles, register-staged
 //   16-bit kernels    bf16 / Q8_0 / Q4_0 weights: v_mfma_f32_32x32x16_{bf16,f16}; activations are
 //                     rounded to the matrix-core input type (bf16 for bf16 weights, f16 for
 //                     quantised weights, which are expanded to f16(q * d) first).
@@ -14,6 +14,7 @@
 //     gemm_qskinny_kernel  up to 64 rows on quantised weights: streams the quantised blocks
 //     gemm_split_reduce_kernel, gemm_tail_reduce_kernel: sums behind launches split along k
 #include "device_utils.hpp"
+#include <type_traits>
 
 namespace coeus {
 
@@ -23,17 +24,7 @@ constexpr int BM = 64, BN = 64, BK = 32, F32_AHEAD = 3;
 // operand = 512 pieces over 256 threads), zero past the edges.
 struct F32Slice { float4 a0, a1, w0, w1; };
 
-// VEC (k % 4 == 0): one unconditional 16-byte load from a clamped address, zeroed afterwards if the
-// piece lies outside the matrix.  (A load under a branch would make the compiler wait for every
-// load in flight, the slices requested ahead included, before the first use.)
-template <bool VEC>
-__device__ __forceinline__ float4 f32_piece(const float *__restrict__ base, uint64_t row, uint64_t rows,
-                                            uint64_t k, uint64_t kk) {
-    if (VEC) {
-        const bool in = row < rows && kk < k;  // k % 4 == 0: a piece is all in or all out
-        const float4 t = *(const float4 *)(base + (row < rows ? row : rows - 1) * k + (kk < k ? kk : 0));
-        return in ? t : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+__device__ __forceinline__ float4 f32_piece(const float *__restrict__ base, uint64_t row, uint64_t rows, uint64_t k, uint64_t kk) {
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (row >= rows) return v;
     if (kk < k) v.x = base[row * k + kk];
@@ -43,8 +34,9 @@ __device__ __forceinline__ float4 f32_piece(const float *__restrict__ base, uint
     return v;
 }
 
-template <bool VEC, bool KV>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__ a,
+// Rows that 16-byte pieces do not lie in (k % 4 != 0, or an input that starts between two of them); every other product is gemm_f32_tile's.
+template <bool KV>
+__global__ __launch_bounds__(256) void gemm_f32_any_kernel(const float *__restrict__ a,
                                                        const float *__restrict__ w, uint64_t m,
                                                        uint64_t n, uint64_t k, EpiArgs e) {
     // k-major tiles: element (row, kk) at [kk][row]; +4 padding keeps the transposing stores
@@ -65,10 +57,10 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__
     auto fetch = [&](uint64_t sl) -> F32Slice {
         F32Slice f;
         const uint64_t kk = sl * BK + lk;
-        f.a0 = f32_piece<VEC>(a, m0 + lrow, m, k, kk);
-        f.a1 = f32_piece<VEC>(a, m0 + lrow + 32, m, k, kk);
-        f.w0 = f32_piece<VEC>(w, n0 + lrow, n, k, kk);
-        f.w1 = f32_piece<VEC>(w, n0 + lrow + 32, n, k, kk);
+        f.a0 = f32_piece(a, m0 + lrow, m, k, kk);
+        f.a1 = f32_piece(a, m0 + lrow + 32, m, k, kk);
+        f.w0 = f32_piece(w, n0 + lrow, n, k, kk);
+        f.w1 = f32_piece(w, n0 + lrow + 32, n, k, kk);
         return f;
     };
     auto put = [&](uint32_t buf, const F32Slice &f) {
@@ -130,8 +122,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__
 constexpr int SM = 32, SN = 32, F32S_AHEAD = 6;
 struct F32SliceS { float4 a, w; };
 
-template <bool VEC, bool KV>
-__global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float *__restrict__ a,
+template <bool KV>
+__global__ __launch_bounds__(256) void gemm_f32_any_small_kernel(const float *__restrict__ a,
                                                              const float *__restrict__ w, uint64_t m,
                                                              uint64_t n, uint64_t k, uint32_t splits, EpiArgs e) {
     __shared__ float as[4][2][8][SM + 4];  // per wave: two buffers of 8 k x 32 rows, k-major
@@ -150,8 +142,8 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float *__rest
     if (splits > 1) e.out_f32 += (uint64_t)blockIdx.z * m * e.n_eff;
     auto fetch = [&](uint64_t sl) -> F32SliceS {
         F32SliceS f;
-        f.a = f32_piece<VEC>(a, m0 + lrow, m, k, sl * BK + 8 * wave + lk);
-        f.w = f32_piece<VEC>(w, n0 + lrow, n, k, sl * BK + 8 * wave + lk);
+        f.a = f32_piece(a, m0 + lrow, m, k, sl * BK + 8 * wave + lk);
+        f.w = f32_piece(w, n0 + lrow, n, k, sl * BK + 8 * wave + lk);
         return f;
     };
     auto put = [&](uint32_t buf, const F32SliceS &f) {
@@ -203,74 +195,6 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float *__rest
         if (!gated) epi_store<KV>(e, row, col, v);
         else if ((lane & 1) == 0) epi_store_gated(e, row, col >> 1, v, other);
     }
-}
-
-__global__ void gemm_split_reduce_kernel(const float *__restrict__ part, uint32_t splits, uint64_t m, uint64_t n,
-                                         EpiArgs e);  // (defined with the 16-bit kernels below)
-
-static bool gemm_f32_is_small(const Weight &w, uint64_t m) {
-    return ceil_div(w.n, BN) * ceil_div(m, BM) < 256;  // fewer 64x64 tiles than CUs
-}
-
-// The 32x32-tile kernel takes 7-8 us plus about 0.3 us per 32-wide slice of k whatever the launch's
-// size, so a long k on few tiles (the FFN's second matmul on a 128-token prompt: 96 slices, 96
-// workgroups, 36-41 us) is split along k over up to 8 workgroups per tile, at least 12 slices each
-// and about three workgroups per CU in all, and gemm_split_reduce_kernel sums the planes in split
-// order and runs the epilogue (8 + 5 us).  Below 48 slices the second launch costs what the split
-// saves (768-long k, 128 rows: 16.5 us unsplit, 17.7 + 4.7 us in two shares).
-static uint32_t gemm_f32_splits_wanted(const Weight &w, uint64_t m) {
-    if (w.dtype != COEUS_W_F32 || m == 0 || !gemm_f32_is_small(w, m) || gemv_takes_f32_rows(w, m)) return 1;
-    const uint64_t wgs = ceil_div(w.n, SN) * ceil_div(m, SM), slices = ceil_div(w.k, BK);
-    if (slices < 48) return 1;
-    uint64_t s = 768 / wgs;
-    if (s > slices / 12) s = slices / 12;
-    if (s > 8) s = 8;
-    return s < 2 ? 1 : (uint32_t)s;
-}
-
-static int launch_gemm_f32(const Weight &w, const float *a, uint64_t m, const Epilogue &ep,
-                           const GemmScratch &scr, hipStream_t st) {
-    // Up to 16 rows: the decode matmul, which gives a weight row's k to 16 waves instead of 4 and requests all of it at
-    // once (5 rows, 768 x 2304 / 768 x 768 / 768 x 3072 / 3072 x 768: 11.5 / 12.3 / 12.1 / 7.9 + 4.7 us here).
-    if (gemv_takes_f32_rows(w, m)) {
-        if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
-        for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) COEUS_TRY(launch_gemv(w, a, m, ep, st));
-        if (scr.ev_end) COEUS_HIP(hipEventRecord(scr.ev_end, st));
-        return COEUS_OK;
-    }
-    const EpiArgs e = make_epi(ep, w.n);
-    const dim3 grid((unsigned)ceil_div(w.n, BN), (unsigned)ceil_div(m, BM));
-    const bool small = gemm_f32_is_small(w, m);
-    uint32_t splits = gemm_f32_splits_wanted(w, m);
-    if (splits > 1 && (!scr.partials || scr.partials_bytes < (uint64_t)splits * m * w.n * 4)) splits = 1;
-    const dim3 sgrid((unsigned)ceil_div(w.n, SN), (unsigned)ceil_div(m, SM), splits);
-    EpiArgs plain;  // a split launch stores bare products: [split][m][n] f32
-    if (splits > 1) {
-        Epilogue pe;
-        pe.out_f32 = scr.partials;
-        plain = make_epi(pe, w.n);
-    }
-    const EpiArgs &ke = splits > 1 ? plain : e;
-    const uint64_t groups = ceil_div(w.n, epi_gated(e.act) ? 8 : 4);
-    if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
-    for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) {
-        // (KV: cache rows; their code in every epilogue costs launches of 128 rows 2 - 3 %, 768 x 768 9.4 -> 9.6 us)
-#define COEUS_F32(VECV, KVV)                                                                                                                        \
-    do {                                                                                                                                            \
-        if (small) hipLaunchKernelGGL((gemm_f32_small_kernel<VECV, KVV>), sgrid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, splits, ke); \
-        else hipLaunchKernelGGL((gemm_f32_kernel<VECV, KVV>), grid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, e);                      \
-    } while (0)
-        if ((w.k & 3) == 0) { if (ke.kv_k) COEUS_F32(true, true); else COEUS_F32(true, false); }
-        else if (ke.kv_k) COEUS_F32(false, true);
-        else COEUS_F32(false, false);
-#undef COEUS_F32
-        if (splits > 1)
-            hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)ceil_div(m * groups, 256)), dim3(256), 0, st,
-                               (const float *)scr.partials, splits, m, w.n, e);
-    }
-    if (scr.ev_end) COEUS_HIP(hipEventRecord(scr.ev_end, st));
-    COEUS_HIP(hipGetLastError());
-    return COEUS_OK;
 }
 
 // ---------------------------------------------------------------- 16-bit inputs
@@ -1664,6 +1588,307 @@ static int launch_narrow_plan(uint32_t rows, uint32_t cols, const uint16_t *a, c
     return cols == 96 ? launch_narrow<BF16, 4, 1, 3>(a, wp, m, w.n, w.k, lda, ldw, splits, period, e, st) : launch_narrow<BF16, 4, 1, 2>(a, wp, m, w.n, w.k, lda, ldw, splits, period, e, st);
 }
 
+
+// ---------------------------------------------------------------- f32 weights
+// k % 4 == 0: slices of 32 L floats a row (L lines of 128 bytes, laid out like the 64-wide slices of the 16-bit kernels) straight into a ring of D
+// regions, two of them on their way while one is multiplied by v_mfma_f32_32x32x2_f32.  A reduction index is only a label: a lane's 16 bytes of a row
+// are four k, and instruction i of four sums over the i-th of lanes 0 - 31 and the i-th of lanes 32 - 63.  WM x WN x KH waves: wave (m, n, h) has
+// RB x NB blocks of 32 x 32 and multiplies steps h, h + KH ... of a slice's 4 L steps of 8 k; the KH sums of an output meet in LDS.
+// A chain of f32 sums is no longer than the 4 L / KH steps of PERIOD slices: their sums are added to those of the slices before.
+// Bound: up to some 128 rows by the way of the first slices from memory and the chain of a workgroup's products (6 slices of 768 k, 0.43 us each where
+// eight waves share a 32x32 tile), beyond that by the products (157 TF at most).  The kernels before took operands through registers into k-major tiles, with
+// 32-byte requests and all requests waited for at each slice.  us, before / this: 768 x 2304, 768 x 768, 768 x 3072, 3072 x 768
+//   17 rows    9.4 / 8.1   9.2 / 7.9   9.2 / 7.9   10.8 / 10.2
+//   128 rows  12.9 / 11.0  9.4 / 8.2  12.9 / 11.1  19.8 / 15.5
+//   512 rows  40.8 / 26.9 13.1 / 11.1 41.1 / 27.1  43.4 / 31.1
+//   1024 rows 56.7 / 41.8 22.2 / 18.5 59.6 / 45.5  74.8 / 49.5
+// and 4096 x 4096 x 4096 1329 / 1075 (128 TF); 768 x 50257 with 17, 128, 1024 rows 75 / 37, 122 / 101, 805 / 682.
+template <int WM, int WN, int RB, int NB, int KH, int L, int D, int PERIOD>
+struct F32Tile {
+    static constexpr int WAVES = WM * WN * KH, ROWS = WM * RB * 32, COLS = WN * NB * 32, SK = 32 * L, STEPS = 4 * L / KH;
+    static constexpr int QA = ROWS / 8 * L / WAVES, QW = COLS / 8 * L / WAVES;  // requests of a wave and slice, 8 rows x 128 bytes each
+    static_assert(QA * WAVES * 8 == ROWS * L && QW * WAVES * 8 == COLS * L && STEPS * KH == 4 * L && D >= 2, "whole requests and steps a wave");
+    static constexpr size_t region = (size_t)(ROWS + COLS) * L * 128, sums = (size_t)KH * ROWS * (COLS + 4) * 4, lds = D * region > sums ? D * region : sums;
+    static_assert(lds <= 160 * 1024, "fits the LDS of a CU");
+};
+
+template <int WM, int WN, int RB, int NB, int KH, int L, int D, int PERIOD>
+__device__ __forceinline__ void gemm_f32_tile(const float *a, const float *w, uint64_t m, uint64_t n, uint32_t k, uint32_t tiles_m, uint32_t tiles_n, uint32_t splits,
+                                              EpiArgs &e) {
+    using T = F32Tile<WM, WN, RB, NB, KH, L, D, PERIOD>;
+    extern __shared__ __attribute__((aligned(16))) char f32_sm[];
+    // consecutive tiles, rows first, on one XCD (see gemm_narrow_kernel; the grid is a multiple of 8)
+    const uint32_t tiles = tiles_m * tiles_n, id = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+    if (id >= tiles * splits) return;
+    const uint32_t split = id / tiles, r = id - split * tiles, tn = r / tiles_m, tm = r - tn * tiles_m;
+    const uint32_t tid = threadIdx.x, lane = tid & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), part = wave % KH, wrow = wave / KH / WN * RB * 32, wcol = wave / KH % WN * NB * 32;
+    const uint64_t m0 = (uint64_t)tm * T::ROWS, n0 = (uint64_t)tn * T::COLS;
+    const uint32_t slices = (k + T::SK - 1) / T::SK, sbeg = (uint32_t)((uint64_t)slices * split / splits), send = (uint32_t)((uint64_t)slices * (split + 1) / splits);
+    if (splits > 1) e.out_f32 += (uint64_t)split * m * e.n_eff;
+    // what this lane requests: bytes of its rows from the tile's first, and its four k of a slice
+    uint32_t row_at[T::QA + T::QW], col_at[T::QA + T::QW];
+    {
+        const uint32_t last_a = (uint32_t)min((uint64_t)T::ROWS - 1, m - 1 - m0), last_w = (uint32_t)min((uint64_t)T::COLS - 1, n - 1 - n0);
+#pragma unroll
+        for (int q = 0; q < T::QA + T::QW; q++) {
+            const bool is_a = q < T::QA;
+            const uint32_t unit = (is_a ? q : q - T::QA) * T::WAVES + wave, per = (is_a ? T::ROWS : T::COLS) / 8;
+            const uint32_t row = unit % per * 8 + (lane >> 3);
+            row_at[q] = min(row, is_a ? last_a : last_w) * (k * 4);
+            col_at[q] = unit / per * 32 + 4 * ((lane & 7) ^ ((row >> 1) & 7));
+        }
+    }
+    const char *const a0 = (const char *)(a + m0 * k), *const w0 = (const char *)(w + n0 * k);
+    auto request = [&](uint32_t s, char *region) {  // (behind the end of a row its last four again, behind the last slice that one)
+        typedef const __attribute__((address_space(1))) void *gptr_t;
+        typedef __attribute__((address_space(3))) void *lptr_t;
+        const uint32_t kk = min(s, send - 1) * T::SK;
+#pragma unroll
+        for (int q = 0; q < T::QA + T::QW; q++) {
+            const bool is_a = q < T::QA;
+            char *to = region + ((is_a ? q : q - T::QA) * T::WAVES + wave) * 1024 + (is_a ? 0 : T::ROWS * L * 128);
+            __builtin_amdgcn_global_load_lds((gptr_t)((is_a ? a0 : w0) + (row_at[q] + 4 * min(kk + col_at[q], k - 4))), (lptr_t)to, 16, 0, 0);
+        }
+    };
+    float16_t acc[RB][NB], total[RB][NB];
+#pragma unroll
+    for (int x = 0; x < RB; x++)
+#pragma unroll
+        for (int y = 0; y < NB; y++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) { acc[x][y][i] = 0.f; total[x][y][i] = 0.f; }
+    const uint32_t frow = lane & 31, fsw = (lane >> 1) & 7;
+    // the products of a slice; EDGE: k ends inside it (what lies behind takes part as zeros)
+    auto multiply = [&](const char *__restrict__ region, uint32_t kk, auto edge) {
+        constexpr bool EDGE = decltype(edge)::value;
+#pragma unroll
+        for (int t = 0; t < T::STEPS; t++) {
+            const uint32_t step = t * KH + part, line = step >> 2, piece = 2 * (step & 3) + (lane >> 5);
+            const uint32_t at = frow * 128 + 16 * (piece ^ fsw);
+            float4_t af[RB], wf[NB];
+#pragma unroll
+            for (int x = 0; x < RB; x++) af[x] = *(const float4_t *)(region + (line * T::ROWS + wrow + 32 * x) * 128 + at);
+#pragma unroll
+            for (int y = 0; y < NB; y++) wf[y] = *(const float4_t *)(region + (T::ROWS * L + line * T::COLS + wcol + 32 * y) * 128 + at);
+            if (EDGE && kk + 32 * line + 4 * piece >= k) {
+#pragma unroll
+                for (int x = 0; x < RB; x++) af[x] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int y = 0; y < NB; y++) wf[y] = float4_t{0.f, 0.f, 0.f, 0.f};
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int x = 0; x < RB; x++)
+#pragma unroll
+                    for (int y = 0; y < NB; y++) acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(wf[y][i], af[x][i], acc[x][y], 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D - 1; d++) request(sbeg + d, f32_sm + d * T::region);
+    uint32_t at = 0, until = PERIOD;
+    for (uint32_t s = sbeg; s < send; s++) {
+        // every wave's requests of slice s have landed (all but the D - 2 newest slices'), and it has read all of slice s - 1
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_s_waitcnt(wait_vm_lds((D - 2) * (T::QA + T::QW)));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t before = at == 0 ? D - 1 : at - 1;
+        request(s + D - 1, f32_sm + before * T::region);
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t kk = s * T::SK;
+        if (kk + T::SK <= k) multiply(f32_sm + at * T::region, kk, std::false_type{});
+        else multiply(f32_sm + at * T::region, kk, std::true_type{});
+        at = at + 1 == D ? 0 : at + 1;
+        if (--until == 0) {
+            until = PERIOD;
+#pragma unroll
+            for (int x = 0; x < RB; x++)
+#pragma unroll
+                for (int y = 0; y < NB; y++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) { total[x][y][i] += acc[x][y][i]; acc[x][y][i] = 0.f; }
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0070);  // the repeats have landed too
+    __syncthreads();
+    constexpr uint32_t TS = T::COLS + 4;
+    float *sums = (float *)f32_sm;
+    {
+        float *mine = sums + (part * T::ROWS + wrow + frow) * TS + wcol + 4 * (lane >> 5);
+#pragma unroll
+        for (int x = 0; x < RB; x++)
+#pragma unroll
+            for (int y = 0; y < NB; y++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const float16_t &c = acc[x][y], &o = total[x][y];
+                    *(float4 *)(mine + x * 32 * TS + y * 32 + 8 * g) = make_float4(o[4 * g] + c[4 * g], o[4 * g + 1] + c[4 * g + 1], o[4 * g + 2] + c[4 * g + 2], o[4 * g + 3] + c[4 * g + 3]);
+                }
+    }
+    __syncthreads();
+    const bool vec4 = epi_vec4(e);
+    const uint32_t live = (uint32_t)min((uint64_t)T::ROWS, m - m0);
+    auto gather = [&](uint32_t q, uint32_t c4) {
+        const float *p = sums + q * TS + c4;
+        float4 v = *(const float4 *)p;
+#pragma unroll
+        for (int h = 1; h < KH; h++) {
+            const float4 o = *(const float4 *)(p + h * T::ROWS * TS);
+            v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
+        }
+        return v;
+    };
+    if (!epi_gated(e.act)) {
+        constexpr uint32_t CG = T::COLS / 4, RP = T::WAVES * 64 / CG;
+        const uint32_t c4 = tid % CG * 4;
+        if (n0 + c4 >= n) return;
+        const KvCols kc = epi_kv_cols(e, n0 + c4, n);
+        for (uint32_t q = tid / CG; q < live; q += RP) {
+            const float4 t = gather(q, c4);
+            float v[4] = {t.x, t.y, t.z, t.w};
+            epi_row4<true>(e, vec4, kc, m0 + q, n0 + c4, n, v);
+        }
+    } else {
+        constexpr uint32_t CG = T::COLS / 8, RP = T::WAVES * 64 / CG;
+        const uint32_t c8 = tid % CG * 8;
+        if (n0 + c8 >= n) return;
+        for (uint32_t q = tid / CG; q < live; q += RP) {
+            const float4 p0 = gather(q, c8), p1 = gather(q, c8 + 4);
+            const float gv[4] = {p0.x, p0.z, p1.x, p1.z}, uv[4] = {p0.y, p0.w, p1.y, p1.w};
+            epi_row4_gated<true>(e, vec4, m0 + q, (n0 + c8) >> 1, n0 + c8, n, gv, uv);
+        }
+    }
+}
+
+template <int WM, int WN, int RB, int NB, int KH, int L, int D, int PERIOD>
+__global__ __launch_bounds__(WM *WN *KH * 64) void gemm_f32_small_kernel(const float *a, const float *w, uint64_t m, uint64_t n, uint32_t k, uint32_t tiles_m,
+                                                                         uint32_t tiles_n, uint32_t splits, EpiArgs e) {
+    gemm_f32_tile<WM, WN, RB, NB, KH, L, D, PERIOD>(a, w, m, n, k, tiles_m, tiles_n, splits, e);
+}
+template <int WM, int WN, int RB, int NB, int KH, int L, int D, int PERIOD>
+__global__ __launch_bounds__(WM *WN *KH * 64) void gemm_f32_kernel(const float *a, const float *w, uint64_t m, uint64_t n, uint32_t k, uint32_t tiles_m,
+                                                                   uint32_t tiles_n, uint32_t splits, EpiArgs e) {
+    gemm_f32_tile<WM, WN, RB, NB, KH, L, D, PERIOD>(a, w, m, n, k, tiles_m, tiles_n, splits, e);
+}
+
+// The tiles, and what a launch of them takes: us = 3.0 + max(alone k, rounds rate k + fixed), k in thousands of one share and `rounds` of 256 workgroups;
+// a split launch's sums cost 3.8 us and 0.35 us for each MB of partial products.  Fitted to 2600 launches (17 to 1024 rows; k 512 to 4096; n 260 to 50257;
+// 1 to 12 shares): the tile and split of least estimated time is on average 0.7 % and at most 9 % slower than the best one of 17 tiles timed.  us, best:
+//   rows             32x32 k128      32x32 k64       64x32           64x64           128x64
+//   128 x 768 x 768  8.2             9.3             10.9            18              -
+//   128 x 3072 x 768 15.7 (2 shares) 15.5 (8)        15.1 (4)        16 (8)          -
+//   256 x 768 x 2304 21              16.7            18.2            19.0            34
+//   1024 x 768 x 2304 62             45.3            41.8            45.4            56
+//   256 x 768 x 50257 350            230             206             183             193
+//   1024 x 768 x 50257 1470          893             796             823             709
+struct F32Shape { uint32_t rows, cols, slice, waves; double rate, fixed, alone; };
+static constexpr F32Shape kF32Shapes[] = {{32, 32, 128, 8, 6.9, 0.1, 0.}, {32, 32, 64, 4, 5.7, 0.9, 8.1}, {64, 32, 64, 8, 9.4, 0.9, 10.4},
+                                          {64, 64, 32, 8, 17., 2., 21.},  {128, 64, 32, 8, 32., 2.4, 37.7}};
+struct F32Plan { uint32_t shape, splits; };
+static F32Plan gemm_f32_plan(const Weight &w, uint64_t m, bool may_split) {
+    F32Plan best{0, 1};
+    double least = 0.;
+    for (uint32_t i = 0; i < sizeof(kF32Shapes) / sizeof(kF32Shapes[0]); i++) {
+        const F32Shape &t = kF32Shapes[i];
+        const uint64_t tiles = ceil_div(m, t.rows) * ceil_div(w.n, t.cols), slices = ceil_div(w.k, t.slice);
+        for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
+            if (s > 1 && (!may_split || slices < 2 * s)) break;
+            const double k = (double)(ceil_div(slices, s) * t.slice) / 1000.;
+            const double us = std::max(t.alone * k, (double)ceil_div(tiles * s, 256) * t.rate * k + t.fixed) + (s > 1 ? 3.8 + 1.4e-6 * s * (double)m * (double)w.n : 0.);
+            if ((i == 0 && s == 1) || us < least) { least = us; best = {i, s}; }
+        }
+    }
+    return best;
+}
+
+// 16-byte requests, and 32-bit places in a tile and in its launch
+static bool gemm_f32_has_tiles(const Weight &w, uint64_t m) {
+    return (w.k & 3) == 0 && w.k < (1u << 22) && ceil_div(m, 32) * ceil_div(w.n, 32) < (1u << 28);
+}
+
+template <int WM, int WN, int RB, int NB, int KH, int L, int D, int PERIOD>
+static int launch_f32_tile(const Weight &w, const float *a, uint64_t m, uint32_t splits, const EpiArgs &e, hipStream_t st) {
+    using T = F32Tile<WM, WN, RB, NB, KH, L, D, PERIOD>;
+    void (*kern)(const float *, const float *, uint64_t, uint64_t, uint32_t, uint32_t, uint32_t, uint32_t, EpiArgs);
+    if constexpr (T::ROWS == 32) kern = gemm_f32_small_kernel<WM, WN, RB, NB, KH, L, D, PERIOD>;
+    else kern = gemm_f32_kernel<WM, WN, RB, NB, KH, L, D, PERIOD>;
+    static const hipError_t room = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::lds);
+    COEUS_HIP(room);
+    const uint32_t tiles_m = (uint32_t)ceil_div(m, T::ROWS), tiles_n = (uint32_t)ceil_div(w.n, T::COLS);
+    hipLaunchKernelGGL(kern, dim3((uint32_t)round_up((uint64_t)tiles_m * tiles_n * splits, 8)), dim3(T::WAVES * 64), T::lds, st, a, (const float *)w.data, m, w.n,
+                       (uint32_t)w.k, tiles_m, tiles_n, splits, e);
+    return COEUS_OK;
+}
+
+// Any k: 64x64 tiles, or 32x32 where there are fewer of those than CUs.  A long k on few tiles is split: at least 12 slices a share and about three
+// workgroups a CU in all (below 48 slices the second launch costs what the split saves).
+static bool gemm_f32_any_is_small(const Weight &w, uint64_t m) { return ceil_div(w.n, BN) * ceil_div(m, BM) < 256; }
+static uint32_t gemm_f32_any_splits(const Weight &w, uint64_t m) {
+    const uint64_t slices = ceil_div(w.k, BK);
+    if (m == 0 || !gemm_f32_any_is_small(w, m) || slices < 48) return 1;
+    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({768 / (ceil_div(w.n, SN) * ceil_div(m, SM)), slices / 12, 8}));
+}
+static uint32_t gemm_f32_splits_wanted(const Weight &w, uint64_t m) {
+    if (m == 0 || gemv_takes_f32_rows(w, m)) return 1;
+    return gemm_f32_has_tiles(w, m) ? gemm_f32_plan(w, m, true).splits : gemm_f32_any_splits(w, m);
+}
+
+static int launch_gemm_f32(const Weight &w, const float *a, uint64_t m, const Epilogue &ep,
+                           const GemmScratch &scr, hipStream_t st) {
+    // Up to 16 rows: the decode matmul, which gives a weight row's k to 16 waves and requests all of it at once (768 x 2304 / 768 x 768 /
+    // 768 x 3072 / 3072 x 768: 16 rows 4.3 / 4.1 / 4.4 / 9.4 us there, 17 rows 8.1 / 7.9 / 7.9 / 10.2 us here).
+    if (gemv_takes_f32_rows(w, m)) {
+        if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
+        for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) COEUS_TRY(launch_gemv(w, a, m, ep, st));
+        if (scr.ev_end) COEUS_HIP(hipEventRecord(scr.ev_end, st));
+        return COEUS_OK;
+    }
+    const EpiArgs e = make_epi(ep, w.n);
+    const bool tiled = gemm_f32_has_tiles(w, m) && ((uintptr_t)a & 15) == 0, small = gemm_f32_any_is_small(w, m);
+    F32Plan plan{0, 1};
+    for (bool may : {true, false}) {
+        plan = tiled ? gemm_f32_plan(w, m, may) : F32Plan{0, may ? gemm_f32_any_splits(w, m) : 1};
+        if (plan.splits == 1 || (scr.partials && scr.partials_bytes >= (uint64_t)plan.splits * m * w.n * 4)) break;
+    }
+    const uint32_t splits = plan.splits;
+    EpiArgs plain;  // a split launch stores bare products: [split][m][n] f32
+    if (splits > 1) {
+        Epilogue pe;
+        pe.out_f32 = scr.partials;
+        plain = make_epi(pe, w.n);
+    }
+    const EpiArgs &ke = splits > 1 ? plain : e;
+    const uint64_t groups = ceil_div(w.n, epi_gated(e.act) ? 8 : 4);
+    const dim3 any_grid((unsigned)ceil_div(w.n, small ? SN : BN), (unsigned)ceil_div(m, small ? SM : BM), splits);
+    if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
+    for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) {
+        if (tiled) {
+            switch (plan.shape) {
+                case 0: COEUS_TRY((launch_f32_tile<1, 1, 1, 1, 8, 4, 3, 2>(w, a, m, splits, ke, st))); break;
+                case 1: COEUS_TRY((launch_f32_tile<1, 1, 1, 1, 4, 2, 3, 4>(w, a, m, splits, ke, st))); break;
+                case 2: COEUS_TRY((launch_f32_tile<2, 1, 1, 1, 4, 2, 3, 4>(w, a, m, splits, ke, st))); break;
+                case 3: COEUS_TRY((launch_f32_tile<2, 2, 1, 1, 2, 1, 3, 4>(w, a, m, splits, ke, st))); break;
+                default: COEUS_TRY((launch_f32_tile<4, 2, 1, 1, 1, 1, 3, 2>(w, a, m, splits, ke, st))); break;
+            }
+        } else if (small) {
+            auto kern = ke.kv_k ? gemm_f32_any_small_kernel<true> : gemm_f32_any_small_kernel<false>;
+            hipLaunchKernelGGL(kern, any_grid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, splits, ke);
+        } else {
+            auto kern = ke.kv_k ? gemm_f32_any_kernel<true> : gemm_f32_any_kernel<false>;
+            hipLaunchKernelGGL(kern, any_grid, dim3(256), 0, st, a, (const float *)w.data, m, w.n, w.k, ke);
+        }
+        if (splits > 1)
+            hipLaunchKernelGGL(gemm_split_reduce_kernel, dim3((unsigned)ceil_div(m * groups, 256)), dim3(256), 0, st,
+                               (const float *)scr.partials, splits, m, w.n, e);
+    }
+    if (scr.ev_end) COEUS_HIP(hipEventRecord(scr.ev_end, st));
+    COEUS_HIP(hipGetLastError());
+    return COEUS_OK;
+}
+
 // Any number of rows: a short prompt leaves most of a 256-row tile empty (rows past the end are
 // clamped on the way in and not stored), and is still several times faster here than in the
 // 128x128 register-staged kernel (1B shape, 16 rows: 24.5 ms per prompt pass there).
@@ -1783,8 +2008,13 @@ uint64_t gemm_split_scratch_bytes(const Weight &w, uint64_t m) {
 coeus_matmul_plan gemm_launch_plan(const Weight &w, uint64_t m) {
     if (w.dtype == COEUS_W_F32) {
         if (gemv_takes_f32_rows(w, m)) return gemv_plan(w, m);
-        if (gemm_f32_is_small(w, m)) return {"gemm_f32_small_kernel", SM, SN, 4, gemm_f32_splits_wanted(w, m), 1};
-        return {"gemm_f32_kernel", BM, BN, 4, 1, 1};
+        if (!gemm_f32_has_tiles(w, m)) {
+            if (gemm_f32_any_is_small(w, m)) return {"gemm_f32_any_small_kernel", SM, SN, 4, gemm_f32_any_splits(w, m), 1};
+            return {"gemm_f32_any_kernel", BM, BN, 4, 1, 1};
+        }
+        const F32Plan plan = gemm_f32_plan(w, m, true);
+        const F32Shape &t = kF32Shapes[plan.shape];
+        return {t.rows == 32 ? "gemm_f32_small_kernel" : "gemm_f32_kernel", t.rows, t.cols, t.waves, plan.splits, 1};
     }
     if (gemm_uses_qskinny(w, m)) return {"gemm_qskinny_kernel", 64, 0, 4, qskinny_splits(w), 1};
     if (!gemm_uses_h256(w, m)) return {"gemm_h_kernel", HM, HN, 4, 1, 1};
