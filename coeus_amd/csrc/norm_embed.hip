@@ -186,7 +186,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float *__restrict_
 }
 
 // Whole-slice statistics, single workgroup: exists for parity with the reference, and serves
-// small slices and callers without a scratch buffer.  Sums are carried in f64 so the result is
+// callers without a scratch buffer and small slices that 16-byte pieces do not fit.  Sums are carried in f64 so the result is
 // within an ulp or two of the reference's sequential Welford update.
 template <bool RMS>
 __global__ __launch_bounds__(1024) void norm_sequence_kernel(const float *__restrict__ x, uint64_t n,
@@ -304,6 +304,56 @@ __global__ __launch_bounds__(256) void norm_sequence_part_kernel(const float *__
     }
 }
 
+// Slices of up to 4096 VM elements in one launch of one workgroup that holds them in registers: bound by one trip to memory for everything and one
+// exchange of both sums (shifted like those above), where the kernel with a loop per sum and one for the results makes three trips after another.
+// us, that one / this, 5, 17, 24, 42 rows of 768: 5.6 / 3.7, 10.5 / 4.7, 13.6 / 6.8, 20.7 / 8.4; one CU's reads and f64 sums grow with the slice.
+template <bool RMS, int VM>
+__global__ __launch_bounds__(1024) void norm_sequence_small_kernel(const float *__restrict__ x, uint32_t n, uint32_t hidden, const float *__restrict__ scale,
+                                                                   const float *__restrict__ bias, float eps, float *y) {
+    __shared__ double sh[2][16];
+    const uint32_t tid = threadIdx.x;
+    float4 v[VM], sc[VM], bi[VM];
+    const float x0 = x[0];
+#pragma unroll
+    for (int u = 0; u < VM; u++) v[u] = *(const float4 *)(x + min((u * 1024 + tid) * 4, n - 4));
+#pragma unroll
+    for (int u = 0; u < VM; u++) {
+        const uint32_t col = min((u * 1024 + tid) * 4, n - 4) % hidden;
+        sc[u] = *(const float4 *)(scale + col);
+        if (!RMS) bi[u] = *(const float4 *)(bias + col);
+    }
+    const double c = RMS ? 0.0 : (double)x0;
+    double s1 = 0.0, s2 = 0.0;
+#pragma unroll
+    for (int u = 0; u < VM; u++) {
+        if ((u * 1024 + tid) * 4 >= n) break;
+        const float p[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const double d = (double)p[i] - c;
+            s1 += d;
+            s2 += d * d;
+        }
+    }
+    s1 = wave_sum_f64(s1);
+    s2 = wave_sum_f64(s2);
+    if ((tid & 63) == 0) { sh[0][tid >> 6] = s1; sh[1][tid >> 6] = s2; }
+    lds_barrier();
+    s1 = 0.0; s2 = 0.0;
+#pragma unroll
+    for (int i = 0; i < 16; i++) { s1 += sh[0][i]; s2 += sh[1][i]; }
+    const double mc = RMS ? 0.0 : s1 / (double)n;
+    const float var = (float)(s2 / (double)n - mc * mc);
+    const float sd = sqrtf(var + eps), meanf = (float)(c + mc);
+#pragma unroll
+    for (int u = 0; u < VM; u++) {
+        if ((u * 1024 + tid) * 4 >= n) break;
+        float4 o = make_float4(sc[u].x * (v[u].x - meanf) / sd, sc[u].y * (v[u].y - meanf) / sd, sc[u].z * (v[u].z - meanf) / sd, sc[u].w * (v[u].w - meanf) / sd);
+        if (!RMS) { o.x += bi[u].x; o.y += bi[u].y; o.z += bi[u].z; o.w += bi[u].w; }
+        *(float4 *)(y + (u * 1024 + tid) * 4) = o;
+    }
+}
+
 size_t norm_sequence_scratch_bytes() { return 2 * kNormSeqMaxGroups * sizeof(double); }
 
 int launch_norm(uint32_t kind, uint32_t scope, const float *x, uint64_t rows, uint64_t hidden,
@@ -317,13 +367,30 @@ int launch_norm(uint32_t kind, uint32_t scope, const float *x, uint64_t rows, ui
     if (scope == COEUS_SCOPE_SEQUENCE) {
         if (y_xq || lp) return fail(COEUS_INVALID_INPUT, "whole-sequence norm has no 16-bit output");
         const uint64_t n = rows * hidden;
-        if (partials && n >= 32768) {
+        const bool rms = kind == COEUS_NORM_RMSNORM;
+        const bool vec = hidden % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)scale | (rms ? 0 : (uintptr_t)bias)) & 15) == 0;
+        // Two launches from 16384 elements (a pass over 32 ids of the 250M model, 25 norms: 0.83 ms with the one-workgroup kernel, 0.75 with two launches;
+        // over 17 ids 0.75 and 0.75); single elements from 32768.
+        const bool parts = partials && n > (vec ? 16384u : 32767u);
+        if (vec && n <= 32768 && !parts) {
+#define COEUS_NSS(VMV)                                                                                                                              \
+    do {                                                                                                                                            \
+        auto kern = rms ? norm_sequence_small_kernel<true, VMV> : norm_sequence_small_kernel<false, VMV>;                                           \
+        hipLaunchKernelGGL(kern, dim3(1), dim3(1024), 0, st, x, (uint32_t)n, (uint32_t)hidden, scale, bias, eps, y);                                \
+    } while (0)
+            if (n <= 4096) COEUS_NSS(1);
+            else if (n <= 8192) COEUS_NSS(2);
+            else if (n <= 16384) COEUS_NSS(4);
+            else COEUS_NSS(8);
+#undef COEUS_NSS
+            COEUS_HIP(hipGetLastError());
+            return COEUS_OK;
+        }
+        if (parts) {
             // at least 1024 elements per workgroup (128 x 768: 96 workgroups; with 4096 per workgroup
             // 24 CUs did the work of a launch that is all latency: 6.4 + 8.2 us)
             const uint64_t chunk = round_up(ceil_div(n, std::min<uint64_t>(kNormSeqMaxGroups, n / 1024)), 4);
             const uint32_t G = (uint32_t)ceil_div(n, chunk);
-            const bool rms = kind == COEUS_NORM_RMSNORM;
-            const bool vec = hidden % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)scale | (rms ? 0 : (uintptr_t)bias)) & 15) == 0;
 #define COEUS_NSP(RMSV, PH, V)                                                                          \
     hipLaunchKernelGGL((norm_sequence_part_kernel<RMSV, PH, V>), dim3(G), dim3(256), 0, st, x, n, chunk, \
                        hidden, scale, bias, eps, partials, y)
