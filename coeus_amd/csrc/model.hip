@@ -90,7 +90,7 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
     auto size = [&](uint64_t r) { return std::min(kHalf, bytes - r * kHalf); };
     auto launch = [&](uint64_t r) -> hipError_t {
         if (++turn == 0) turn = 1;
-        hipLaunchKernelGGL(copy_out_kernel, dim3(16), dim3(256), 0, st, (const uint32_t *)((const char *)src_dev + r * kHalf),
+        hipLaunchKernelGGL(copy_out_kernel, dim3(32), dim3(256), 0, st, (const uint32_t *)((const char *)src_dev + r * kHalf),
                            (uint32_t *)(pin + r % 2 * kHalf), size(r) / 4, flags + r % 2 * kPieces, turn);
         return hipGetLastError();
     };
@@ -99,7 +99,8 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
         return t > before ? t : t + 1;
     };
     for (uint64_t r = 0; r < rounds && r < 2; r++) COEUS_HIP(launch(r));
-    const uint32_t threads = bytes >= kThreadsFrom ? 3 : 1;
+    const uint32_t cpus = std::max(3u, std::thread::hardware_concurrency() / 2);
+    const uint32_t threads = bytes >= kThreadsFrom ? (uint32_t)std::min<uint64_t>({bytes / kPerThread + 1, kThreads, cpus}) : 1;
     std::atomic<bool> stop{false};
     std::atomic<uint64_t> copied[2] = {};  // pieces out of each half, over all rounds
     auto arrived = [&](uint64_t r, uint64_t p) { return __atomic_load_n(flags + r % 2 * kPieces + p, __ATOMIC_ACQUIRE) == turn_of(r); };
@@ -145,7 +146,7 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
             copy(r, p);
         }
     };
-    std::thread others[2];
+    std::thread others[kThreads - 1];
     for (uint32_t t = 1; t < threads; t++) {
         try {
             others[t - 1] = std::thread(helper, t);
