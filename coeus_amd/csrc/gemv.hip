@@ -1575,8 +1575,11 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
     // Every second pair adds up in accumulators of its own, f32's halves of one too, so that few waves' sums are no longer than many's: not
     // shares of two pairs, unless of bf16 in two parts (8 rows of 2560 x 12352, whose waves would have one sum of twice the products they have
     // in one part: error to 64 bits 1.1e-7 in one part, 1.24e-7 with one sum, 9.9e-8 so), and not where sixteen rows of bf16 leave no registers.  f32 in four parts: the quarters of both pairs, which
-    // makes two or three rows as exact as a wave per row (768 x 768, error to that form's 1.04 with halves, 0.94 so; 1.6 with one).
-    constexpr int AS = (KEEP && (BF16 ? TS != 2 : TS < 4)) || (BF16 && XQ == 4 && TS == 1) ? 1 : 2, AH = (KEEP && TS < 4) || BF16 ? 1 : KEEP ? 4 : 2;
+    // makes two or three rows as exact as a wave per row (768 x 768, error to that form's 1.04 with halves, 0.94 so; 1.6 with one).  A pair of bf16
+    // a wave (PD 1, short rows behind a norm): its halves, 9.2e-8 at 768 and 9.0e-8 at 512 (one sum 1.03e-7 and 1.01e-7, a wave per row 1.09e-7 and 9.9e-8).
+    static_assert(PD > 1 || (BF16 && KEEP), "one pair a wave: short rows of bf16");
+    constexpr int AS = (KEEP && (BF16 ? TS != 2 : TS < 4)) || (BF16 && XQ == 4 && TS == 1) ? 1 : 2,
+                  AH = PD == 1 ? 2 : (KEEP && TS < 4) || BF16 ? 1 : KEEP ? 4 : 2;
     // What a group of PD pairs adds up to starts anew with the next one and joins the sum of the groups, so that the chains of eight waves are no
     // longer than those of sixteen (error to 64 bits, 8 rows of bf16 11008 x 4096 with sixteen waves / eight / so: 2.0e-7 / 2.9e-7 / 1.3e-7, 4 of f32 5632 x 8192 in parts of
     // k / eight waves / so: 1.3e-7 / 2.5e-7 / 1.2e-7; 324 launches, time: f32 0.998, bf16 1.003).  bf16 only for more than four pairs a wave (2048 x 2048, 4 rows, 1.02
@@ -1664,15 +1667,15 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
     }
 }
 
-// The staging of a folded norm for mfma_rows: wave b normalises row b in its registers (16 bytes of every 256 elements a
+// The staging of a folded norm for mfma_rows: wave b normalises row b (every row in front of a norm over all) in its registers (16 bytes of every 256 elements a
 // lane, k <= 256 VM) and puts it into LDS split.  stage_normed_rows spreads every row over all waves, a trip through
 // LDS and a barrier for each of two sums and a chain of 16 reads behind them: 13.9 us for a folded launch of 8 rows of
 // 768 x 2304 in f32, whose product alone takes 4.3.
 template <int NORM, int VM, class Rows>
 __device__ __forceinline__ void stage_rows_by_wave(float *sh, const float *__restrict__ x, uint32_t k, uint32_t batch,
                                                    const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
-                                                   uint64_t ldx, const PostNorm &post, const Rows &xs) {
-    const uint32_t lane = threadIdx.x & 63, b = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n4 = k / 4;
+                                                   uint64_t ldx, const PostNorm &post, const Rows &xs, uint32_t b) {
+    const uint32_t lane = threadIdx.x & 63, n4 = k / 4;
     const bool on = b < batch;
     const float *row = NORM == 3 ? post.y + (uint64_t)b * k : x + (uint64_t)b * ldx;
     auto row_sum = [](float t) { return xor32_sum(xor16_sum(group_sum<16>(t))); };
@@ -1772,8 +1775,8 @@ static constexpr size_t kDenseNormLdsLimit = 64 * 1024;
 // rows + scale + bias + per-wave partial sums + statistics
 static constexpr size_t gemv_dense_norm_lds(uint64_t k, uint32_t bp) { return ((size_t)(bp + 2) * k + 16 * bp + 32) * 4; }
 static constexpr size_t gemv_dense_post_lds(uint64_t k, uint32_t bp) { return gemv_dense_norm_lds(k, bp) + (size_t)bp * k * 4; }
-// The most pairs of chunks in a row that a folded norm over bp rows leaves room for, and of these in the share of one of 16 waves
-// (0: a wave has none).  Nothing is built for more.
+// The most pairs of chunks in a row that a folded norm over bp rows leaves room for, and of these in the share of one of up to 16 waves
+// (f32, which is always 16 of them, 0: a wave has none).  Nothing is built for more.
 template <bool BF16>
 static constexpr uint32_t gemv_fold_row_pairs(int norm, uint32_t bp) {
     const uint64_t ku = MfmaType<BF16>::KU;
@@ -1784,7 +1787,7 @@ static constexpr uint32_t gemv_fold_row_pairs(int norm, uint32_t bp) {
 template <bool BF16>
 static constexpr uint32_t gemv_fold_share(int norm, uint32_t bp) {
     const uint32_t pairs = gemv_fold_row_pairs<BF16>(norm, bp);
-    return pairs < 16 ? 0 : (pairs + 15) / 16;
+    return BF16 || pairs >= 16 ? (pairs + 15) / 16 : 0;
 }
 
 // NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
@@ -1802,8 +1805,14 @@ __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType
     mfma_rows<BF16, PD, KEEP, XQ, TS, FOLD>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
         if constexpr (NORM != 0) {
             constexpr uint32_t LONGEST = gemv_fold_row_pairs<BF16>(NORM, BP) * MfmaType<BF16>::KU;
-            if (LONGEST <= 1024 || k <= 1024) stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
-            else if (LONGEST <= 2048 || k <= 2048) stage_rows_by_wave<NORM, 8>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs);
+            const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+            if (LONGEST <= 1024 || k <= 1024) {
+                stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs, wave);
+                // (a pair a wave: there may be more rows than waves)
+                if constexpr (PD == 1 && NORM != 4)
+                    for (uint32_t b = wave + waves; b < batch; b += waves)
+                        stage_rows_by_wave<NORM, 4>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs, b);
+            } else if (LONGEST <= 2048 || k <= 2048) stage_rows_by_wave<NORM, 8>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post, xs, wave);
             else
                 stage_normed_rows<BP, NORM>((float *)corners, x, k, batch, nscale, nbias, eps, ldx, post,
                                             [&](uint32_t b, uint32_t i, float v) { xs.put(b, i, v); });
@@ -1853,9 +1862,18 @@ static uint32_t gemv_mfma_waves(uint64_t pairs) { return (uint32_t)std::max<uint
 bool gemv_takes_f32_rows(const Weight &w, uint64_t rows) {
     return w.dtype == COEUS_W_F32 && rows >= 2 && rows <= 16 && gemv_mfma_shape(w, gemv_mfma_waves(w.k / 32));
 }
+// Waves behind a folded norm: sixteen, or one for each pair of a shorter row of bf16.  Those took the kernel with a wave per output row, whose
+// workgroups convert every row again for each of them.  Decode steps of 12 layers of 768, ms, that one / the norm a launch of its own / this: 2, 4, 8 and
+// 16 rows 0.42 / 0.46 / 0.38, 0.50 / 0.46 / 0.38, 0.72 / 0.50 / 0.43, 1.19 / 0.62 / 0.56; of 512 0.41 / 0.44 / 0.37, 0.48 / 0.45 / 0.39, 0.66 / 0.47 / 0.40,
+// 1.08 / 0.56 / 0.49.  (f32 below 512 stays: sums of pairs, even in quarters, are 1 % less exact than a wave per row's.)
+static uint32_t gemv_fold_waves(const Weight &w) { return w.dtype == COEUS_W_BF16 ? (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(16, w.k / 64)) : 16; }
 static size_t gemv_mfma_norm_lds(const Weight &w, uint32_t bp, size_t staging) {
     const bool bf = w.dtype == COEUS_W_BF16;
     return (bf ? SplitRows::bytes(bp, w.k) : PlainRows::bytes(bp, w.k)) + std::max((size_t)16 * 16 * 128, staging);
+}
+static bool gemv_folds_on_mfma(const Weight &w, uint64_t batch, size_t staging) {
+    const uint32_t waves = gemv_fold_waves(w);
+    return gemv_uses_mfma(w, batch, waves, true) && gemv_mfma_norm_lds(w, pad_batch(batch), staging) <= 160 * 1024;
 }
 bool gemv_can_fuse_whole_norm(const Weight &w, uint64_t batch) {
     if (w.dtype != COEUS_W_F32 || batch < 2 || batch > 16 || !gemv_can_fuse_norm_dense(w, batch) || !gemv_uses_mfma(w, batch, 16, true)) return false;
@@ -2321,12 +2339,12 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
     }
     {
         // plain: workgroups enough to fill the compute units' 16 waves;
-        // a folded norm: one workgroup of 16 waves per compute unit, which stages the rows once
+        // a folded norm: one workgroup of up to 16 waves per compute unit, which stages the rows once
         const uint32_t pairs = (uint32_t)std::min<uint64_t>(w.k / MfmaType<BF16>::KU, 1u << 20);
         const MfmaPlain plain = gemv_mfma_plain<BF16>(w, batch);
-        const uint32_t mw = nf ? 16u : plain.waves;
+        const uint32_t mw = nf ? gemv_fold_waves(w) : plain.waves;
         const size_t mlds = nf ? gemv_mfma_norm_lds(w, bp, lds) : plain.lds;
-        if (aligned && (nf ? gemv_uses_mfma(w, batch, 16, true) && mlds <= 160 * 1024 : plain.runs)) {
+        if (aligned && (nf ? gemv_folds_on_mfma(w, batch, lds) : plain.runs)) {
             const uint32_t parts = nf ? 1u : plain.parts, tiles = (uint32_t)ceil_div(w.n, 16 / parts), np = (pairs / parts + mw - 1) / mw;
             const dim3 mgrid(std::min(tiles, 256 * (16 / mw))), mblock(mw * 64);
 #define COEUS_MFMA6(BPV, NV, PV, KV, TV, FV)                                                                                  \
@@ -2351,8 +2369,9 @@ static int launch_gemv_dense(const Weight &w, const float *x, uint64_t batch, co
 #define COEUS_MFMA3(BPV, NV) do { if (np <= 2) COEUS_MFMA4(BPV, NV, 2, true); else if (pairs > 4 * mw) COEUS_MFMAL(BPV, NV, (BF16 && NV == 0 && BPV < 16)); else COEUS_MFMAL(BPV, NV, false); } while (0)
 #define COEUS_MFMAN(BPV, NV)                                                                               \
     do {                                                                                                   \
-        if constexpr (gemv_fold_share<BF16>(NV, BPV) > 2) COEUS_MFMA3(BPV, NV);                             \
-        else if constexpr (gemv_fold_share<BF16>(NV, BPV) > 0) COEUS_MFMA4(BPV, NV, 2, true);               \
+        if (BF16 && np == 1) COEUS_MFMA4(BPV, NV, (BF16 ? 1 : 2), true);                                    \
+        else if constexpr (gemv_fold_share<BF16>(NV, BPV) > 2) COEUS_MFMA3(BPV, NV);                        \
+        else if constexpr (gemv_fold_share<BF16>(NV, BPV) > (BF16 ? 1 : 0)) COEUS_MFMA4(BPV, NV, 2, true);  \
         else return fail(COEUS_INVALID_INPUT, "norm fusion needs the normalised activations to fit in LDS"); \
     } while (0)
 #define COEUS_MFMA(BPV) do { if (norm == 4) { if constexpr (!BF16) COEUS_MFMAN(BPV, 4); } else if (norm == 1) COEUS_MFMAN(BPV, 1); else if (norm == 2) COEUS_MFMAN(BPV, 2); else COEUS_MFMAN(BPV, 3); } while (0)
