@@ -3,8 +3,9 @@
 //
 //   memory_local_kernel   prompt: what each chunk of 64 tokens adds to the state, all chunks at once
 //   memory_carry_kernel   prompt: the state in front of every chunk (element by element over the chunks)
-//   memory_read_kernel    prompt: the outputs of every chunk, normalised and gated, all chunks at once
-//   memory_scan_kernel    short prompts and odd sizes: token by token, state in registers
+//   memory_read_kernel    prompt: the outputs of every chunk, normalised and gated, all chunks at once; of prompts that are one chunk,
+//                         the state behind it too, and no other launch
+//   memory_scan_kernel    odd sizes and places, few tokens: token by token, state in registers
 //   memory_finish_kernel  its outputs: normaliser, RMS norm, gate
 //   memory_step_kernel    decode: all of it for one token per sequence
 //
@@ -63,10 +64,15 @@ struct MemoryChunks {
 static uint64_t chunk_floats(const MemoryDims &dm, uint64_t units, uint64_t chunks) {
     return units * (chunks * (ceil_div(dm.d, 16) * ceil_div(dm.e, 16) * 256 + dm.d + 2) + chunks + 1) + 64;
 }
+static bool chunk_shape(const MemoryDims &dm) {
+    return dm.d % 4 == 0 && dm.e % 4 == 0 && dm.in_ld % 4 == 0 && dm.d <= kMaxChunkDim && dm.e <= kMaxChunkDim;
+}
 static bool chunked(const MemoryDims &dm, uint64_t n) {
     // (a few dozen tokens are quicker one by one than through three launches)
-    return n >= 48 && dm.d % 4 == 0 && dm.e % 4 == 0 && dm.in_ld % 4 == 0 && dm.d <= kMaxChunkDim && dm.e <= kMaxChunkDim;
+    return n >= 48 && chunk_shape(dm);
 }
+// The prompt is one chunk: one launch reads the state, answers and stores the state behind it (rows in 16-byte pieces).
+static bool one_chunk(const MemoryDims &dm, uint64_t n, const float *proj) { return n >= 2 && n <= kChunk && chunk_shape(dm) && ((uintptr_t)proj & 15) == 0; }
 
 struct ChunkGates {
     double F, a, top;  // running sum of the log forget gates, log input gate - F, running maximum of that
@@ -240,11 +246,17 @@ __global__ __launch_bounds__(256) void memory_carry_kernel(MemoryDims dm, Memory
 // One workgroup of eight waves per (chunk, head, sequence); wave w owns the 16-column tiles w, w + 8, .. of all 64
 // rows, so that a chunk's state is read once and the values once.  Queries and keys are in LDS (rows of an odd
 // number of quads); the weighted scores take the keys' place.
+// ONE: the prompt's only chunk.  The state is the session's, and a wave stores its columns' new one, keep S + K^T diag(w) V, next to its products
+// with the old one; rows of 16 tokens that the prompt does not reach are left out.  Bound: one compute unit's trips for a head's state (64 KB in and
+// out of 128 x 128) and rows, and chains of f32 products.
+// 16 heads of 128 x 128, us a layer, token by token or (from 48) three launches / this: 8 sequences of 24 tokens 280 / 21, one of 8 tokens 34 / 16.  Prompt
+// passes of the 2048-wide design (9 such layers of 12), ms: one sequence of 2 / 8 / 24 / 47 tokens 1.12 / 1.26 / 1.72 / 2.38 and 1.11 / 1.09 / 1.14 / 1.21, 16
+// of them 1.82 / 3.05 / 6.09 / 10.4 and 1.23 / 1.46 / 1.87 / 2.47.  Error to 64 bits of what is remembered after 24 tokens 2.6e-7 and 1.7e-7, of the outputs 4.5e-7 and 3.3e-7.
 static uint32_t read_ld(const MemoryDims &dm) { return 16 * (uint32_t)ceil_div(dm.d, 16) + 4; }
 constexpr uint32_t kScoreLd = kChunk + 4;
 static size_t read_lds_bytes(const MemoryDims &dm) { return kChunk * (size_t)(read_ld(dm) + std::max(read_ld(dm), kScoreLd)) * 4; }
 
-template <int NCT>
+template <int NCT, bool ONE>
 __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restrict__ proj, MemoryDims dm, MemoryParams pr, MemoryState st,
                                                           uint64_t n, uint64_t t0, uint64_t seg, MemoryChunks cb,
                                                           float *__restrict__ out, uint16_t *__restrict__ out_lp, uint64_t lp_ld,
@@ -252,34 +264,48 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
     constexpr uint32_t PLD = kScoreLd, W = 8;
     extern __shared__ __attribute__((aligned(16))) float lds[];
     __shared__ double rs[kChunk], as[kChunk];  // F - m of a row, a of a column
-    __shared__ __attribute__((aligned(16))) float carry[kChunk], floor_[kChunk], psum[4][kChunk], qn[kChunk], dinv[kChunk], rsum[W][kChunk];
+    __shared__ __attribute__((aligned(16))) float carry[kChunk], floor_[kChunk], psum[4][kChunk], qn[kChunk], dinv[kChunk], rsum[W][kChunk], adds[ONE ? kChunk : 1];
+    __shared__ float keep;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
     const uint32_t chunk = blockIdx.x, h = blockIdx.y, H = dm.heads, d = dm.d, e = dm.e, LD = 16 * cb.dtiles + 4;
     const uint64_t b = blockIdx.z, left = seg - (uint64_t)chunk * kChunk, row0 = b * n + t0 + (uint64_t)chunk * kChunk;
-    const uint32_t live = left < kChunk ? (uint32_t)left : kChunk;
+    const uint32_t live = left < kChunk ? (uint32_t)left : kChunk, tiles = ONE ? (live + 15) / 16 : 4;
     const uint64_t unit = b * H + h, ci = unit * cb.chunks + chunk;
     const float *p = proj + row0 * dm.in_ld, *qp = p + h * d, *kp = p + dm.k_off() + h * d, *vp = p + dm.v_off() + h * e;
     float *const ql = lds, *const kl = ql + kChunk * LD, *const pl = kl;
     const float qs = 1.0f / sqrtf((float)d);
     // the first tiles of the state and the values are requested before anything else
-    const float *sp = cb.s + ci * cb.dtiles * cb.etiles * 256 + lane * 4;
+    const float *sp = ONE ? nullptr : cb.s + ci * cb.dtiles * cb.etiles * 256 + lane * 4;
+    float *const state = st.s + unit * d * e;
     auto sload = [&](uint32_t m, float4_t (&x)[NCT]) {
 #pragma unroll
-        for (int t = 0; t < NCT; t++) x[t] = *(const float4_t *)(sp + (min(m, cb.dtiles - 1) * cb.etiles + min(wave + W * t, cb.etiles - 1)) * 256);
+        for (int t = 0; t < NCT; t++) {
+            if constexpr (ONE) {
+                const uint32_t col = min(16 * (wave + W * t) + c, e - 1), row = 16 * m + 4 * g;  // (d % 4 == 0)
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[t][i] = state[(uint64_t)(min(row, d - 4) + i) * e + col];
+            } else {
+                x[t] = *(const float4_t *)(sp + (min(m, cb.dtiles - 1) * cb.etiles + min(wave + W * t, cb.etiles - 1)) * 256);
+            }
+        }
     };
     float4_t s[4][NCT], v[4][NCT];
 #pragma unroll
     for (int q = 0; q < 4; q++) sload(q, s[q]);
+    bool odd = false;  // ONE: a value is infinite or not a number
 #pragma unroll
-    for (int m = 0; m < 4; m++)
+    for (int m = 0; m < 4; m++) {
+        if (ONE && m >= (int)tiles) break;
 #pragma unroll
         for (int t = 0; t < NCT; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) v[m][t][i] = vp[(uint64_t)min(16u * m + 4 * g + i, live - 1) * dm.in_ld + min(16 * (wave + W * t) + c, e - 1)];
+    }
     // queries and keys, half a wave per row: rows behind the end repeat the last one, dims behind the end are zero
     for (uint32_t x = 4 * (tid & 31); x < 16 * cb.dtiles; x += 128)
 #pragma unroll
         for (uint32_t r = tid >> 5; r < kChunk; r += 16) {
+            if (ONE && r >= 16 * tiles) break;
             const uint64_t at = (uint64_t)min(r, live - 1) * dm.in_ld + min(x, d - 4);
             float4_t qv = *(const float4_t *)(qp + at), kv = *(const float4_t *)(kp + at);
             if (x >= d) qv = kv = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -288,14 +314,44 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
         }
     if (wave == W - 1) {
         const ChunkGates cg = chunk_gates(p, dm, pr, h, lane, live);
-        const double m0 = (double)cb.m0[unit * (cb.chunks + 1) + chunk], top = fmax(m0, cg.top);
+        const double m0 = (double)(ONE ? st.m[unit] : cb.m0[unit * (cb.chunks + 1) + chunk]), top = fmax(m0, cg.top);
         rs[lane] = -top;  // F - m
         as[lane] = cg.a;
         carry[lane] = qs * expf((float)(m0 - top));
         floor_[lane] = expf((float)-(cg.F + top));
-        if (chunk == cb.chunks - 1 && lane == 0) st.m[unit] = cb.m0[unit * (cb.chunks + 1) + cb.chunks];
+        if constexpr (ONE) {  // the state behind the prompt, relative to its maximum as stored
+            const double F = __shfl(cg.F, 63, 64);
+            const float end = (float)(F + __shfl(top, 63, 64));
+            auto exp64 = [](double x) {  // (an exponent of 8 rounded to f32 is 2e-7 of the result; -infinity stays one)
+                const float hi = (float)x, y = expf(hi);
+                return y > 0.f ? fmaf(y, (float)(x - (double)hi), y) : y;
+            };
+            adds[lane] = exp64(F + cg.a - (double)end);
+            if (lane == 0) {
+                keep = exp64(F + m0 - (double)end);
+                st.m[unit] = end;
+            }
+        } else if (chunk == cb.chunks - 1 && lane == 0) {
+            st.m[unit] = cb.m0[unit * (cb.chunks + 1) + cb.chunks];
+        }
     }
     __syncthreads();
+    // ONE: values weighted for the state; among the others one that is not finite would reach the rows in front of it (times zero)
+    float4_t wv[ONE ? 4 : 1][NCT];
+    if constexpr (ONE) {
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            if (m >= (int)tiles) break;
+            const float4_t w = *(const float4_t *)(adds + 16 * m + 4 * g);
+#pragma unroll
+            for (int t = 0; t < NCT; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    wv[m][t][i] = 16u * m + 4 * g + i < live ? w[i] * v[m][t][i] : 0.f;
+                    if (!(fabsf(v[m][t][i]) < INFINITY)) { odd = true; v[m][t][i] = 0.f; }
+                }
+        }
+    }
     auto operand = [&](const float *rows, uint32_t tile, uint32_t m) { return *(const float4_t *)(rows + (16 * tile + c) * LD + 16 * m + 4 * g); };
     // ---- Q S0
     float4_t acc[4][NCT];
@@ -308,24 +364,61 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
         for (int q = 0; q < 4; q++) {
             const uint32_t m = m0 + q;
             if (m >= cb.dtiles) break;
+            const bool real = 16 * m + 4 * g < d;
+            if constexpr (ONE)
+#pragma unroll
+                for (int t = 0; t < NCT; t++)
+                    if (!real) s[q][t] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int r = 0; r < 4; r++) {
+                if (ONE && r >= (int)tiles) break;
                 const float4_t a = operand(ql, r, m);
 #pragma unroll
                 for (int t = 0; t < NCT; t++) acc[r][t] = mfma4(a, s[q][t], acc[r][t]);
             }
-            if (m + 4 < cb.dtiles) sload(m + 4, s[q]);
+            if constexpr (ONE) {
+                float4_t x[NCT];
+#pragma unroll
+                for (int t = 0; t < NCT; t++) x[t] = keep * s[q][t];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    if (r >= (int)tiles) break;
+                    float4_t a;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) a[i] = kl[(16 * r + 4 * g + i) * LD + 16 * m + c];
+#pragma unroll
+                    for (int t = 0; t < NCT; t++) x[t] = mfma4(a, wv[r][t], x[t]);
+                }
+                if (m + 4 < cb.dtiles) sload(m + 4, s[q]);
+#pragma unroll
+                for (int t = 0; t < NCT; t++) {
+                    const uint32_t col = 16 * (wave + W * t) + c;
+                    if (real && col < e)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) state[(uint64_t)(16 * m + 4 * g + i) * e + col] = x[t][i];
+                }
+            } else if (m + 4 < cb.dtiles) {
+                sload(m + 4, s[q]);
+            }
         }
     // ---- q . n0, eight threads a row
+    const float *const n0 = ONE ? st.n + unit * d : cb.n + ci * d;
     {
-        const float *n0 = cb.n + ci * d;
         float dot = 0.f;
         for (uint32_t dim = 4 * (tid & 7); dim < d; dim += 32) {
-            const float4_t q = *(const float4_t *)(ql + (tid >> 3) * LD + dim), x = *(const float4_t *)(n0 + dim);
+            const float4_t q = *(const float4_t *)(ql + (tid >> 3) * LD + dim);
+            float4_t x;
+            if constexpr (ONE) x = float4_t{n0[dim], n0[dim + 1], n0[dim + 2], n0[dim + 3]};  // (the caller's, aligned to floats)
+            else x = *(const float4_t *)(n0 + dim);
             dot = fmaf(q[0], x[0], dot); dot = fmaf(q[1], x[1], dot); dot = fmaf(q[2], x[2], dot); dot = fmaf(q[3], x[3], dot);
         }
         dot = group_sum<8>(dot);
         if ((tid & 7) == 0) qn[tid >> 3] = dot;
+    }
+    float n1 = 0.f;  // the new normaliser's element of this thread, stored behind the barrier
+    if (ONE && tid < d) {
+        for (uint32_t j = 0; j < live; j++) n1 = fmaf(adds[j], kl[j * LD + tid], n1);
+        n1 = fmaf(keep, n0[tid], n1);
     }
     // ---- scores up to the diagonal: ten 16 x 16 tiles over the eight waves, then weighted
     auto tile_of = [](uint32_t idx, uint32_t &r, uint32_t &t) {
@@ -336,15 +429,16 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
 #pragma unroll
     for (int u = 0; u < 2; u++) {
         sc[u] = float4_t{0.f, 0.f, 0.f, 0.f};
-        if (wave + W * u >= 10) continue;
+        if (wave + W * u >= (ONE ? tiles * (tiles + 1) / 2 : 10)) continue;
         uint32_t r, t;
         tile_of(wave + W * u, r, t);
         for (uint32_t m = 0; m < cb.dtiles; m++) sc[u] = mfma4(operand(ql, r, m), operand(kl, t, m), sc[u]);
     }
     __syncthreads();
+    if (ONE && tid < d) st.n[unit * d + tid] = n1;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-        if (wave + W * u >= 10) continue;
+        if (wave + W * u >= (ONE ? tiles * (tiles + 1) / 2 : 10)) continue;
         uint32_t r, t;
         tile_of(wave + W * u, r, t);
         const uint32_t j = 16 * t + c;
@@ -366,14 +460,16 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
     }
     float4_t gate[4][NCT];
 #pragma unroll
-    for (int r = 0; r < 4; r++)
+    for (int r = 0; r < 4; r++) {
+        if (ONE && r >= (int)tiles) break;
 #pragma unroll
         for (int t = 0; t < NCT; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 gate[r][t][i] = p[(uint64_t)min(16u * r + 4 * g + i, live - 1) * dm.in_ld + dm.gate_off() + h * e + min(16 * (wave + W * t) + c, e - 1)];
+    }
     __syncthreads();
-    if (tid < kChunk) {
+    if (tid < (ONE ? 16 * tiles : kChunk)) {
         float nq = qn[tid] * carry[tid];
         for (uint32_t t = 0; t <= tid / 16; t++) nq += psum[t][tid];
         dinv[tid] = 1.0f / (fmaxf(fabsf(nq), floor_[tid]) + kFloor);
@@ -383,14 +479,31 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
     for (int m = 0; m < 4; m++)
 #pragma unroll
         for (int r = m; r < 4; r++) {
+            if (ONE && r >= (int)tiles) break;
             const float4_t a = *(const float4_t *)(pl + (16 * r + c) * PLD + 16 * m + 4 * g);
 #pragma unroll
             for (int t = 0; t < NCT; t++) acc[r][t] = mfma4(a, v[m][t], acc[r][t]);
         }
+    if constexpr (ONE)
+        if (__any(odd))  // what is not finite takes part in its own row and those behind it alone, as token by token
+            for (uint32_t j = 0; j < live; j++)
+#pragma unroll
+                for (int t = 0; t < NCT; t++) {
+                    const float x = vp[(uint64_t)j * dm.in_ld + min(16 * (wave + W * t) + c, e - 1)];
+                    if (fabsf(x) < INFINITY) continue;
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const uint32_t ri = 16 * r + 4 * g + i;
+                            if (ri >= j && ri < live) acc[r][t][i] += pl[ri * PLD + j] * x;
+                        }
+                }
     __syncthreads();
     // ---- normaliser, norm, gate
 #pragma unroll
     for (int r = 0; r < 4; r++) {
+        if (ONE && r >= (int)tiles) break;
         const float4_t f = *(const float4_t *)(dinv + 16 * r + 4 * g);
         float4_t s2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -419,6 +532,7 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
         const float w = pr.norm[h * e + col];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
+            if (ONE && r >= (int)tiles) break;
             const float4_t f = *(const float4_t *)(dinv + 16 * r + 4 * g);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -521,6 +635,26 @@ int launch_memory_prompt(const float *proj, const MemoryDims &dm, const MemoryPa
     uint16_t *lp = out_lp ? (uint16_t *)out_lp->p : nullptr;
     const uint64_t lp_ld = out_lp ? out_lp->ld : 0;
     const bool lp_bf = out_lp && out_lp->bf16;
+#define COEUS_MR(NV, ONEV)                                                                                                        \
+    do {                                                                                                                          \
+        static const bool once = hipFuncSetAttribute((const void *)memory_read_kernel<NV, ONEV>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                                     136 * 1024) == hipSuccess;                                                   \
+        (void)once;                                                                                                               \
+        hipLaunchKernelGGL((memory_read_kernel<NV, ONEV>), rgrid, dim3(512), read_lds_bytes(dm), st, proj, dm, pr, state, n, t0, seg, cb, out, lp, \
+                           lp_ld, lp_bf);                                                                                         \
+    } while (0)
+    if (may_chunk && one_chunk(dm, n, proj)) {
+        MemoryChunks cb = {};
+        cb.chunks = 1;
+        cb.dtiles = (uint32_t)ceil_div(dm.d, 16);
+        cb.etiles = (uint32_t)ceil_div(dm.e, 16);
+        const uint64_t t0 = 0, seg = n;
+        const dim3 rgrid(1, dm.heads, (unsigned)batch);
+        if (cb.etiles <= 8) COEUS_MR(1, true);
+        else COEUS_MR(2, true);
+        COEUS_HIP(hipGetLastError());
+        return COEUS_OK;
+    }
     if (may_chunk && chunked(dm, n)) {
         const uint64_t units = batch * dm.heads;
         for (uint64_t t0 = 0; t0 < n; t0 += kSegment) {
@@ -551,21 +685,13 @@ int launch_memory_prompt(const float *proj, const MemoryDims &dm, const MemoryPa
             const dim3 cgrid((unsigned)ceil_div(cb.dtiles * cb.etiles * 64 + dm.d + 1, 256), dm.heads, (unsigned)batch);
             hipLaunchKernelGGL(memory_carry_kernel, cgrid, dim3(256), 0, st, dm, state, cb);
             const dim3 rgrid(cb.chunks, dm.heads, (unsigned)batch);
-#define COEUS_MR(NV)                                                                                                              \
-    do {                                                                                                                          \
-        static const bool once = hipFuncSetAttribute((const void *)memory_read_kernel<NV>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                                     136 * 1024) == hipSuccess;                                                   \
-        (void)once;                                                                                                               \
-        hipLaunchKernelGGL(memory_read_kernel<NV>, rgrid, dim3(512), read_lds_bytes(dm), st, proj, dm, pr, state, n, t0, seg, cb, out, lp, \
-                           lp_ld, lp_bf);                                                                                         \
-    } while (0)
-            if (cb.etiles <= 8) COEUS_MR(1);
-            else COEUS_MR(2);
-#undef COEUS_MR
+            if (cb.etiles <= 8) COEUS_MR(1, false);
+            else COEUS_MR(2, false);
         }
         COEUS_HIP(hipGetLastError());
         return COEUS_OK;
     }
+#undef COEUS_MR
     float *raw = scratch, *nq = raw + batch * n * dm.heads * dm.e, *mt = nq + batch * n * dm.heads;
     const dim3 grid((unsigned)ceil_div(dm.e + 1, 16), dm.heads, (unsigned)batch);
 #define COEUS_MS(RV) hipLaunchKernelGGL(memory_scan_kernel<RV>, grid, dim3(256), 0, st, proj, dm, pr, state, n, raw, nq, mt)

@@ -1,0 +1,49 @@
+"""Matrix memory, prompts of one chunk: a launch that reads the state, answers and stores the state behind the prompt.  At the
+edges of the 16-token tiles and of the sizes, from a state that earlier tokens left, with a value that is not finite (which the rows
+in front of it must not see), and for rows that 16-byte pieces do not lie in (token by token, as before)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from coeus_amd import _lib
+from coeus_amd.device import DeviceArray
+from coeus_amd.plugin import _check
+from gpu_util import dev
+from test_gpu_zekilix import Memory, off
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [(4, 24, 64), (2, 128, 128), (1, 256, 256), (2, 36, 132), (3, 4, 4), (2, 128, 40)])
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 32, 33, 48, 49, 63, 64])
+def test_behind_earlier_tokens(shape, n):
+    t = Memory(*shape, batch=2, seed=n)
+    p = t.inputs(3 + n + 1)
+    want, S = t.want(p)
+    got = np.concatenate([t.prompt(p[:, :3], 0), t.prompt(p[:, 3:3 + n], 1), t.step(p[:, 3 + n])[:, None]], axis=1)
+    # (the bounds of the other tests of prompts and states: chains of f32 sums of some 64 terms)
+    assert off(got, want) < 2e-5 and t.state_off(S) < 2e-5
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("n,j", [(5, 3), (30, 0), (40, 39), (64, 20)])
+def test_rows_in_front_of_a_value_that_is_not_finite(bad, n, j):
+    H, d, e = 2, 32, 48
+    a, b = (Memory(H, d, e, batch=1, seed=n) for _ in range(2))
+    p = a.inputs(n)
+    clean = b.prompt(p, 1)
+    p[0, j, 2 * H * d + 5] = bad
+    got = a.prompt(p, 1)
+    assert np.array_equal(got[:, :j], clean[:, :j])  # the same sums of the same values
+    assert not np.isfinite(got[0, j:, 5]).any() and np.isfinite(got[0, :, e:]).all()  # (the other head)
+    assert not np.isfinite(a.state[0].to_host()[0, 0, :, 5]).any() and np.isfinite(a.state[0].to_host()[0, :, :, 6]).all()
+
+
+def test_rows_off_a_16_byte_boundary():
+    t = Memory(2, 32, 48, batch=1, seed=1)
+    p = t.inputs(20)
+    x, out = dev(np.concatenate([np.zeros(1, np.float32), p.ravel()])), DeviceArray((1, 20, 96))
+    _check(_lib.load().coeus_op_memory_prompt(C.byref(t.s), C.byref(t.w), x.ptr + 4, *[a.ptr for a in t.state], 1, 20, 1, out.ptr, None))
+    want, S = t.want(p)
+    assert off(out.to_host(), want) < 2e-5 and t.state_off(S) < 2e-5
