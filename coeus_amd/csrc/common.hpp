@@ -90,6 +90,7 @@ struct Weight {
     __half *scales = nullptr;    // Q* only
     uint64_t bytes = 0;
     bool infinite = false;       // bf16: some value is infinite (weights_check)
+    bool few_rows = true;        // prompts of up to 16 rows may take the decode matmul's kernels (gemm_uses_few)
     __half *xq_scratch = nullptr; // [k_pad/8][16][8] f16 staging for the operator-level API
     // Q* only: dense f16 copy [n] rows of gemm_ld(k) elements for the prefill matmul, made on first
     // use and kept while the owner's budget lasts (7B: 13.7 GB next to 4.2 GB of quants; the card
@@ -128,7 +129,7 @@ int launch_fill_seeded(float *dst, uint64_t n, uint64_t seed, uint64_t base, flo
 // Row stride (elements) of the 16-bit staging matrices of the prefill matmul.  Rows that lie a
 // power of two apart would send a tile's 256 row slices to the same few memory channels; one
 // extra 128-byte line per row rotates them over all channels.
-static inline uint64_t gemm_ld(uint64_t k) { return k + 64; }
+static constexpr uint64_t gemm_ld(uint64_t k) { return k + 64; }
 // [rows][k] f32 -> 16-bit (bf16 or f16) rows of stride ld
 int launch_f32_to_16(const float *src, void *dst, uint64_t rows, uint64_t k, uint64_t ld, bool bf16,
                      hipStream_t st);
@@ -273,6 +274,10 @@ coeus_matmul_plan gemv_plan(const Weight &w, uint64_t batch);
 coeus_matmul_plan gemm_launch_plan(const Weight &w, uint64_t m);
 // Short prompts on quantised weights: the matmul that streams the quantised blocks (gemv.hip).
 struct EpiArgs;
+// ... and prompts of up to 16 rows, on the decode matmul's kernels.
+bool gemm_uses_few(const Weight &w, uint64_t m);
+coeus_matmul_plan gemm_few_plan(const Weight &w, uint64_t m);
+int launch_gemm_few(const Weight &w, const uint16_t *a, uint64_t lda, uint64_t m, const EpiArgs &e, hipStream_t st);
 uint32_t qskinny_splits(const Weight &w);
 bool gemm_uses_qskinny(const Weight &w, uint64_t m);
 uint64_t gemm_qskinny_scratch_bytes(const Weight &w, uint64_t m);

@@ -11,7 +11,8 @@
 //     gemm_narrow_kernel   k % 64 == 0, launches of few tiles: 128 or 256 rows by 64 to 128 columns
 //     gemm_h256_kernel     k % 32 == 0: 256x256 tile, eight waves of 128x64, 32-wide slices
 //     gemm_h_kernel        any k: 128x128 tile, register-staged
-//     gemm_qskinny_kernel  up to 64 rows on quantised weights: streams the quantised blocks
+//     gemm_qskinny_kernel  17 to 64 rows on quantised weights: streams the quantised blocks
+//     up to 16 rows        the decode matmul's kernels (launch_gemm_few)
 //     gemm_split_reduce_kernel, gemm_tail_reduce_kernel: sums behind launches split along k
 #include "device_utils.hpp"
 #include <type_traits>
@@ -1995,6 +1996,7 @@ uint64_t gemm_split_scratch_bytes(const Weight &w, uint64_t m) {
         const uint32_t sf = gemm_f32_splits_wanted(w, m);
         return sf > 1 ? (uint64_t)sf * m * w.n * 4 : 0;
     }
+    if (gemm_uses_few(w, m)) return 0;
     if (gemm_uses_qskinny(w, m)) return gemm_qskinny_scratch_bytes(w, m);
     const GemmPlan plan = gemm_plan(w, m, true);
     if (plan.splits > 1) return (uint64_t)plan.splits * m * w.n * 4;
@@ -2016,6 +2018,7 @@ coeus_matmul_plan gemm_launch_plan(const Weight &w, uint64_t m) {
         const F32Shape &t = kF32Shapes[plan.shape];
         return {t.rows == 32 ? "gemm_f32_small_kernel" : "gemm_f32_kernel", t.rows, t.cols, t.waves, plan.splits, 1};
     }
+    if (gemm_uses_few(w, m)) return gemm_few_plan(w, m);
     if (gemm_uses_qskinny(w, m)) return {"gemm_qskinny_kernel", 64, 0, 4, qskinny_splits(w), 1};
     if (!gemm_uses_h256(w, m)) return {"gemm_h_kernel", HM, HN, 4, 1, 1};
     const GemmPlan plan = gemm_plan(w, m, true);
@@ -2028,6 +2031,7 @@ coeus_matmul_plan gemm_launch_plan(const Weight &w, uint64_t m) {
 bool gemm_appends_kv(const Weight &w, uint64_t m, uint64_t inner, uint64_t hd) {
     // (f32: element by element, or by the kernel that sums a split launch's planes, four columns at a time)
     if (w.dtype == COEUS_W_F32) return m < (1ull << 32) && w.n == 3 * inner && (inner & 3) == 0 && (hd & 3) == 0;
+    if (gemm_uses_few(w, m)) return w.n == 3 * inner;  // (element by element)
     // rows fit 32 bits; a lane's 4 columns stay inside one head.  (The short-prompt kernel for
     // quantised weights qualifies when it is split along k: the kernel that sums its partial
     // planes runs this same epilogue.)
@@ -2058,6 +2062,13 @@ int launch_gemm(const Weight &w, const void *a_in, uint64_t m, const Epilogue &e
                         (unsigned long long)scr.a_lp_bytes, (unsigned long long)a_bytes);
         COEUS_TRY(launch_f32_to_16(a, scr.a_lp, m, w.k, lda, bf, st));
         ap = (const uint16_t *)scr.a_lp;
+    }
+    if (gemm_uses_few(w, m)) {
+        const EpiArgs e = make_epi(ep, w.n);
+        if (scr.ev_begin) COEUS_HIP(hipEventRecord(scr.ev_begin, st));
+        for (uint32_t rep = 0; rep < (scr.repeat ? scr.repeat : 1); rep++) COEUS_TRY(launch_gemm_few(w, ap, lda, m, e, st));
+        if (scr.ev_end) COEUS_HIP(hipEventRecord(scr.ev_end, st));
+        return COEUS_OK;
     }
     const uint64_t qs_bytes = gemm_uses_qskinny(w, m) ? gemm_qskinny_scratch_bytes(w, m) : 0;
     if (gemm_uses_qskinny(w, m) && (qs_bytes ? scr.partials && scr.partials_bytes >= qs_bytes : !ep.kv_rows_per_seq)) {

@@ -6,7 +6,7 @@
 //                      wave owns four consecutive 128-k chunks, stages exactly their activations
 //                      (with or without the folded norm) into its private slice of LDS and feeds
 //                      the quants to v_mfma_f32_16x16x32_f16 as f16 subnormals.
-//   gemv_rows_kernel   the same weights for batches of 3 to 16.  One workgroup owns one to six tiles
+//   gemv_rows_kernel   the same weights for batches of 3 to 16 and prompts of up to 16 rows.  One workgroup owns one to six tiles
 //                      of 16 output rows; its waves take 128-k chunks (1 KiB of Q4_0 quants = one
 //                      fully coalesced 16 B/lane load per wave).  Each 32-k block is one
 //                      v_mfma_f32_16x16x32_f16 between the 16 activation rows (f16, straight from
@@ -18,8 +18,10 @@
 //                      wave's registers, no LDS and no barrier.
 //   gemv_many_kernel   one plain activation row: two weight rows a wave, up to four steps of both in flight.
 //   gemv_mfma_kernel   2 - 16 activation rows on f32 / bf16 weights: 16 output rows a workgroup on
-//                      the matrix cores (bf16: the f32 activations as three bf16 each).
+//                      the matrix cores (bf16: the f32 activations as three bf16 each, or prompts'
+//                      rows of bf16).
 #include "device_utils.hpp"
+#include <type_traits>
 
 namespace coeus {
 
@@ -215,15 +217,20 @@ int launch_norm_from_stats(const NormFuse &nf, uint64_t batch, uint64_t k, uint6
 // against 64 bits 2.3e-6 of the result for Q4_0 and 2-7e-7 for Q8_0, 6e-8 - 1.1e-7 so), 4 rows, Q4_0: 4096 x 22016 20.6 -> 15.2, 11008 x 4096
 // 15.1 -> 12.5, 8192 x 2048 10.3 -> 9.5, 2048 x 8192 7.8 -> 6.9, 2048 x 32000 15.2 -> 12.7; Q8_0: 11008 x 4096 16.3 -> 14.1, 4096 x 12288 15.1
 // -> 13.8.  Two chunks of a wave in flight instead of one changed nothing (11008 x 4096 12.2 and 13.0, 8192 x 2048 9.2 and 9.5 us).
-template <bool Q4, int BP, int TPW>
+// W16 (prompts): a weight is its f16(q d), as in every other prompt matmul, one rounding of the exact product; a chunk's blocks add
+// up in the matrix cores, and a wave's chunks behind them (error to 64 bits of 11008 x 4096 Q4_0, 16 rows: 2.0e-7 all in one chain, 1.07e-7 so, 1.69e-7 of the kernel for 17 to 64).
+template <bool Q4, int BP, int TPW, bool W16>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds, const uint4 *__restrict__ xq, uint32_t ngroups,
                       uint32_t tiles, uint32_t batch, EpiArgs e) {
+    // 16-byte pieces from one eight of k to the next, and from row to row: of the interchange format, or of rows gemm_ld(k) elements apart
+    const uint32_t xk = W16 ? 1 : BP, xr = W16 ? ngroups * 16 + 8 : 1;
     static_assert(BP == 4 || BP == 8 || BP == 16, "batch padded to 4, 8 or 16");
+    static_assert(gemm_ld(128) == 192, "rows of a prompt");
     extern __shared__ float rows_red[];  // [TPW][nwaves][4][64]
     const uint32_t lane = threadIdx.x & 63, nwaves = blockDim.x >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t T0 = blockIdx.x * TPW, j = lane & 15, ig = lane >> 4, xb = j & (BP - 1);
+    const uint32_t T0 = blockIdx.x * TPW, j = lane & 15, ig = lane >> 4, xb = W16 ? min(j & (BP - 1), batch - 1) * xr : j & (BP - 1);
     const float4_t zero = {0.f, 0.f, 0.f, 0.f};
     // Output o of the workgroup = (tile, batch row, column); a thread finishes o = threadIdx.x and every blockDim.x-th behind it.
     constexpr uint32_t OUTS = TPW * 16 * BP;
@@ -250,8 +257,9 @@ void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds
     for (uint32_t G = wave; G < ngroups; G += nwaves) {
         uint4 xv[4];
         ChunkRegs<Q4> r[TPW];
+        float4_t chunk[W16 ? TPW : 1];
 #pragma unroll
-        for (int jj = 0; jj < 4; jj++) xv[jj] = xq[((G * 4 + jj) * 4 + ig) * BP + xb];
+        for (int jj = 0; jj < 4; jj++) xv[jj] = xq[((G * 4 + jj) * 4 + ig) * xk + xb];
 #pragma unroll
         for (int t = 0; t < TPW; t++) load_chunk<Q4>(r[t], qs, ds, cb[t] + G, lane);
         __builtin_amdgcn_sched_barrier(0);
@@ -268,6 +276,13 @@ void gemv_rows_kernel(const uint4 *__restrict__ qs, const uint2 *__restrict__ ds
                 union { uint2 u2; _Float16 h[4]; } s;
                 s.u2 = c.s;
                 const half8_t wv = Q4 ? unpack_q4(qw[jj]) : unpack_q8(qw[2 * jj], qw[2 * jj + 1]);
+                if constexpr (W16) {
+                    chunk[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.h, wv * s.h[jj], jj ? chunk[t] : zero, 0, 0, 0);
+                    if (jj == 3)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[t][i] += chunk[t][i];
+                    continue;
+                }
                 const float4_t part = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.h, wv, zero, 0, 0, 0);
                 const float d = (float)s.h[jj];
 #pragma unroll
@@ -846,19 +861,40 @@ static void gemv_rows_shape(bool q4, uint32_t ngroups, uint32_t tiles, uint32_t 
     waves = std::min(waves, ngroups);
 }
 
-template <bool Q4, int BP, int TPW>
-static int launch_gemv_rows(const Weight &w, const __half *xq, uint32_t batch, uint32_t waves, const EpiArgs &e, hipStream_t st) {
+template <bool Q4, int BP, int TPW, bool W16>
+static int launch_gemv_rows(const Weight &w, const void *xq, uint32_t batch, uint32_t waves, const EpiArgs &e, hipStream_t st) {
     const size_t lds = (size_t)TPW * waves * 4 * 64 * 4;
     if (lds > 48 * 1024) {
-        static const hipError_t once = hipFuncSetAttribute((const void *)gemv_rows_kernel<Q4, BP, TPW>,
+        static const hipError_t once = hipFuncSetAttribute((const void *)gemv_rows_kernel<Q4, BP, TPW, W16>,
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         COEUS_HIP(once);
     }
     const uint32_t ngroups = (uint32_t)(w.k_pad / 128), tiles = (uint32_t)(w.n_pad / 16);
-    hipLaunchKernelGGL((gemv_rows_kernel<Q4, BP, TPW>), dim3((uint32_t)ceil_div(tiles, TPW)), dim3(waves * 64), lds, st, (const uint4 *)w.data,
+    hipLaunchKernelGGL((gemv_rows_kernel<Q4, BP, TPW, W16>), dim3((uint32_t)ceil_div(tiles, TPW)), dim3(waves * 64), lds, st, (const uint4 *)w.data,
                        (const uint2 *)w.scales, (const uint4 *)xq, ngroups, tiles, batch, e);
     COEUS_HIP(hipGetLastError());
     return COEUS_OK;
+}
+
+// x: rows of the interchange format, or (W16) plain f16 rows gemm_ld(k) elements apart.
+template <bool Q4, bool W16 = false>
+static int launch_gemv_rows_of(const Weight &w, const void *x, uint64_t batch, const EpiArgs &e, hipStream_t st) {
+    uint32_t tpw, waves;
+    gemv_rows_shape(Q4, (uint32_t)(w.k_pad / 128), (uint32_t)(w.n_pad / 16), tpw, waves);
+    auto with = [&](auto bp) -> int {
+        constexpr int BP = decltype(bp)::value;
+        const uint32_t b = (uint32_t)batch;
+        switch (tpw) {
+            case 1: return launch_gemv_rows<Q4, BP, 1, W16>(w, x, b, waves, e, st);
+            case 2: return launch_gemv_rows<Q4, BP, 2, W16>(w, x, b, waves, e, st);
+            case 3: return launch_gemv_rows<Q4, BP, 3, W16>(w, x, b, waves, e, st);
+            case 4: return launch_gemv_rows<Q4, BP, 4, W16>(w, x, b, waves, e, st);
+            default: if constexpr (Q4) return launch_gemv_rows<Q4, BP, 6, W16>(w, x, b, waves, e, st);
+        }
+        return fail(COEUS_INVALID_INPUT, "decode matmul: no kernel for %u tiles a workgroup", tpw);
+    };
+    const uint32_t bp = pad_batch(batch);
+    return bp <= 4 ? with(std::integral_constant<int, 4>{}) : bp == 8 ? with(std::integral_constant<int, 8>{}) : with(std::integral_constant<int, 16>{});
 }
 
 template <bool Q4>
@@ -870,24 +906,7 @@ static int launch_gemv_quant(const Weight &w, const __half *xq, uint64_t batch, 
     if (nf) return fail(COEUS_INVALID_INPUT, "norm fusion is for batches of up to 4");
     if (e.stats_out && e.act == COEUS_EPI_SILU_GATE)
         return fail(COEUS_INVALID_INPUT, "statistics records are not produced by the gated epilogue");
-    uint32_t tpw, waves;
-    gemv_rows_shape(Q4, (uint32_t)(w.k_pad / 128), (uint32_t)(w.n_pad / 16), tpw, waves);
-    auto with = [&](auto bp) -> int {
-        constexpr int BP = decltype(bp)::value;
-        switch (tpw) {
-            case 1: return launch_gemv_rows<Q4, BP, 1>(w, xq, (uint32_t)batch, waves, e, st);
-            case 2: return launch_gemv_rows<Q4, BP, 2>(w, xq, (uint32_t)batch, waves, e, st);
-            case 3: return launch_gemv_rows<Q4, BP, 3>(w, xq, (uint32_t)batch, waves, e, st);
-            case 4: return launch_gemv_rows<Q4, BP, 4>(w, xq, (uint32_t)batch, waves, e, st);
-            default: if constexpr (Q4) return launch_gemv_rows<Q4, BP, 6>(w, xq, (uint32_t)batch, waves, e, st);
-        }
-        return fail(COEUS_INVALID_INPUT, "decode matmul: no kernel for %u tiles a workgroup", tpw);
-    };
-    switch (pad_batch(batch)) {
-        case 4: return with(std::integral_constant<int, 4>{});
-        case 8: return with(std::integral_constant<int, 8>{});
-        default: return with(std::integral_constant<int, 16>{});
-    }
+    return launch_gemv_rows_of<Q4>(w, xq, batch, e, st);
 }
 
 // ---------------------------------------------------------------- dense kernel (f32 / bf16)
@@ -1464,15 +1483,29 @@ template <> struct MfmaType<false> {
         b = __builtin_amdgcn_mfma_f32_16x16x4f32(uw.v[3], ux.v[3], b, 0, 0, 0);
     }
 };
+// bf16 weights and rows of activations that are bf16 already (prompts)
+struct MfmaRows16 : MfmaType<true> {
+    static constexpr int PIECES = 1, XROWS = 8;
+    struct Frag { uint4 p[1]; };
+    static __device__ __forceinline__ float4_t mul(const uint4 &w, const Frag &x, float4_t acc) {
+        union { uint4 u; bf16x8_t v; } uw, ux;
+        uw.u = w;
+        ux.u = x.p[0];
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(uw.v, ux.v, acc, 0, 0, 0);
+    }
+};
 // uint4 of a wave's corner: 16 weight rows x 128 bytes; per request of x its rows' KU values in pieces
-template <bool BF16>
-static constexpr uint32_t mfma_wave_lds(int xq) { return 128 + (BF16 ? 96 : 64) * xq; }
-template <bool BF16, int PD, bool KEEP, int XQ, int TS, bool FOLD, class Stage>
-__device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
+template <bool BF16, bool X16 = false>
+static constexpr uint32_t mfma_wave_lds(int xq) { return 128 + (BF16 && !X16 ? 96 : 64) * xq; }
+// X16: x is rows of bf16, ldx elements apart
+template <bool BF16, int PD, bool KEEP, int XQ, int TS, bool FOLD, bool X16, class Stage>
+__device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__restrict__ w, const void *__restrict__ xp, uint64_t ldx, uint32_t k,
                                           uint32_t n, uint32_t batch, uint32_t nw, uint32_t grid, const EpiArgs &e, uint4 *lds,
                                           const typename MfmaType<BF16>::Rows &xs, Stage stage) {
-    typedef MfmaType<BF16> MT;
+    typedef std::conditional_t<X16, MfmaRows16, MfmaType<BF16>> MT;
+    typedef std::conditional_t<X16, uint16_t, float> X;
     typedef typename MT::W W;
+    const X *__restrict__ x = (const X *)xp;
     typedef typename MT::Frag Frag;
     constexpr uint32_t KU = MT::KU, EPP = KU / 8;  // k per pair, elements per 16-byte piece
     constexpr int XR = MT::XROWS, XN = XQ ? XQ : 1;
@@ -1482,7 +1515,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
     const uint32_t c = lane & 15, g = lane >> 4, cb = TS > 1 ? c : min(c, batch - 1);
     const uint32_t pairs = k / (KU * TS), pb = pairs * wave / nw, np = pairs * (wave + 1) / nw - pb, groups = (np + PD - 1) / PD;
     const uint32_t tiles = (n + R - 1) / R;
-    uint4 *wl = lds + wave * mfma_wave_lds<BF16>(XQ), *xl = wl + 128;
+    uint4 *wl = lds + wave * mfma_wave_lds<BF16, X16>(XQ), *xl = wl + 128;
     // (a pair behind the wave's share is the share's last one again: no branches around the requests)
     auto pair_at = [&](uint32_t i) { return min(i, np - 1) * (KU * TS); };
     struct WRows { const W *p[2]; };
@@ -1495,7 +1528,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
         }
         return r;
     };
-    const float *xr[XN];
+    const X *xr[XN];
     uint4 wr[PD][2];
     u32x4_t xv[XQ ? PD : 1][XN];  // (arrays of the struct type would be copied through scratch memory)
     auto x_request = [&](int s, uint32_t i) {
@@ -1511,7 +1544,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
 #pragma unroll
         for (int q = 0; q < XQ; q++) {
             const u32x4_t v = xv[s][q];
-            if constexpr (BF16) {
+            if constexpr (BF16 && !X16) {
                 const uint32_t r = 4 * q + (lane >> 4), at = (r * 8 + (((lane & 15) >> 1) ^ ((r >> 1) & 7))) * 2 + (lane & 1);
                 const Split2 lo = split2(__uint_as_float(v.x), __uint_as_float(v.y)), hi = split2(__uint_as_float(v.z), __uint_as_float(v.w));
 #pragma unroll
@@ -1542,7 +1575,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
 #pragma unroll
         for (int q = 0; q < XQ; q++) {
             const uint32_t line = XR * q + lane / LPR;
-            xr[q] = x + (uint64_t)min(TS > 1 ? line % R : line, batch - 1) * k + (TS > 1 ? pb * TS + line / R : pb) * KU + (lane % LPR) * 4;
+            xr[q] = x + (uint64_t)min(TS > 1 ? line % R : line, batch - 1) * (X16 ? ldx : k) + (TS > 1 ? pb * TS + line / R : pb) * KU + (lane % LPR) * (16 / sizeof(X));
         }
     }
     uint32_t tile = blockIdx.x, gi = 0;
@@ -1648,7 +1681,7 @@ __device__ __forceinline__ void mfma_rows(const typename MfmaType<BF16>::W *__re
                 // lane (c, g) adds line c of every fourth wave, in the column of its part
                 float sum = 0.f;
                 for (uint32_t v = g; v < nw; v += 4)
-                    sum += ((const float *)(lds + v * mfma_wave_lds<BF16>(XQ) + (c >> 2) * 16 + (TS > 1 ? c / R * R : 0) + b))[c & 3];
+                    sum += ((const float *)(lds + v * mfma_wave_lds<BF16, X16>(XQ) + (c >> 2) * 16 + (TS > 1 ? c / R * R : 0) + b))[c & 3];
                 sum = xor32_sum(xor16_sum(sum));
                 if (TS == 4) sum += dpp_f32<DPP_ROW_ROR4>(sum);
                 if (TS >= 2) sum += dpp_f32<DPP_ROW_ROR8>(sum);
@@ -1791,18 +1824,18 @@ static constexpr uint32_t gemv_fold_share(int norm, uint32_t bp) {
 }
 
 // NORM 0: BP rows (padded to 4, 8 or 16) in global memory; else staged normalised in LDS behind the waves' corners.
-template <bool BF16, int BP, int NORM, int PD, bool KEEP, int TS = 1, bool FOLD = false>
+template <bool BF16, int BP, int NORM, int PD, bool KEEP, int TS = 1, bool FOLD = false, bool X16 = false>
 __global__ __launch_bounds__(1024) void gemv_mfma_kernel(const typename MfmaType<BF16>::W *__restrict__ w, const float *__restrict__ x, uint32_t k,
                                                          uint32_t n, uint32_t batch, uint32_t waves, uint32_t grid, EpiArgs e,
                                                          const float *__restrict__ nscale, const float *__restrict__ nbias, float eps,
                                                          uint64_t ldx, PostNorm post) {
     extern __shared__ uint4 mlds[];
     typedef typename MfmaType<BF16>::Rows Rows;
-    constexpr int XQ = NORM ? 0 : ((TS > 1 ? 16 : BP) + MfmaType<BF16>::XROWS - 1) / MfmaType<BF16>::XROWS;
+    constexpr int XROWS = X16 ? MfmaRows16::XROWS : MfmaType<BF16>::XROWS, XQ = NORM ? 0 : ((TS > 1 ? 16 : BP) + XROWS - 1) / XROWS;
     // a folded norm: the split rows first; what its staging needs lies where the corners will be
     const Rows xs{(decltype(Rows::p))mlds, k, (uint32_t)BP};
     uint4 *corners = NORM ? (uint4 *)((char *)mlds + Rows::bytes(BP, k)) : mlds;
-    mfma_rows<BF16, PD, KEEP, XQ, TS, FOLD>(w, x, k, n, batch, waves, grid, e, corners, xs, [&]() {
+    mfma_rows<BF16, PD, KEEP, XQ, TS, FOLD, X16>(w, x, ldx, k, n, batch, waves, grid, e, corners, xs, [&]() {
         if constexpr (NORM != 0) {
             constexpr uint32_t LONGEST = gemv_fold_row_pairs<BF16>(NORM, BP) * MfmaType<BF16>::KU;
             const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2068,7 +2101,7 @@ __global__ __launch_bounds__(1024) void gemv_hyper_kernel(const void *__restrict
     };
     if constexpr (MF) {
         __builtin_amdgcn_sched_barrier(0);
-        mfma_rows<true, 2, true, 0, 1, false>((const uint16_t *)wdata, nullptr, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
+        mfma_rows<true, 2, true, 0, 1, false, false>((const uint16_t *)wdata, nullptr, k, k, (uint32_t)e.n, batch, 16, gridDim.x, e, (uint4 *)hyper_lds, xs, [&]() {
             __builtin_amdgcn_sched_barrier(0);
             normalise();
         });
@@ -2609,6 +2642,56 @@ static uint32_t qskinny_gpw(const Weight &w) {
 uint32_t qskinny_splits(const Weight &w) {
     const uint32_t ngroups = (uint32_t)(w.k_pad / 128), gpw = qskinny_gpw(w);
     return (ngroups + gpw - 1) / gpw;
+}
+
+// Prompts of up to 16 rows: the decode step's kernels on the 16-bit rows that the prompt's producers leave.  The tiles of the longer prompts are mostly rows
+// that are not there, and their launches on small matrices are shares of k with a second launch that sums them.
+// Prompt passes, ms, those (gemm_narrow_kernel, gemm_qskinny_kernel) / these, of 2, 8 and 16 ids: 250M bf16 0.65 / 0.37, 0.66 / 0.42, 0.69 / 0.48; 250M Q8_0 0.64 /
+// 0.38, 0.66 / 0.42, 0.65 / 0.41; 1B Q4_0 1.45 / 0.88, 1.54 / 1.03, 1.51 / 1.01; 7B Q4_0 2.52 / 1.68, 2.68 / 1.95, 2.82 / 2.03; matrix-memory layers 4096 wide
+// 1.32 / 0.93, 1.32 / 0.98, 1.33 / 1.15.  The weights cross the memory interface once, so that beyond 16 rows these would read them twice.  Rules for waves and parts are the
+// decode step's.  Errors to 64 bits of the same operands are smaller (bf16 11008 x 4096 9.1e-8, 1.6e-7 before, 768 x 2304 7.5e-8 and 8.4e-8; Q4_0 4096 x 4096 9.8e-8 and 1.3e-7).
+bool gemm_uses_few(const Weight &w, uint64_t m) {
+    if (m < 1 || m > 16 || w.dtype == COEUS_W_F32 || !w.few_rows) return false;
+    if (w.dtype >= COEUS_W_Q8_0) return w.k == w.k_pad;
+    return gemv_mfma_plain<true>(w, std::max<uint64_t>(m, 3)).runs;
+}
+coeus_matmul_plan gemm_few_plan(const Weight &w, uint64_t m) {
+    const uint32_t bp = std::max(pad_batch(m), 4u);
+    if (w.dtype == COEUS_W_BF16) {
+        const MfmaPlain plain = gemv_mfma_plain<true>(w, std::max<uint64_t>(m, 3));
+        return {"gemv_mfma_kernel", bp, 16 / plain.parts, plain.waves, 1, 1};
+    }
+    uint32_t tpw, waves;
+    gemv_rows_shape(w.dtype == COEUS_W_Q4_0, (uint32_t)(w.k_pad / 128), (uint32_t)(w.n_pad / 16), tpw, waves);
+    return {"gemv_rows_kernel", bp, 16 * tpw, waves, 1, 1};
+}
+int launch_gemm_few(const Weight &w, const uint16_t *a, uint64_t lda, uint64_t m, const EpiArgs &e, hipStream_t st) {
+    if (w.dtype >= COEUS_W_Q8_0 && lda != gemm_ld(w.k)) return fail(COEUS_INVALID_INPUT, "matmul of few rows: rows %llu elements apart", (unsigned long long)lda);
+    if (w.dtype == COEUS_W_Q8_0) return launch_gemv_rows_of<false, true>(w, a, m, e, st);
+    if (w.dtype == COEUS_W_Q4_0) return launch_gemv_rows_of<true, true>(w, a, m, e, st);
+    const MfmaPlain plain = gemv_mfma_plain<true>(w, std::max<uint64_t>(m, 3));
+    const uint32_t bp = std::max(pad_batch(m), 4u), parts = plain.parts, mw = plain.waves, pairs = (uint32_t)(w.k / 64), np = (pairs / parts + mw - 1) / mw;
+    const uint32_t tiles = (uint32_t)ceil_div(w.n, 16 / parts), rows = parts > 1 ? 16 : bp;
+    const dim3 grid(std::min(tiles, 256 * (16 / mw))), block(mw * 64);
+    const size_t lds = (size_t)mw * 16 * mfma_wave_lds<true, true>((int)ceil_div(rows, MfmaRows16::XROWS));
+#define COEUS_FEW(BPV, KV, TV, FV)                                                                                             \
+    do {                                                                                                                       \
+        auto kern = gemv_mfma_kernel<true, BPV, 0, 2, KV, TV, FV, true>;                                                       \
+        static const hipError_t room = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+        COEUS_HIP(room);                                                                                                       \
+        hipLaunchKernelGGL(kern, grid, block, lds, st, (const uint16_t *)w.data, (const float *)a, (uint32_t)w.k, (uint32_t)w.n, (uint32_t)m, mw, grid.x, e, \
+                           nullptr, nullptr, 0.f, lda, PostNorm{nullptr, nullptr, nullptr});                                   \
+    } while (0)
+#define COEUS_FEW2(BPV) do { if (np <= 2) COEUS_FEW(BPV, true, 1, false); else if (pairs > 4 * mw) COEUS_FEW(BPV, false, 1, true); else COEUS_FEW(BPV, false, 1, false); } while (0)
+    if (parts == 4) { if (np <= 2) COEUS_FEW(4, true, 4, false); else COEUS_FEW(4, false, 4, false); }
+    else if (parts == 2) { if (np <= 2) COEUS_FEW(8, true, 2, false); else COEUS_FEW(8, false, 2, false); }
+    else if (bp == 4) COEUS_FEW2(4);
+    else if (bp == 8) COEUS_FEW2(8);
+    else COEUS_FEW2(16);
+#undef COEUS_FEW2
+#undef COEUS_FEW
+    COEUS_HIP(hipGetLastError());
+    return COEUS_OK;
 }
 
 // Up to 64 rows: with 128 (8 fragments of 16 rows per wave) the kernel needs 348 registers and
