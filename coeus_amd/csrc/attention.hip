@@ -120,7 +120,8 @@ __device__ __forceinline__ void kv_piece(const uint4 &r, float (&v)[EPL]) {
         else { union { uint32_t u32; half2_t h2; } cv; cv.u32 = w[u]; v[2 * u] = (float)cv.h2.x; v[2 * u + 1] = (float)cv.h2.y; }
     }
 }
-template <int HD, int KV, int NW, int TILE, bool ROWS = false>
+// ROWS: prompts (see below); LP: their results as 16-bit rows at out_xq, bp elements apart, for the output projection (1 f16, 2 bf16).
+template <int HD, int KV, int NW, int TILE, bool ROWS = false, int LP = 0>
 __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__restrict__ qkv,
                                                           const void *__restrict__ kc,
                                                           const void *__restrict__ vc,
@@ -251,6 +252,10 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(const float *__res
         if (nsplit == 1) {
             // the whole context in one workgroup: this is the result, nothing to publish or merge
             const float r = a / lt;
+            if constexpr (LP != 0) {
+                ((uint16_t *)out_xq)[(uint64_t)b * bp + h * HD + threadIdx.x] = f32_to_lp_bits(r, LP == 2);
+                return;
+            }
             if (out) out[(uint64_t)b * inner + h * HD + threadIdx.x] = r;
             if (out_xq) out_xq[xq_index(h * HD + threadIdx.x, b, bp)] = __float2half_rn(r);
             return;
@@ -838,6 +843,9 @@ bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype) {
 
 // Prompts of fewer than 16 rows with a workgroup per row and head (attn_decode_kernel's ROWS form; grid.z holds the sequences).
 static bool attn_rows_apart(uint64_t batch, uint64_t n, uint64_t hd) { return n < 16 && (hd == 64 || hd == 128) && batch <= 65535; }
+bool attn_writes_lp(uint64_t batch, uint64_t n, uint64_t hd, uint32_t kv_dtype) {
+    return attn_prefill_on_matrix_cores(n, hd, kv_dtype) || (attn_rows_apart(batch, n, hd) && kv_dtype != COEUS_KV_F32);
+}
 
 // Queries of a workgroup of f32 prompt attention: one up to 15 rows; then 32, with four key shares, while 128 queries give few workgroups.  us, 128 queries / 32:
 // heads of 64, up to 384 workgroups: 12 heads at 64 / 128 / 512 / 1024 rows 7.6 / 5.0, 13.0 / 6.1, 42 / 16, 81 / 49; 48 at 1024 1.28x as
@@ -956,7 +964,8 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
         COEUS_HIP(hipGetLastError());
         return COEUS_OK;
     }
-    if (lp) return fail(COEUS_INVALID_INPUT, "16-bit attention output needs the matrix-core prefill kernel");
+    if (lp && (!attn_writes_lp(batch, n, hd, kv_dtype) || pos_dev || out || out_xq || lp_ld >> 32))
+        return fail(COEUS_INVALID_INPUT, "16-bit attention output needs a prompt, heads of 64 or 128 and a 16-bit cache");
     if (kv_dtype == COEUS_KV_F32 && attn_prefill_f32_queries(batch, n, pos0, heads, hd) > 4 && !pos_dev && out && !out_xq) {
         const dim3 pgrid((unsigned)ceil_div(n, 128), (unsigned)heads, (unsigned)batch);
         if (attn_prefill_f32_queries(batch, n, pos0, heads, hd) == 32) {
@@ -980,14 +989,17 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
     }
     // Fewer than 16 rows: a workgroup per row and head, as in a decode step whose keys stay in one piece.  Bound by the launch and one trip to
     // memory behind the queries'; attn_generic_kernel's lanes walk a key each, dimension by dimension (5 rows x 12 heads of 64, f32: 5.3 us,
-    // 3.3 here).
+    // 3.3 here).  16-bit rows for the output projection spare it a launch that converts them (prompt passes of 3 and 12 ids, ms,
+    // with it / so: 250M bf16 0.377 / 0.351, 0.460 / 0.434, 250M Q8_0 0.386 / 0.362, 0.419 / 0.403, 1B Q4_0 0.937 / 0.883, 1.008 / 0.950, 7B Q4_0 1.755 / 1.708, 1.880 / 1.850).
     if (attn_rows_apart(batch, n, hd)) {
         const dim3 rgrid((unsigned)n, (unsigned)heads, (unsigned)batch);
         const uint32_t kpl = 64 / ((uint32_t)hd / (kv_dtype == COEUS_KV_F32 ? 4 : 8));
         const bool few = !pos_dev && pos0 + n <= 16 * kpl;
-#define COEUS_AR2(HDV, KVV, TV)                                                                                                    \
-    hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV, 4, TV, true>), rgrid, dim3(256), 0, st, qkv, kc, vc, (uint32_t)heads, (uint32_t)max_ctx, \
-                       (uint32_t)pos0, pos_dev, (uint32_t)max_ctx, nullptr, nullptr, out, out_xq, bp)
+#define COEUS_AR3(HDV, KVV, TV, LPV)                                                                                               \
+    hipLaunchKernelGGL((attn_decode_kernel<HDV, KVV, 4, TV, true, LPV>), rgrid, dim3(256), 0, st, qkv, kc, vc, (uint32_t)heads, (uint32_t)max_ctx, \
+                       (uint32_t)pos0, pos_dev, (uint32_t)max_ctx, nullptr, nullptr, out, LPV ? (__half *)lp : out_xq, LPV ? (uint32_t)lp_ld : bp)
+#define COEUS_AR2(HDV, KVV, TV) do { if (KVV != COEUS_KV_F32 && lp && lp_bf) COEUS_AR3(HDV, KVV, TV, (KVV == COEUS_KV_F32 ? 0 : 2)); \
+        else if (KVV != COEUS_KV_F32 && lp) COEUS_AR3(HDV, KVV, TV, (KVV == COEUS_KV_F32 ? 0 : 1)); else COEUS_AR3(HDV, KVV, TV, 0); } while (0)
 #define COEUS_AR(HDV, KVV) do { if (few) COEUS_AR2(HDV, KVV, 4); else COEUS_AR2(HDV, KVV, (KVV == COEUS_KV_F32 ? 8 : 16)); } while (0)
 #define COEUS_ARH(HDV) do { if (kv_dtype == COEUS_KV_F32) COEUS_AR(HDV, COEUS_KV_F32); \
         else if (kv_dtype == COEUS_KV_BF16) COEUS_AR(HDV, COEUS_KV_BF16); else COEUS_AR(HDV, COEUS_KV_F16); } while (0)
@@ -995,6 +1007,7 @@ int launch_attention(const float *qkv, const void *kc, const void *vc, uint32_t 
 #undef COEUS_ARH
 #undef COEUS_AR
 #undef COEUS_AR2
+#undef COEUS_AR3
         COEUS_HIP(hipGetLastError());
         return COEUS_OK;
     }

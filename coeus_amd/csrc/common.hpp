@@ -345,6 +345,8 @@ uint32_t attn_decode_splits(uint64_t batch, uint64_t heads, uint64_t hd, uint32_
 // output rows) rather than the generic one.
 uint32_t attn_prefill_f32_queries(uint64_t batch, uint64_t n, uint64_t pos0, uint64_t heads, uint64_t hd);
 bool attn_prefill_on_matrix_cores(uint64_t n, uint64_t hd, uint32_t kv_dtype);
+// ... and that launch_attention can write 16-bit rows: those, and prompts of fewer than 16 rows.
+bool attn_writes_lp(uint64_t batch, uint64_t n, uint64_t hd, uint32_t kv_dtype);
 // Attention of n new rows per sequence (positions pos..pos+n-1) against the cache.
 // part_scratch: [batch*heads*nsplit*(head_dim+2)] f32 for the split decode kernel (nullable);
 // counters: [batch*heads] zeroed u32 -> the last split merges in-kernel (else a merge kernel runs).

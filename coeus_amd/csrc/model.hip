@@ -460,7 +460,7 @@ int run_blocks_prefill(Model &m, Workspace &ws, const Cache &cache, uint64_t bat
     // reference-parity mode and stays on the f32 route).
     const bool lp = c.weight_dtype != COEUS_W_F32 && c.norm_scope == COEUS_SCOPE_TOKEN && ws.a_lp.p && ws.b_lp.p;
     const bool lp_bf = c.weight_dtype == COEUS_W_BF16;
-    const bool attn_lp = lp && attn_prefill_on_matrix_cores(n, hd, c.kv_dtype);
+    const bool attn_lp = lp && attn_writes_lp(batch, n, hd, c.kv_dtype);
     const LpOut x_lp{ws.a_lp.p, gemm_ld(H), lp_bf};
     const LpOut att_lp{ws.b_lp.p, gemm_ld(m.L.inner_dim), lp_bf};
     const LpOut ff_lp{ws.b_lp.p, gemm_ld(c.intermediate_dim), lp_bf};
