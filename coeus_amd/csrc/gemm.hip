@@ -1789,25 +1789,28 @@ struct F32Shape { uint32_t rows, cols, slice, waves; double rate, fixed, alone; 
 static constexpr F32Shape kF32Shapes[] = {{32, 32, 128, 8, 6.9, 0.1, 0.}, {32, 32, 64, 4, 5.7, 0.9, 8.1}, {64, 32, 64, 8, 9.4, 0.9, 10.4},
                                           {64, 64, 32, 8, 17., 2., 21.},  {128, 64, 32, 8, 32., 2.4, 37.7}};
 struct F32Plan { uint32_t shape, splits; };
+// A launch of that many workgroups of `waves` waves fits a grid's 2^32 threads (it is rounded up to a multiple of 8).
+static constexpr bool f32_grid_fits(uint64_t workgroups, uint32_t waves) { return workgroups < (1ull << 32) / (64 * waves) - 8; }
 static F32Plan gemm_f32_plan(const Weight &w, uint64_t m, bool may_split) {
-    F32Plan best{0, 1};
+    F32Plan best{0, 0};
     double least = 0.;
     for (uint32_t i = 0; i < sizeof(kF32Shapes) / sizeof(kF32Shapes[0]); i++) {
         const F32Shape &t = kF32Shapes[i];
         const uint64_t tiles = ceil_div(m, t.rows) * ceil_div(w.n, t.cols), slices = ceil_div(w.k, t.slice);
         for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
-            if (s > 1 && (!may_split || slices < 2 * s)) break;
+            if ((s > 1 && (!may_split || slices < 2 * s)) || !f32_grid_fits(tiles * s, t.waves)) break;
             const double k = (double)(ceil_div(slices, s) * t.slice) / 1000.;
             const double us = std::max(t.alone * k, (double)ceil_div(tiles * s, 256) * t.rate * k + t.fixed) + (s > 1 ? 3.8 + 1.4e-6 * s * (double)m * (double)w.n : 0.);
-            if ((i == 0 && s == 1) || us < least) { least = us; best = {i, s}; }
+            if (best.splits == 0 || us < least) { least = us; best = {i, s}; }
         }
     }
     return best;
 }
 
-// 16-byte requests, and 32-bit places in a tile and in its launch
+// 16-byte requests, 32-bit places in a tile, and a grid for the largest tiles at least
 static bool gemm_f32_has_tiles(const Weight &w, uint64_t m) {
-    return (w.k & 3) == 0 && w.k < (1u << 22) && ceil_div(m, 32) * ceil_div(w.n, 32) < (1u << 28);
+    const F32Shape &largest = kF32Shapes[sizeof(kF32Shapes) / sizeof(kF32Shapes[0]) - 1];
+    return (w.k & 3) == 0 && w.k < (1u << 22) && f32_grid_fits(ceil_div(m, largest.rows) * ceil_div(w.n, largest.cols), largest.waves);
 }
 
 template <int WM, int WN, int RB, int NB, int KH, int L, int D, int PERIOD>

@@ -146,3 +146,15 @@ def test_other_prompts():
     assert plan(_lib.W_Q4_0, 4096, 22016, 4071, 1).tail_shares == 2 and plan(_lib.W_BF16, 512, 4090, 4100, 1).tail_shares == 2
     assert plan(_lib.W_F32, 768, 768, 5, 1).kernel == b"gemv_mfma_kernel" and plan(_lib.W_F32, 768, 768, 128, 1).kernel == b"gemm_f32_small_kernel"
     assert plan(_lib.W_F32, 3072, 768, 128, 1).shares == 8 and plan(_lib.W_F32, 768, 50257, 128, 1).kernel == b"gemm_f32_kernel"
+
+
+# f32 prompts of very many outputs: the tiles' grid has one dimension, of at most 2^32 threads (17 rows of 4 x 2^29, 36 GB of results: 2^24 tiles of four waves would be one thread too many)
+@pytest.mark.parametrize("k,n,m", [(4, 1 << 28, 17), (4, 1 << 28, 32), (4, (1 << 28) - 256, 32), (4, (1 << 28) + 4, 33), (4, 1 << 29, 17), (4, 1 << 29, 200), (8192, 1 << 22, 1024), (64, 1 << 24, 5000),
+                                   (4, 1 << 20, 100000), (4, 1 << 16, 1 << 22), (4, 1 << 31, 17), (1 << 20, 256, 1 << 20)])
+def test_the_grid_of_f32_tiles(k, n, m):
+    p = plan(_lib.W_F32, k, n, m, 1)
+    tiles = -(-m // p.tile_rows) * -(-n // p.tile_cols)
+    if p.kernel in (b"gemm_f32_small_kernel", b"gemm_f32_kernel"):
+        assert -(-tiles * p.shares // 8) * 8 * p.waves * 64 < 1 << 32
+    else:
+        assert p.kernel == b"gemm_f32_any_kernel" and tiles >= 1 << 22
