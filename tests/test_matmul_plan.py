@@ -148,7 +148,7 @@ def test_other_prompts():
     assert plan(_lib.W_F32, 3072, 768, 128, 1).shares == 8 and plan(_lib.W_F32, 768, 50257, 128, 1).kernel == b"gemm_f32_kernel"
 
 
-# f32 prompts of very many outputs: the tiles' grid has one dimension, of at most 2^32 threads (17 rows of 4 x 2^29, 36 GB of results: 2^24 tiles of four waves would be one thread too many)
+# f32 prompts of very many outputs: the tiles' grid has one dimension, of at most 2^32 threads (17 rows of 4 x 2^29, 36 GB of results: 2^23 tiles of eight waves are one thread too many)
 @pytest.mark.parametrize("k,n,m", [(4, 1 << 28, 17), (4, 1 << 28, 32), (4, (1 << 28) - 256, 32), (4, (1 << 28) + 4, 33), (4, 1 << 29, 17), (4, 1 << 29, 200), (8192, 1 << 22, 1024), (64, 1 << 24, 5000),
                                    (4, 1 << 20, 100000), (4, 1 << 16, 1 << 22), (4, 1 << 31, 17), (1 << 20, 256, 1 << 20)])
 def test_the_grid_of_f32_tiles(k, n, m):
