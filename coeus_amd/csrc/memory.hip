@@ -301,7 +301,8 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
 #pragma unroll
             for (int i = 0; i < 4; i++) v[m][t][i] = vp[(uint64_t)min(16u * m + 4 * g + i, live - 1) * dm.in_ld + min(16 * (wave + W * t) + c, e - 1)];
     }
-    // queries and keys, half a wave per row: rows behind the end repeat the last one, dims behind the end are zero
+    // queries and keys, half a wave per row: rows behind the end repeat the last one, dims behind the end are zero (ONE: so are keys behind the end, whose
+    // products with weights of zero the state takes)
     for (uint32_t x = 4 * (tid & 31); x < 16 * cb.dtiles; x += 128)
 #pragma unroll
         for (uint32_t r = tid >> 5; r < kChunk; r += 16) {
@@ -309,6 +310,7 @@ __global__ __launch_bounds__(512) void memory_read_kernel(const float *__restric
             const uint64_t at = (uint64_t)min(r, live - 1) * dm.in_ld + min(x, d - 4);
             float4_t qv = *(const float4_t *)(qp + at), kv = *(const float4_t *)(kp + at);
             if (x >= d) qv = kv = float4_t{0.f, 0.f, 0.f, 0.f};
+            if (ONE && r >= live) kv = float4_t{0.f, 0.f, 0.f, 0.f};
             *(float4_t *)(ql + r * LD + x) = qv;
             *(float4_t *)(kl + r * LD + x) = kv;
         }

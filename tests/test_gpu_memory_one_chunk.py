@@ -1,6 +1,6 @@
 """Matrix memory, prompts of one chunk: a launch that reads the state, answers and stores the state behind the prompt.  At the
 edges of the 16-token tiles and of the sizes, from a state that earlier tokens left, with a value that is not finite (which the rows
-in front of it must not see), and for rows that 16-byte pieces do not lie in (token by token, as before)."""
+in front of it must not see) or a key that is infinite, and for rows that 16-byte pieces do not lie in (token by token, as before)."""
 import ctypes as C
 
 import numpy as np
@@ -38,6 +38,20 @@ def test_rows_in_front_of_a_value_that_is_not_finite(bad, n, j):
     assert np.array_equal(got[:, :j], clean[:, :j])  # the same sums of the same values
     assert not np.isfinite(got[0, j:, 5]).any() and np.isfinite(got[0, :, e:]).all()  # (the other head)
     assert not np.isfinite(a.state[0].to_host()[0, 0, :, 5]).any() and np.isfinite(a.state[0].to_host()[0, :, :, 6]).all()
+
+
+@pytest.mark.parametrize("n,j", [(2, 1), (5, 4), (16, 15), (17, 16), (30, 29), (30, 7), (63, 62)])
+def test_infinite_key_as_token_by_token(n, j):
+    H, d, e = 2, 32, 48
+    a, b = (Memory(H, d, e, batch=1, seed=n) for _ in range(2))
+    p = a.inputs(n)
+    p[0, j, H * d + 3] = np.inf
+    got, want = a.prompt(p, 1), b.prompt(p, 0)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want)) and np.isfinite(got[0, :j]).all()
+    for x, y in zip(a.state, b.state):
+        x, y = x.to_host(), y.to_host()
+        assert np.array_equal(x[~np.isfinite(y)], y[~np.isfinite(y)]) and np.isfinite(x).sum() == np.isfinite(y).sum()
+    assert (np.abs(a.state[0].to_host()[0, 0, 3]) == np.inf).all() and a.state[1].to_host()[0, 0, 3] == np.inf
 
 
 def test_rows_off_a_16_byte_boundary():
