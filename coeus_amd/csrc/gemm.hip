@@ -326,8 +326,10 @@ __device__ __forceinline__ void epi_store4(const EpiArgs &e, uint64_t row, uint6
         *(uint2 *)(e.out_lp + row * e.lp_ld + col) = p;
     }
 }
+// Four columns at a time: rows of whole fours, and pointers of the caller's that 16-byte (8-byte: 16-bit rows) pieces fit.
 __device__ __forceinline__ bool epi_vec4(const EpiArgs &e) {
-    return (e.n_eff & 3) == 0 && (e.lp_ld & 3) == 0 && (e.out_f32 || e.out_lp) && !e.out_xq;
+    return (e.n_eff & 3) == 0 && (e.lp_ld & 3) == 0 && (e.out_f32 || e.out_lp) && !e.out_xq &&
+           (((uintptr_t)e.out_f32 | (uintptr_t)e.bias | (uintptr_t)e.residual) & 15) == 0 && ((uintptr_t)e.out_lp & 7) == 0;
 }
 // Columns col .. col + 3 of activation row `row` (bias, cache append or activation, residual, store).
 // OWN: GELU and SiLU by times_sigmoid where the caller sees f32 results (no further off than the math library's forms), else on the
@@ -2032,7 +2034,7 @@ coeus_matmul_plan gemm_launch_plan(const Weight &w, uint64_t m) {
 }
 
 bool gemm_appends_kv(const Weight &w, uint64_t m, uint64_t inner, uint64_t hd) {
-    // (f32: element by element, or by the kernel that sums a split launch's planes, four columns at a time)
+    // (f32: element by element, or four columns at a time, which stay inside one head)
     if (w.dtype == COEUS_W_F32) return m < (1ull << 32) && w.n == 3 * inner && (inner & 3) == 0 && (hd & 3) == 0;
     if (gemm_uses_few(w, m)) return w.n == 3 * inner;  // (element by element)
     // rows fit 32 bits; a lane's 4 columns stay inside one head.  (The short-prompt kernel for

@@ -1,4 +1,4 @@
-"""The f32 prompt matmul at the edges of its tiles, of a slice of k and of its shares, against float64."""
+"""The f32 prompt matmul at the edges of its tiles, of a slice of k, of its shares and of 16-byte pieces of what it reads and writes, against float64."""
 import ctypes as C
 
 import numpy as np
@@ -80,3 +80,34 @@ def test_rows_between_pieces():
     synchronize()
     out = out.to_host()
     assert np.all(np.abs(out - exact) <= 256 * 2.0 ** -24 * size)  # (sums of up to 192 products in each of four waves)
+
+
+# outputs that whole groups of four fill and that they do not (a row of 2050 weight rows gives 1025 gated ones); one share and several; all from 17 rows on
+@pytest.mark.parametrize("k,n,m", [(100, 98, 33), (3072, 104, 40), (768, 2050, 300), (772, 2304, 257)])
+@pytest.mark.parametrize("epilogue", [_lib.EPI_NONE, _lib.EPI_GELU, _lib.EPI_SILU_GATE])
+@pytest.mark.parametrize("off", [(0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (3, 2, 1)])
+def test_epilogues_between_pieces(k, n, m, epilogue, off):
+    """Results, bias and residual that start between two 16-byte pieces (by `off` floats), with every activation."""
+    rng = np.random.default_rng(n + m)
+    gated = epilogue == _lib.EPI_SILU_GATE
+    w, a = Weight(_lib.W_F32, seed=9, shape=(k, n)), rng.standard_normal((m, k)).astype(np.float32)
+    b, r = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n // 2 if gated else n)).astype(np.float32)
+    at = lambda x, o: dev(np.r_[np.zeros(o, np.float32), x.ravel()])  # noqa: E731
+    da, out, db, dr = dev(a), at(np.full(r.size + 4, 7, np.float32), off[0]), at(b, off[1]), at(r, off[2])
+    ptr = lambda x, o: C.c_void_p(C.cast(x.ptr, C.c_void_p).value + 4 * o)  # noqa: E731
+    _check(_lib.load().coeus_op_gemm(w.h, da.ptr, m, ptr(db, off[1]), ptr(dr, off[2]), epilogue, ptr(out, off[0]), None))
+    synchronize()
+    got = out.to_host()
+    assert not got[:off[0]].any() and np.all(got[off[0] + r.size:] == 7)
+    got = got[off[0]:off[0] + r.size].reshape(r.shape)
+    size, pb = ROUNDINGS * (np.abs(a).astype(np.float64) @ np.abs(w.dequantize()) + np.abs(b)), a.astype(np.float64) @ w.dequantize() + b
+    # GELU has slopes of up to 1.13, SiLU of 1.1; some 16 roundings each of their own, the residual one
+    if gated:
+        g, u = pb[:, 0::2], pb[:, 1::2]
+        s = g / (1 + np.exp(-g))
+        want, bound = s * u, 1.1 * size[:, 0::2] * np.abs(u) + np.abs(s) * size[:, 1::2] + 2.0 ** -20 * np.abs(s * u) + 1e-6
+    elif epilogue == _lib.EPI_GELU:
+        want, bound = 0.5 * pb * (1 + np.tanh(0.7978845608028654 * pb * (1 + 0.044715 * pb * pb))), 1.2 * size + 2.0 ** -20 * (1 + np.abs(pb))
+    else:
+        want, bound = pb, size
+    assert np.all(np.abs(got - (want + r)) <= bound + 2.0 ** -23 * (np.abs(want) + np.abs(r)))
