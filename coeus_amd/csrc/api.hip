@@ -958,13 +958,22 @@ int coeus_op_memory_prompt(const coeus_memory_shape *shape, const coeus_memory_w
         return fail(COEUS_INVALID_INPUT, "null pointer argument or size out of range");
     if (batch == 0 || n == 0 || batch > 65535 || n > 0x7fffffffull)
         return fail(COEUS_INVALID_INPUT, "matrix memory: %llu x %llu rows out of range", (unsigned long long)batch, (unsigned long long)n);
+    COEUS_TRY(memory_check_args(dm, batch, n));
     hipStream_t st = (hipStream_t)stream;
-    DeviceBuf scratch;
+    DeviceBuf scratch, rows;
     int rc = scratch.ensure(memory_prompt_scratch_bytes(dm, batch, n, chunked != 0));
+    if (rc == COEUS_OK && chunked && ((uintptr_t)proj_dev & 15) && memory_prompt_in_pieces(dm, n)) {
+        // rows between two 16-byte pieces: their copy (of the last row what it holds), not token by token
+        const uint64_t bytes = ((batch * n - 1) * dm.in_ld + dm.forget_off() + dm.heads) * 4;
+        rc = rows.ensure(bytes);
+        if (rc == COEUS_OK && hipMemcpyAsync(rows.p, proj_dev, bytes, hipMemcpyDeviceToDevice, st) != hipSuccess)
+            rc = fail(COEUS_DEVICE_ERROR, "matrix memory: copy of the rows failed");
+        proj_dev = (const float *)rows.p;
+    }
     if (rc == COEUS_OK)
         rc = launch_memory_prompt(proj_dev, dm, pr, MemoryState{state_dev, norm_state_dev, max_dev}, batch, n, out_dev, nullptr,
                                   (float *)scratch.p, scratch.bytes, st, chunked != 0);
-    return finish_op(rc, st, {&scratch}, "matrix memory");
+    return finish_op(rc, st, {&scratch, &rows}, "matrix memory");
     COEUS_GUARD_END
 }
 

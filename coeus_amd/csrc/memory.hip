@@ -5,7 +5,7 @@
 //   memory_carry_kernel   prompt: the state in front of every chunk (element by element over the chunks)
 //   memory_read_kernel    prompt: the outputs of every chunk, normalised and gated, all chunks at once; of prompts that are one chunk,
 //                         the state behind it too, and no other launch
-//   memory_scan_kernel    odd sizes and places, few tokens: token by token, state in registers
+//   memory_scan_kernel    sizes or rows that 16-byte pieces do not fit, single tokens: token by token, state in registers
 //   memory_finish_kernel  its outputs: normaliser, RMS norm, gate
 //   memory_step_kernel    decode: all of it for one token per sequence
 //
@@ -28,7 +28,7 @@ __device__ __forceinline__ void log_gates(const float *__restrict__ p, const Mem
 __device__ __forceinline__ float sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float normaliser(float nq, float m) { return fmaxf(fabsf(nq), expf(-m)) + kFloor; }
 
-static int check_args(const MemoryDims &dm, uint64_t batch, uint64_t n) {
+int memory_check_args(const MemoryDims &dm, uint64_t batch, uint64_t n) {
     if (dm.heads == 0 || dm.heads > 65535 || dm.d == 0 || dm.d > kMaxDim || dm.e == 0 || dm.e > 1024 ||
         dm.in_ld < dm.forget_off() + dm.heads || !(dm.cap > 0.f))
         return fail(COEUS_INVALID_INPUT, "matrix memory: sizes out of range");
@@ -67,12 +67,10 @@ static uint64_t chunk_floats(const MemoryDims &dm, uint64_t units, uint64_t chun
 static bool chunk_shape(const MemoryDims &dm) {
     return dm.d % 4 == 0 && dm.e % 4 == 0 && dm.in_ld % 4 == 0 && dm.d <= kMaxChunkDim && dm.e <= kMaxChunkDim;
 }
-static bool chunked(const MemoryDims &dm, uint64_t n) {
-    // (a few dozen tokens are quicker one by one than through three launches)
-    return n >= 48 && chunk_shape(dm);
-}
-// The prompt is one chunk: one launch reads the state, answers and stores the state behind it (rows in 16-byte pieces).
-static bool one_chunk(const MemoryDims &dm, uint64_t n, const float *proj) { return n >= 2 && n <= kChunk && chunk_shape(dm) && ((uintptr_t)proj & 15) == 0; }
+// More than one chunk: three launches.  (One: a single launch that reads the state, answers and stores the state behind it.)
+static bool chunked(const MemoryDims &dm, uint64_t n) { return n > kChunk && chunk_shape(dm); }
+static bool one_chunk(const MemoryDims &dm, uint64_t n) { return n >= 2 && n <= kChunk && chunk_shape(dm); }
+bool memory_prompt_in_pieces(const MemoryDims &dm, uint64_t n) { return n >= 2 && chunk_shape(dm); }
 
 struct ChunkGates {
     double F, a, top;  // running sum of the log forget gates, log input gate - F, running maximum of that
@@ -624,6 +622,7 @@ __global__ __launch_bounds__(256) void memory_finish_kernel(const float *__restr
 }
 
 uint64_t memory_prompt_scratch_bytes(const MemoryDims &dm, uint64_t batch, uint64_t n, bool may_chunk) {
+    if (may_chunk && one_chunk(dm, n)) return 0;
     if (may_chunk && chunked(dm, n)) return chunk_floats(dm, batch * dm.heads, ceil_div(n < kSegment ? n : kSegment, kChunk)) * 4;
     return batch * n * dm.heads * (dm.e + 2ull) * 4;
 }
@@ -631,8 +630,10 @@ uint64_t memory_prompt_scratch_bytes(const MemoryDims &dm, uint64_t batch, uint6
 int launch_memory_prompt(const float *proj, const MemoryDims &dm, const MemoryParams &pr, const MemoryState &state, uint64_t batch,
                          uint64_t n, float *out, const LpOut *out_lp, float *scratch, uint64_t scratch_bytes, hipStream_t st,
                          bool may_chunk) {
-    COEUS_TRY(check_args(dm, batch, n));
-    if (!scratch || scratch_bytes < memory_prompt_scratch_bytes(dm, batch, n, may_chunk))
+    COEUS_TRY(memory_check_args(dm, batch, n));
+    if ((uintptr_t)proj & 15) may_chunk = false;
+    const uint64_t needs = memory_prompt_scratch_bytes(dm, batch, n, may_chunk);
+    if (needs && (!scratch || scratch_bytes < needs))
         return fail(COEUS_INVALID_INPUT, "matrix memory: scratch too small");
     uint16_t *lp = out_lp ? (uint16_t *)out_lp->p : nullptr;
     const uint64_t lp_ld = out_lp ? out_lp->ld : 0;
@@ -645,7 +646,7 @@ int launch_memory_prompt(const float *proj, const MemoryDims &dm, const MemoryPa
         hipLaunchKernelGGL((memory_read_kernel<NV, ONEV>), rgrid, dim3(512), read_lds_bytes(dm), st, proj, dm, pr, state, n, t0, seg, cb, out, lp, \
                            lp_ld, lp_bf);                                                                                         \
     } while (0)
-    if (may_chunk && one_chunk(dm, n, proj)) {
+    if (may_chunk && one_chunk(dm, n)) {
         MemoryChunks cb = {};
         cb.chunks = 1;
         cb.dtiles = (uint32_t)ceil_div(dm.d, 16);
@@ -810,7 +811,7 @@ __global__ __launch_bounds__(512) void memory_step_kernel(const float *__restric
 
 int launch_memory_step(const float *proj, const MemoryDims &dm, const MemoryParams &pr, const MemoryState &state, uint64_t batch,
                        float *out, hipStream_t st) {
-    COEUS_TRY(check_args(dm, batch, 1));
+    COEUS_TRY(memory_check_args(dm, batch, 1));
     const bool vec = dm.e % 4 == 0;
     const uint32_t cg = vec ? dm.e / 4 : dm.e;
     if (cg > 512) return fail(COEUS_INVALID_INPUT, "matrix memory: a value size above 512 must be a multiple of 4");

@@ -78,12 +78,14 @@ struct MemoryParams {
 struct MemoryState {
     float *s, *n, *m;  // [batch][heads][d][e], [batch][heads][d], [batch][heads]
 };
-// n new tokens per sequence: f32 rows (out) and / or 16-bit rows (out_lp), state moved on.  may_chunk false:
-// token by token whatever the length.
+int memory_check_args(const MemoryDims &dm, uint64_t batch, uint64_t n);  // sizes that there are kernels for
+// n new tokens per sequence: f32 rows (out) and / or 16-bit rows (out_lp), state moved on.  may_chunk false, or a proj
+// that does not start on 16 bytes: token by token whatever the length.
 int launch_memory_prompt(const float *proj, const MemoryDims &dm, const MemoryParams &pr, const MemoryState &state, uint64_t batch,
                          uint64_t n, float *out, const LpOut *out_lp, float *scratch, uint64_t scratch_bytes, hipStream_t st,
                          bool may_chunk = true);
 uint64_t memory_prompt_scratch_bytes(const MemoryDims &dm, uint64_t batch, uint64_t n, bool may_chunk = true);
+bool memory_prompt_in_pieces(const MemoryDims &dm, uint64_t n);  // whether such a prompt is read 16 bytes at a time
 int launch_memory_step(const float *proj, const MemoryDims &dm, const MemoryParams &pr, const MemoryState &state, uint64_t batch,
                        float *out, hipStream_t st);
 

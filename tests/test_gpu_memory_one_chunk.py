@@ -1,6 +1,7 @@
 """Matrix memory, prompts of one chunk: a launch that reads the state, answers and stores the state behind the prompt.  At the
 edges of the 16-token tiles and of the sizes, from a state that earlier tokens left, with a value that is not finite (which the rows
-in front of it must not see) or a key that is infinite, and for rows that 16-byte pieces do not lie in (token by token, as before)."""
+in front of it must not see) or a key that is infinite, and for rows that
+16-byte pieces do not lie in, in one chunk and in several."""
 import ctypes as C
 
 import numpy as np
@@ -61,3 +62,17 @@ def test_rows_off_a_16_byte_boundary():
     _check(_lib.load().coeus_op_memory_prompt(C.byref(t.s), C.byref(t.w), x.ptr + 4, *[a.ptr for a in t.state], 1, 20, 1, out.ptr, None))
     want, S = t.want(p)
     assert off(out.to_host(), want) < 2e-5 and t.state_off(S) < 2e-5
+
+
+@pytest.mark.parametrize("shape", [(2, 32, 48), (1, 20, 8), (2, 9, 5)])
+@pytest.mark.parametrize("n", [2, 48, 64, 65, 130])
+def test_rows_off_a_boundary_in_chunks(shape, n):
+    """The same bits as rows on a boundary, nothing behind the last row's gates read (the buffer ends there)."""
+    H, d, e = shape
+    a, b = (Memory(*shape, batch=2, seed=n) for _ in range(2))
+    p = a.inputs(n)
+    want = a.prompt(p, 1)
+    x, out = dev(np.r_[np.zeros(1, np.float32), p.ravel()[:p.size - (a.ld - a.nb - 2 * H)]]), DeviceArray((2, n, H * e))
+    _check(_lib.load().coeus_op_memory_prompt(C.byref(b.s), C.byref(b.w), x.ptr + 4, *[s.ptr for s in b.state], 2, n, 1, out.ptr, None))
+    assert np.array_equal(out.to_host(), want)
+    assert all(np.array_equal(s.to_host(), t.to_host()) for s, t in zip(a.state, b.state))
