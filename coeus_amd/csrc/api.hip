@@ -598,7 +598,8 @@ int coeus_op_norm(uint32_t kind, uint32_t scope, const float *x_dev, uint64_t ro
     if (!x_dev || !scale_dev || !y_dev || (kind == COEUS_NORM_LAYERNORM && !bias_dev))
         return fail(COEUS_INVALID_INPUT, "null pointer argument");
     // whole-slice statistics over a large slice: many workgroups, through a scratch buffer that
-    // lives for this call (the model keeps one in its workspace instead)
+    // lives for this call (the model keeps one in its workspace instead, and uses it from 16384 elements on;
+    // a call without one neither allocates nor waits, and may be captured)
     double *part = nullptr;
     if (scope == COEUS_SCOPE_SEQUENCE && rows * hidden >= 32768)
         COEUS_HIP(hipMalloc((void **)&part, norm_sequence_scratch_bytes()));

@@ -370,7 +370,8 @@ int launch_norm(uint32_t kind, uint32_t scope, const float *x, uint64_t rows, ui
         const bool rms = kind == COEUS_NORM_RMSNORM;
         const bool vec = hidden % 4 == 0 && (((uintptr_t)x | (uintptr_t)y | (uintptr_t)scale | (rms ? 0 : (uintptr_t)bias)) & 15) == 0;
         // Two launches from 16384 elements (a pass over 32 ids of the 250M model, 25 norms: 0.83 ms with the one-workgroup kernel, 0.75 with two launches;
-        // over 17 ids 0.75 and 0.75); single elements from 32768.
+        // over 17 ids 0.75 and 0.75); single elements from 32768.  One workgroup up to 32768 is for the operator, which takes no scratch, and so may be captured
+        // and does not wait, below that.
         const bool parts = partials && n > (vec ? 16384u : 32767u);
         if (vec && n <= 32768 && !parts) {
 #define COEUS_NSS(VMV)                                                                                                                              \
