@@ -99,8 +99,11 @@ int HostCopy::out(void *dst, const void *src_dev, uint64_t bytes, hipStream_t st
         return t > before ? t : t + 1;
     };
     for (uint64_t r = 0; r < rounds && r < 2; r++) COEUS_HIP(launch(r));
-    const uint32_t cpus = std::max(3u, std::thread::hardware_concurrency() / 2);
-    const uint32_t threads = bytes >= kThreadsFrom ? (uint32_t)std::min<uint64_t>({bytes / kPerThread + 1, kThreads, cpus}) : 1;
+    uint32_t threads = 1;
+    if (bytes >= kThreadsFrom) {
+        static const uint32_t half = std::max(3u, std::thread::hardware_concurrency() / 2);  // (asks the system: once)
+        threads = (uint32_t)std::min<uint64_t>({bytes / kPerThread + 1, kThreads, half});
+    }
     std::atomic<bool> stop{false};
     std::atomic<uint64_t> copied[2] = {};  // pieces out of each half, over all rounds
     auto arrived = [&](uint64_t r, uint64_t p) { return __atomic_load_n(flags + r % 2 * kPieces + p, __ATOMIC_ACQUIRE) == turn_of(r); };

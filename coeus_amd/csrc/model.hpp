@@ -29,9 +29,10 @@ struct DeviceBuf {
 // mapped while the GPU still computes, and a piece is copied out as soon as its flag is there.  Copies and events of the
 // runtime's instead (1 MiB each) cost 15 us of the GPU's time a piece and 12 us between the last one's end and the
 // waiting thread; us behind the step, copies / this: 128 KB 33 / 14, 200 KB 35 / 18, 512 KB 48 / 28, 1.6 MB 94 / 60, 2 MB 117 / 70.
-// From 8 MB on more threads map and copy, one for 4 MB and five at most (no more than three where the process has not twice as many CPUs): a pass with
+// From 8 MB on more threads map and copy: three, another for each 4 MB more, five at most, and beyond three no more than half of the CPUs that the process may
+// be scheduled on (a quota of their time is not seen).  A pass with
 // every row's logits, 3 / 5 / 6 / 8 / 10 threads: 25.7 MB 1.80 / 1.58 / 1.54 / 1.56 / 1.58 ms, 50 MB 3.14 / 2.70 / 2.77 / 2.60 / 3.08, 103 MB 5.6 / 5.0 / 5.1 / 5.1 / 5.8.
-// Six and more are the slower ones for a new model's first pass (25.7 MB, 3 / 4 / 5 / 6: 2.05 / 1.83 / 1.80 / 3.4 ms).
+// Six and more are the slower ones for a new model's first pass (25.7 MB, 3 / 4 / 5 / 6: 2.05 / 1.83 / 1.80 / 3.4 ms; why is not known).
 // A launch of 32 workgroups writes 4 MB as fast as the link takes them (16 / 32 / 64, eight threads: 25.7 MB 1.62 / 1.57 / 1.57).
 // Into pinned (or device) memory the copy is the runtime's, without a stop.
 struct HostCopy {
