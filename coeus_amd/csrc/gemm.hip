@@ -12,7 +12,8 @@
 //     gemm_h256_kernel     k % 32 == 0: 256x256 tile, eight waves of 128x64, 32-wide slices
 //     gemm_h_kernel        any k: 128x128 tile, register-staged
 //     gemm_qskinny_kernel  17 to 64 rows on quantised weights: streams the quantised blocks
-//     up to 16 rows        the decode matmul's kernels (launch_gemm_few)
+//     up to 16 rows        the decode matmul's kernels (launch_gemm_few): bf16 with k % 64 == 0 and no infinity, quantised weights with
+//                          k % 128 == 0, none of a layered stack with a delta rule
 //     gemm_split_reduce_kernel, gemm_tail_reduce_kernel: sums behind launches split along k
 #include "device_utils.hpp"
 #include <type_traits>

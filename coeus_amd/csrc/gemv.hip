@@ -2694,11 +2694,11 @@ int launch_gemm_few(const Weight &w, const uint16_t *a, uint64_t lda, uint64_t m
     return COEUS_OK;
 }
 
-// Up to 64 rows: with 128 (8 fragments of 16 rows per wave) the kernel needs 348 registers and
+// 17 to 64 rows (fewer: gemm_uses_few): with 128 (8 fragments of 16 rows per wave) the kernel needs 348 registers and
 // is slower than the 256x256 kernel on the f16 copies.  Matrices of at least 4 M weights: below
 // (the 250M shape) the 256x256 kernel split along k is as fast or faster.
 bool gemm_uses_qskinny(const Weight &w, uint64_t m) {
-    return w.dtype >= COEUS_W_Q8_0 && m >= 1 && m <= 64 && w.k == w.k_pad && w.k >= 128 &&
+    return w.dtype >= COEUS_W_Q8_0 && m > 16 && m <= 64 && w.k == w.k_pad && w.k >= 128 &&
            w.k * w.n >= 4000000ull;
 }
 
