@@ -1,9 +1,10 @@
 """The prompt matmul on up to 16 rows of 16-bit operands, which takes the decode step's kernels: float64 of the rounded operands, at
-the edges of the padded row counts, of a tile's 16 outputs, of whole chunks of k, and of the shares that bf16 tiles are dealt in."""
+the edges of the padded row counts, of a tile's 16 outputs, of whole chunks of k, and of the shares that bf16 tiles are dealt in; and the stacks
+that do not take them."""
 import numpy as np
 import pytest
 
-from coeus_amd import _lib
+from coeus_amd import PLUGINS, LayeredConfig, _lib
 from gpu_util import Weight, dev, oracle_roundtrip
 from test_matmul_plan import plan
 
@@ -50,3 +51,22 @@ def test_rows_do_not_meet(orc):
         a[2, 7] = np.inf
         got = wt.gemm(dev(a))
         assert np.array_equal(np.delete(got, 2, 0), np.delete(clean, 2, 0)) and not np.isfinite(got[2]).any()
+
+
+def stack(mixer, attention):
+    mlp = {"kind": "dense", "ff": 512}
+    layers = [dict(mixer, mlp=mlp), dict(attention, mlp=mlp)]
+    cfg = {"architecture": "Bofirax", "vocab": 300, "width": 1024, "norm": {"eps": 1e-5}, "layers": layers}
+    return PLUGINS["layered_model"].create_builder().build(LayeredConfig(cfg, max_seq_len=32, max_batch=1), seed=5)
+
+
+@pytest.mark.parametrize("rows", [2, 5, 16])
+def test_stacks_with_a_delta_rule_keep_the_longer_prompts_sums(rows):
+    """Such a stack's rows are, bit for bit, those of a prompt of one token more than the decode step's kernels take; one without it has other sums."""
+    latent = {"type": "latent_attention", "mixer": dict(heads=4, dim=128, vdim=128, q_rank=192, kv_rank=128, scale=128 ** -0.5, mask={"size": 32})}
+    delta = {"type": "delta", "mixer": dict(heads=4, kv_heads=2, dim=128, vdim=128, conv=4)}
+    ids = np.random.default_rng(1).integers(0, 300, (1, 17), dtype=np.uint64)
+    for mixer, same in ((delta, True), (latent, False)):
+        model = stack(mixer, latent)
+        few, more = (model.session(batch=1, max_ctx=32).feed(ids[:, :n], want=(0,), want_residuals=True)[1] for n in (rows, 17))
+        assert np.array_equal(few, more[:, :rows]) == same
