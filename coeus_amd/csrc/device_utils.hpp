@@ -222,6 +222,7 @@ struct EpiArgs {
     __half *out_xq;
     uint32_t act, bp_out;
     float limit;
+    uint32_t vec4;   // prompt matmuls: four columns at a time (rows of whole fours, pointers that 16-byte pieces fit, 8-byte ones for 16-bit rows)
     uint64_t n;      // weight rows (outputs before gating)
     uint64_t n_eff;  // outputs written per activation row (n, or n/2 when gated)
     // fused q|k|v projection of a decode step: columns >= kv_inner go straight into the cache
@@ -342,6 +343,8 @@ static inline EpiArgs make_epi(const Epilogue &ep, uint64_t n) {
     e.out_lp = (uint16_t *)ep.out_lp.p;
     e.lp_ld = (uint32_t)ep.out_lp.ld;
     e.lp_bf16 = ep.out_lp.bf16 ? 1u : 0u;
+    e.vec4 = (e.n_eff & 3) == 0 && (e.lp_ld & 3) == 0 && (e.out_f32 || e.out_lp) && !e.out_xq &&
+             (((uintptr_t)e.out_f32 | (uintptr_t)e.bias | (uintptr_t)e.residual) & 15) == 0 && ((uintptr_t)e.out_lp & 7) == 0;
     return e;
 }
 

@@ -327,11 +327,6 @@ __device__ __forceinline__ void epi_store4(const EpiArgs &e, uint64_t row, uint6
         *(uint2 *)(e.out_lp + row * e.lp_ld + col) = p;
     }
 }
-// Four columns at a time: rows of whole fours, and pointers of the caller's that 16-byte (8-byte: 16-bit rows) pieces fit.
-__device__ __forceinline__ bool epi_vec4(const EpiArgs &e) {
-    return (e.n_eff & 3) == 0 && (e.lp_ld & 3) == 0 && (e.out_f32 || e.out_lp) && !e.out_xq &&
-           (((uintptr_t)e.out_f32 | (uintptr_t)e.bias | (uintptr_t)e.residual) & 15) == 0 && ((uintptr_t)e.out_lp & 7) == 0;
-}
 // Columns col .. col + 3 of activation row `row` (bias, cache append or activation, residual, store).
 // OWN: GELU and SiLU by times_sigmoid where the caller sees f32 results (no further off than the math library's forms), else on the
 // hardware's exp2 and reciprocal: at most 17 of 2^-24 off, where the rounding to f16 takes 2^12 of them (root mean square error of a gate to f16 2.0794e-4
@@ -398,7 +393,7 @@ __device__ __forceinline__ void epi_row4_gated(const EpiArgs &e, bool vec4, uint
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float *__restrict__ part, uint32_t splits,
                                                                 uint64_t m, uint64_t n, EpiArgs e) {
     const bool gated = epi_gated(e.act);
-    const bool vec4 = epi_vec4(e);
+    const bool vec4 = e.vec4;
     const uint64_t raw_per_thread = gated ? 8 : 4;
     const uint64_t groups = (n + raw_per_thread - 1) / raw_per_thread;  // per row
     const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -453,7 +448,7 @@ __global__ __launch_bounds__(256) void gemm_tail_reduce_kernel(const float *__re
                                                                uint32_t full_tiles, uint32_t tiles_m,
                                                                uint32_t tiles_n, uint64_t m, uint64_t n, EpiArgs e) {
     const bool gated = epi_gated(e.act);
-    const bool vec4 = epi_vec4(e);
+    const bool vec4 = e.vec4;
     const uint32_t rpt = gated ? 8 : 4, gpr = 256 / rpt;  // raw columns per thread, threads per tile row
     const uint32_t j = blockIdx.x >> 6, within = (blockIdx.x & 63) * 256 + threadIdx.x;
     const uint32_t r = within / gpr, g = within - r * gpr;
@@ -671,11 +666,12 @@ __global__ __launch_bounds__(512) void gemm_h256_kernel(const uint16_t *a, const
         EpiArgs pe = {};
         pe.out_f32 = tail_part + ((uint64_t)split * (total - full_tiles) + tail_idx) * (TM * TN);
         pe.n = pe.n_eff = TN;
+        pe.vec4 = 1;
         e = pe;
         em = TM; en = TN; em0 = 0; en0 = 0;
     }
     const bool gated = epi_gated(e.act);
-    const bool vec4 = epi_vec4(e);
+    const bool vec4 = e.vec4;
     auto strip_out = [&](const float16_t (&t)[2], uint32_t x) {
 #pragma unroll
         for (int y = 0; y < 2; y++)
@@ -1296,11 +1292,12 @@ __global__ __launch_bounds__(256) void gemm_h256k64_kernel(const uint16_t *a, co
         EpiArgs pe = {};
         pe.out_f32 = tail_part + ((uint64_t)split * (total - full_tiles) + tail_idx) * (TM * TN);
         pe.n = pe.n_eff = TN;
+        pe.vec4 = 1;
         e = pe;
         em = TM; en = TN; em0 = 0; en0 = 0;
     }
     const bool gated = epi_gated(e.act);
-    const bool vec4 = epi_vec4(e);
+    const bool vec4 = e.vec4;
     uint32_t bits;
     const uint32_t kind = k64_epilogue_kind(e, vec4, en0 + wn, en, bits);
     __syncthreads();  // every wave has finished reading the operand slices
@@ -1546,7 +1543,7 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(const uint16_t *a, con
                 }
     }
     __syncthreads();
-    const bool vec4 = epi_vec4(e);
+    const bool vec4 = e.vec4;
     const uint32_t live = (uint32_t)min((uint64_t)T::ROWS, m - m0);
     if (!epi_gated(e.act)) {
         constexpr uint32_t CG = T::COLS / 4, RP = 512 / CG;
@@ -1691,6 +1688,9 @@ __device__ __forceinline__ void gemm_f32_tile(const float *a, const float *w, ui
     };
 #pragma unroll
     for (int d = 0; d < D - 1; d++) request(sbeg + d, f32_sm + d * T::region);
+    // (fetched here: behind the products their trip takes 0.5 us of 11)
+    const uint32_t act = e.act, vec4 = e.vec4;
+    asm volatile("" ::"s"(act), "s"(vec4));
     uint32_t at = 0, until = PERIOD;
     for (uint32_t s = sbeg; s < send; s++) {
         // every wave's requests of slice s have landed (all but the D - 2 newest slices'), and it has read all of slice s - 1
@@ -1733,7 +1733,6 @@ __device__ __forceinline__ void gemm_f32_tile(const float *a, const float *w, ui
                 }
     }
     __syncthreads();
-    const bool vec4 = epi_vec4(e);
     const uint32_t live = (uint32_t)min((uint64_t)T::ROWS, m - m0);
     auto gather = [&](uint32_t q, uint32_t c4) {
         const float *p = sums + q * TS + c4;
@@ -1745,7 +1744,7 @@ __device__ __forceinline__ void gemm_f32_tile(const float *a, const float *w, ui
         }
         return v;
     };
-    if (!epi_gated(e.act)) {
+    if (!epi_gated(act)) {
         constexpr uint32_t CG = T::COLS / 4, RP = T::WAVES * 64 / CG;
         const uint32_t c4 = tid % CG * 4;
         if (n0 + c4 >= n) return;
